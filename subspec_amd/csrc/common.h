@@ -292,5 +292,13 @@ int dense_gate_up_silu_ex(const void* x, const void* w, const void* bias, void* 
 int dense_linear_ex(const void* x, const void* w, const void* bias, const void* residual, void* y, int dtype, int64_t M,
                     int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream, int* pending_splits = nullptr);
 
+// The same products for more than 64 rows (tile.hip).  tile_linear with *splits > 1: the fp32 partials [*splits][M][N] are in
+// the workspace (tile_workspace bytes) and y is untouched; 1: y is complete.
+bool tile_applies(int64_t M, int64_t N, int64_t K, bool silu, const void* y, const void* residual);
+size_t tile_workspace(int64_t M, int64_t N, int64_t K);
+int tile_linear(const void* x, const void* w, const void* bias, const void* residual, void* y, int dtype, int64_t M, int64_t N,
+                int64_t K, void* workspace, hipStream_t st, int* splits);
+int tile_gate_up_silu(const void* x, const void* w, const void* bias, void* act, int dtype, int64_t M, int64_t N, int64_t K,
+                      hipStream_t st);
 
 }  // namespace subspec

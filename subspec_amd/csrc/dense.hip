@@ -7,8 +7,9 @@
 // max_verify_tokens, 1 + 48 * 6 = 289 in configs/exp_offloading/subspec_sd_qwen_7b.yaml:16-19) go through the layer at
 // once.  Up to 64 rows every projection streams its whole weight matrix for a handful of rows and is bound by HBM
 // (algorithmic bytes = N*K*2 + (M*K + M*N)*2); a library GEMM tiled for large M leaves more than half of that bandwidth
-// unused at this shape.  Three kernels: 1 to 32 rows the 16 x 16 x 32 kernel below, 33 to 384 rows the 32 x 32 x 16
-// kernel behind it.
+// unused at this shape.  Three kernels: 1 to 32 rows the 16 x 16 x 32 kernel below, 33 to 64 rows the 32 x 32 x 16
+// kernel behind it, more rows the tiled kernel of tile.hip (dense_wide_kernel keeps those whose output is not 16-byte
+// aligned).
 //
 // Same skeleton as the int4 kernel next door: the activations are the MFMA A operand, a 16-row
 // weight tile the B operand (v_mfma_f32_16x16x32, k permutation "step s, lane group c, element e ->
@@ -255,16 +256,29 @@ __global__ __launch_bounds__(kDnThreads) void dense_gemm_kernel(
   }
 }
 
+// Sum of the fp32 partials of a split K in split order, plus bias and residual: four columns per thread, the requests of
+// four partials in flight (289 x 3584, 6 partials: 9.2 -> 7.5 us; 64 x 3584, 4 partials: 4.6 us either way).
 template <int DT>
 __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restrict__ partial, const uint16_t* __restrict__ bias,
                                                            const uint16_t* residual, uint16_t* y, int64_t M, int64_t N,
                                                            int splits) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= M * N) return;
-  float v = 0.f;
-  for (int s = 0; s < splits; ++s) v += partial[(int64_t)s * M * N + i];
-  if (bias) v += Elem<DT>::load(bias, i % N);
-  store_linear_out<DT>(y, i, v, residual);
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= M * N) return;                                        // N is a multiple of 16
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int s0 = 0; s0 < splits; s0 += 4) {
+    float4 q[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) q[s] = *(const float4*)(partial + (int64_t)min(s0 + s, splits - 1) * M * N + i);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s0 + s < splits) { v.x += q[s].x; v.y += q[s].y; v.z += q[s].z; v.w += q[s].w; }
+  }
+  float o[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (bias) o[e] += Elem<DT>::load(bias, i % N + e);
+    store_linear_out<DT>(y, i + e, o[e], residual);
+  }
 }
 
 // ------------------------------------------------------------------ 33 <= M <= 384
@@ -283,7 +297,7 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restri
 // registers r and r + 8 of one lane.
 // Measured on the four projections of a 7B layer, weights from HBM: M = 64 16.8 / 14.6 / 50.8 / 34.6 us (q|k|v, o,
 // gate|up with SwiGLU, down with its reduction; the 16 x 16 x 32 kernel above: 16.2 / 14.8 / 64.2 / 37.6); M = 289
-// 33 / 29 / 97 / 70 us.  At 289 rows the kernel is bound by the activation copies: a chunk is 40 KB per workgroup, LDS
+// 33 / 29 / 97 / 70 us (dense_tile_kernel: 20 / 16 / 88 / 58).  At 289 rows the kernel is bound by the activation copies: a chunk is 40 KB per workgroup, LDS
 // holds two of them beside three weight chunks, and one chunk in flight does not cover the L2 latency (M = 256 with
 // three activation slots: 79 us against 94 us with two).
 typedef float wd_v16f __attribute__((ext_vector_type(16)));
@@ -606,6 +620,7 @@ static DnPlan dn_plan(int64_t M, int64_t N, int64_t K) {
 template <int DT>
 static int run_dense_silu(const void* x, const void* w, const void* bias, void* act, int64_t M, int64_t N, int64_t K,
                           hipStream_t st) {
+  if (tile_applies(M, N, K, true, act, nullptr)) return tile_gate_up_silu(x, w, bias, act, DT, M, N, K, st);
   if (wide_applies(M, N)) {
     const WidePlan pl = wide_plan(N, K, true);
     const WideParams p{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, nullptr, (uint16_t*)act, nullptr,
@@ -642,6 +657,19 @@ template <int DT>
 static int run_dense(const void* x, const void* w, const void* bias, const void* residual, void* y, int64_t M, int64_t N,
                      int64_t K, void* workspace, hipStream_t st, int* pending_splits) {
   if (pending_splits) *pending_splits = 1;
+  auto reduce = [&](int splits) {
+    if (splits > 1 && pending_splits) *pending_splits = splits;
+    else if (splits > 1)
+      hipLaunchKernelGGL((dense_reduce_kernel<DT>), dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, st, (const float*)workspace,
+                         (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, M, N, splits);
+  };
+  if (tile_applies(M, N, K, false, y, residual)) {
+    int splits = 1;
+    tile_linear(x, w, bias, residual, y, DT, M, N, K, workspace, st, &splits);
+    reduce(splits);
+    SUBSPEC_CHECK_HIP(hipGetLastError());
+    return SUBSPEC_OK;
+  }
   if (wide_applies(M, N)) {
     const WidePlan pl = wide_plan(N, K, false);
     const WideParams p{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y,
@@ -650,10 +678,7 @@ static int run_dense(const void* x, const void* w, const void* bias, const void*
       DominantKernelTimer timer(st);
       launch_wide<DT, false>(p, pl, st);
     }
-    if (pl.splits > 1 && pending_splits) *pending_splits = pl.splits;
-    else if (pl.splits > 1)
-      hipLaunchKernelGGL((dense_reduce_kernel<DT>), dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st, (const float*)workspace,
-                         (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, M, N, pl.splits);
+    reduce(pl.splits);
     SUBSPEC_CHECK_HIP(hipGetLastError());
     return SUBSPEC_OK;
   }
@@ -678,10 +703,7 @@ static int run_dense(const void* x, const void* w, const void* bias, const void*
   }
 #undef SUBSPEC_DN_LAUNCH_MT
 #undef SUBSPEC_DN_LAUNCH
-  if (pl.splits > 1 && pending_splits) *pending_splits = pl.splits;
-  else if (pl.splits > 1)
-    hipLaunchKernelGGL((dense_reduce_kernel<DT>), dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st, partial,
-                       (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, M, N, pl.splits);
+  reduce(pl.splits);
   SUBSPEC_CHECK_HIP(hipGetLastError());
   return SUBSPEC_OK;
 }
@@ -694,7 +716,9 @@ extern "C" size_t subspec_dense_linear_workspace(int64_t M, int64_t N, int64_t K
   if (M <= 0 || N <= 0 || K <= 0) return 256;
   if (wide_applies(M, N)) {
     const WidePlan wp = wide_plan(N, K, false);
-    return (wp.splits > 1 ? align_up((size_t)wp.splits * M * N * sizeof(float), 256) : 0) + 256;
+    // above 64 rows either kernel may run (the tiled one needs a 16-byte aligned y)
+    const size_t wide = wp.splits > 1 ? (size_t)wp.splits * M * N * sizeof(float) : 0;
+    return align_up(std::max(wide, M > 64 ? tile_workspace(M, N, K) : 0), 256) + 256;
   }
   const DnPlan pl = dn_plan(M, N, K);
   return (pl.splits > 1 ? align_up((size_t)pl.splits * M * N * sizeof(float), 256) : 0) + 256;

@@ -1,0 +1,459 @@
+// Dense 16-bit linear layers for many activation rows on gfx950:
+//   y[M, N] = x[M, K] * W[N, K]^T (+ bias) (+ residual),   W row-major bf16 / fp16
+// and the gate|up projection of a SwiGLU MLP with the activation in its output stage: the target's projections over a
+// large draft tree (1 + 48 * 6 = 289 rows in configs/exp_offloading/subspec_sd_qwen_7b.yaml:16-19, through
+// ClassicSDGeneratorBase._tree_decoding, specdecodes/models/generators/classic_sd.py:75-109) and over a prefill.
+//
+// A workgroup of eight wavefronts multiplies a BM x BN tile (BM activation rows, BN weight rows) with
+// v_mfma_f32_16x16x32, the WEIGHT rows as A operand and the activation rows as B operand: both are k-contiguous 16-byte
+// pieces of row-major rows, and a lane ends up with four consecutive output columns of one row.  K advances in chunks of
+// 64: both operands' chunks are copied straight into LDS rings as whole 128-byte lines (global_load_lds_dwordx4, a
+// request moves 8 rows; 16-byte piece p of row r sits at p ^ (r / 2) % 8, conflict-free for the operand reads).
+//
+// What bounds it (measured on the gate|up projection of a 7B layer, 37888 x 3584):
+// * Issue.  A compute unit copies 64 bytes per cycle from the L2 and reads 256 bytes per cycle from LDS, both less than
+//   the products of a 256 x 256 tile take, but copies, operand reads and products of a wavefront are issued in order: with
+//   the copies in a block behind the barrier and the reads in front of the products, a chunk of that tile cost 3500
+//   cycles against 2048 of products.  Here copies and reads are issued BETWEEN the products (a read or a copy every few of
+//   them, the operands one 32-k step ahead), and the last chunk is peeled so that no branch sits between products.
+// * Distance.  Vector memory returns in order, so an activation chunk requested behind a weight chunk waits for it: with two
+//   slots of each ring every chunk waits for a request to HBM (2500 cycles and more).  Three slots of both (256 x 160 at 256
+//   rows: 83 -> 73 us), or three of weights and two of activations with the weights requested half a chunk later (256 x 256,
+//   2048 rows: 490 -> 441 us), are what LDS holds.  Chunks of 32 k in twice as many slots lose (half-line requests).
+// 2048 rows: 441 us = 1.26 PFLOP/s with the activation included (library GEMM alone: 520 us; an 8192^3 product reaches
+// 1.38 PFLOP/s on this card), 289 rows: 87 us (dense_wide_kernel: 106), 128 rows: 54 us = 5.0 TB/s of weights.
+#include "common.h"
+#include <algorithm>
+#include <type_traits>
+
+namespace subspec {
+
+typedef float tl_v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t tl_u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t tl_u2 __attribute__((ext_vector_type(2)));
+typedef __bf16 tl_v8bf __attribute__((ext_vector_type(8)));
+typedef _Float16 tl_v8h __attribute__((ext_vector_type(8)));
+
+template <int DT>
+__device__ __forceinline__ tl_v4f tl_mfma(tl_u4 a, tl_u4 b, tl_v4f c) {
+  if constexpr (DT == SUBSPEC_BF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tl_v8bf, a), __builtin_bit_cast(tl_v8bf, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(tl_v8h, a), __builtin_bit_cast(tl_v8h, b), c, 0, 0, 0);
+}
+// 16 bytes per lane from base + voffset into LDS (lds_base + 16 * lane); NT: as streaming data
+template <bool NT>
+__device__ __forceinline__ void tl_dma16(uint32_t lds_base, uint32_t voffset, const void* base) {
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
+}
+// a wavefront-uniform address in scalar registers
+__device__ __forceinline__ const uint8_t* tl_uniform(const uint8_t* p) {
+  const uint64_t a = (uint64_t)(uintptr_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return (const uint8_t*)(uintptr_t)((uint64_t)hi << 32 | lo);
+}
+template <int N> __device__ __forceinline__ void tl_wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+struct TileParams {
+  const uint16_t* x; const uint16_t* w; const uint16_t* bias; const uint16_t* residual; uint16_t* y; float* partial;
+  int M, K; int64_t N;               // N: rows of w (SILU: 2 F)
+  int tiles_m, tiles_n, splits, chunks_per_split;
+};
+
+template <int DT, int GM, int GN, int GK, int TA, int TB, int SW, int SX, bool NT, bool SILU>
+__global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParams p) {
+  constexpr int kWaves = GM * GN * GK;
+  constexpr int BM = GM * TB * 16, BN = GN * TA * 16;
+  constexpr int kWSlots = BN / 8, kXSlots = BM / 8;                        // 1 KB requests per chunk ...
+  constexpr int RW = (kWSlots + kWaves - 1) / kWaves, RX = (kXSlots + kWaves - 1) / kWaves;   // ... of one wavefront
+  constexpr uint32_t kWStride = BN * 128, kXStride = BM * 128, kXRing = SW * kWStride;
+  constexpr int kRingBytes = SW * BN * 128 + SX * BM * 128;
+  constexpr int kOutRow = TA * (SILU ? 16 : 32) + 16;                     // bytes of a parked output row
+  constexpr int kEpi = kWaves * 16 * kOutRow, kRed = GK > 1 ? GM * GN * TA * TB * 1024 : 0;
+  constexpr int kLds = kRingBytes > kEpi ? (kRingBytes > kRed ? kRingBytes : kRed) : (kEpi > kRed ? kEpi : kRed);
+  static_assert(kLds <= 160 * 1024, "LDS");
+  static_assert(GK <= 2 && SX >= 2 && (SW == SX || (SW == SX + 1 && GK == 1)) , "k groups, ring depths");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 15, c = lane >> 4;
+  const int M = p.M, K = p.K;
+
+  // XCD-aware order: consecutive ids go to different XCDs; each XCD takes a contiguous run of the tile list, rows fastest
+  const int total = p.tiles_m * p.tiles_n * p.splits;
+  const int id = blockIdx.x, xcd = id & 7, per = total >> 3, rem = total & 7;
+  int lin = xcd * per + min(xcd, rem) + (id >> 3);
+  const int tm = lin % p.tiles_m; lin /= p.tiles_m;
+  const int tn = lin % p.tiles_n, ks = lin / p.tiles_n;
+  const int m0 = tm * BM;
+  const int64_t n0 = (int64_t)tn * (SILU ? BN / 2 : BN);                  // SILU: first output column
+  const int64_t F = p.N >> 1;
+  const int n_chunks = K >> 6;
+  const int st0 = ks * p.chunks_per_split, nst = min(n_chunks, st0 + p.chunks_per_split) - st0;
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  // ---- copies: request = 8 rows x 128 bytes; lane -> row lane / 8, position lane % 8 holding piece position ^ (row / 2) % 8
+  uint32_t woff[RW], wdst[RW], xoff[RX], xdst[RX];
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const int slot = (i * kWaves + wave) % kWSlots;                       // surplus requests repeat earlier ones
+    const int r = slot * 8 + (lane >> 3);
+    const int pc = (lane & 7) ^ ((r >> 1) & 7);
+    int64_t row;
+    if constexpr (SILU) {
+      const int q = r & 15, f_in = (r >> 4) * 8 + (q >> 2) * 2 + (q & 1);
+      row = min(n0 + f_in, F - 1) - n0 + ((q >> 1) & 1) * F;
+    } else {
+      row = min(n0 + r, p.N - 1) - n0;
+    }
+    woff[i] = (uint32_t)(row * K * 2 + pc * 16);
+    wdst[i] = lds0 + slot * 1024;
+  }
+#pragma unroll
+  for (int i = 0; i < RX; ++i) {
+    const int slot = (i * kWaves + wave) % kXSlots;
+    const int r = slot * 8 + (lane >> 3);
+    const int pc = (lane & 7) ^ ((r >> 1) & 7);
+    xoff[i] = (uint32_t)((min(m0 + r, M - 1) - m0) * K * 2 + pc * 16);
+    xdst[i] = lds0 + kXRing + slot * 1024;
+  }
+  const uint8_t* const wbase = (const uint8_t*)(p.w + n0 * K) + (int64_t)st0 * 128;
+  const uint8_t* const xbase = (const uint8_t*)(p.x + (int64_t)m0 * K) + (int64_t)st0 * 128;
+  // source of chunk s (relative to st0; beyond the last one: the last one again, into a slot nobody reads any more)
+  auto chunk_src = [&](const uint8_t* base, int s) { return tl_uniform(base + (int64_t)min(s, nst - 1) * 128); };
+  auto copy_w = [&](int i, const uint8_t* src, uint32_t slot_off) {
+    tl_dma16<NT>(__builtin_amdgcn_readfirstlane(wdst[i] + slot_off), woff[i], src);
+  };
+  auto copy_x = [&](int i, const uint8_t* src, uint32_t slot_off) {
+    tl_dma16<false>(__builtin_amdgcn_readfirstlane(xdst[i] + slot_off), xoff[i], src);
+  };
+  auto fill_w = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < RW; ++i) copy_w(i, chunk_src(wbase, s), s * kWStride);
+  };
+  auto fill_x = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < RX; ++i) copy_x(i, chunk_src(xbase, s), s * kXStride);
+  };
+  // Order of a wavefront's requests, here and in the loop (they return in order): two slots each: X(c), W(c), ...;
+  // three and more: the weights of a chunk half a chunk later than its activations; one weight slot more than
+  // activation slots: W(c + 1) behind X(c).
+  constexpr bool kWLate = GK == 1 && SW > 2;                               // weights are requested in step 0 of the next chunk
+  if constexpr (SW > SX) {
+#pragma unroll
+    for (int s = 0; s < SX; ++s) { fill_w(s); fill_x(s); }
+  } else {
+#pragma unroll
+    for (int s = 0; s < SX; ++s) {
+      fill_x(s);
+      if (!kWLate || s < SX - 1) fill_w(s);
+    }
+  }
+  constexpr int kFirstWait = SW > SX ? (SX - 1) * (RX + RW) : kWLate ? (SX - 2) * (RX + RW) + RX : (SX - 1) * (RX + RW);
+  constexpr int kWait = SW > SX ? (SX - 1) * RW + (SX - 2) * RX : (SX - 2) * (RX + RW);
+  static_assert(kFirstWait < 64, "request counter");
+
+  const int kg = wave / (GM * GN), wmn = wave % (GM * GN), wm = wmn % GM, wn = wmn / GM;
+  tl_v4f acc[TA][TB];
+#pragma unroll
+  for (int i = 0; i < TA; ++i)
+#pragma unroll
+    for (int k = 0; k < TB; ++k) acc[i][k] = tl_v4f{0.f, 0.f, 0.f, 0.f};
+  uint32_t opoff[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+    opoff[s] = (uint32_t)ln * 128 + ((uint32_t)(4 * (GK == 2 ? kg : s) + c) ^ (uint32_t)((ln >> 1) & 7)) * 16;
+  const uint32_t wop = wn * TA * 2048, xop = kXRing + wm * TB * 2048;
+
+  tl_u4 a0[TA], b0[TB], a1[TA], b1[TB];
+  int wslot = 0, xslot = 0;                                               // slots of the chunk being multiplied
+  // One 32-k step of this wavefront: TB groups of TA products; between the groups, so that they are issued while the
+  // matrix core works: the operands of the next step (from wsrc / xsrc) and this wavefront's copies into freed slots.
+  auto step = [&](tl_u4 (&A)[TA], tl_u4 (&B)[TB], tl_u4 (&An)[TA], tl_u4 (&Bn)[TB], auto read_c, auto cx_c, auto cw_c,
+                  const uint8_t* wsrc, const uint8_t* xsrc, const uint8_t* xg, uint32_t xo, const uint8_t* wg, uint32_t wo)
+                  __attribute__((always_inline)) {
+    constexpr bool kRead = decltype(read_c)::value, kCx = decltype(cx_c)::value, kCw = decltype(cw_c)::value;
+    constexpr int kReads = TA + TB, kReadGroups = TB >= 4 ? TB * 3 / 4 : TB, D = (kCx ? RX : 0) + (kCw ? RW : 0);
+#pragma unroll
+    for (int k = 0; k < TB; ++k) {
+      if constexpr (D > 0) {
+#pragma unroll
+        for (int d = k * D / TB; d < (k + 1) * D / TB; ++d) {
+          if (kCx && d < RX) copy_x(d, xg, xo);
+          else copy_w(d - (kCx ? RX : 0), wg, wo);
+        }
+      }
+      if constexpr (kRead) {
+        if (k < kReadGroups) {
+#pragma unroll
+          for (int r = k * kReads / kReadGroups; r < (k + 1) * kReads / kReadGroups; ++r) {
+            if (r < TA) An[r] = *(const tl_u4*)(wsrc + r * 2048);
+            else Bn[r - TA] = *(const tl_u4*)(xsrc + (r - TA) * 2048);
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < TA; ++i) acc[i][k] = tl_mfma<DT>(A[i], B[k], acc[i][k]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto sync = [&](auto wait_c) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    tl_wait_vmcnt<decltype(wait_c)::value>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  const uint8_t* const wop_p = lds + wop;
+  const uint8_t* const xop_p = lds + xop;
+  sync(std::integral_constant<int, kFirstWait>{});
+#pragma unroll
+  for (int i = 0; i < TA; ++i) a0[i] = *(const tl_u4*)(wop_p + opoff[0] + i * 2048);
+#pragma unroll
+  for (int k = 0; k < TB; ++k) b0[k] = *(const tl_u4*)(xop_p + opoff[0] + k * 2048);
+  // the last chunk is peeled off: a branch inside the loop would make the accumulators cross basic blocks
+  auto advance = [&]() __attribute__((always_inline)) {
+    wslot = wslot + 1 == SW ? 0 : wslot + 1;
+    xslot = xslot + 1 == SX ? 0 : xslot + 1;
+  };
+  auto last_step = [&](tl_u4 (&A)[TA], tl_u4 (&B)[TB]) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    step(A, B, A, B, no, no, no, nullptr, nullptr, nullptr, 0u, nullptr, 0u);
+  };
+  if constexpr (GK == 1) {
+    for (int it = 0; it < nst - 1; ++it) {
+      const uint32_t wcur = wslot * kWStride, xcur = xslot * kXStride;
+      const int wprev = wslot == 0 ? SW - 1 : wslot - 1;
+      step(a0, b0, a1, b1, yes, no, std::integral_constant<bool, kWLate>{}, wop_p + wcur + opoff[1], xop_p + xcur + opoff[1],
+           nullptr, 0u, kWLate ? chunk_src(wbase, it - 1 + SW) : nullptr, wprev * kWStride);
+      advance();
+      sync(std::integral_constant<int, kWait>{});
+      step(a1, b1, a0, b0, yes, yes, std::integral_constant<bool, !kWLate>{}, wop_p + wslot * kWStride + opoff[0],
+           xop_p + xslot * kXStride + opoff[0], chunk_src(xbase, it + SX), xcur, kWLate ? nullptr : chunk_src(wbase, it + SW), wcur);
+    }
+    step(a0, b0, a1, b1, yes, no, no, wop_p + wslot * kWStride + opoff[1], xop_p + xslot * kXStride + opoff[1], nullptr, 0u, nullptr, 0u);
+    last_step(a1, b1);
+  } else {
+    // two wavefront groups share a chunk: group g multiplies its 16-byte pieces 4 g .. 4 g + 3 (32 of the 64 k)
+    auto half = [&](tl_u4 (&A)[TA], tl_u4 (&B)[TB], tl_u4 (&An)[TA], tl_u4 (&Bn)[TB], int it) __attribute__((always_inline)) {
+      const uint32_t wcur = wslot * kWStride, xcur = xslot * kXStride;
+      advance();
+      sync(std::integral_constant<int, kWait>{});
+      step(A, B, An, Bn, yes, yes, yes, wop_p + wslot * kWStride + opoff[0], xop_p + xslot * kXStride + opoff[0],
+           chunk_src(xbase, it + SX), xcur, chunk_src(wbase, it + SW), wcur);
+    };
+    int it = 0;
+    for (; it + 2 < nst; it += 2) {
+      half(a0, b0, a1, b1, it);
+      half(a1, b1, a0, b0, it + 1);
+    }
+    if (it + 1 < nst) {
+      half(a0, b0, a1, b1, it);
+      last_step(a1, b1);
+    } else {
+      last_step(a0, b0);
+    }
+  }
+  // every copy into the rings has landed and every wavefront is done reading them: the space is reused below
+  tl_wait_vmcnt<0>();
+  __syncthreads();
+
+  if constexpr (GK == 2) {
+    tl_v4f* red = (tl_v4f*)lds + (wmn * TA * TB) * 64 + lane;
+    if (kg == 1) {
+#pragma unroll
+      for (int i = 0; i < TA; ++i)
+#pragma unroll
+        for (int k = 0; k < TB; ++k) red[(i * TB + k) * 64] = acc[i][k];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+      for (int k = 0; k < TB; ++k) {
+        const tl_v4f o = red[(i * TB + k) * 64];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][k][r] += o[r];
+      }
+  }
+
+  // ---- output.  acc[i][k][r]: row m0 + (wm TB + k) 16 + ln, column (wn TA + i) 16 + 4 c + r of the tile
+  if (!SILU && p.splits > 1) {
+#pragma unroll
+    for (int k = 0; k < TB; ++k) {
+      const int m = m0 + (wm * TB + k) * 16 + ln;
+      if (m >= M) continue;
+      float* row = p.partial + ((int64_t)ks * M + m) * p.N;
+#pragma unroll
+      for (int i = 0; i < TA; ++i) {
+        const int64_t n = n0 + (wn * TA + i) * 16 + 4 * c;
+        if (n < p.N) *(float4*)(row + n) = make_float4(acc[i][k][0], acc[i][k][1], acc[i][k][2], acc[i][k][3]);
+      }
+    }
+    return;
+  }
+  // 16 rows at a time through a wavefront-private LDS block, so that rows leave as 16-byte pieces of whole segments
+  constexpr int kCols = SILU ? TA * 8 : TA * 16;                           // output columns of this wavefront
+  constexpr int kPieces = kCols / 8;
+  // (two k groups: the block lies in the part of the exchange that only this wavefront reads)
+  static_assert(GK == 1 || TA * TB * 1024 >= 16 * kOutRow, "output block inside the exchange");
+  uint8_t* const mine = lds + (GK == 2 ? wmn * TA * TB * 1024 : wmn * 16 * kOutRow);
+  const int64_t ncol0 = n0 + (int64_t)wn * kCols, ncols = SILU ? F : p.N;
+#pragma unroll
+  for (int k = 0; k < TB; ++k) {
+#pragma unroll
+    for (int i = 0; i < TA; ++i) {
+      if constexpr (SILU) {
+        const int64_t f = n0 + (wn * TA + i) * 8 + 2 * c;
+        float o[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const bool in = p.bias && f + e < F;
+          const float bg = in ? Elem<DT>::load(p.bias, f + e) : 0.f, bu = in ? Elem<DT>::load(p.bias, F + f + e) : 0.f;
+          const float gate = Elem<DT>::round(acc[i][k][e] + bg), up = Elem<DT>::round(acc[i][k][2 + e] + bu);
+          o[e] = Elem<DT>::round(gate / (1.f + __expf(-gate))) * up;
+        }
+        *(uint32_t*)(mine + ln * kOutRow + i * 16 + c * 4) = pack2<DT>(o[0], o[1]);
+      } else {
+        const int64_t n = n0 + (wn * TA + i) * 16 + 4 * c;
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = acc[i][k][r] + (p.bias && n + r < p.N ? Elem<DT>::load(p.bias, n + r) : 0.f);
+        *(tl_u2*)(mine + ln * kOutRow + i * 32 + c * 8) = tl_u2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < (16 * kPieces + 63) / 64; ++q) {
+      const int pi = q * 64 + lane, row = pi / kPieces, piece = pi % kPieces;
+      const int m = m0 + (wm * TB + k) * 16 + row;
+      const int64_t n = ncol0 + piece * 8;
+      if (row < 16 && m < M && n < ncols) {
+        dec_u4 v = *(const dec_u4*)(mine + row * kOutRow + piece * 16);
+        if (p.residual) {
+          float a[8], b[8];
+          unpack8<DT>(v, a);
+          unpack8<DT>(*(const dec_u4*)(p.residual + (int64_t)m * ncols + n), b);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) a[j] += b[j];
+          v = pack8<DT>(a);
+        }
+        *(dec_u4*)(p.y + (int64_t)m * ncols + n) = v;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// ------------------------------------------------------------------ launch shapes
+// Tile shapes and what a chunk of one takes when the chip is full of them (us, measured on the projections of a 7B layer:
+// 4608 / 3584 / 37888 x 3584 and 3584 x 18944 at 65 to 2048 rows).  The shapes of 160 columns cut 37888 rows into 237
+// workgroups, one per compute unit; those that serve up to 192 rows request their weights as streaming data (every
+// workgroup holds all rows, so a weight is read once: 128 rows 58.5 -> 53.8 us).
+#define SUBSPEC_TILE_SHAPES(X)                      \
+  X(0, 2, 4, 1, 4, 8, 3, 2, false, 1.55f)           \
+  X(1, 4, 2, 1, 5, 5, 3, 2, false, 1.48f)           \
+  X(2, 4, 2, 1, 5, 4, 3, 3, false, 1.10f)           \
+  X(3, 4, 2, 1, 5, 3, 4, 3, true, 0.95f)            \
+  X(4, 4, 2, 1, 5, 2, 4, 4, true, 0.83f)            \
+  X(5, 4, 2, 1, 4, 4, 3, 3, false, 0.90f)           \
+  X(6, 2, 4, 1, 4, 4, 3, 3, false, 0.93f)           \
+  X(7, 4, 2, 1, 4, 2, 4, 4, false, 0.65f)           \
+  X(8, 2, 2, 2, 2, 4, 6, 6, false, 0.40f)
+struct TileShape { int bm, bn; float chunk_us; };
+static constexpr TileShape kShapes[] = {
+#define X(ID, GM, GN, GK, TA, TB, SW, SX, NT, US) {GM * TB * 16, GN * TA * 16, US},
+    SUBSPEC_TILE_SHAPES(X)
+#undef X
+};
+constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
+constexpr int kTileMaxSplits = 8;
+
+struct TilePlan { int shape, tiles_m, tiles_n, splits, chunks_per_split; };
+// Cheapest (shape, number of K ranges) under: 5.5 us for launch, first chunks and output; rounds of 256 workgroups, one
+// per compute unit, of chunk_us per chunk; never less than the weights take from HBM at 5.5 TB/s; fp32 partials written
+// and read back at 4.5 TB/s.  Within 7 % of the best measured shape on the matrices above.
+static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool silu) {
+  TilePlan best{};
+  float best_us = 1e30f;
+  const int chunks = (int)(K / 64);
+  const float hbm_us = 8.f + (float)N * (float)K * 2.f / 5.5e6f;
+  for (int i = 0; i < kNumShapes; ++i) {
+    const int64_t tm = (M + kShapes[i].bm - 1) / kShapes[i].bm, cols = silu ? N / 2 : N, bn = silu ? kShapes[i].bn / 2 : kShapes[i].bn;
+    const int64_t tn = (cols + bn - 1) / bn;
+    for (int s = 1; s <= (silu ? 1 : kTileMaxSplits); ++s) {
+      const int cps = (chunks + s - 1) / s;
+      if (s > 1 && (cps < 8 || (chunks + cps - 1) / cps != s)) continue;
+      const int64_t rounds = (tm * tn * s + 255) / 256;
+      float us = std::max(5.5f + (float)rounds * (float)cps * kShapes[i].chunk_us, hbm_us);
+      if (s > 1) us += 1.f + 2.f * (float)s * (float)M * (float)N * 4.f / 4.5e6f;
+      if (us < best_us) {
+        best_us = us;
+        best = TilePlan{i, (int)tm, (int)tn, s, cps};
+      }
+    }
+  }
+  return best;
+}
+
+template <int DT, bool SILU>
+static void launch_tile(TileParams p, const TilePlan& pl, hipStream_t st) {
+  p.tiles_m = pl.tiles_m;
+  p.tiles_n = pl.tiles_n;
+  p.splits = pl.splits;
+  p.chunks_per_split = pl.chunks_per_split;
+  const dim3 grid((unsigned)((int64_t)pl.tiles_m * pl.tiles_n * pl.splits));
+  switch (pl.shape) {
+#define X(ID, GM, GN, GK, TA, TB, SW, SX, NT, US)                                                                       \
+  case ID:                                                                                                              \
+    hipLaunchKernelGGL((dense_tile_kernel<DT, GM, GN, GK, TA, TB, SW, SX, NT, SILU>), grid, dim3(512), 0, st, p);       \
+    break;
+    SUBSPEC_TILE_SHAPES(X)
+#undef X
+  }
+}
+
+// More than 64 rows: below, dense_wide_kernel with its four weight slots is level or ahead (64 rows: q|k|v and o together
+// 23.3 against 22.8 us here, gate|up 50.3 against 53.4, down 33 against 36 us with their reductions).  16-byte stores of
+// whole output pieces; 32-bit offsets inside a tile (a SwiGLU tile spans gate and up rows).
+bool tile_applies(int64_t M, int64_t N, int64_t K, bool silu, const void* y, const void* residual) {
+  return M > 64 && N % (silu ? 32 : 16) == 0 && K % 64 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)residual % 16 == 0 &&
+         (silu ? N / 2 + 512 : 512) * K * 2 < ((int64_t)1 << 31) && M < (1 << 24) && N < ((int64_t)1 << 31);
+}
+
+size_t tile_workspace(int64_t M, int64_t N, int64_t K) {
+  const TilePlan pl = tile_plan(M, N, K, false);
+  return pl.splits > 1 ? (size_t)pl.splits * M * N * sizeof(float) : 0;
+}
+
+int tile_linear(const void* x, const void* w, const void* bias, const void* residual, void* y, int dtype, int64_t M, int64_t N,
+                int64_t K, void* workspace, hipStream_t st, int* splits) {
+  const TilePlan pl = tile_plan(M, N, K, false);
+  const TileParams p{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y,
+                     (float*)workspace, (int)M, (int)K, N, 0, 0, 0, 0};
+  *splits = pl.splits;
+  DominantKernelTimer timer(st);
+  if (dtype == SUBSPEC_BF16) launch_tile<SUBSPEC_BF16, false>(p, pl, st);
+  else launch_tile<SUBSPEC_F16, false>(p, pl, st);
+  return SUBSPEC_OK;
+}
+
+int tile_gate_up_silu(const void* x, const void* w, const void* bias, void* act, int dtype, int64_t M, int64_t N, int64_t K,
+                      hipStream_t st) {
+  const TilePlan pl = tile_plan(M, N, K, true);
+  const TileParams p{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, nullptr, (uint16_t*)act, nullptr,
+                     (int)M, (int)K, N, 0, 0, 0, 0};
+  DominantKernelTimer timer(st);
+  if (dtype == SUBSPEC_BF16) launch_tile<SUBSPEC_BF16, true>(p, pl, st);
+  else launch_tile<SUBSPEC_F16, true>(p, pl, st);
+  SUBSPEC_CHECK_HIP(hipGetLastError());
+  return SUBSPEC_OK;
+}
+
+}  // namespace subspec

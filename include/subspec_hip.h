@@ -463,6 +463,17 @@ int subspec_dense_decoder_layer(const subspec_decoder_layer_dims* dims, const su
                                 void* x, const int32_t* positions, const int32_t* cache_rows, const uint64_t* anc_bits,
                                 void* k_cache, void* v_cache, void* workspace, size_t workspace_bytes, void* stream);
 
+/* One decoder layer over a chunk of a prompt: the sequence of subspec_dense_decoder_layer with causal attention -- row i is
+ * the token at cache row prefix_len + i (cache_rows[i] must say so) and sees every row up to its own.  1 <= n_rows <= 65536;
+ * dims->n_tree_slots is ignored, dims->prefix_len_dev must be NULL.
+ *
+ * Replaces  the target's forward over a chunk of the prompt (specdecodes/models/generators/base.py:204-263). */
+size_t subspec_prefill_layer_workspace(const subspec_decoder_layer_dims* dims);
+
+int subspec_prefill_layer(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights, void* x,
+                          const int32_t* positions, const int32_t* cache_rows, void* k_cache, void* v_cache, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * RMSNorm of [rows, hidden] activations in one launch: y = weight * round(x * rsqrt(mean(x^2) + eps)), the sum
  * in fp32, the normalized value rounded to the activation dtype before the gain is applied (HuggingFace's

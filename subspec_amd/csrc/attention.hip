@@ -921,7 +921,14 @@ __device__ __forceinline__ void pp_softmax_phase(int64_t kb, const PPRow& rw, v1
   rf.l += (lsum[0][0] + lsum[0][1]) + (lsum[1][0] + lsum[1][1]);
 }
 
-template <int DT, int WPH>
+// CAUSAL (a prefill: query row i of the call sits at cache row prefix + i): window w sees prefix + 64 w rows in full and the
+// rows of its own window up to the query's, so its row masks are (2 << row) - 1 and come from no memory.  Windows have
+// different lengths: the longest start first, chunks behind a window's last key end at once, and the partial results of a
+// window cut into several chunks stay fp32 (unnormalised O and sum).
+// 28 : 4 heads, bf16: 2048 rows of a prompt 72 us + 11 us merge, the last 256 of 2048 20 + 9 us (a library's attention with the
+// mask it needs and K / V repeated for the heads: 275 and 190 us).  Bound by the softmax and matrix phases of the blocks, like
+// the tree form; what is left is the uneven length of the windows.
+template <int DT, int WPH, bool CAUSAL = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void tree_attention_pp_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const uint64_t* __restrict__ anc, AttnParams ap, uint16_t* __restrict__ out, float* __restrict__ part_o,
@@ -939,7 +946,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if ((int64_t)unit >= ap.units) return;
   const int chunk = (int)(unit % (uint32_t)ap.chunks);
   const uint32_t bkv = unit / (uint32_t)ap.chunks;
-  const int kvh = (int)(bkv % (uint32_t)ap.hkv), vb = (int)(bkv / (uint32_t)ap.hkv);
+  const int kvh = (int)(bkv % (uint32_t)ap.hkv);
+  const int vb = CAUSAL ? ap.windows - 1 - (int)(bkv / (uint32_t)ap.hkv) : (int)(bkv / (uint32_t)ap.hkv);
   const AttnWindow aw = attn_window(ap, vb);          // (sequence, window of 64 query rows) of this unit
   const int b = aw.b;
   const int group = (int)((uint32_t)ap.hq / (uint32_t)ap.hkv);
@@ -953,8 +961,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int qh = kvh * group + (head_ok ? head_in_group : 0);
   const int bh = b * (int)ap.hq + qh, vbh = vb * (int)ap.hq + qh;   // q / out rows; partial slots
   const int n = (int)ap.n_rows;
-  const int64_t prefix = ap.prefix_dev ? min(max(*ap.prefix_dev, (int64_t)0), ap.prefix) : ap.prefix;
-  const int64_t kv_len = prefix + ap.n_slots;
+  const int64_t prefix = CAUSAL ? ap.prefix + aw.row0
+                                : ap.prefix_dev ? min(max(*ap.prefix_dev, (int64_t)0), ap.prefix) : ap.prefix;
+  const int64_t kv_len = prefix + (CAUSAL ? (int64_t)aw.win_rows : ap.n_slots);
   const int tile = wave % WPH;
   const int row = tile * 32 + lr;
   const bool live = head_ok && tile * 32 < aw.win_rows;     // (wave-uniform) this wavefront has rows to work on
@@ -964,6 +973,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const int64_t key0 = (int64_t)chunk * ap.chunk_keys;
+  if (CAUSAL && key0 >= kv_len) return;                     // (the whole workgroup, before its first barrier)
   const int64_t key1 = min(key0 + ap.chunk_keys, kv_len);
   const int nkeys = (int)(key1 - key0);
   const int nb = (nkeys + kKeyBlock - 1) / kKeyBlock;
@@ -1005,7 +1015,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int i = tid + u * 512, r = i / kPPMaskWords, w = i % kPPMaskWords;
-    mword[u] = (i < kAttnRows * kPPMaskWords && r < aw.win_rows && w < ap.mask_words)
+    if constexpr (CAUSAL) mword[u] = (w == 0 && r < aw.win_rows) ? (2ull << r) - 1ull : 0ull;
+    else mword[u] = (i < kAttnRows * kPPMaskWords && r < aw.win_rows && w < ap.mask_words)
                    ? anc[((int64_t)b * ap.anc_batch_stride + aw.row0 + r) * ap.mask_words + w] : 0ull;
   }
 
@@ -1085,7 +1096,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const float l = rf.l + __shfl_xor(rf.l, 32, kWave);
   if (!live) return;
-  if (ap.chunks == 1) {
+  if (CAUSAL ? kv_len <= ap.chunk_keys : ap.chunks == 1) {
     if (!row_ok) return;
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     uint16_t* op = out + (((int64_t)b * n + aw.row0 + row) * ap.hq + qh) * kAttnD + g * 4;
@@ -1095,6 +1106,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int q4 = 0; q4 < 4; ++q4)
         *(uint2*)(op + dt * 32 + q4 * 8) = make_uint2(pack2<DT>(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
                                                       pack2<DT>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv));
+  } else if constexpr (CAUSAL) {
+    float* po = part_o + (((int64_t)vbh * ap.chunks + chunk) * 2 + tile) * kTileElems + lane * 4;
+#pragma unroll
+    for (int dt = 0; dt < kAttnD / 32; ++dt)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *(float4*)(po + (dt * 4 + q4) * 256) =
+            make_float4(oacc[dt][4 * q4], oacc[dt][4 * q4 + 1], oacc[dt][4 * q4 + 2], oacc[dt][4 * q4 + 3]);
+    if (g == 0) {
+      const int64_t pslot = ((int64_t)vbh * ap.chunks + chunk) * kAttnRows + row;
+      *(v2f_t*)(part_ml + pslot * 2) = v2f_t{rf.have ? rf.ref * ap.scale_log2 : -INFINITY, l};
+    }
   } else {
     // the chunk's own softmax-weighted average of V, in the 16-bit dtype (a convex combination of such averages is what the
     // merge forms, so their rounding error does not grow); every store instruction writes 512 consecutive bytes
@@ -1184,6 +1207,39 @@ __global__ __launch_bounds__(256) void tree_attention32_merge_kernel(
   const int d0 = (idx16 >> 2) * 32 + (idx16 & 3) * 8 + g * 4;
   *(uint2*)(out + (((int64_t)b * ap.n_rows + aw.row0 + row) * ap.hq + qh) * kAttnD + d0) =
       make_uint2(pack2<DT>(num[0] * inv, num[1] * inv), pack2<DT>(num[2] * inv, num[3] * inv));
+}
+
+// Merge of a causal call's chunks (fp32): blocks and threads as above; windows of one chunk are complete already.
+template <int DT>
+__global__ __launch_bounds__(256) void causal_attention_merge_kernel(const float* __restrict__ part_o,
+                                                                     const float* __restrict__ part_ml, AttnParams ap,
+                                                                     uint16_t* __restrict__ out) {
+  const int tile = blockIdx.x & 1, vbh = blockIdx.x >> 1;
+  const int lane = threadIdx.x & 63, idx16 = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int row = tile * 32 + (lane & 31), g = lane >> 5;
+  const int vb = vbh / (int)ap.hq, qh = vbh % (int)ap.hq;
+  const AttnWindow aw = attn_window(ap, vb);
+  const int64_t kv_len = ap.prefix + aw.row0 + aw.win_rows;
+  const int chunks = (int)((kv_len + ap.chunk_keys - 1) / ap.chunk_keys);
+  if (chunks == 1 || row >= aw.win_rows) return;
+  const float* ml = part_ml + ((int64_t)vbh * ap.chunks * kAttnRows + row) * 2;
+  const float* po = part_o + ((int64_t)vbh * ap.chunks * 2 + tile) * kTileElems + (idx16 * 64 + lane) * 4;
+  float m = -INFINITY, den = 0.f;
+  float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (int c = 0; c < chunks; ++c) m = fmaxf(m, ml[c * 2 * kAttnRows]);
+#pragma unroll 4
+  for (int c = 0; c < chunks; ++c) {
+    const v2f_t v = *(const v2f_t*)(ml + c * 2 * kAttnRows);
+    const float4 o = *(const float4*)(po + (int64_t)c * 2 * kTileElems);
+    const float w = v[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(v[0] - m);
+    num.x = fmaf(w, o.x, num.x); num.y = fmaf(w, o.y, num.y); num.z = fmaf(w, o.z, num.z); num.w = fmaf(w, o.w, num.w);
+    den = fmaf(w, v[1], den);
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  const int d0 = (idx16 >> 2) * 32 + (idx16 & 3) * 8 + g * 4;
+  *(uint2*)(out + ((int64_t)(aw.row0 + row) * ap.hq + qh) * kAttnD + d0) =
+      make_uint2(pack2<DT>(num.x * inv, num.y * inv), pack2<DT>(num.z * inv, num.w * inv));
 }
 
 // Launch shape of one window of query rows.
@@ -1416,3 +1472,76 @@ int subspec::tree_attention_ex(const void* q, const void* k_cache, const void* v
   return tree_attention_impl("tree_attention", q, k_cache, v_cache, out, dtype, 1, n_q_heads, n_kv_heads, n_rows, n_tree_slots, kAttnD,
                              kv_seq_stride, prefix_len, anc_bits, 0, scale, nullptr, prefix_dev, workspace, workspace_bytes, stream);
 }
+
+// ------------------------------------------------------------------------------------------- causal attention (prefill)
+namespace subspec {
+// Windows of 64 rows, each cut into chunks of equal length: as many key blocks per workgroup as an even share of all blocks
+// over 256 compute units (a workgroup fills one), at least two.  A long prompt ends up with one chunk per window.
+struct CausalPlan { int windows, wph, pairs, chunks; int64_t chunk_keys; };
+static CausalPlan causal_plan(int64_t hq, int64_t hkv, int64_t n_rows, int64_t prefix) {
+  CausalPlan pl;
+  const int64_t group = hq / hkv, last = (prefix + n_rows + kKeyBlock - 1) / kKeyBlock;
+  pl.windows = (int)((n_rows + kAttnRows - 1) / kAttnRows);
+  pl.wph = n_rows <= 32 ? 1 : 2;
+  pl.pairs = (int)((group + 8 / pl.wph - 1) / (8 / pl.wph));
+  int64_t blocks = 0;
+  for (int w = 0; w < pl.windows; ++w)
+    blocks += (prefix + std::min<int64_t>(n_rows, (int64_t)(w + 1) * kAttnRows) + kKeyBlock - 1) / kKeyBlock;
+  blocks *= hkv * pl.pairs;
+  int64_t share = std::max<int64_t>(2, (blocks + 255) / 256);
+  share = std::max<int64_t>(share, (last + 63) / 64);                     // at most 64 chunks
+  pl.chunks = (int)((last + share - 1) / share);
+  pl.chunk_keys = (last + pl.chunks - 1) / pl.chunks * kKeyBlock;
+  pl.chunks = (int)((last * kKeyBlock + pl.chunk_keys - 1) / pl.chunk_keys);
+  return pl;
+}
+
+size_t causal_attention_workspace(int64_t hq, int64_t hkv, int64_t n_rows, int64_t prefix) {
+  const CausalPlan pl = causal_plan(hq, hkv, n_rows, prefix);
+  size_t o_bytes;
+  return pl.chunks == 1 ? 256 : attn_partial_bytes(pl.windows, hq, pl.chunks, &o_bytes);
+}
+
+template <int DT>
+static void causal_launch(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const AttnParams& ap, const CausalPlan& pl,
+                          uint16_t* out, float* part_o, float* part_ml, hipStream_t st) {
+  const dim3 grid((unsigned)((ap.units + kXcds - 1) / kXcds * kXcds * ap.pairs_per_kv));
+  {
+    DominantKernelTimer timer(st);
+    if (pl.wph == 1)
+      hipLaunchKernelGGL((tree_attention_pp_kernel<DT, 1, true>), grid, dim3(512), 0, st, q, kc, vc, (const uint64_t*)nullptr, ap,
+                         out, part_o, part_ml);
+    else
+      hipLaunchKernelGGL((tree_attention_pp_kernel<DT, 2, true>), grid, dim3(512), 0, st, q, kc, vc, (const uint64_t*)nullptr, ap,
+                         out, part_o, part_ml);
+  }
+  if (pl.chunks > 1)
+    hipLaunchKernelGGL((causal_attention_merge_kernel<DT>), dim3((unsigned)(pl.windows * ap.hq * 2), 4), dim3(256), 0, st, part_o,
+                       part_ml, ap, out);
+}
+
+// q [Hq, n_rows, 128] of the rows at cache rows prefix .. prefix + n_rows - 1; k / v [Hkv, seq_stride, 128]; out [n_rows, Hq, 128].
+// Shapes, alignment and workspace are the caller's (subspec_prefill_layer) to check.
+int causal_attention(const void* q, const void* k, const void* v, void* out, int dtype, int64_t hq, int64_t hkv, int64_t n_rows,
+                     int64_t seq_stride, int64_t prefix, float scale, void* workspace, hipStream_t st) {
+  const CausalPlan pl = causal_plan(hq, hkv, n_rows, prefix);
+  AttnParams ap{};
+  ap.batch = 1; ap.hq = hq; ap.hkv = hkv; ap.n_rows = n_rows; ap.seq_stride = seq_stride; ap.prefix = prefix;
+  ap.win_rows = (int)std::min<int64_t>(n_rows, kAttnRows);
+  ap.windows = pl.windows;
+  ap.chunks = pl.chunks;
+  ap.chunk_keys = pl.chunk_keys;
+  ap.pairs_per_kv = pl.pairs;
+  ap.units = (int64_t)pl.windows * hkv * pl.chunks;
+  ap.scale_log2 = scale * kLog2e;
+  size_t o_bytes = 0;
+  attn_partial_bytes(pl.windows, hq, pl.chunks, &o_bytes);
+  float *part_o = (float*)workspace, *part_ml = (float*)((char*)workspace + o_bytes);
+  if (dtype == SUBSPEC_BF16)
+    causal_launch<SUBSPEC_BF16>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, ap, pl, (uint16_t*)out, part_o, part_ml, st);
+  else
+    causal_launch<SUBSPEC_F16>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, ap, pl, (uint16_t*)out, part_o, part_ml, st);
+  SUBSPEC_CHECK_HIP(hipGetLastError());
+  return SUBSPEC_OK;
+}
+}  // namespace subspec

@@ -269,6 +269,11 @@ int tree_attention_ex(const void* q, const void* k_cache, const void* v_cache, v
                       const int64_t* prefix_dev, const KvPages* pages, const uint64_t* anc_bits, float scale, void* workspace,
                       size_t workspace_bytes, void* stream);
 
+// Causal attention of a prefill (batch 1, head_dim 128): query row i is the token at cache row prefix + i
+size_t causal_attention_workspace(int64_t hq, int64_t hkv, int64_t n_rows, int64_t prefix);
+int causal_attention(const void* q, const void* k, const void* v, void* out, int dtype, int64_t hq, int64_t hkv, int64_t n_rows,
+                     int64_t seq_stride, int64_t prefix, float scale, void* workspace, hipStream_t st);
+
 // Linear layers with a fused residual add (y = x W^T + bias + residual; residual may alias y); the C entry points
 // are these with residual = NULL.  Used by the decoder-layer sequence.
 int int4_linear_ex(const void* x, const uint32_t* wq, const uint32_t* sz, const void* bias, const void* residual, void* y,
@@ -288,7 +293,7 @@ int dense_gate_up_silu_ex(const void* x, const void* w, const void* bias, void* 
                           int64_t K, void* stream);
 // pending_splits != NULL: when K is split over workgroups the launch that sums the fp32 partials
 // (workspace: [splits][M][N]) is left to the caller's next kernel, *pending_splits = number of partials (then neither bias
-// nor residual has been applied and y is untouched); 1: y is complete
+// nor residual has been applied and y is untouched); 1: y is complete.  More than 384 rows (a prefill) where tile_applies.
 int dense_linear_ex(const void* x, const void* w, const void* bias, const void* residual, void* y, int dtype, int64_t M,
                     int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream, int* pending_splits = nullptr);
 

@@ -20,7 +20,8 @@
 //
 // The target model's layer in the tree-decoding forward (HF Qwen2DecoderLayer under
 // ClassicSDGeneratorBase._tree_decoding, specdecodes/models/generators/classic_sd.py:75-109) is the
-// same sequence with dense 16-bit projections (dense.hip) in place of the int4 ones.
+// same sequence with dense 16-bit projections (dense.hip) in place of the int4 ones.  A chunk of a prompt (generators/base.py:204-263)
+// is that sequence with causal attention and any number of rows.
 #include "common.h"
 #include <algorithm>
 
@@ -163,12 +164,27 @@ __global__ __launch_bounds__(64) void rope_write_kernel(const uint16_t* __restri
   Elem<DT>::store(dst, i + half, o_hi);
 }
 
+// Rows 0 .. rows - 1 of a paged layer as contiguous [Hkv, rows, 128] K and V: a prefill's attention reads every row many
+// times, so one copy (4 MB at 2048 rows of four heads) lets it run on the contiguous kernel, with the contiguous cache's bits.
+__global__ __launch_bounds__(256) void gather_pages_kernel(KvRowMap kv, int64_t rows, dec_u4* __restrict__ k_out,
+                                                           dec_u4* __restrict__ v_out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;               // 16-byte piece i % 16 of (row, head)
+  const int64_t row = i / (16 * kv.hkv);
+  if (row >= rows) return;
+  const int piece = (int)(i & 15), head = (int)(i / 16 % kv.hkv);
+  uint16_t *k, *v;
+  if (!kv_row_ptrs(kv, head, row, &k, &v)) return;
+  const int64_t o = ((int64_t)head * rows + row) * 16 + piece;
+  k_out[o] = ((const dec_u4*)k)[piece];
+  v_out[o] = ((const dec_u4*)v)[piece];
+}
+
 // rows of one call: the int4 stack serves draft levels and post-verify windows, the dense stack also whole large trees
-constexpr int kInt4LayerMaxRows = 64, kDenseLayerMaxRows = 384;
+constexpr int kInt4LayerMaxRows = 64, kDenseLayerMaxRows = 384, kPrefillMaxRows = 65536;
 struct LayerPlan {
-  size_t h, qkv, q, a, o, gu, act, sub, sub_bytes, total;
+  size_t h, qkv, q, a, o, gu, act, kv, sub, sub_bytes, total;
 };
-static LayerPlan layer_plan(const subspec_decoder_layer_dims& s) {
+static LayerPlan layer_plan(const subspec_decoder_layer_dims& s, bool causal = false) {
   LayerPlan p;
   const size_t es = 2, M = (size_t)s.n_rows, H = (size_t)s.hidden, Q = (size_t)s.n_q_heads * s.head_dim,
                KV = (size_t)s.n_kv_heads * s.head_dim, F = (size_t)s.intermediate;
@@ -179,10 +195,12 @@ static LayerPlan layer_plan(const subspec_decoder_layer_dims& s) {
   p.q = take(M * Q * es);
   p.a = take(M * Q * es);
   p.o = take(M * H * es);
-  p.gu = take(M * 2 * F * es);
+  // (a prefill's gate|up projection always ends in the activation)
+  p.gu = take(causal ? 0 : M * 2 * F * es);
   p.act = take(M * F * es);
+  p.kv = take(causal && s.page_indices ? 2 * KV * (size_t)(s.prefix_len + s.n_rows) * es : 0);
   size_t sub = 256;
-  if (s.n_rows <= kInt4LayerMaxRows) {                 // wider windows are dense only
+  if (!causal && s.n_rows <= kInt4LayerMaxRows) {                 // wider windows are dense only
     sub = std::max(sub, subspec_int4_linear_workspace(s.n_rows, Q + 2 * KV, H));
     sub = std::max(sub, subspec_int4_linear_workspace(s.n_rows, H, Q));
     sub = std::max(sub, subspec_int4_linear_workspace(s.n_rows, 2 * F, H));
@@ -190,9 +208,10 @@ static LayerPlan layer_plan(const subspec_decoder_layer_dims& s) {
   }
   sub = std::max(sub, subspec_dense_linear_workspace(s.n_rows, Q + 2 * KV, H));
   sub = std::max(sub, subspec_dense_linear_workspace(s.n_rows, H, Q));
-  sub = std::max(sub, subspec_dense_linear_workspace(s.n_rows, 2 * F, H));
+  if (!causal) sub = std::max(sub, subspec_dense_linear_workspace(s.n_rows, 2 * F, H));
   sub = std::max(sub, subspec_dense_linear_workspace(s.n_rows, H, F));
-  sub = std::max(sub, subspec_tree_attention_workspace(1, s.n_q_heads, s.n_kv_heads, s.n_rows, s.prefix_len, s.n_tree_slots));
+  if (causal) sub = std::max(sub, causal_attention_workspace(s.n_q_heads, s.n_kv_heads, s.n_rows, s.prefix_len));
+  else sub = std::max(sub, subspec_tree_attention_workspace(1, s.n_q_heads, s.n_kv_heads, s.n_rows, s.prefix_len, s.n_tree_slots));
   p.sub_bytes = align_up(sub, 256);
   p.sub = take(p.sub_bytes);
   p.total = off;
@@ -248,8 +267,8 @@ static int project(const LayerWeights& w, const Projection& p, const void* x, co
 template <int DT>
 static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w, uint16_t* x,
                      const int32_t* positions, const int32_t* cache_rows, const uint64_t* anc_bits, uint16_t* k_cache,
-                     uint16_t* v_cache, char* ws, hipStream_t st) {
-  const LayerPlan p = layer_plan(s);
+                     uint16_t* v_cache, char* ws, hipStream_t st, bool causal = false) {
+  const LayerPlan p = layer_plan(s, causal);
   const int M = (int)s.n_rows, H = (int)s.hidden, Hq = (int)s.n_q_heads, Hkv = (int)s.n_kv_heads, D = (int)s.head_dim,
             F = (int)s.intermediate;
   const int64_t Q = (int64_t)Hq * D, KV = (int64_t)Hkv * D;
@@ -278,7 +297,18 @@ static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w,
                        M, Hq, Hkv, D, log2f(s.rope_theta), s.rope_inv_freq, (const float*)sub, pending > 1 ? pending : 0,
                        (const uint16_t*)w.qkv_bias);
   }
-  if ((rc = tree_attention_ex(q, k_cache, v_cache, a, DT, Hq, Hkv, M, s.n_tree_slots, s.kv_seq_stride, s.prefix_len,
+  if (causal) {
+    const int64_t rows = s.prefix_len + M;
+    const uint16_t *kk = k_cache, *vv = v_cache;
+    if (pg) {
+      kk = (const uint16_t*)(ws + p.kv);
+      vv = kk + KV * rows;
+      const int64_t pieces = rows * KV / 8;
+      hipLaunchKernelGGL(gather_pages_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, kv, rows, (dec_u4*)kk, (dec_u4*)vv);
+    }
+    if ((rc = causal_attention(q, kk, vv, a, DT, Hq, Hkv, M, pg ? rows : s.kv_seq_stride, s.prefix_len, 1.f / sqrtf((float)D), sub, st)))
+      return rc;
+  } else if ((rc = tree_attention_ex(q, k_cache, v_cache, a, DT, Hq, Hkv, M, s.n_tree_slots, s.kv_seq_stride, s.prefix_len,
                               s.prefix_len_dev, pg, anc_bits, 1.f / sqrtf((float)D), sub, p.sub_bytes, st)))
     return rc;
   if (fused) {
@@ -389,4 +419,59 @@ extern "C" int subspec_dense_decoder_layer(const subspec_decoder_layer_dims* dim
   const LayerWeights w{s.input_norm, s.post_norm, s.qkv_bias, {s.qkv_w, nullptr}, {s.o_w, nullptr},
                        {s.gate_up_w, nullptr}, {s.down_w, nullptr}, true};
   return decoder_layer_entry(dims, w, x, positions, cache_rows, anc_bits, k_cache, v_cache, workspace, workspace_bytes, stream);
+}
+
+// A prefill takes dense layers whose projections the kernels above cover at its number of rows
+static int check_prefill(const subspec_decoder_layer_dims* s) {
+  if (!s) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: null dims");
+  subspec_decoder_layer_dims d = *s;
+  d.n_tree_slots = 1;                                 // (no tree: the rows of the call bound the cache below)
+  const int rc = check_dims(&d, kPrefillMaxRows);
+  if (rc != SUBSPEC_OK) return rc;
+  if (s->prefix_len + s->n_rows > s->kv_seq_stride)
+    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: prefix_len=%lld + n_rows=%lld exceed a cache of %lld rows", (long long)s->prefix_len,
+                 (long long)s->n_rows, (long long)s->kv_seq_stride);
+  if (s->prefix_len_dev) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: no device-side prefix length");
+  const int64_t M = s->n_rows, H = s->hidden, F = s->intermediate, Q = s->n_q_heads * s->head_dim, KV = s->n_kv_heads * s->head_dim;
+  if (std::max(std::max(H, F), Q) > 65536)
+    SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "prefill_layer: a projection longer than 65536");
+  // up to 64 rows: kernels with a 2 GiB descriptor range
+  if (M <= 64 && std::max(2 * F * H, (Q + 2 * KV) * H) >= ((int64_t)1 << 30))
+    SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "prefill_layer: up to 64 rows take matrices below 2 GiB");
+  if (M > 64 && !(tile_applies(M, Q + 2 * KV, H, false, nullptr, nullptr) && tile_applies(M, H, Q, false, nullptr, nullptr) &&
+                  tile_applies(M, 2 * F, H, true, nullptr, nullptr) && tile_applies(M, H, F, false, nullptr, nullptr)))
+    SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "prefill_layer: projection sizes outside the tiled kernel's range");
+  if ((Q + 2 * KV) / s->head_dim > 65535 || s->n_q_heads * ((M + 63) / 64) * 2 > 0x7fffff)
+    SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "prefill_layer: %lld heads over %lld rows", (long long)s->n_q_heads, (long long)M);
+  return SUBSPEC_OK;
+}
+
+extern "C" size_t subspec_prefill_layer_workspace(const subspec_decoder_layer_dims* dims) {
+  return check_prefill(dims) == SUBSPEC_OK ? layer_plan(*dims, true).total : 0;
+}
+
+extern "C" int subspec_prefill_layer(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights, void* x,
+                                     const int32_t* positions, const int32_t* cache_rows, void* k_cache, void* v_cache,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+  const int rc = check_prefill(dims);
+  if (rc != SUBSPEC_OK) return rc;
+  if (!weights) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: null weights");
+  const subspec_dense_layer_weights& s = *weights;
+  if (!x || !positions || !cache_rows || !k_cache || (!v_cache && !dims->page_indices) || !s.input_norm || !s.post_norm ||
+      !s.qkv_w || !s.o_w || !s.gate_up_w || !s.down_w)
+    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: null pointer argument");
+  if ((uintptr_t)x % 16 || (uintptr_t)s.input_norm % 16 || (uintptr_t)s.post_norm % 16 || (uintptr_t)k_cache % 16 ||
+      (uintptr_t)v_cache % 16)
+    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: x, norm weights and caches must be 16-byte aligned");
+  const size_t need = layer_plan(*dims, true).total;
+  if (!workspace || workspace_bytes < need)
+    SUBSPEC_FAIL(SUBSPEC_ERR_WORKSPACE, "prefill_layer: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
+  if ((uintptr_t)workspace % 256) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: workspace must be 256-byte aligned");
+  const LayerWeights w{s.input_norm, s.post_norm, s.qkv_bias, {s.qkv_w, nullptr}, {s.o_w, nullptr},
+                       {s.gate_up_w, nullptr}, {s.down_w, nullptr}, true};
+  if (dims->dtype == SUBSPEC_BF16)
+    return run_layer<SUBSPEC_BF16>(*dims, w, (uint16_t*)x, positions, cache_rows, nullptr, (uint16_t*)k_cache, (uint16_t*)v_cache,
+                                   (char*)workspace, (hipStream_t)stream, true);
+  return run_layer<SUBSPEC_F16>(*dims, w, (uint16_t*)x, positions, cache_rows, nullptr, (uint16_t*)k_cache, (uint16_t*)v_cache,
+                                (char*)workspace, (hipStream_t)stream, true);
 }

@@ -714,6 +714,7 @@ using namespace subspec;
 
 extern "C" size_t subspec_dense_linear_workspace(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 256;
+  if (M > kWideMaxRows) return align_up(tile_workspace(M, N, K), 256) + 256;
   if (wide_applies(M, N)) {
     const WidePlan wp = wide_plan(N, K, false);
     // above 64 rows either kernel may run (the tiled one needs a 16-byte aligned y)
@@ -726,6 +727,7 @@ extern "C" size_t subspec_dense_linear_workspace(int64_t M, int64_t N, int64_t K
 
 extern "C" int subspec_dense_linear(const void* x, const void* w, const void* bias, void* y, int dtype, int64_t M,
                                     int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream) {
+  if (M > kWideMaxRows) SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "dense_linear: M=%lld exceeds the %d-row limit", (long long)M, kWideMaxRows);
   return dense_linear_ex(x, w, bias, nullptr, y, dtype, M, N, K, workspace, workspace_bytes, stream);
 }
 
@@ -734,7 +736,7 @@ int subspec::dense_gate_up_silu_ex(const void* x, const void* w, const void* bia
   if (dtype != SUBSPEC_BF16 && dtype != SUBSPEC_F16)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_gate_up_silu: dtype %d not supported (bf16 / fp16 only)", dtype);
   if (!x || !w || !act) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_gate_up_silu: null pointer argument");
-  if (M <= 0 || M > kWideMaxRows || N <= 0 || K <= 0 || N % 32 != 0 || K % kDnGroup != 0 || K > 65536)
+  if (M <= 0 || (M > kWideMaxRows && !tile_applies(M, N, K, true, act, nullptr)) || N <= 0 || K <= 0 || N % 32 != 0 || K % kDnGroup != 0 || K > 65536)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_gate_up_silu: M=%lld N=%lld K=%lld; 1 <= M <= %d, N a multiple of 32, K of 64",
                  (long long)M, (long long)N, (long long)K, kWideMaxRows);
   // up to 32 rows: a workgroup's weight descriptor spans from its gate tiles to its up tiles, more than half the matrix
@@ -749,6 +751,8 @@ int subspec::dense_gate_up_silu_ex(const void* x, const void* w, const void* bia
 
 extern "C" int subspec_dense_gate_up_silu(const void* x, const void* w, const void* bias, void* act, int dtype, int64_t M,
                                           int64_t N, int64_t K, void* stream) {
+  if (M > kWideMaxRows)
+    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_gate_up_silu: M=%lld exceeds the %d-row limit", (long long)M, kWideMaxRows);
   return subspec::dense_gate_up_silu_ex(x, w, bias, act, dtype, M, N, K, stream);
 }
 
@@ -760,7 +764,8 @@ int subspec::dense_linear_ex(const void* x, const void* w, const void* bias, con
   if (M <= 0 || N <= 0 || K <= 0 || N % 16 != 0 || K % kDnGroup != 0)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_linear: M=%lld N=%lld K=%lld; N must be a multiple of 16 and K of 64",
                  (long long)M, (long long)N, (long long)K);
-  if (M > kWideMaxRows) SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "dense_linear: M=%lld exceeds the %d-row limit", (long long)M, kWideMaxRows);
+  if (M > kWideMaxRows && !tile_applies(M, N, K, false, y, residual))
+    SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "dense_linear: M=%lld exceeds the %d-row limit", (long long)M, kWideMaxRows);
   if (M > 64 && N % 32 != 0)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_linear: N=%lld must be a multiple of 32 for more than 64 rows", (long long)N);
   if (K > 65536) SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "dense_linear: K=%lld too large", (long long)K);

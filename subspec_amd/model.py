@@ -2,9 +2,9 @@
 against the shared static KV cache, SwiGLU MLP.  Random-init weights of the real shapes; nothing is
 downloaded.
 
-Plain library work (bf16 GEMMs, norms, rotary, the causal prefill attention) goes through torch;
-the hot-path pieces are the HIP kernels: tree-masked attention for every tree forward, int4
-GEMV / GEMM for the draft's projections, layer streaming for the target's offloaded layers.
+The hot-path pieces are the HIP kernels: whole decoder layers for tree forwards and prompt chunks, int4
+GEMV / GEMM for the draft's projections, layer streaming for the target's offloaded layers.  torch and
+its libraries serve what those kernels do not cover (float32, other head sizes, int4 prompts).
 q/k/v and gate/up are stored fused (rows concatenated), which leaves every output row and its
 quantization groups unchanged.
 """
@@ -199,6 +199,49 @@ class Decoder:
             self.streamer.run(step)
         return x
 
+    def _prefill_plan(self, x: torch.Tensor, start: int):
+        """What the one-call layers need for a chunk of a prompt, or None where they do not apply: 16-bit device tensors, one
+        sequence, head_dim 128, the sizes ``subspec_prefill_layer`` takes.  The workspace lives as long as the forward: a long
+        prompt's is large (150 MB at 2048 rows), and nothing else needs that much."""
+        cfg, cache, n = self.cfg, self.kv.cache, x.shape[0]
+        paged = not cache.contiguous
+        if not (self.use_native_layers and n and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and cfg.head_dim == 128
+                and x.shape[1] == cfg.hidden_size) or (paged and not hasattr(cache, "pool")):
+            return None
+        data = cache.pool.cache_data if paged else cache.data
+        heads = data.shape[4 if paged else 3]
+        if data.dtype != x.dtype or not data.is_contiguous() or heads != cfg.num_key_value_heads or data.device != x.device \
+                or (not paged and data.shape[2] != 1):
+            return None
+        stride, paging = cache.max_cache_len, {}
+        if paged:
+            table = cache.table()
+            paging = dict(page_indices=table, max_pages=cache.pool.max_pages, page_len=cache.page_len)
+            stride = table.numel() * cache.page_len
+        dims = ops.decoder_layer_dims(x.dtype, n, cfg.hidden_size, cfg.intermediate_size, cfg.num_attention_heads,
+                                      cfg.num_key_value_heads, cfg.head_dim, stride, start, 1, cfg.rms_norm_eps, cfg.rope_theta,
+                                      self._inv_freq, **paging)
+        need = ops.prefill_layer_workspace(dims)
+        if need == 0:
+            return None
+        rows = torch.arange(start, start + n, device=x.device, dtype=torch.int32)
+        return {"dims": dims, "rows": rows, "ws": torch.empty(need, dtype=torch.uint8, device=x.device), "paging": paging,
+                "shapes": layer_shapes(cfg), "kv": (lambda i: (data[i], data[i])) if paged else (lambda i: (data[i, 0], data[i, 1]))}
+
+    def _prefill_layer(self, plan, i: int, w: Dict[str, torch.Tensor], x: torch.Tensor) -> Optional[torch.Tensor]:
+        """One layer of a prompt chunk on the one-call kernels (in place), or None when this layer's weights are not dense
+        contiguous 16-byte aligned matrices of the expected shapes."""
+        if not x.is_contiguous():
+            return None
+        for name, shape in plan["shapes"].items():
+            t = w.get(name)
+            if t is None:
+                if name != "qkv_proj.bias":
+                    return None
+            elif (t.shape != shape or t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16):
+                return None
+        return ops.prefill_layer_(x, plan["dims"], ops.dense_layer_weights(w), plan["rows"], plan["rows"], *plan["kv"](i), plan["ws"])
+
     # ------------------------------------------------------------------ pieces
     def _rope(self, t: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         """t: [n, heads, D]"""
@@ -209,7 +252,11 @@ class Decoder:
         return t * cos + rot * sin
 
     def _layer(self, i: int, w: Dict[str, torch.Tensor], x: torch.Tensor, positions: torch.Tensor,
-               rows: torch.Tensor, attn: Callable[[int, torch.Tensor], torch.Tensor]) -> torch.Tensor:
+               rows: torch.Tensor, attn: Callable[[int, torch.Tensor], torch.Tensor], plan=None) -> torch.Tensor:
+        if plan is not None:
+            y = self._prefill_layer(plan, i, w, x)
+            if y is not None:
+                return y
         cfg = self.cfg
         n = x.shape[0]
         h = rms_norm(x, w["input_layernorm.weight"], cfg.rms_norm_eps)
@@ -225,15 +272,15 @@ class Decoder:
         gate, up = _linear(w, "gate_up_proj", h).chunk(2, dim=-1)
         return x + _linear(w, "down_proj", F.silu(gate) * up)
 
-    def _run_layers(self, x, positions, rows, attn) -> torch.Tensor:
+    def _run_layers(self, x, positions, rows, attn, plan=None) -> torch.Tensor:
         state = {"x": x}
         for i in range(min(self.first_streamed, len(self.layers))):
-            state["x"] = self._layer(i, self.layers[i], state["x"], positions, rows, attn)
+            state["x"] = self._layer(i, self.layers[i], state["x"], positions, rows, attn, plan)
         if self.streamer is not None and self.streamer.n:
             base = self.first_streamed
 
             def step(j, w):
-                state["x"] = self._layer(base + j, w, state["x"], positions, rows, attn)
+                state["x"] = self._layer(base + j, w, state["x"], positions, rows, attn, plan)
 
             self.streamer.run(step)
         return state["x"]
@@ -255,7 +302,8 @@ class Decoder:
     # ------------------------------------------------------------------ forwards
     def prefill(self, token_ids: torch.Tensor, start: int, all_logits: bool = False) -> torch.Tensor:
         """Causal forward of ``token_ids`` [n] at cache rows start..start+n-1; returns the last logits [1, V]
-        (``all_logits``: the logits of every position [n, V], e.g. to score a sequence by teacher forcing)."""
+        (``all_logits``: the logits of every position [n, V], e.g. to score a sequence by teacher forcing).  16-bit dense
+        layers run as one call each (``subspec_prefill_layer``); other layers module by module on library GEMMs."""
         n = token_ids.numel()
         self.kv.cache.ensure(start + n)
         self._rope_tables(start + n)
@@ -270,7 +318,8 @@ class Decoder:
             o = F.scaled_dot_product_attention(q, k, v, attn_mask=mask)
             return o.transpose(1, 2).reshape(n, cfg.q_size)
 
-        x = self._run_layers(self.embed[token_ids], positions, positions, attn)
+        x = self.embed[token_ids]
+        x = self._run_layers(x, positions, positions, attn, self._prefill_plan(x, start))
         return self.logits(x if all_logits else x[-1:])
 
     def tree_forward(self, token_ids: torch.Tensor, depths: Optional[torch.Tensor], anc_bits: torch.Tensor, prefix_len: int,

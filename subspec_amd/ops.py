@@ -544,6 +544,29 @@ def int4_decoder_layer_(x: torch.Tensor, dims: "L.DecoderLayerDims", weights: "L
     return x
 
 
+def prefill_layer_workspace(dims: "L.DecoderLayerDims") -> int:
+    """Bytes for ``prefill_layer_``; 0 where it does not cover these dimensions."""
+    return int(L.lib().subspec_prefill_layer_workspace(ctypes.byref(dims)))
+
+
+def prefill_layer_(x: torch.Tensor, dims: "L.DecoderLayerDims", weights: "L.DenseLayerWeights", positions: torch.Tensor,
+                   cache_rows: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, workspace: torch.Tensor) -> torch.Tensor:
+    """In-place update of the residual stream ``x`` [n_rows, hidden] by one dense layer over a chunk of a prompt: row i is
+    the token at cache row ``dims.prefix_len + i`` (``cache_rows``, int32 like ``positions``) and sees all rows up to its own."""
+    dev = _require_gpu(x, positions, cache_rows, k_cache, v_cache, workspace)
+    if positions.dtype != torch.int32 or cache_rows.dtype != torch.int32:
+        raise ValueError("prefill layer: positions / cache_rows must be int32")
+    if not (x.is_contiguous() and k_cache.is_contiguous() and v_cache.is_contiguous()):
+        raise ValueError("prefill layer: x and the layer's cache views must be contiguous")
+    if x.shape != (dims.n_rows, dims.hidden) or positions.numel() != dims.n_rows or cache_rows.numel() != dims.n_rows:
+        raise ValueError("prefill layer: tensor shapes do not match the dimensions given")
+    code = L.lib().subspec_prefill_layer(ctypes.byref(dims), ctypes.byref(weights), x.data_ptr(), positions.data_ptr(),
+                                         cache_rows.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), workspace.data_ptr(),
+                                         workspace.numel() * workspace.element_size(), _stream(dev))
+    L.check(code, "subspec_prefill_layer")
+    return x
+
+
 decoder_layer_ = int4_decoder_layer_     # either weight storage: the pointer table's type selects the entry point
 
 

@@ -275,10 +275,10 @@ int causal_attention(const void* q, const void* k, const void* v, void* out, int
                      int64_t seq_stride, int64_t prefix, float scale, void* workspace, hipStream_t st);
 
 // Linear layers with a fused residual add (y = x W^T + bias + residual; residual may alias y); the C entry points
-// are these with residual = NULL.  Used by the decoder-layer sequence.
+// are these with residual = NULL.  Used by the decoder-layer sequence.  pending_splits: see dense_linear_ex.
 int int4_linear_ex(const void* x, const uint32_t* wq, const uint32_t* sz, const void* bias, const void* residual, void* y,
                    int dtype, int64_t M, int64_t N, int64_t K, int64_t group_size, void* workspace, size_t workspace_bytes,
-                   void* stream);
+                   void* stream, int* pending_splits = nullptr);
 // act[M, F] = round(silu(round(gate))) * round(up) with gate | up = x * W^T (+ bias), W of N = 2F rows (gate rows first):
 // the SwiGLU MLP's first projection and its activation in one launch
 // norm_gain != NULL: x is the un-normalized residual stream and RMSNorm (gain [K], eps) is the projection's prologue (M <= 32)
@@ -296,6 +296,13 @@ int dense_gate_up_silu_ex(const void* x, const void* w, const void* bias, void* 
 // nor residual has been applied and y is untouched); 1: y is complete.  More than 384 rows (a prefill) where tile_applies.
 int dense_linear_ex(const void* x, const void* w, const void* bias, const void* residual, void* y, int dtype, int64_t M,
                     int64_t N, int64_t K, void* workspace, size_t workspace_bytes, void* stream, int* pending_splits = nullptr);
+
+// The int4 products for 33 to 64 rows (int4_tile.hip); returns the number of K ranges: with more than one their fp32 partials
+// [ranges][M][N] are in the workspace (int4_tile_workspace bytes) and y is untouched.
+bool int4_tile_applies(int64_t M, int64_t N, int64_t K, bool silu);
+size_t int4_tile_workspace(int64_t M, int64_t N, int64_t K);
+int int4_tile_linear(const void* x, const void* wq, const void* sz, const void* bias, const void* residual, void* y, int dtype,
+                     int64_t M, int64_t N, int64_t K, bool silu, void* workspace, hipStream_t st);
 
 // The same products for more than 64 rows (tile.hip).  tile_linear with *splits > 1: the fp32 partials [*splits][M][N] are in
 // the workspace (tile_workspace bytes) and y is untouched; 1: y is complete.

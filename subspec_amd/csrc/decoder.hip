@@ -261,7 +261,7 @@ static int project(const LayerWeights& w, const Projection& p, const void* x, co
                    int* pending_splits = nullptr) {
   if (pending_splits) *pending_splits = 1;
   if (w.dense) return dense_linear_ex(x, p.w, bias, residual, y, dtype, M, N, K, sub, sub_bytes, st, pending_splits);
-  return int4_linear_ex(x, (const uint32_t*)p.w, (const uint32_t*)p.sz, bias, residual, y, dtype, M, N, K, 64, sub, sub_bytes, st);
+  return int4_linear_ex(x, (const uint32_t*)p.w, (const uint32_t*)p.sz, bias, residual, y, dtype, M, N, K, 64, sub, sub_bytes, st, pending_splits);
 }
 
 template <int DT>
@@ -290,7 +290,7 @@ static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w,
   } else {
     hipLaunchKernelGGL((add_rmsnorm_kernel<DT, false>), dim3(M), dim3(kNormThreads), 0, st, x, (const uint16_t*)nullptr,
                        (const uint16_t*)w.input_norm, h, H, s.rms_eps);
-    // dense projections whose K is split leave the sum of their partials to the kernel that reads them next
+    // projections whose K is split leave the sum of their partials to the kernel that reads them next
     int pending = 0;
     if ((rc = project(w, w.qkv, h, w.qkv_bias, nullptr, qkv, DT, M, Q + 2 * KV, H, sub, p.sub_bytes, st, &pending))) return rc;
     hipLaunchKernelGGL((rope_write_kernel<DT>), dim3(M, Hq + 2 * Hkv), dim3(64), 0, st, qkv, positions, cache_rows, q, kv,

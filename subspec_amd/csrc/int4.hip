@@ -26,6 +26,7 @@
 //           compute unit), where a pipeline of a few groups is bound by round trips, not by bytes.
 //           A K of more than 56 groups over at least 128 tiles (the down projection): int4_rows8_long_kernel, one
 //           workgroup per tile over the whole of K, in rounds whose registers refill while they are used.
+// M = 33-64, K a multiple of 256: int4_tile.hip, a workgroup's wavefronts share the activations.
 // M = 2-64: int4_gemm_kernel, v_mfma_f32_16x16x32 with the activations as A and the weight tile as
 //           B operand; the 32 k of one MFMA step all come from one quantization group, so the raw
 //           accumulator of a group is scaled once.  The wavefronts of a workgroup split K, their
@@ -1072,6 +1073,11 @@ static I4Plan i4_plan(int64_t M, int64_t N, int64_t K) {
 template <int DT, int EPI>
 static int run_int4_paired(const void* x, const uint32_t* wq, const uint32_t* sz, const void* bias, void* out, int64_t M,
                            int64_t N, int64_t K, const I4Fused& fz, hipStream_t st) {
+  if (EPI == kEpiSilu && !fz.norm_gain && int4_tile_applies(M, N, K, true)) {
+    int4_tile_linear(x, wq, sz, bias, nullptr, out, DT, M, N, K, true, nullptr, st);
+    SUBSPEC_CHECK_HIP(hipGetLastError());
+    return SUBSPEC_OK;
+  }
   const int64_t pairs = N / 32, slots = i4_slots(M);
   // one or two pairs per workgroup; two only with few activation rows (the accumulators of four tiles
   // times four row blocks would fill the register file)
@@ -1127,7 +1133,17 @@ static int run_int4_paired(const void* x, const uint32_t* wq, const uint32_t* sz
 
 template <int DT>
 static int run_int4(const void* x, const uint32_t* wq, const uint32_t* sz, const void* bias, const void* residual, void* y,
-                    int64_t M, int64_t N, int64_t K, void* workspace, hipStream_t st) {
+                    int64_t M, int64_t N, int64_t K, void* workspace, hipStream_t st, int* pending_splits) {
+  if (pending_splits) *pending_splits = 1;
+  if (int4_tile_applies(M, N, K, false)) {
+    const int splits = int4_tile_linear(x, wq, sz, bias, residual, y, DT, M, N, K, false, workspace, st);
+    if (splits > 1 && pending_splits) *pending_splits = splits;
+    else if (splits > 1)
+      hipLaunchKernelGGL((int4_reduce_kernel<DT>), dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st, (const float*)workspace,
+                         (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, M, N, splits);
+    SUBSPEC_CHECK_HIP(hipGetLastError());
+    return SUBSPEC_OK;
+  }
   // One row: the GEMV kernel, unless the matrix has few rows and a long K (down projection): then its one workgroup
   // per 16-row tile leaves most of the chip idle and the split-K GEMM path is faster (3584x18944 from HBM: 22 against 32 us).
   if (M == 1 && !i4_rows8_plain(M, (int)(K / kGroup)) && i4_plan(M, N, K).splits == 1) {
@@ -1217,6 +1233,7 @@ extern "C" int subspec_int4_linear(const void* x, const uint32_t* wq, const uint
 }
 
 static size_t i4_workspace_one(int64_t M, int64_t N, int64_t K) {
+  if (int4_tile_applies(M, N, K, false)) return align_up(int4_tile_workspace(M, N, K), 256) + 256;
   const I4Plan pl = i4_plan(M, N, K);
   return (pl.splits > 1 ? align_up((size_t)pl.splits * M * N * sizeof(float), 256) : 0) + 256;
 }
@@ -1290,7 +1307,7 @@ int subspec::int4_qkv_rope_ex(const void* x, const uint32_t* wq, const uint32_t*
 
 int subspec::int4_linear_ex(const void* x, const uint32_t* wq, const uint32_t* sz, const void* bias, const void* residual,
                             void* y, int dtype, int64_t M, int64_t N, int64_t K, int64_t group_size, void* workspace,
-                            size_t workspace_bytes, void* stream) {
+                            size_t workspace_bytes, void* stream, int* pending_splits) {
   if (dtype != SUBSPEC_BF16 && dtype != SUBSPEC_F16)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "int4_linear: dtype %d not supported (bf16 / fp16 activations only)", dtype);
   if (!x || !wq || !sz || !y) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "int4_linear: null pointer argument");
@@ -1312,6 +1329,6 @@ int subspec::int4_linear_ex(const void* x, const uint32_t* wq, const uint32_t* s
                    workspace_bytes, need);
     if ((uintptr_t)workspace % 16) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "int4_linear: workspace must be 16-byte aligned");
   }
-  if (dtype == SUBSPEC_BF16) return run_int4<SUBSPEC_BF16>(x, wq, sz, bias, residual, y, M, N, K, workspace, (hipStream_t)stream);
-  return run_int4<SUBSPEC_F16>(x, wq, sz, bias, residual, y, M, N, K, workspace, (hipStream_t)stream);
+  if (dtype == SUBSPEC_BF16) return run_int4<SUBSPEC_BF16>(x, wq, sz, bias, residual, y, M, N, K, workspace, (hipStream_t)stream, pending_splits);
+  return run_int4<SUBSPEC_F16>(x, wq, sz, bias, residual, y, M, N, K, workspace, (hipStream_t)stream, pending_splits);
 }

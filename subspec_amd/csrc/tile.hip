@@ -22,7 +22,7 @@
 //   2048 rows: 490 -> 441 us), are what LDS holds.  Chunks of 32 k in twice as many slots lose (half-line requests).
 // 2048 rows: 441 us = 1.26 PFLOP/s with the activation included (library GEMM alone: 520 us; an 8192^3 product reaches
 // 1.38 PFLOP/s on this card), 289 rows: 87 us (dense_wide_kernel: 106), 128 rows: 54 us = 5.0 TB/s of weights.
-#include "common.h"
+#include "dma.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -41,22 +41,6 @@ __device__ __forceinline__ tl_v4f tl_mfma(tl_u4 a, tl_u4 b, tl_v4f c) {
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(tl_v8h, a), __builtin_bit_cast(tl_v8h, b), c, 0, 0, 0);
 }
-// 16 bytes per lane from base + voffset into LDS (lds_base + 16 * lane); NT: as streaming data
-template <bool NT>
-__device__ __forceinline__ void tl_dma16(uint32_t lds_base, uint32_t voffset, const void* base) {
-  if constexpr (NT)
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
-}
-// a wavefront-uniform address in scalar registers
-__device__ __forceinline__ const uint8_t* tl_uniform(const uint8_t* p) {
-  const uint64_t a = (uint64_t)(uintptr_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-  return (const uint8_t*)(uintptr_t)((uint64_t)hi << 32 | lo);
-}
-template <int N> __device__ __forceinline__ void tl_wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 struct TileParams {
   const uint16_t* x; const uint16_t* w; const uint16_t* bias; const uint16_t* residual; uint16_t* y; float* partial;
   int M, K; int64_t N;               // N: rows of w (SILU: 2 F)
@@ -123,12 +107,12 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
   const uint8_t* const wbase = (const uint8_t*)(p.w + n0 * K) + (int64_t)st0 * 128;
   const uint8_t* const xbase = (const uint8_t*)(p.x + (int64_t)m0 * K) + (int64_t)st0 * 128;
   // source of chunk s (relative to st0; beyond the last one: the last one again, into a slot nobody reads any more)
-  auto chunk_src = [&](const uint8_t* base, int s) { return tl_uniform(base + (int64_t)min(s, nst - 1) * 128); };
+  auto chunk_src = [&](const uint8_t* base, int s) { return uniform_ptr(base + (int64_t)min(s, nst - 1) * 128); };
   auto copy_w = [&](int i, const uint8_t* src, uint32_t slot_off) {
-    tl_dma16<NT>(__builtin_amdgcn_readfirstlane(wdst[i] + slot_off), woff[i], src);
+    dma16<NT>(__builtin_amdgcn_readfirstlane(wdst[i] + slot_off), woff[i], src);
   };
   auto copy_x = [&](int i, const uint8_t* src, uint32_t slot_off) {
-    tl_dma16<false>(__builtin_amdgcn_readfirstlane(xdst[i] + slot_off), xoff[i], src);
+    dma16<false>(__builtin_amdgcn_readfirstlane(xdst[i] + slot_off), xoff[i], src);
   };
   auto fill_w = [&](int s) {
 #pragma unroll
@@ -202,7 +186,7 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
   };
   auto sync = [&](auto wait_c) __attribute__((always_inline)) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    tl_wait_vmcnt<decltype(wait_c)::value>();
+    wait_vmcnt<decltype(wait_c)::value>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -259,7 +243,7 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
     }
   }
   // every copy into the rings has landed and every wavefront is done reading them: the space is reused below
-  tl_wait_vmcnt<0>();
+  wait_vmcnt<0>();
   __syncthreads();
 
   if constexpr (GK == 2) {

@@ -179,3 +179,32 @@ def test_gate_up_projection_with_the_activation_in_its_output_stage(dtype):
     with pytest.raises(ValueError):
         ops.int4_gate_up_silu(torch.zeros(65, 64, dtype=dtype, device=DEV), torch.zeros(2 * 32 * 64 // 8, dtype=torch.int32, device=DEV),
                               torch.zeros(2 * 32, dtype=torch.int32, device=DEV), 32)          # more than 64 rows
+
+
+@pytest.mark.parametrize("N,K,M", [(16, 256, 33), (48, 256, 64), (160, 512, 47), (336, 1280, 64), (1056, 2048, 50), (4608, 3584, 64),
+                                   (3584, 18944, 41), (28672, 4096, 64), (12288, 256, 63)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_shared_activation_kernel(N, K, M, dtype):
+    """33 to 64 rows, K a multiple of 256: one chunk, fewer and more chunks than ring slots, partial last workgroups, K ranges."""
+    print("int4 tile", N, K, M, dtype, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(N + K + M)
+    codes = torch.randint(0, 16, (N, K), generator=g, device=DEV, dtype=torch.uint8)
+    scale = (torch.rand(N, K // 64, generator=g, device=DEV) * 0.02 + 0.001).half()
+    zero = (torch.rand(N, K // 64, generator=g, device=DEV) * 15).half()
+    wq, sz = quant.pack_tiled(codes, scale, zero)
+    x, b = torch.randn(M, K, generator=g, device=DEV).to(dtype), torch.randn(N, generator=g, device=DEV).to(dtype)
+    w = (codes.double().view(N, -1, 64) - zero.double()[..., None]) * scale.double()[..., None]
+    w = w.view(N, K)
+    # one rounding of the result; fp32 sums of K products of (offset + code) x scale: 2^-24 sqrt(K) times their size, eightfold
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    slack = 8 * 2.0 ** -24 * K ** 0.5 * 0.021 * (143 if dtype == torch.bfloat16 else 1039) * x.abs().max().item()
+    ref = x.double() @ w.T + b.double()
+    got = ops.int4_linear(x, wq, sz, N, b).double()
+    assert ((got - ref).abs() <= ulp * ref.abs() + slack).all()
+    if N % 32 == 0:
+        act = ops.int4_gate_up_silu(x, wq, sz, N // 2, b).float()
+        gate, up = ref.to(dtype).float().chunk(2, dim=-1)
+        want = torch.nn.functional.silu(gate).to(dtype).float() * up
+        # gate and up may each land on the neighbouring value of their type (silu' < 1.1): three roundings
+        assert ((act - want).abs() <= 4 * 2 * ulp * want.abs() + 1.1 * (2 * ulp * gate.abs() + slack) * up.abs()
+                + (2 * ulp * up.abs() + slack) * gate.abs()).all()

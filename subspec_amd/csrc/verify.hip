@@ -28,6 +28,7 @@
 // row maximum; the normalized entropy of a 16-bit row is sum(entr(p)) with p, log p and p*log p
 // each rounded to that dtype, the sum rounded once, divided by float(ln V) and rounded again.
 #include "common.h"
+#include <string.h>
 #include <mutex>
 #include <algorithm>
 
@@ -141,11 +142,29 @@ struct VerifyParams {
   uint32_t offset[2];   // Philox counter words 2, 3: the caller's 64-bit stream offset
 };
 
-// TemperatureLogitsWarper on one element: IEEE quotient, one rounding to the row dtype
-template <int DT, bool WARP>
+// TemperatureLogitsWarper on one element: IEEE quotient, one rounding to the row dtype.  kWarpMul: the reciprocal product
+// rounds to the same value for every element of the dtype (warp_by_product), which saves four instructions per element.
+constexpr int kWarpNone = 0, kWarpDiv = 1, kWarpMul = 2;
+template <int DT, int WARP>
 __device__ __forceinline__ float warped(float x, const Divisor& temperature) {
-  if constexpr (WARP) return Elem<DT>::round(div_rn(x, temperature));
+  if constexpr (WARP == kWarpDiv) return Elem<DT>::round(div_rn(x, temperature));
+  if constexpr (WARP == kWarpMul) return Elem<DT>::round(x * temperature.inv_t);
   return x;
+}
+// bf16(float(x / T)) == bf16(float(x * (1 / T))) for every x: a bf16 is one of 128 mantissas times a power of two, and both
+// roundings scale with that power while nothing leaves the normal range (T within 2^+-20; an overflow is infinite either way),
+// so the 128 mantissas decide.  They agree unless a quotient lies within an fp32 ulp of a bf16 midpoint: some 0.4 % of all T.
+// (fp16 has 1024 mantissas and results in its subnormal range, fp32 no second rounding: they keep the division.)
+inline bool warp_by_product(int dtype, const Divisor& d) {
+  if (dtype != SUBSPEC_BF16 || !(d.t >= 0x1p-20f && d.t <= 0x1p20f)) return false;
+  auto bf16 = [](float v) {
+    uint32_t u;
+    memcpy(&u, &v, 4);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+  };
+  for (int x = 128; x < 256; ++x)
+    if (bf16((float)x / d.t) != bf16((float)x * d.inv_t)) return false;
+  return true;
 }
 template <int DT>
 __device__ __forceinline__ float load_warped(const void* logits, int64_t i, const VerifyParams& vp) {
@@ -241,7 +260,7 @@ __global__ __launch_bounds__(kRowThreads) void row_exact_kernel(
 // ------------------------------------------------------------------ kernel 1: one pass over HBM
 // sum exp and sum t*exp of one tile relative to the reference `mb = -ref * log2(e)`;
 // t is clamped so that exp2(t) == 0 implies t * exp2(t) == 0 (x may be -inf).
-template <int DT, int VEC, bool WARP>
+template <int DT, int VEC, int WARP>
 __device__ __forceinline__ float tile_accumulate(const Tile<DT, VEC>& t, float mb, const Divisor& temperature,
                                                  float (&s)[2], float (&u)[2]) {
   float x[VEC];
@@ -249,7 +268,7 @@ __device__ __forceinline__ float tile_accumulate(const Tile<DT, VEC>& t, float m
   // fp32 maximum): t stays finite, and whatever lies that far below the reference contributes exp2(t) == 0
   // and t * 0 == 0 either way.  The maximum of a fully masked tile is then the floor instead of -inf; it
   // can only surface as a row maximum when the whole row is masked.
-  constexpr bool kPackedFloor = !WARP && DT != SUBSPEC_F32 && VEC == 8;
+  constexpr bool kPackedFloor = WARP == kWarpNone && DT != SUBSPEC_F32 && VEC == 8;
   if constexpr (kPackedFloor) {
     Tile<DT, VEC> tc = t;
     tc.floor_neg_inf();
@@ -273,7 +292,7 @@ __device__ __forceinline__ float tile_accumulate(const Tile<DT, VEC>& t, float m
   return tmax;
 }
 
-template <int DT, int VEC, int U, bool WARP>
+template <int DT, int VEC, int U, int WARP>
 __global__ __launch_bounds__(kRowThreads) void row_partial_kernel(
     const void* __restrict__ logits, VerifyParams vp, Part1* __restrict__ part, Part2* __restrict__ part2) {
   const int64_t vocab = vp.vocab, chunk = vp.chunk;
@@ -381,21 +400,28 @@ __global__ __launch_bounds__(kRowThreads) void row_partial_kernel(
 }
 
 // ------------------------------------------------------------------ kernel 2b: one draw per row
-// Philox4x32-10 (Salmon et al., "Parallel random numbers: as easy as 1, 2, 3", SC'11).
-__device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
-                                              uint32_t k1, uint32_t (&out)[4]) {
+// Philox4x32-10 (Salmon et al., "Parallel random numbers: as easy as 1, 2, 3", SC'11); `out` holds the COMPLEMENT of the four
+// words.  A round is two 32 x 32 -> 64 bit multiplies and two three-way exclusive ors.
+__device__ __forceinline__ void philox4x32_10_not(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
+                                                  uint32_t k1, uint32_t (&out)[4]) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
-    const uint64_t p0 = (uint64_t)0xD2511F53u * c0;    // one 32 x 32 -> 64 bit multiply each
+    const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
     const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-    c0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
+    // truth tables: 0x96 a ^ b ^ c, 0x69 its complement
+    if (r < 9) {
+      c0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x96);
+      c2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c3, k1, 0x96);
+    } else {
+      c0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x69);
+      c2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c3, k1, 0x69);
+    }
     c1 = (uint32_t)p1;
-    c2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
     c3 = (uint32_t)p0;
     k0 += 0x9E3779B9u;
     k1 += 0xBB67AE85u;
   }
-  out[0] = c0; out[1] = c1; out[2] = c2; out[3] = c3;
+  out[0] = c0; out[1] = ~c1; out[2] = c2; out[3] = ~c3;
 }
 
 // Relative and absolute rounding bounds of one value stored in the row dtype (generous).
@@ -408,11 +434,15 @@ template <> struct RoundBound<SUBSPEC_BF16> { static constexpr float rel = 0x1p-
 // u = ((word >> 9) + 0.5) * 2^-23 lies strictly inside (0, 1) and is exact in fp32.
 // A slice starts at a multiple of 4, so a 4-element group never straddles two workgroups.
 //
-// The race key of an element is p / -log(u), evaluated exactly as defined (rounded probability,
-// accurate logarithm, IEEE quotient) only for the few elements that can still win: -log(u) >= 1 - u
-// and p <= an upper bound from the hardware exponential give key <= bound / (1 - u), and an
-// element whose bound stays below the best key any lane of the wavefront has seen is skipped.
-// What is left per element is the Philox block, one exponential and a compare.
+// The race key of an element is p / -log(u), evaluated exactly as defined (rounded probability, accurate logarithm, IEEE
+// quotient) only for the few elements that can still win.  -log(u) >= 1 - u, so key <= p / (1 - u), and an element with
+// log2(bound of p) - log2(best key any lane of the wavefront has seen) < log2(1 - u) is skipped.  The test needs no
+// exponential: its left side is linear in the logit, and the bit pattern of a float, read as an integer, is 2^23 (127 + log2)
+// from below (exact at powers of two, at most 0.087 low), so an element costs six instructions -- unpack, one fused
+// multiply-add, a shift, two conversions, a compare -- and only lets a few more candidates through.
+// What is left is the Philox block: 18 multiplies and 18 exclusive ors per four elements.  Two blocks per lane and trip, the
+// logits of the next trip in flight.  2048 x 152064 bf16 at T = 0.8, rows in the L3: the call 388 -> 317 us, of which the draw takes
+// two thirds, bound by the vector ALU (the multiplies alone are 60 % of it).
 // QUAD: the slice starts and ends on multiples of four elements and the rows are aligned for it, so the four logits
 // of a Philox block are one load (8 bytes of a 16-bit row, 16 of an fp32 row) and need no bounds.
 template <int DT, bool QUAD>
@@ -424,28 +454,29 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
   const int c = blockIdx.x;
   const RowStat rs = combine_row<DT>(part1 + row * vp.splits, vp);
   const int64_t c0 = (int64_t)c * vp.chunk;
-  const int64_t n = min(vp.chunk, vp.vocab - c0);
-  const int64_t base = row * vp.vocab + c0;
+  const int n = (int)min(vp.chunk, vp.vocab - c0);
+  const int blocks = (n + 3) / 4;                      // Philox blocks of the slice
   const bool warp = vp.temperature.t != 1.0f;
   const float inv_t = warp ? vp.temperature.inv_t : 1.0f;
-  const float round_up = warp ? RoundBound<DT>::rel : 0.f;          // x / T rounded to the dtype, relative
+  const float round_rel = warp ? RoundBound<DT>::rel : 0.f;         // x / T rounded to the dtype, relative
   const float round_abs = warp ? RoundBound<DT>::abs + 1e-30f : 0.f;
-  const float mb = -rs.m * kLog2e;
-  // p <= exp2((x' - m) log2 e) / S * (1 + rounding of p, of the hardware exp2 and of this arithmetic)
-  const float p_scale = (1.0f / rs.S) * (1.0f + 4.0f * RoundBound<DT>::rel + 1e-4f);
+  // p <= exp2((x' - m) log2 e) / S * (1 + its rounding), x' <= x / T (1 - round_rel) + 2 round_rel max(m, 0) + round_abs; the
+  // last term covers the fp32 arithmetic of the test.  In units of 2^-23 of log2, the exponent bias added:
+  const float slope = inv_t * (1.0f - round_rel) * kLog2e * 0x1p23f;
+  const float level = (127.0f + (2.02f * round_rel * fmaxf(rs.m, 0.f) + round_abs - rs.m) * kLog2e +
+                       log2f((1.0f / rs.S) * (1.0f + 4.0f * RoundBound<DT>::rel + 1e-4f)) + 1e-3f + 1e-6f * fabsf(rs.m)) * 0x1p23f;
+  constexpr bool kAbs = RoundBound<DT>::abs > 0.f;      // fp16: a probability may round up to the smallest subnormal
   float best = -1.f;
   int idx = 0x7fffffff;
-  float thr = 0.f;                                     // 0.9999 * 2^-23 * best key of the wavefront
-  for (int64_t g0 = 0; g0 * 4 < n; g0 += kRowThreads) {   // same trip count for every lane: the votes below see whole wavefronts
-    const int64_t g = g0 + threadIdx.x;
-    float xs[4];
+  float from = INFINITY, floor_from = INFINITY;         // level less log2 of the wavefront's best key; the same for p = abs
+  auto load = [&](int g, float (&xs)[4]) __attribute__((always_inline)) {
     if constexpr (QUAD) {                              // one load, clamped to the last block of the slice
-      const int64_t q = min(g, n / 4 - 1);
+      const int64_t at = row * vp.vocab + c0 + (int64_t)min(g, blocks - 1) * 4;
       if constexpr (DT == SUBSPEC_F32) {
-        const float4 v = *(const float4*)((const float*)logits + base + q * 4);
+        const float4 v = *(const float4*)((const float*)logits + at);
         xs[0] = v.x; xs[1] = v.y; xs[2] = v.z; xs[3] = v.w;
       } else {
-        const uint2 v = *(const uint2*)((const uint16_t*)logits + base + q * 4);
+        const uint2 v = *(const uint2*)((const uint16_t*)logits + at);
         if constexpr (DT == SUBSPEC_BF16) {
           xs[0] = __uint_as_float(v.x << 16); xs[1] = __uint_as_float(v.x & 0xffff0000u);
           xs[2] = __uint_as_float(v.y << 16); xs[3] = __uint_as_float(v.y & 0xffff0000u);
@@ -456,38 +487,60 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
       }
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)                      // unconditional loads (clamped index), in flight during the Philox rounds
-        xs[e] = Elem<DT>::load(logits, base + min(g * 4 + e, n - 1));
+      for (int e = 0; e < 4; ++e) xs[e] = Elem<DT>::load(logits, row * vp.vocab + c0 + min((int64_t)g * 4 + e, (int64_t)n - 1));
     }
-    uint32_t w[4];
-    philox4x32_10((uint32_t)(c0 / 4 + g), (uint32_t)row, vp.offset[0], vp.offset[1], vp.key[0], vp.key[1], w);
-    bool cand[4];
+  };
+  constexpr int U = 2;                                 // blocks per lane and trip
+  float xs[U][4];
+#pragma unroll
+  for (int b = 0; b < U; ++b) load(threadIdx.x + b * kRowThreads, xs[b]);
+  for (int g0 = 0; g0 < blocks; g0 += U * kRowThreads) {   // same trip count for every lane: the votes below see whole wavefronts
+    const int g = g0 + threadIdx.x;
+    float xn[U][4];
+#pragma unroll
+    for (int b = 0; b < U; ++b) load(g + (U + b) * kRowThreads, xn[b]);
+    uint32_t w[U][4];                                  // complements of the random words
+    bool cand[U][4];
     bool any_cand = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t i = g * 4 + e;
-      const float xa = fmaxf(xs[e] * inv_t, -1e30f);                 // masked (-inf) logits stay finite below
-      const float xu = fmaf(fabsf(xa), round_up, xa) + round_abs;
-      const float bound = fmaf(__builtin_amdgcn_exp2f(fmaf(xu, kLog2e, mb)), p_scale, RoundBound<DT>::abs);
-      const float one_minus_u = (float)((~w[e]) >> 9) + 0.5f;        // (1 - u) * 2^23, exact
-      cand[e] = (QUAD ? g * 4 < n : i < n) && !(bound < thr * one_minus_u);
-      any_cand |= cand[e];
-    }
-    // one vote per block of four: the threshold only prunes, so refreshing it less often changes no result
-    if (__any(any_cand)) {                             // wavefront-uniform
+    for (int b = 0; b < U; ++b)
+      philox4x32_10_not((uint32_t)(c0 / 4 + g + b * kRowThreads), (uint32_t)row, vp.offset[0], vp.offset[1], vp.key[0], vp.key[1], w[b]);
+#pragma unroll
+    for (int b = 0; b < U; ++b) {
+      const bool in = g + b * kRowThreads < blocks;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        if (cand[e]) {
-          const float x = xs[e];
-          const float xw = warp ? Elem<DT>::round(div_rn(x, vp.temperature)) : x;
-          const float p = rounded_prob<DT>(xw, rs.m, rs.S);
-          const float u = ((float)(w[e] >> 9) + 0.5f) * 0x1p-23f;
-          const float key = p / -logf(u);
-          if (key > best) { best = key; idx = (int)(c0 + g * 4 + e); }   // indices ascend: the first maximum stays
+        float z = fmaf(xs[b][e], slope, from);         // (a masked logit's -inf never passes, a NaN row has no candidate)
+        if constexpr (kAbs) z = fmaxf(z, floor_from) + 0x1p23f;
+        const float below = (float)(int)__float_as_uint((float)(w[b][e] >> 9));   // (1 - u) 2^23 - 1/2
+        cand[b][e] = in && z >= below && (QUAD || (g + b * kRowThreads) * 4 + e < n);
+        any_cand |= cand[b][e];
+      }
+    }
+    // one vote per trip: the threshold only prunes, so refreshing it less often changes no result
+    if (__any(any_cand)) {                             // wavefront-uniform
+#pragma unroll
+      for (int b = 0; b < U; ++b) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (cand[b][e]) {
+            const float x = xs[b][e];
+            const float xw = warp ? Elem<DT>::round(div_rn(x, vp.temperature)) : x;
+            const float p = rounded_prob<DT>(xw, rs.m, rs.S);
+            const float u = ((float)(~w[b][e] >> 9) + 0.5f) * 0x1p-23f;
+            const float key = p / -logf(u);
+            if (key > best) { best = key; idx = (int)(c0 + (g + b * kRowThreads) * 4 + e); }   // indices ascend: the first maximum stays
+          }
         }
       }
-      thr = fmaxf(wave_max(best), 0.f) * (0.9999f * 0x1p-23f);
+      const float seen = log2f(fmaxf(wave_max(best), 0.f) * (0.9999f * 0x1p-23f)) * 0x1p23f;
+      from = level - seen;
+      if constexpr (kAbs) floor_from = (127.0f + log2f(RoundBound<DT>::abs)) * 0x1p23f - seen;
     }
+#pragma unroll
+    for (int b = 0; b < U; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xs[b][e] = xn[b][e];
   }
   const float top = block_max<kRowThreads>(best, red_f);
   idx = block_min_i<kRowThreads>(best == top ? idx : 0x7fffffff, red_i);
@@ -833,12 +886,15 @@ static void launch_partial(dim3 grid, hipStream_t st, const void* logits, const 
   // loads in flight per thread: 8 when a slice is long enough for whole trips of that size (whole rows of a
   // large batch: 111 against 113 us at 2048 x 152064 bf16), 4 for the short slices of a few rows split many ways
   const bool long_slices = vp.chunk / VEC >= 2 * (int64_t)kRowThreads * 8;
-  if (vp.temperature.t != 1.0f)
-    hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 4, true>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
+  if (DT == SUBSPEC_BF16 && vp.temperature.t != 1.0f && warp_by_product(DT, vp.temperature))
+    hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 4, DT == SUBSPEC_BF16 ? kWarpMul : kWarpDiv>), grid, dim3(kRowThreads), 0, st, logits,
+                       vp, p1, p2);
+  else if (vp.temperature.t != 1.0f)
+    hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 4, kWarpDiv>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
   else if (long_slices)
-    hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 8, false>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
+    hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 8, kWarpNone>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
   else
-    hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 4, false>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
+    hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 4, kWarpNone>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
 }
 
 template <int DT>

@@ -53,6 +53,23 @@ def test_draws_match_oracle(dtype, vocab):
     assert near <= 4
 
 
+@pytest.mark.parametrize("temperature", [0.8, 1.3, 0.6, 0.26, 2.0 ** -21, 2.0 ** 21])
+def test_bf16_temperatures_by_product_and_by_division(temperature):
+    """bf16 rows are warped by the reciprocal's product where all 128 mantissas round like the quotient (0.8, 1.3), by division
+    otherwise (0.6 and 0.26 have a mantissa that does not, the powers of two lie outside the range); every mantissa, both signs,
+    masked elements, and slices that end inside a trip of the draw."""
+    g = torch.Generator().manual_seed(5)
+    rows, vocab = 6, 8 * 1283
+    mantissas = torch.arange(128, 256).float().repeat(vocab // 128 + 1)[:vocab] / 128
+    logits = (mantissas * 2.0 ** torch.randint(-2, 3, (rows, vocab), generator=g).float()
+              * torch.where(torch.rand(rows, vocab, generator=g) < 0.5, -1.0, 1.0)).to(torch.bfloat16)
+    logits[2, ::3] = float("-inf")
+    if temperature < 1e-3:
+        logits = (logits.float() * 2.0 ** -18).to(torch.bfloat16)     # keep the quotients in the range of logits
+    near = _check_draws(logits, temperature, ops.sample_tokens(logits.to(DEV), temperature, 3, 1).cpu(), 3, 1)
+    assert near <= 1
+
+
 def test_draw_frequencies_on_device():
     # 256 rows x 300 offsets of one 16-way distribution: chi-square against the rounded probabilities
     p = torch.tensor([0.25, 0.18, 0.14, 0.10, 0.08, 0.06, 0.05, 0.04, 0.03, 0.02, 0.02, 0.01, 0.01, 0.005, 0.003, 0.002])

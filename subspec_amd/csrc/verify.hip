@@ -220,32 +220,46 @@ __device__ __forceinline__ float rounded_prob(float x, float m, float S) {
 }
 
 // ------------------------------------------------------------------ rare exact pass over one slice
-// Re-reads the slice (normally still in L2) and evaluates what the reference evaluates element by
+// Re-reads the slice (normally still in the caches) and evaluates what the reference evaluates element by
 // element: the entropy terms with p, log p and p*log p rounded to the row dtype, and the first
-// index whose rounded probability equals the rounded maximum.
-template <int DT>
+// index whose rounded probability equals the rounded maximum.  Usually a handful of a batch's rows lies in the guard band, and
+// when one of them comes last its workgroup works alone, so what counts is the time of ONE row: element by element it waited for
+// a 2-byte load per element; now the next tile is requested while a tile is worked on and the quotient takes three
+// instructions, and the vector ALU bounds it (expf and logf are the accurate ones).  2048 x 152064 bf16 with such a row
+// 156 -> 119 us (105 without one).  Dealing the flagged rows out to all workgroups in a second launch: 116 and 112 us.
+template <int DT, int VEC, int WARP>
 __device__ __forceinline__ void row_exact_body(const void* __restrict__ logits, const VerifyParams& vp,
                                                const RowStat& rs, int64_t row, int c, float* red_f, int* red_i,
                                                Part2* __restrict__ part2) {
   const int64_t c0 = (int64_t)c * vp.chunk;
-  const int64_t n = min(vp.chunk, vp.vocab - c0);
+  const int nt = (int)(min(vp.chunk, vp.vocab - c0) / VEC);   // tiles of this slice
   const int64_t base = row * vp.vocab + c0;
+  const Divisor sum{rs.S, 1.0f / rs.S};
   float acc = 0.f;
   int tie = 0x7fffffff;
-  for (int64_t i = threadIdx.x; i < n; i += kRowThreads) {
-    const float x = load_warped<DT>(logits, base + i, vp);
-    const float p = rounded_prob<DT>(x, rs.m, rs.S);
-    if (rs.need_emu && p > 0.f) acc += Elem<DT>::round(-p * Elem<DT>::round(logf(p)));
-    if (p == rs.pmax && tie == 0x7fffffff) tie = (int)(c0 + i);
+  Tile<DT, VEC> next;
+  if ((int)threadIdx.x < nt) next.load_cached(logits, base + (int64_t)threadIdx.x * VEC);
+  for (int j = threadIdx.x; j < nt; j += kRowThreads) {
+    const Tile<DT, VEC> t = next;
+    next.load_cached(logits, base + (int64_t)min(j + kRowThreads, nt - 1) * VEC);
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      const float e = expf(warped<DT, WARP>(t.get(k), vp.temperature) - rs.m);
+      float q = div_rn(e, sum);
+      if (e < 0x1p-100f) q = e / rs.S;                 // where the residual of div_rn may be subnormal
+      const float p = Elem<DT>::round(q);
+      if (rs.need_emu && p > 0.f) acc += Elem<DT>::round(-p * Elem<DT>::round(logf(p)));
+      if (p == rs.pmax) tie = min(tie, (int)(c0 + (int64_t)j * VEC + k));
+    }
   }
   acc = block_sum<kRowThreads>(acc, red_f);
   tie = block_min_i<kRowThreads>(tie, red_i);
   if (threadIdx.x == 0) part2[row * vp.splits + c] = Part2{acc, tie};
 }
 
-// Separate launch, used when a row is split over several workgroups (the slices of a row must all
-// be reduced before any of them knows the row's statistics).
-template <int DT>
+// Separate launch for rows that are split over several workgroups (the slices of a row must all
+// be reduced before any of them knows the row's statistics): one workgroup per slice.
+template <int DT, int VEC, int WARP>
 __global__ __launch_bounds__(kRowThreads) void row_exact_kernel(
     const void* __restrict__ logits, VerifyParams vp, const Part1* __restrict__ part1,
     Part2* __restrict__ part2) {
@@ -254,7 +268,7 @@ __global__ __launch_bounds__(kRowThreads) void row_exact_kernel(
   const int64_t row = blockIdx.y;
   const RowStat rs = combine_row<DT>(part1 + row * vp.splits, vp);
   if (!rs.need_emu && !rs.need_tie) return;           // uniform across the workgroup
-  row_exact_body<DT>(logits, vp, rs, row, blockIdx.x, red_f, red_i, part2);
+  row_exact_body<DT, VEC, WARP>(logits, vp, rs, row, blockIdx.x, red_f, red_i, part2);
 }
 
 // ------------------------------------------------------------------ kernel 1: one pass over HBM
@@ -395,7 +409,7 @@ __global__ __launch_bounds__(kRowThreads) void row_partial_kernel(
     // the workgroup holds the statistics of the whole row: decide here whether the row needs the
     // exact pass and run it while the row is still in cache
     const RowStat rs = combine_row<DT>(&mine, vp);
-    if (rs.need_emu || rs.need_tie) row_exact_body<DT>(logits, vp, rs, row, 0, red_f, red_i, part2);
+    if (rs.need_emu || rs.need_tie) row_exact_body<DT, VEC, WARP>(logits, vp, rs, row, 0, red_f, red_i, part2);
   }
 }
 
@@ -897,6 +911,14 @@ static void launch_partial(dim3 grid, hipStream_t st, const void* logits, const 
     hipLaunchKernelGGL((row_partial_kernel<DT, VEC, 4, kWarpNone>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
 }
 
+template <int DT, int VEC>
+static void launch_exact(dim3 grid, hipStream_t st, const void* logits, const VerifyParams& vp, const Part1* p1, Part2* p2) {
+  if (vp.temperature.t != 1.0f)
+    hipLaunchKernelGGL((row_exact_kernel<DT, VEC, kWarpDiv>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
+  else
+    hipLaunchKernelGGL((row_exact_kernel<DT, VEC, kWarpNone>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
+}
+
 template <int DT>
 static int run_verify(const void* logits, int64_t batch, int64_t rows, int64_t vocab, const Plan& pl,
                       const VerifyParams& vp, const TreeParams& tp, Part1* p1, Part2* p2, Part3* p3,
@@ -910,8 +932,10 @@ static int run_verify(const void* logits, int64_t batch, int64_t rows, int64_t v
   };
   // the timed kernel is the longest one: the statistics pass, or the draw when sampling
   if (vp.sample) partial(); else { DominantKernelTimer timer(st); partial(); }
-  if (pl.splits > 1 && !vp.ties_in_accept)
-    hipLaunchKernelGGL((row_exact_kernel<DT>), grid, dim3(kRowThreads), 0, st, logits, vp, p1, p2);
+  if (pl.splits > 1 && !vp.ties_in_accept) {
+    if (pl.vec == 1) launch_exact<DT, 1>(grid, st, logits, vp, p1, p2);
+    else launch_exact<DT, (DT == SUBSPEC_F32 ? 4 : 8)>(grid, st, logits, vp, p1, p2);
+  }
   if (vp.sample) {
     DominantKernelTimer timer(st);
     // slices are whole numbers of 512-thread tiles of pl.vec elements: with pl.vec > 1 rows and slices are quad-aligned

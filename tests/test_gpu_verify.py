@@ -172,6 +172,31 @@ def test_config2_lossy_entropy_full_vocab(dtype):
     assert accepts[0] == 0 and accepts[-1] == 8
 
 
+@pytest.mark.parametrize("temperature", [1.0, 0.8])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("batch,n,vocab", [(4, 64, 520), (5, 60, 33003), (33, 64, 1000), (130, 33, 4104)])
+def test_exact_pass_in_tiles(batch, n, vocab, dtype, temperature):
+    """The exact pass behind the entropy gate, tile by tile: rows shorter and longer than a trip of the workgroup, ragged and
+    odd ones, in one slice and in several; every fp16 row takes it, of the bf16 rows those around the threshold."""
+    gen = torch.Generator().manual_seed(vocab)
+    logits = (torch.randn(batch, n, vocab, generator=gen) * (torch.rand(batch, n, 1, generator=gen) * 2.5 + 0.5)).to(DT[dtype])
+    logits[:, ::7, 3] = 9.0
+    logits[:, ::7, vocab - 2] = 9.0
+    parents, tokens, _ = W.random_tree(gen, n=n, vocab=vocab, chain_depth=8)
+    probs = torch.softmax((logits.float() / temperature).to(DT[dtype]).float(), -1).to(DT[dtype])
+    ref = torch.special.entr(probs).float().sum(-1).to(DT[dtype]) / math.log(vocab)      # float32 sum, rounded as stored
+    theta = float(ref.float().median())
+    kw = dict(do_sample=True, temperature=temperature, seed=1, offset=2) if temperature != 1.0 else {}
+    out = _run(logits, [tokens] * batch, [parents] * batch, verify_method="lossy", threshold_method="entropy", threshold=theta,
+               window_size=2, **kw)
+    assert (out["counts"][:, 3] == 0).all()
+    if not kw:                                         # greedy: first index of the rounded maximum
+        assert torch.equal(out["target"], (probs == probs.amax(-1, keepdim=True)).float().argmax(-1))
+    near = torch.ones_like(ref, dtype=torch.bool) if dtype == "float16" else (ref.float() - theta).abs() < 0.01 * theta
+    assert near.sum() > (0 if dtype == "bfloat16" else batch * n - 1)
+    _assert_entropy_matches(out["entropy"].float()[near], ref.float()[near], (batch, n, vocab, dtype))
+
+
 def test_near_threshold_rows_take_the_rounded_path():
     # rows whose entropy sits right at the threshold: decisions must still equal the oracle's
     torch.manual_seed(7)

@@ -69,9 +69,16 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
   // XCD-aware order: consecutive ids go to different XCDs; each XCD takes a contiguous run of the tile list, rows fastest
   const int total = p.tiles_m * p.tiles_n * p.splits;
   const int id = blockIdx.x, xcd = id & 7, per = total >> 3, rem = total & 7;
-  int lin = xcd * per + min(xcd, rem) + (id >> 3);
-  const int tm = lin % p.tiles_m; lin /= p.tiles_m;
-  const int tn = lin % p.tiles_n, ks = lin / p.tiles_n;
+  // The quotients are pinned to scalar registers: the compiler divides in the vector ALU and would keep the tile's origin, and
+  // with it the base address of every copy, in vector registers.  A copy's scalar base then comes out of a vector instruction
+  // one to four instructions ahead of it, where the architecture asks for five wait states -- which the compiler inserts in front
+  // of its own memory instructions, not in front of assembly text.
+  const int lin = xcd * per + min(xcd, rem) + (id >> 3);
+  int cell = lin / p.tiles_m;
+  asm volatile("" : "+s"(cell));
+  int ks = cell / p.tiles_n;
+  asm volatile("" : "+s"(ks));
+  const int tm = lin - cell * p.tiles_m, tn = cell - ks * p.tiles_n;
   const int m0 = tm * BM;
   const int64_t n0 = (int64_t)tn * (SILU ? BN / 2 : BN);                  // SILU: first output column
   const int64_t F = p.N >> 1;

@@ -199,6 +199,96 @@ def test_the_wide_dense_kernel_waits_only_where_it_says(tmp_path):
         assert waits and waits <= expected, f"{kernel}: waits {sorted(waits)} between its products, expected {sorted(expected)}"
 
 
+def _registers(operand: str) -> set:
+    """Numbers of the scalar registers of one operand: s5, s[4:5]."""
+    m = re.fullmatch(r"s(\d+)|s\[(\d+):(\d+)\]", operand.strip())
+    if not m:
+        return set()
+    return {int(m.group(1))} if m.group(1) else set(range(int(m.group(2)), int(m.group(3)) + 1))
+
+
+def _control_flow(lines):
+    """(instructions of every basic block, predecessors of every block) of one kernel body."""
+    blocks, names = [[]], {None: 0}
+    for line in lines:
+        m = re.match(r"^(\.LBB\w+):", line)
+        if m:
+            names[m.group(1)] = len(blocks)
+            blocks.append([])
+            continue
+        text = line.split(";")[0].strip()
+        if text and not text.startswith("."):
+            blocks[-1].append(text)
+            if text.startswith("s_cbranch"):
+                blocks.append([])
+    before = [set() for _ in blocks]
+    for i, body in enumerate(blocks):
+        for text in body:
+            m = re.match(r"s_c?branch\w*\s+(\S+)", text)
+            if m and m.group(1) in names:
+                before[names[m.group(1)]].add(i)
+        if i + 1 < len(blocks) and not (body and re.match(r"s_(branch|endpgm)\b", body[-1])):
+            before[i + 1].add(i)
+    return blocks, before
+
+
+def _vector_writes_close_to(blocks, before, block, at, wanted, states, seen):
+    """Vector ALU instructions that write one of the `wanted` scalar registers less than `states` wait states (one per
+    instruction, s_nop N: N + 1) ahead of instruction `at` of `block`, along every path that leads there."""
+    found = []
+    for text in reversed(blocks[block][:at]):
+        if states <= 0:
+            return found
+        name, _, operands = text.partition(" ")
+        outputs = operands.split(",")[:2 if "_co_" in name or "div_scale" in name else 1]
+        if name.startswith("v_") and any(_registers(o) & wanted for o in outputs):
+            found.append(text)
+        nop = re.match(r"s_nop (\d+)", text)
+        states -= int(nop.group(1)) + 1 if nop else 1
+    if states > 0:
+        for b in before[block]:
+            if (b, states) not in seen:
+                seen.add((b, states))
+                found += _vector_writes_close_to(blocks, before, b, len(blocks[b]), wanted, states, seen)
+    return found
+
+
+def test_the_parser_of_vector_writes_sees_paths_and_wait_states():
+    body = ["\tv_readfirstlane_b32 s12, v2", "\ts_add_i32 s3, s3, 1", "\ts_cbranch_scc1 .LBB0_2", "\ts_nop 1", ".LBB0_2:",
+            "\tv_cmp_gt_i32_e64 s[4:5], v0, v1", "\ts_mov_b32 m0, s8", "\tglobal_load_lds_dwordx4 v1, s[12:13]"]
+    blocks, before = _control_flow(body)
+    close = lambda wanted, states: _vector_writes_close_to(blocks, before, 2, 2, wanted, states, set())
+    assert close({12, 13}, 5) == ["v_readfirstlane_b32 s12, v2"]          # over the branch: four instructions lie between
+    assert close({12, 13}, 4) == [] and close({13}, 5) == []
+    assert close({5}, 2) == ["v_cmp_gt_i32_e64 s[4:5], v0, v1"] and close({5}, 1) == []
+
+
+@pytest.mark.parametrize("source, kernel, min_kernels", [
+    ("tile.hip", "dense_tile_kernel", 36), ("int4_tile.hip", "int4_tile_kernel", 12),
+    ("dense.hip", "dense_wide_kernel", 12), ("attention.hip", "tree_attention_pp_kernel", 8),
+])
+def test_copies_into_lds_do_not_read_a_scalar_address_too_early(source, kernel, min_kernels, tmp_path):
+    """A vector memory instruction may read a scalar register only five wait states after a vector ALU instruction has
+    written it.  The compiler keeps that distance for the memory instructions it knows; the copies into LDS are assembly
+    text to it.  No copy may therefore follow the instruction that writes its base address so closely, on any path."""
+    asm = _assembly(os.path.join(build_mod.CSRC, source), tmp_path)
+    _recognised(asm, kernel)
+    bodies = _kernel_bodies(asm, kernel)
+    assert len(bodies) >= min_kernels, "the parser found too few kernel variants"
+    for name, lines in bodies.items():
+        blocks, before = _control_flow(lines)
+        copies = 0
+        for b, body in enumerate(blocks):
+            for i, text in enumerate(body):
+                if not text.startswith("global_load_lds"):
+                    continue
+                copies += 1
+                base = set().union(*(_registers(o) for o in re.findall(r"\bs\d+\b|s\[\d+:\d+\]", text)))
+                close = _vector_writes_close_to(blocks, before, b, i, base, 5, set())
+                assert not close, f"{name}: '{text}' follows {close}"
+        assert copies, f"{name}: no copies found"
+
+
 def test_no_hand_written_vector_instruction_sits_next_to_an_mfma():
     """With MFMA results kept in ordinary vector registers (-amdgpu-mfma-vgpr-form=1) the compiler inserts the wait
     states between an MFMA and the vector ALU instruction that reads its result, but only for instructions it emitted

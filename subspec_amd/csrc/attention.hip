@@ -754,7 +754,7 @@ constexpr int kPPLdsBytes = kPPMaskOff + kAttnRows * kPPMaskWords * 8;
 
 __device__ __forceinline__ void pp_wait_vmcnt4() { asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); }
 __device__ __forceinline__ void pp_dma16(uint32_t lds_base, const uint16_t* src) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(src) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(src) : "memory", "m0");
 }
 
 // The matrix work of an M phase as steps of one matrix instruction each.  MODE 2 (the steady state) alternates the two

@@ -1,5 +1,6 @@
 // Copies from memory straight into LDS, waited for by hand: the compiler waits for every LDS copy that it knows of before any
-// LDS read, so the requests are inline assembly and the kernels that use them place their own waits.
+// LDS read, so the requests are inline assembly and the kernels that use them place their own waits.  (s_nop: the wait state that
+// M0 needs before a copy reads it.  The base must have been in scalar registers for five wait states: see dense_tile_kernel.)
 #pragma once
 #include "common.h"
 
@@ -9,9 +10,9 @@ namespace subspec {
 template <bool NT>
 __device__ __forceinline__ void dma16(uint32_t lds_base, uint32_t voffset, const void* base) {
   if constexpr (NT)
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
   else
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voffset), "s"(base) : "memory", "m0");
 }
 // a wavefront-uniform address in scalar registers
 __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {

@@ -289,16 +289,30 @@ def test_copies_into_lds_do_not_read_a_scalar_address_too_early(source, kernel, 
         assert copies, f"{name}: no copies found"
 
 
+def test_copies_into_lds_wait_for_their_destination_register():
+    """A copy into LDS takes its destination from M0, and one wait state has to lie between the scalar move that writes M0 and
+    the copy.  The compiler puts it there for its own copies; in assembly text it must be part of the text."""
+    texts = []
+    for name in sorted(os.listdir(build_mod.CSRC)):
+        if name.endswith((".hip", ".h")):
+            with open(os.path.join(build_mod.CSRC, name)) as f:
+                texts += [(name, t) for t in re.findall(r"\basm\s*(?:volatile)?\s*\(\s*\"([^\"]*global_load_lds[^\"]*)\"", f.read())]
+    assert len(texts) >= 4, "the pattern no longer finds the copies"
+    for name, text in texts:
+        steps = [t.split()[:2] for t in text.replace("\\t", "").split("\\n")]
+        assert [s[0] for s in steps] == ["s_mov_b32", "s_nop", "global_load_lds_dwordx4"] and steps[0][1] == "m0,", f"{name}: {text}"
+
+
 def test_no_hand_written_vector_instruction_sits_next_to_an_mfma():
     """With MFMA results kept in ordinary vector registers (-amdgpu-mfma-vgpr-form=1) the compiler inserts the wait
     states between an MFMA and the vector ALU instruction that reads its result, but only for instructions it emitted
     itself: a vector ALU instruction written as inline assembly is opaque to that pass and has read half-written
     accumulators.  The kernels therefore contain no vector ALU instruction as assembly TEXT -- asm statements are empty
     ones that only pin a value to a register class (the constants of v_and_or_b32 are made opaque by arithmetic on
-    run-time values instead), waits, and the attention kernel's copies from memory into LDS (which the compiler must NOT
+    run-time values instead), waits and wait states, and the attention kernel's copies from memory into LDS (which the compiler must NOT
     know about: it would wait for all of them before every LDS read) -- and this test keeps it that way."""
     pattern = re.compile(r"\basm\s*(?:volatile)?\s*\(\s*\"([^\"]*)\"")
-    allowed = re.compile(r"^(s_waitcnt\b|s_mov_b32 m0,|global_load_lds_dwordx4\b)")
+    allowed = re.compile(r"^(s_waitcnt\b|s_nop \d+$|s_mov_b32 m0,|global_load_lds_dwordx4\b)")
     seen = 0
     for name in sorted(os.listdir(build_mod.CSRC)):
         if not name.endswith((".hip", ".h")):

@@ -893,7 +893,8 @@ __device__ __forceinline__ void pp_softmax_phase(int64_t kb, const PPRow& rw, v1
   const bool move = mloc > -INFINITY && (!rf.have || mloc * rw.scale_log2 > kPPSlack);
   if (__any(move)) {
     const float d = move ? mloc : 0.f;                              // the row's reference goes up (first time: anywhere) by d
-    const float alpha = __builtin_amdgcn_exp2f(-d * rw.scale_log2);
+    // (only the first time does the reference go down, and nothing is accumulated then: 2^-d of scores far below zero is infinite)
+    const float alpha = __builtin_amdgcn_exp2f(fminf(-d * rw.scale_log2, 0.f));
     rf.ref += d;
     rf.l *= alpha;
 #pragma unroll

@@ -74,6 +74,22 @@ def test_many_pairs_peaked_rows():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_many_pairs_rows_far_below_zero(dtype):
+    """Rows whose scores in a whole first block of keys, of the sequence and of every chunk, lie near -1500 (a query against a
+    common component of the keys): the reference exponent of such a row starts far below zero.  Odd heads find ordinary
+    scores later on, even heads none at all."""
+    B, Hq, Hkv, n, P, S = 8, 16, 2, 64, 1000, 1064
+    parents, q, k, v = _case(78, B, Hq, Hkv, n, P, S, dtype)
+    common = 2.0 * torch.randn(128, generator=torch.Generator().manual_seed(1)).sign()
+    k = k / 4 + common                                                 # |common|^2 = 512
+    k[:, 1, 700:750] -= common.to(dtype)
+    q = q / 4
+    q[:, :, ::2] -= 3 * common.to(dtype)
+    assert (q.float() @ k.float().repeat_interleave(8, 1).transpose(-1, -2))[:, :, ::2, :700].max() < -1100
+    _check(parents, q.to(dtype), k.to(dtype), v, P, "far below zero")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_many_pairs_large_trees(dtype):
     """Trees beyond 64 slots (two and more mask words per row) with many (sequence, head) pairs: every window of 64 rows."""
     for seed, (B, n_slots, P, S, depth) in enumerate([(16, 128, 70, 256, 16), (16, 289, 200, 512, 48), (20, 100, 0, 128, 12)]):

@@ -56,6 +56,36 @@ def test_prefill_matches_float32(n, start, dtype, hq, hkv):
     assert torch.equal(rows[..., :start, :], past[..., :start, :]) and torch.equal(rows[..., start + n:, :], past[..., start + n:, :])
 
 
+@pytest.mark.parametrize("n,start", [(20, 0), (70, 0), (300, 0), (130, 200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prefill_with_scores_far_below_zero(n, start, dtype):
+    """Biases that put every score of a prompt's own keys near -1500 before the softmax (softmax over them is the ordinary one:
+    they share the shift); with past rows, which lack the bias, ordinary scores lie in front of them and in chunks without any."""
+    cfg = _cfg(4, 2)
+    w = M.init_weights(cfg, 6, DEV, dtype)
+    w["embed"].mul_(50.0)
+    slow = torch.tensor([d for d in range(128) if d % 64 >= 60], device=DEV)       # dimensions that the rotation leaves alone
+    for layer in w["layers"]:
+        heads = layer["qkv_proj.bias"].view(-1, 128)
+        heads[:cfg.num_attention_heads, slow] = -14.0
+        heads[cfg.num_attention_heads:cfg.num_attention_heads + cfg.num_key_value_heads, slow] = 14.0
+    g = torch.Generator(device=DEV).manual_seed(n + start)
+    tokens = torch.randint(0, cfg.vocab_size, (n,), generator=g, device=DEV)
+    past = torch.randn((2, 2, 1, 2, start + n + 9, 128), generator=g, device=DEV).to(dtype)
+    past[:, 0, :, :, :100, 60:64] += 14.0                                          # the first chunk's keys have it too
+    past[:, 0, :, :, :100, 124:] += 14.0
+    out = {}
+    with torch.no_grad():
+        for name, dt, native in (("exact", torch.float32, False), ("module", dtype, False), ("native", dtype, True)):
+            d = _stack(cfg, w, dt, start + n + 9)
+            d.use_native_layers = native
+            d.kv.cache.data.copy_(past)
+            out[name] = d.prefill(tokens, start, all_logits=True)
+    assert torch.isfinite(out["native"]).all()
+    module, native = (_rel(out[k], out["exact"]) for k in ("module", "native"))
+    assert native <= 2 * module, (native, module)
+
+
 @pytest.mark.parametrize("chunks", [(70,), (40, 30), (5, 64, 1)])
 def test_paged_prefill_equals_contiguous(chunks):
     cfg = _cfg(7, 1)

@@ -476,8 +476,10 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
   const float round_abs = warp ? RoundBound<DT>::abs + 1e-30f : 0.f;
   // p <= exp2((x' - m) log2 e) / S * (1 + its rounding), x' <= x / T (1 - round_rel) + 2 round_rel max(m, 0) + round_abs; the
   // last term covers the fp32 arithmetic of the test.  In units of 2^-23 of log2, the exponent bias added:
-  const float slope = inv_t * (1.0f - round_rel) * kLog2e * 0x1p23f;
-  const float level = (127.0f + (2.02f * round_rel * fmaxf(rs.m, 0.f) + round_abs - rs.m) * kLog2e +
+  // Where that leaves the range of a float (a maximum or 1 / T of 2^90 and more), every element is a candidate.
+  const bool in_range = fabsf(rs.m) < 0x1p90f && inv_t < 0x1p90f;
+  const float slope = in_range ? inv_t * (1.0f - round_rel) * kLog2e * 0x1p23f : 0.f;
+  const float level = !in_range ? INFINITY : (127.0f + (2.02f * round_rel * fmaxf(rs.m, 0.f) + round_abs - rs.m) * kLog2e +
                        log2f((1.0f / rs.S) * (1.0f + 4.0f * RoundBound<DT>::rel + 1e-4f)) + 1e-3f + 1e-6f * fabsf(rs.m)) * 0x1p23f;
   constexpr bool kAbs = RoundBound<DT>::abs > 0.f;      // fp16: a probability may round up to the smallest subnormal
   float best = -1.f;

@@ -70,6 +70,26 @@ def test_bf16_temperatures_by_product_and_by_division(temperature):
     assert near <= 1
 
 
+@pytest.mark.parametrize("scale,temperature", [(1.0, 2.0 ** -70), (1.0, 2.0 ** -101), (1.0, 2.0 ** -123), (2.0 ** 101, 1.0), (2.0 ** 122, 0.5),
+                                               (2.0 ** -40, 2.0 ** -126), (1.0, 2.0 ** 100), (1.0, 2.0 ** 127)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_draws_at_the_ends_of_the_range(dtype, scale, temperature):
+    """Quotients up to 2^126 and down to nothing: many equal maxima (the draw decides among them), masked elements, slices of
+    many trips.  Maxima are powers of two, whose exponent arguments are exact at any size."""
+    g = torch.Generator().manual_seed(9)
+    rows, vocab = 5, 30011
+    logits = torch.randint(-8, 9, (rows, vocab), generator=g).float()
+    logits[1] = logits[1].clamp(max=6.0)
+    logits[1, 29000] = 8.0                                # one maximum
+    logits[2, 5:] = float("-inf")
+    logits[2, :3] = torch.tensor([4.0, -1.0, 4.0])
+    logits[2, 3:5] = -2.0
+    logits[3] = -logits[3].abs() - 1.0                    # a negative maximum
+    logits = (logits * scale).to(dtype)
+    near = _check_draws(logits, temperature, ops.sample_tokens(logits.to(DEV), temperature, 5, 2).cpu(), 5, 2)
+    assert near <= 1
+
+
 def test_draw_frequencies_on_device():
     # 256 rows x 300 offsets of one 16-way distribution: chi-square against the rounded probabilities
     p = torch.tensor([0.25, 0.18, 0.14, 0.10, 0.08, 0.06, 0.05, 0.04, 0.03, 0.02, 0.02, 0.01, 0.01, 0.005, 0.003, 0.002])

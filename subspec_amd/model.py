@@ -230,8 +230,9 @@ class Decoder:
 
     def _prefill_layer(self, plan, i: int, w: Dict[str, torch.Tensor], x: torch.Tensor) -> Optional[torch.Tensor]:
         """One layer of a prompt chunk on the one-call kernels (in place), or None when this layer's weights are not dense
-        contiguous 16-byte aligned matrices of the expected shapes."""
-        if not x.is_contiguous():
+        contiguous 16-byte aligned matrices of the expected shapes, or when `_linear` would read more than those (int4 codes,
+        biases other than that of q|k|v)."""
+        if not x.is_contiguous() or any(n + ".wq" in w or (n != "qkv_proj" and w.get(n + ".bias") is not None) for n in QUANTIZED):
             return None
         for name, shape in plan["shapes"].items():
             t = w.get(name)

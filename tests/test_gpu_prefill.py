@@ -116,6 +116,32 @@ def test_layers_outside_the_one_call_path_keep_running():
         assert _rel(d.prefill(tokens, 0), want) < 0.02               # two bf16 layers: see the distances above
 
 
+@pytest.mark.parametrize("extra", ["o_proj.bias", "gate_up_proj.bias", "down_proj.bias", "codes"])
+def test_layers_that_hold_more_than_the_one_call_form_run_module_by_module(extra):
+    """The one-call layer has a bias for q|k|v only and reads dense weights; a layer with other biases, or with int4 codes
+    beside its dense matrices (the codes count), keeps its results."""
+    cfg = _cfg(4, 2)
+    w = M.init_weights(cfg, 7, DEV, torch.bfloat16)
+    w["embed"].mul_(50.0)
+    layer = w["layers"][1]
+    g = torch.Generator(device=DEV).manual_seed(2)
+    if extra == "codes":
+        layer.update({k: v for k, v in M.quantize_layers([layer])[0].items() if k.startswith("gate_up_proj.")})
+        layer["gate_up_proj.weight"] = torch.zeros_like(layer["gate_up_proj.weight"])
+    else:
+        rows = layer[extra.replace("bias", "weight")].shape[0]
+        layer[extra] = torch.randn(rows, generator=g, device=DEV).to(torch.bfloat16)
+    tokens = torch.randint(0, cfg.vocab_size, (40,), generator=g, device=DEV)
+    out = []
+    with torch.no_grad():
+        for native in (False, True):
+            kv = create_kv_cache("static", max_cache_len=64, config=cfg, device=DEV, dtype=torch.bfloat16)
+            d = M.Decoder(cfg, w["embed"], w["layers"], w["norm"], w["lm_head"], kv)
+            d.use_native_layers = native
+            out.append(d.prefill(tokens, 0, all_logits=True))
+    assert _rel(out[1], out[0]) < 0.02                               # one bf16 layer in another order of sums
+
+
 def test_prefill_layer_refuses_what_it_cannot_hold():
     d = lambda **k: ops.decoder_layer_dims(**{**dict(dtype=torch.bfloat16, n_rows=8, hidden=512, intermediate=1088, n_q_heads=4,
                                                      n_kv_heads=2, head_dim=128, kv_seq_stride=64, prefix_len=0, n_tree_slots=1,

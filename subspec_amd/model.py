@@ -201,8 +201,8 @@ class Decoder:
 
     def _prefill_plan(self, x: torch.Tensor, start: int):
         """What the one-call layers need for a chunk of a prompt, or None where they do not apply: 16-bit device tensors, one
-        sequence, head_dim 128, the sizes ``subspec_prefill_layer`` takes.  The workspace lives as long as the forward: a long
-        prompt's is large (150 MB at 2048 rows), and nothing else needs that much."""
+        sequence, head_dim 128, the sizes ``subspec_prefill_layer`` takes.  The workspace lives from the first layer that uses
+        it to the end of the forward: a long prompt's is large (150 MB at 2048 rows), and nothing else needs that much."""
         cfg, cache, n = self.cfg, self.kv.cache, x.shape[0]
         paged = not cache.contiguous
         if not (self.use_native_layers and n and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and cfg.head_dim == 128
@@ -225,7 +225,7 @@ class Decoder:
         if need == 0:
             return None
         rows = torch.arange(start, start + n, device=x.device, dtype=torch.int32)
-        return {"dims": dims, "rows": rows, "ws": torch.empty(need, dtype=torch.uint8, device=x.device), "paging": paging,
+        return {"dims": dims, "rows": rows, "need": need, "ws": None, "paging": paging,
                 "shapes": layer_shapes(cfg), "kv": (lambda i: (data[i], data[i])) if paged else (lambda i: (data[i, 0], data[i, 1]))}
 
     def _prefill_layer(self, plan, i: int, w: Dict[str, torch.Tensor], x: torch.Tensor) -> Optional[torch.Tensor]:
@@ -241,6 +241,8 @@ class Decoder:
                     return None
             elif (t.shape != shape or t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16):
                 return None
+        if plan["ws"] is None:
+            plan["ws"] = torch.empty(plan["need"], dtype=torch.uint8, device=x.device)
         return ops.prefill_layer_(x, plan["dims"], ops.dense_layer_weights(w), plan["rows"], plan["rows"], *plan["kv"](i), plan["ws"])
 
     # ------------------------------------------------------------------ pieces

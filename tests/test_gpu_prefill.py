@@ -142,6 +142,27 @@ def test_layers_that_hold_more_than_the_one_call_form_run_module_by_module(extra
     assert _rel(out[1], out[0]) < 0.02                               # one bf16 layer in another order of sums
 
 
+def test_int4_stacks_allocate_no_workspace_for_layers_that_decline_it():
+    """int4 layers of a prompt run module by module; the one-call layers' workspace (69 MB here) is for those that use it."""
+    cfg = M.DecoderConfig(num_hidden_layers=1, hidden_size=512, num_attention_heads=4, num_key_value_heads=2, head_dim=128,
+                          intermediate_size=11264, vocab_size=1024)
+    w = M.init_weights(cfg, 9, DEV, torch.bfloat16)
+    tokens = torch.randint(0, cfg.vocab_size, (1500,), generator=torch.Generator(device=DEV).manual_seed(3), device=DEV)
+    peak = []
+    with torch.no_grad():
+        for native in (False, True, False, True):                    # (the first round also sets up what the libraries keep)
+            kv = create_kv_cache("static", max_cache_len=1500, config=cfg, device=DEV, dtype=torch.bfloat16)
+            d = M.Decoder(cfg, w["embed"], M.quantize_layers(w["layers"]), w["norm"], w["lm_head"], kv)
+            d.use_native_layers = native
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            d.prefill(tokens, 0)
+            peak.append(torch.cuda.max_memory_allocated() - before)
+            del d, kv
+    assert peak[3] <= peak[2] + 65536, peak                          # (row numbers and the like)
+
+
 def test_prefill_layer_refuses_what_it_cannot_hold():
     d = lambda **k: ops.decoder_layer_dims(**{**dict(dtype=torch.bfloat16, n_rows=8, hidden=512, intermediate=1088, n_q_heads=4,
                                                      n_kv_heads=2, head_dim=128, kv_seq_stride=64, prefix_len=0, n_tree_slots=1,

@@ -345,8 +345,9 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
 // ------------------------------------------------------------------ launch shapes
 // Tile shapes and what a chunk of one takes when the chip is full of them (us, measured on the projections of a 7B layer:
 // 4608 / 3584 / 37888 x 3584 and 3584 x 18944 at 65 to 2048 rows).  The shapes of 160 columns cut 37888 rows into 237
-// workgroups, one per compute unit; those that serve up to 192 rows request their weights as streaming data (every
-// workgroup holds all rows, so a weight is read once: 128 rows 58.5 -> 53.8 us).
+// workgroups, one per compute unit; those that serve up to 192 rows request their weights as streaming data while one row tile
+// holds all rows, and a weight is read once (128 rows 58.5 -> 53.8 us).  Several row tiles share a weight through the L2, which
+// streaming defeats: 11264 x 2048 with the activation at 289 rows, 24 layers, 2.83 -> 2.73 ms without it.
 #define SUBSPEC_TILE_SHAPES(X)                      \
   X(0, 2, 4, 1, 4, 8, 3, 2, false, 1.55f)           \
   X(1, 4, 2, 1, 5, 5, 3, 2, false, 1.48f)           \
@@ -403,7 +404,10 @@ static void launch_tile(TileParams p, const TilePlan& pl, hipStream_t st) {
   switch (pl.shape) {
 #define X(ID, GM, GN, GK, TA, TB, SW, SX, NT, US)                                                                       \
   case ID:                                                                                                              \
-    hipLaunchKernelGGL((dense_tile_kernel<DT, GM, GN, GK, TA, TB, SW, SX, NT, SILU>), grid, dim3(512), 0, st, p);       \
+    if (NT && pl.tiles_m == 1)                                                                                          \
+      hipLaunchKernelGGL((dense_tile_kernel<DT, GM, GN, GK, TA, TB, SW, SX, NT, SILU>), grid, dim3(512), 0, st, p);     \
+    else                                                                                                                \
+      hipLaunchKernelGGL((dense_tile_kernel<DT, GM, GN, GK, TA, TB, SW, SX, false, SILU>), grid, dim3(512), 0, st, p);  \
     break;
     SUBSPEC_TILE_SHAPES(X)
 #undef X

@@ -32,7 +32,7 @@ def test_dense_linear(M, N, K, dtype):
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 64, 64), (128, 37888, 192), (192, 37888, 64), (256, 37888, 448), (289, 37888, 192),
-                                   (384, 11264, 256), (257, 28672, 128), (130, 2112, 320)])
+                                   (384, 11264, 256), (257, 28672, 128), (130, 2112, 320), (289, 11264, 2048)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gate_up_silu(M, N, K, dtype):
     print("tile gate|up", M, N, K, dtype, flush=True)

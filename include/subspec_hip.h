@@ -444,6 +444,11 @@ size_t subspec_dense_linear_workspace(int64_t M, int64_t N, int64_t K);
 int subspec_dense_linear(const void* x, const void* w, const void* bias, void* y, int dtype, int64_t M, int64_t N,
                          int64_t K, void* workspace, size_t workspace_bytes, void* stream);
 
+/* How a dense projection over more than 64 rows (gate_up != 0: the gate|up projection with its activation) is cut, for tests
+ * and tuning; host only.  plan = {index of the tile shape, row tiles, column tiles, K ranges}; returns 0, or
+ * SUBSPEC_ERR_LIMIT where the tiled kernel does not take these sizes (an aligned output assumed). */
+int subspec_dense_tile_plan(int64_t M, int64_t N, int64_t K, int gate_up, int32_t* plan);
+
 /* One decoder layer with dense 16-bit projections: same sequence of kernels, arguments, workspace
  * (subspec_int4_decoder_layer_workspace) and limits as subspec_int4_decoder_layer, for the target
  * model's layers (HF Qwen2DecoderLayer inside the forward named above), except that n_rows may reach 384 (a whole

@@ -9,7 +9,7 @@
 // (algorithmic bytes = N*K*2 + (M*K + M*N)*2); a library GEMM tiled for large M leaves more than half of that bandwidth
 // unused at this shape.  Three kernels: 1 to 32 rows the 16 x 16 x 32 kernel below, 33 to 64 rows the 32 x 32 x 16
 // kernel behind it, more rows the tiled kernel of tile.hip (dense_wide_kernel keeps those whose output is not 16-byte
-// aligned).
+// aligned, which no tensor has but a direct caller may, and gate|up matrices beyond the tiled kernel's 32-bit offsets).
 //
 // Same skeleton as the int4 kernel next door: the activations are the MFMA A operand, a 16-row
 // weight tile the B operand (v_mfma_f32_16x16x32, k permutation "step s, lane group c, element e ->

@@ -452,3 +452,14 @@ int tile_gate_up_silu(const void* x, const void* w, const void* bias, void* act,
 }
 
 }  // namespace subspec
+
+extern "C" int subspec_dense_tile_plan(int64_t M, int64_t N, int64_t K, int gate_up, int32_t* plan) {
+  using namespace subspec;
+  if (!plan || M <= 0 || N <= 0 || K <= 0) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_tile_plan: null pointer or empty size");
+  if (!tile_applies(M, N, K, gate_up != 0, nullptr, nullptr))
+    SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "dense_tile_plan: M=%lld N=%lld K=%lld outside the tiled kernel's range", (long long)M, (long long)N,
+                 (long long)K);
+  const TilePlan pl = tile_plan(M, N, K, gate_up != 0);
+  plan[0] = pl.shape; plan[1] = pl.tiles_m; plan[2] = pl.tiles_n; plan[3] = pl.splits;
+  return SUBSPEC_OK;
+}

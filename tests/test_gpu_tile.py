@@ -1,13 +1,18 @@
-"""GPU: the tiled dense kernels (more than 64 rows) at the edges of their tiles and for every launch shape the plan can
-choose: one 64-k chunk, fewer chunks than ring slots, rows and columns one past a tile, K split over workgroups, partial
-last tiles of the SwiGLU pairs, an output that is not 16-byte aligned (which takes the other kernel)."""
+"""GPU: the tiled dense kernels (more than 64 rows) at the edges of their tiles: one 64-k chunk, fewer chunks than ring slots,
+rows and columns one past a tile, partial last tiles of the SwiGLU pairs.  Every launch shape, with one and with several row
+tiles, with K whole and split: at a K of more chunks than the rings have slots, the shape checked against the plan.  Shapes
+that only prompts of more than 384 rows take at full size run inside whole layers.  Outputs that are not 16-byte aligned take
+the other kernel."""
+import ctypes
+
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 from subspec_amd import _lib as L
-from subspec_amd import ops
+from subspec_amd import model, ops
+from subspec_amd.cache import create_kv_cache
 
 DEV = "cuda:0"
 
@@ -45,6 +50,99 @@ def test_gate_up_silu(M, N, K, dtype):
     # gate and up may each land on the neighbouring value of their type (and silu' < 1.1): three roundings
     ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
     assert ((act - want).abs() <= 4 * ulp * want.abs() + 2 * ulp * up.abs() * 1e-1 + 1e-4).all()
+
+
+def _plan(M, N, K, gate_up):
+    """(tile shape, row tiles, column tiles, K ranges)"""
+    plan = (ctypes.c_int32 * 4)()
+    L.check(L.lib().subspec_dense_tile_plan(M, N, K, gate_up, plan), "subspec_dense_tile_plan")
+    return tuple(plan)
+
+
+# M, N, K; tile shape, row tiles, K ranges
+@pytest.mark.parametrize("M,N,K,shape,row_tiles,ranges", [
+    (129, 41536, 512, 0, 1, 1), (333, 22816, 512, 0, 2, 1), (129, 20736, 5632, 0, 1, 3), (333, 7296, 18944, 0, 2, 4),
+    (257, 22816, 512, 1, 1, 1), (257, 7296, 5632, 1, 1, 5), (200, 33216, 512, 2, 1, 1), (200, 16576, 3584, 2, 1, 2),
+    (129, 33216, 1024, 3, 1, 1), (129, 4736, 5632, 3, 1, 7), (65, 33216, 3584, 4, 1, 1), (257, 12416, 512, 4, 3, 1),
+    (65, 16576, 5632, 4, 1, 2), (300, 5856, 2048, 4, 3, 2), (129, 20736, 512, 5, 1, 1), (257, 14496, 512, 5, 2, 1),
+    (129, 4256, 3584, 5, 1, 6), (257, 3616, 3584, 5, 2, 4), (257, 16576, 512, 6, 3, 1), (257, 5536, 2048, 6, 3, 3),
+    (65, 16576, 640, 7, 1, 1), (257, 5536, 512, 7, 3, 1), (65, 5536, 5632, 7, 1, 4), (257, 2816, 2048, 7, 3, 3),
+    (65, 96, 512, 8, 1, 1), (129, 96, 512, 8, 2, 1), (65, 96, 1024, 8, 1, 2), (129, 96, 1024, 8, 2, 2),
+    (300, 4608, 3584, 8, 3, 1), (300, 3584, 18944, 6, 3, 6)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_shape_of_a_linear_layer(M, N, K, shape, row_tiles, ranges, dtype):
+    plan = _plan(M, N, K, 0)
+    assert (plan[0], plan[1], plan[3]) == (shape, row_tiles, ranges)
+    test_dense_linear(M, N, K, dtype)
+
+
+@pytest.mark.parametrize("M,N,K,shape,row_tiles", [
+    (129, 41536, 512, 0, 1), (333, 22816, 512, 0, 2), (333, 28672, 4096, 0, 2), (257, 22816, 512, 1, 1), (300, 37888, 3584, 1, 1),
+    (200, 33216, 512, 2, 1), (129, 33216, 1024, 3, 1), (160, 37888, 3584, 3, 1), (100, 37888, 3584, 4, 1), (257, 12416, 512, 4, 3),
+    (129, 20736, 512, 5, 1), (257, 14496, 512, 5, 2), (200, 28672, 4096, 5, 1), (257, 16576, 512, 6, 3), (333, 37888, 3584, 6, 3),
+    (65, 16576, 640, 7, 1), (257, 5536, 512, 7, 3), (65, 96, 512, 8, 1), (129, 96, 512, 8, 2), (100, 11264, 2048, 8, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_shape_of_gate_up(M, N, K, shape, row_tiles, dtype):
+    plan = _plan(M, N, K, 1)
+    assert (plan[0], plan[1], plan[3]) == (shape, row_tiles, 1)
+    test_gate_up_silu(M, N, K, dtype)
+
+
+# shapes of q|k|v, o, gate|up, down and the K ranges of down, at the widths of a 7B layer and of a wider one
+@pytest.mark.parametrize("rows,widths,shapes,ranges", [(2000, (3584, 28, 4, 18944), (2, 5, 0, 0), 2), (1000, (3584, 28, 4, 18944), (4, 7, 2, 0), 4),
+                                                       (1930, (4096, 32, 8, 14336), (0, 5, 0, 5), 1), (1590, (4096, 32, 8, 14336), (1, 5, 2, 0), 2)])
+def test_shapes_of_long_prompts(rows, widths, shapes, ranges):
+    """One whole layer against float32, the module-by-module path of the same dtype as the yardstick: both round at the same
+    points, so neither may be twice as far off as the other, in the 2-norm and in any one element."""
+    hidden, hq, hkv, mlp = widths
+    sizes = [((hq + 2 * hkv) * 128, hidden, 0), (hidden, hq * 128, 0), (2 * mlp, hidden, 1), (hidden, mlp, 0)]
+    plans = [_plan(rows, *s) for s in sizes]
+    assert tuple(p[0] for p in plans) == shapes and plans[3][3] == ranges
+    cfg = model.DecoderConfig(num_hidden_layers=1, hidden_size=hidden, num_attention_heads=hq, num_key_value_heads=hkv, head_dim=128,
+                          intermediate_size=mlp, vocab_size=512)
+    w = model.init_weights(cfg, 1, DEV, torch.bfloat16)
+    w["embed"].mul_(50.0)
+    tokens = torch.randint(0, 512, (rows,), generator=torch.Generator(device=DEV).manual_seed(rows), device=DEV)
+    out = {}
+    with torch.no_grad():
+        for name, dt, native in (("exact", torch.float32, False), ("module", torch.bfloat16, False), ("native", torch.bfloat16, True)):
+            print("long prompt", rows, hidden, name, flush=True)
+            kv = create_kv_cache("static", max_cache_len=rows, config=cfg, device=DEV, dtype=dt)
+            layers = [{k: v.to(dt) for k, v in w["layers"][0].items()}]
+            d = model.Decoder(cfg, w["embed"].to(dt), layers, w["norm"].to(dt), w["lm_head"].to(dt), kv)
+            d.use_native_layers = native
+            out[name] = (d.prefill(tokens, 0, all_logits=True).double(), kv.cache.data.double())
+    for exact, module, native in zip(out["exact"], out["module"], out["native"]):
+        assert (native - exact).norm() <= 2 * (module - exact).norm()
+        assert (native - exact).abs().max() <= 2 * (module - exact).abs().max()
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 96, 256), (200, 96, 2048), (257, 160, 2048), (384, 3584, 3584)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_unaligned_outputs_of_every_row_count(M, N, K, dtype):
+    """Two bytes past a 16-byte boundary, as only a direct caller of the library has them: dense_wide_kernel for 65 to 256 and
+    for 257 to 384 rows, K whole and split, and its SwiGLU form; nothing outside the output is written."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x, b = torch.randn(M, K, generator=g).to(dtype).to(DEV), torch.randn(N, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype).to(DEV)
+    lib, st, code = L.lib(), torch.cuda.current_stream().cuda_stream, L.BF16 if dtype == torch.bfloat16 else L.F16
+    ws = torch.empty(lib.subspec_dense_linear_workspace(M, N, K), dtype=torch.uint8, device=DEV)
+    ref = _ref(x, w, b)
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    room = torch.zeros(M * N + 16, dtype=dtype, device=DEV)
+    L.check(lib.subspec_dense_linear(x.data_ptr(), w.data_ptr(), b.data_ptr(), room[1:].data_ptr(), code, M, N, K, ws.data_ptr(),
+                                     ws.numel(), st), "subspec_dense_linear")
+    assert room[:1].abs().max() == 0 and room[1 + M * N:].abs().max() == 0
+    assert ((room[1:1 + M * N].view(M, N).double() - ref).abs() <= ulp * ref.abs() + 1e-4).all()      # see test_dense_linear
+    F = N // 2
+    room = torch.zeros(M * F + 16, dtype=dtype, device=DEV)
+    L.check(lib.subspec_dense_gate_up_silu(x.data_ptr(), w.data_ptr(), b.data_ptr(), room[1:].data_ptr(), code, M, N, K, st),
+            "subspec_dense_gate_up_silu")
+    assert room[:1].abs().max() == 0 and room[1 + M * F:].abs().max() == 0
+    gate, up = ref.to(dtype).float().chunk(2, dim=-1)
+    want = torch.nn.functional.silu(gate).to(dtype).float() * up
+    act = room[1:1 + M * F].view(M, F).float()
+    assert ((act - want).abs() <= 8 * ulp * want.abs() + 4 * ulp * up.abs() * 1e-1 + 1e-4).all()      # see test_gate_up_silu
 
 
 def test_unaligned_output_takes_the_other_kernel():

@@ -51,9 +51,10 @@ def test_config5_cycle_at_full_size():
     seq, log, rows, target, kv = _generate(cfg, base, cfg.num_hidden_layers, prompt)
     assert seq.numel() == PROMPT + NEW and log["n_tokens"] == NEW
     assert torch.equal(seq[:PROMPT], prompt[0])
-    # teacher forcing through the same target, on the device, in chunks of the prefill path
+    # teacher forcing through the same target, on the device, module by module on torch and its libraries
     print("config 5: teacher forcing", flush=True)
     kv.reset()
+    target.use_native_layers = False
     logits = target.prefill(seq[:-1], 0, all_logits=True)[PROMPT - 1:].float()       # row t scores token PROMPT + t
     emitted = seq[PROMPT:]
     scale = logits.abs().amax().item()

@@ -93,8 +93,9 @@ def test_cycle_emits_target_greedy_tokens_and_compacts_kv(method, kwargs):
     log = wandb_logger.log_data
     assert log["n_tokens"] == 24 and log["n_iter"] >= 1 and log["avg_sampled"] >= 1.0 and log["tput"] > 0
     assert kv.get_seq_length() == out.shape[1] - 1            # everything but the last sampled token is cached
-    # the compacted cache equals what a fresh prefill of the produced sequence writes (same weights)
+    # the compacted cache equals what a fresh prefill of the produced sequence writes (same weights, module by module on torch)
     kv2, target2, _, _ = _models(first_streamed=None)
+    target2.use_native_layers = False
     target2.prefill(out[0, :-1], 0)
     L = out.shape[1] - 1
     a, b = kv.cache.data[..., :L, :].float(), kv2.cache.data[..., :L, :].float()
@@ -269,6 +270,7 @@ def test_agreeing_draft_accepts_deep_paths():
         rounding of the window it was scored in: two correct runs may part ways at such a position)."""
         kv = create_kv_cache("static", max_cache_len=256, config=CFG, device=DEV, dtype=torch.bfloat16)
         target, _, _ = build_models(CFG, kv, device=DEV, weights=weights)
+        target.use_native_layers = False                              # module by module on torch: none of the kernels under test
         logits = target.prefill(seq[:-1].to(DEV), 0, all_logits=True).float().cpu()
         scale, exact = logits.abs().amax().item(), 0
         for t in range(31, seq.numel() - 1):

@@ -34,11 +34,12 @@ def _weights(agreeing, seed=9):
 
 
 def _assert_greedy_continuation(weights, seq, start, tag):
-    """Teacher forcing through the target (resident, torch prefill path): every token from ``start`` on is the argmax
+    """Teacher forcing through the target (resident, module by module on torch): every token from ``start`` on is the argmax
     of the logits at its prefix, or within what bf16 can tell apart of it (different tree shapes change the order of
     the attention sums, and this random model has many near-ties)."""
     kv = create_kv_cache("static", max_cache_len=512, config=CFG, device=DEV, dtype=torch.bfloat16)
     target, _, _ = build_models(CFG, kv, device=DEV, weights=weights)
+    target.use_native_layers = False
     logits = target.prefill(seq[:-1].to(DEV), 0, all_logits=True).float().cpu()      # row t scores token t + 1
     scale = logits.abs().amax().item()
     exact = 0
@@ -79,10 +80,11 @@ def test_v2_emits_what_v1_emits(agreeing, first_streamed):
         if steps == 0:
             assert torch.equal(out, ref)                     # without extension the two drivers are the same program
         assert kv.get_seq_length() == out.numel() - 1
-        # the cache holds the rows of the emitted sequence: compare with a fresh prefill of it
+        # the cache holds the rows of the emitted sequence: compare with a fresh prefill of it, module by module on torch
         L = kv.get_seq_length()
         kv2 = create_kv_cache("static", max_cache_len=512, config=CFG, device=DEV, dtype=torch.bfloat16)
         t2, _, _ = build_models(CFG, kv2, device=DEV, weights=w)
+        t2.use_native_layers = False
         t2.prefill(out[:-1].to(DEV), 0)
         a, b = kv.cache.data[..., :L, :].float(), kv2.cache.data[..., :L, :].float()
         assert (a - b).abs().amax().item() <= 5e-2 * b.abs().amax().item()
@@ -118,6 +120,7 @@ def test_deep_trees_beyond_one_window(cls, steps):
     assert L == out.numel() - 1
     kv2 = create_kv_cache("static", max_cache_len=512, config=CFG, device=DEV, dtype=torch.bfloat16)
     t2, _, _ = build_models(CFG, kv2, device=DEV, weights=w)
+    t2.use_native_layers = False
     t2.prefill(out[:-1].to(DEV), 0)
     a, b = kv.cache.data[..., :L, :].float(), kv2.cache.data[..., :L, :].float()
     assert (a - b).abs().amax().item() <= 5e-2 * b.abs().amax().item()
@@ -172,6 +175,7 @@ def test_v2_with_a_verify_cap_below_the_tree_size(verify):
     assert log["post_verify_count"] >= 2 and log["avg_sampled"] > 2.5, log
     kv2 = create_kv_cache("static", max_cache_len=512, config=CFG, device=DEV, dtype=torch.bfloat16)
     t2, _, _ = build_models(CFG, kv2, device=DEV, weights=w)
+    t2.use_native_layers = False
     t2.prefill(out[:-1].to(DEV), 0)
     a, b = kv.cache.data[..., :91, :].float(), kv2.cache.data[..., :91, :].float()
     assert (a - b).abs().amax().item() <= 5e-2 * b.abs().amax().item()

@@ -1,5 +1,5 @@
-"""GPU: the product decoder (bf16 target on one-call dense layers, int4 substitute draft on one-call int4
-layers, torch prefill) against a HuggingFace Qwen2 model with the same weights, called the way the
+"""GPU: the product decoder (bf16 target on one-call dense layers, its prefill included, int4 substitute draft on
+one-call int4 layers) against a HuggingFace Qwen2 model with the same weights, called the way the
 reference calls it: prefill into a KV cache, then the draft tree as one sequence with
 ``position_ids = prefix + depth`` and the additive ancestor mask
 (specdecodes/models/generators/classic_sd.py:75-109).  The HuggingFace side runs in fp32 on the CPU on

@@ -26,6 +26,7 @@ def _greedy_continuation(path, seq, start, tag):
     cfg, w = load_hf_checkpoint(path, device=DEV)
     kv = create_kv_cache("static", max_cache_len=512, config=cfg, device=DEV, dtype=torch.bfloat16)
     target, _, _ = build_models(cfg, kv, device=DEV, weights=w)
+    target.use_native_layers = False                                  # module by module on torch: none of the kernels under test
     logits = target.prefill(seq[:-1].to(DEV), 0, all_logits=True).float().cpu()
     scale, exact = logits.abs().amax().item(), 0
     for t in range(start - 1, seq.numel() - 1):

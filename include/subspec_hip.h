@@ -347,6 +347,11 @@ int subspec_int4_linear(const void* x, const uint32_t* wq, const uint32_t* sz, c
 int subspec_int4_gate_up_silu(const void* x, const uint32_t* wq, const uint32_t* sz, const void* bias, void* act,
                               int dtype, int64_t M, int64_t N, int64_t K, void* stream);
 
+/* How an int4 projection over 33 to 64 rows (gate_up != 0: the gate|up projection with its activation) is cut, for tests and
+ * tuning; host only.  plan = {index of the launch shape, workgroups per K range, K ranges}; returns 0, or SUBSPEC_ERR_LIMIT
+ * where these sizes take another kernel. */
+int subspec_int4_tile_plan(int64_t M, int64_t N, int64_t K, int gate_up, int32_t* plan);
+
 /* The same for a dense 16-bit gate|up weight W [2F, K] row-major (gate rows first), as the target's layers hold it:
  * 1 <= M <= 384; up to 32 rows 2F * K * 2 bytes must stay below 2 GiB. */
 int subspec_dense_gate_up_silu(const void* x, const void* w, const void* bias, void* act, int dtype, int64_t M,

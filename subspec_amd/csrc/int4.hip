@@ -26,7 +26,8 @@
 //           compute unit), where a pipeline of a few groups is bound by round trips, not by bytes.
 //           A K of more than 56 groups over at least 128 tiles (the down projection): int4_rows8_long_kernel, one
 //           workgroup per tile over the whole of K, in rounds whose registers refill while they are used.
-// M = 33-64, K a multiple of 256: int4_tile.hip, a workgroup's wavefronts share the activations.
+// M = 33-64, K a multiple of 256, more than a tile per compute unit or a long K (int4_tile_applies): int4_tile.hip, a
+//           workgroup's wavefronts share the activations.
 // M = 2-64: int4_gemm_kernel, v_mfma_f32_16x16x32 with the activations as A and the weight tile as
 //           B operand; the 32 k of one MFMA step all come from one quantization group, so the raw
 //           accumulator of a group is scaled once.  The wavefronts of a workgroup split K, their

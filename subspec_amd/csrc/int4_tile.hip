@@ -270,47 +270,57 @@ __global__ __launch_bounds__(512) void int4_tile_kernel(Int4TileParams p) {
 }
 
 // ------------------------------------------------------------------ launch shapes
-// Tiles of a wavefront, ring slots, and what a chunk takes with the chip full (us; measured with weights from HBM at 64 rows:
-// 4608 x 3584 12.9 us in one K range of shape 2, 3584 x 18944 27.2 in four ranges of shape 1 and 28.5 in eleven of shape 0,
-// 37888 x 3584 with the activation 38.3 in shape 0; int4_gemm_kernel: 18.2, 47.1 and 51.3 us).
+// Tiles of a wavefront, ring slots, and what a chunk takes with the chip full (us; see int4_tile_plan).
 #define SUBSPEC_INT4_TILE_SHAPES(X) \
-  X(0, 5, 2, 4, 2.00f)              \
-  X(1, 2, 3, 6, 0.90f)              \
-  X(2, 1, 3, 8, 0.65f)
+  X(0, 5, 2, 4, 2.10f)              \
+  X(1, 2, 3, 6, 1.05f)              \
+  X(2, 1, 3, 8, 0.60f)
 struct Int4TileShape { int ta; float chunk_us; };
 static constexpr Int4TileShape kInt4Shapes[] = {
 #define X(ID, TA, SX, SW, US) {TA, US},
     SUBSPEC_INT4_TILE_SHAPES(X)
 #undef X
 };
-struct Int4TilePlan { int shape, units, splits, chunks_per_split; };
-// Cheapest (shape, number of K ranges): 8 us for launch, first chunks and output, rounds of one workgroup per compute unit,
-// the sum over the ranges (a launch, or part of the consumer's) and its fp32 partials at 4.5 TB/s.
+struct Int4TilePlan { int shape, units, splits, chunks_per_split; float us; };
+// Cheapest (shape, number of K ranges): 4 us for the launch, rounds of one workgroup per compute unit with 2 us for first chunks
+// and output; the sum over the ranges 2 us (a launch, or part of the consumer's), 0.2 per range and its fp32 partials at
+// 4.5 TB/s.  Fitted to the times of every shape at 78 matrices (512 to 37888 rows of 512 to 18944, weights from HBM) and 33, 48
+// and 64 activation rows: the choice, int4_gemm_kernel included (below), takes 1.006 times the best one's time in the mean, 1.11 at
+// worst (4608 x 3584 shape 2 12.7 us, 3584 x 18944 shape 0 in eleven ranges 27.7, 37888 x 3584 with the activation shape 0 36.0).
+// gate|up never takes shape 2: one pair per workgroup is int4_gemm_kernel's case, several rounds of it lose to shape 1 or 0.
 static Int4TilePlan int4_tile_plan(int64_t M, int64_t N, int64_t K, bool silu) {
   Int4TilePlan best{};
-  float best_us = 1e30f;
+  best.us = 1e30f;
   const int chunks = (int)(K / 256);
   const int64_t cols = silu ? N / 32 : N / 16;
-  for (int i = 0; i < 3; ++i) {
+  for (int i = 0; i < (silu ? 2 : 3); ++i) {
     const int per = silu ? kInt4Shapes[i].ta : 2 * kInt4Shapes[i].ta;
     const int units = (int)((cols + per - 1) / per);
     for (int s = 1; s <= (silu ? 1 : 16); ++s) {
       const int cps = (chunks + s - 1) / s;
       if ((chunks + cps - 1) / cps != s) continue;
       const int64_t rounds = ((int64_t)units * s + 255) / 256;
-      float us = 8.f + (float)rounds * (float)cps * kInt4Shapes[i].chunk_us;
-      if (s > 1) us += 3.f + 2.f * (float)s * (float)M * (float)N * 4.f / 4.5e6f;
-      if (us < best_us) {
-        best_us = us;
-        best = Int4TilePlan{i, units, s, cps};
-      }
+      float us = 4.f + (float)rounds * (2.f + (float)cps * kInt4Shapes[i].chunk_us);
+      if (s > 1) us += 2.f + 0.2f * (float)s + 2.f * (float)s * (float)M * (float)N * 4.f / 4.5e6f;
+      if (us < best.us) best = Int4TilePlan{i, units, s, cps, us};
     }
   }
   return best;
 }
+// int4_gemm_kernel at the same row counts: rounds of one gate|up pair per workgroup and compute unit; a linear layer of up to 256
+// 16-row tiles and K in one range (beyond those it is 0 to 60 % behind at every size measured).
+static float int4_gemm_us(int64_t M, int64_t N, int64_t K, bool silu) {
+  const int64_t units = silu ? N / 32 : N / 16, groups = K / 64, rounds = (units + 255) / 256;
+  if (silu) return 2.5f + (float)rounds * (1.7f + 0.125f * (float)groups) * (rounds > 1 ? 1.f + 0.005f * (float)(M - 48) : 1.f);
+  return units <= 256 && groups < 112 ? 2.7f + 0.135f * (float)groups : 1e30f;
+}
 
+// Where sharing the activations pays, by the two estimates.  Few tiles of a short K are better off with a workgroup each, which
+// is done before the rings have filled: 3584 x 3584 10.2 us in int4_gemm_kernel against 12.7, 2048 x 2048 7.3 against 9.0,
+// 4096 x 4096 11.5 against 13.2.  With more, 4608 x 3584 15.2 against 13.3, 3584 x 18944 41 against 27, 37888 x 3584 with the
+// activation 46 against 36.
 bool int4_tile_applies(int64_t M, int64_t N, int64_t K, bool silu) {
-  return M > 32 && M <= 64 && K % 256 == 0 && N % (silu ? 32 : 16) == 0;
+  return M > 32 && M <= 64 && K % 256 == 0 && N % (silu ? 32 : 16) == 0 && int4_tile_plan(M, N, K, silu).us < int4_gemm_us(M, N, K, silu);
 }
 
 size_t int4_tile_workspace(int64_t M, int64_t N, int64_t K) {
@@ -326,8 +336,11 @@ static void launch_int4_tile(Int4TileParams p, const Int4TilePlan& pl, hipStream
   const dim3 grid((unsigned)(pl.units * pl.splits));
   DominantKernelTimer timer(st);
   switch (pl.shape) {
-#define X(ID, TA, SX, SW, US)                                                                        \
-  case ID: hipLaunchKernelGGL((int4_tile_kernel<DT, TA, SX, SW, SILU>), grid, dim3(512), 0, st, p); break;
+#define X(ID, TA, SX, SW, US)                                                                           \
+  case ID:                                                                                              \
+    if constexpr (!SILU || ID < 2)                                                                      \
+      hipLaunchKernelGGL((int4_tile_kernel<DT, TA, SX, SW, SILU>), grid, dim3(512), 0, st, p);          \
+    break;
     SUBSPEC_INT4_TILE_SHAPES(X)
 #undef X
   }
@@ -347,3 +360,13 @@ int int4_tile_linear(const void* x, const void* wq, const void* sz, const void* 
 }
 
 }  // namespace subspec
+
+extern "C" int subspec_int4_tile_plan(int64_t M, int64_t N, int64_t K, int gate_up, int32_t* plan) {
+  using namespace subspec;
+  if (!plan || M <= 0 || N <= 0 || K <= 0) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "int4_tile_plan: null pointer or empty size");
+  if (!int4_tile_applies(M, N, K, gate_up != 0))
+    SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "int4_tile_plan: M=%lld N=%lld K=%lld take another kernel", (long long)M, (long long)N, (long long)K);
+  const Int4TilePlan pl = int4_tile_plan(M, N, K, gate_up != 0);
+  plan[0] = pl.shape; plan[1] = pl.units; plan[2] = pl.splits;
+  return SUBSPEC_OK;
+}

@@ -1,12 +1,15 @@
 """GPU parity: int4 g64 linear (GEMV for M = 1, MFMA GEMM for M = 2..64) through the C ABI against
 x.float() @ ((Wq - z) * s).T on identical (Wq, scale, zero).  Tolerance 1e-2 relative
 (max |diff| <= 1e-2 * max |ref|, outputs rounded to the activation dtype)."""
+import ctypes
+
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 from oracle import int4 as oi
+from subspec_amd import _lib as L
 from subspec_amd import ops, quant
 
 DEV = "cuda:0"
@@ -185,7 +188,8 @@ def test_gate_up_projection_with_the_activation_in_its_output_stage(dtype):
                                    (3584, 18944, 41), (28672, 4096, 64), (12288, 256, 63)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_shared_activation_kernel(N, K, M, dtype):
-    """33 to 64 rows, K a multiple of 256: one chunk, fewer and more chunks than ring slots, partial last workgroups, K ranges."""
+    """33 to 64 rows, K a multiple of 256 (the small matrices take the other kernel): one chunk, fewer and more chunks than ring
+    slots, partial last workgroups, K ranges."""
     print("int4 tile", N, K, M, dtype, flush=True)
     g = torch.Generator(device=DEV).manual_seed(N + K + M)
     codes = torch.randint(0, 16, (N, K), generator=g, device=DEV, dtype=torch.uint8)
@@ -208,3 +212,39 @@ def test_shared_activation_kernel(N, K, M, dtype):
         # gate and up may each land on the neighbouring value of their type (silu' < 1.1): three roundings
         assert ((act - want).abs() <= 4 * 2 * ulp * want.abs() + 1.1 * (2 * ulp * gate.abs() + slack) * up.abs()
                 + (2 * ulp * up.abs() + slack) * gate.abs()).all()
+
+
+def _tile_plan(M, N, K, gate_up):
+    """(launch shape, K ranges) of the kernel whose wavefronts share the activations; None: another kernel"""
+    plan = (ctypes.c_int32 * 3)()
+    rc = L.lib().subspec_int4_tile_plan(M, N, K, gate_up, plan)
+    return None if rc else (plan[0], plan[2])
+
+
+# every launch shape with one chunk, fewer chunks than ring slots, as many, and more; K whole and split; partial last workgroups
+@pytest.mark.parametrize("M,N,K,shape,ranges", [
+    (33, 16848, 256, 0, 1), (64, 16848, 512, 0, 1), (47, 16848, 1280, 0, 1), (33, 5504, 5120, 0, 7), (33, 8304, 5120, 0, 4),
+    (64, 3584, 18944, 0, 11), (33, 8304, 256, 1, 1), (50, 8304, 512, 1, 1), (64, 8304, 768, 1, 1), (41, 8304, 2048, 1, 1),
+    (33, 2144, 8192, 1, 7), (33, 4160, 5120, 1, 3), (64, 4096, 14336, 1, 4), (33, 4160, 256, 2, 1), (64, 4160, 512, 2, 1),
+    (49, 4160, 768, 2, 1), (64, 4608, 3584, 2, 1), (33, 16, 5120, 2, 7), (33, 912, 18944, 2, 8), (64, 2048, 5632, 2, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_shape_of_the_shared_activation_kernel(M, N, K, shape, ranges, dtype):
+    assert _tile_plan(M, N, K, 0) == (shape, ranges)
+    test_shared_activation_kernel(N, K, M, dtype)
+
+
+@pytest.mark.parametrize("M,N,K,shape", [(33, 16864, 256, 0), (47, 16864, 512, 0), (33, 24704, 1280, 0), (64, 37888, 3584, 0),
+                                         (64, 8320, 256, 1), (60, 8320, 512, 1), (64, 8320, 768, 1), (64, 11264, 2048, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_shape_of_the_shared_activation_kernel_with_gate_up(M, N, K, shape, dtype):
+    assert _tile_plan(M, N, K, 1) == (shape, 1)
+    test_shared_activation_kernel(N, K, M, dtype)
+
+
+def test_few_tiles_of_a_short_k_take_a_workgroup_each():
+    """The sizes at which int4_gemm_kernel measured faster, 33 to 64 rows: up to 256 tiles (gate|up pairs) of K up to 4096."""
+    for M in (33, 48, 64):
+        for N in (2048, 3584, 4096):
+            for K in (256, 2048, 3584, 4096):
+                assert _tile_plan(M, N, K, 0) is None and _tile_plan(M, 2 * N, K, 1) is None
+        assert _tile_plan(M, 4608, 3584, 0) and _tile_plan(M, 3584, 18944, 0) and _tile_plan(M, 37888, 3584, 1)

@@ -352,7 +352,7 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
   X(0, 2, 4, 1, 4, 8, 3, 2, false, 1.55f)           \
   X(1, 4, 2, 1, 5, 5, 3, 2, false, 1.48f)           \
   X(2, 4, 2, 1, 5, 4, 3, 3, false, 1.10f)           \
-  X(3, 4, 2, 1, 5, 3, 4, 3, true, 0.95f)            \
+  X(3, 4, 2, 1, 5, 3, 4, 3, true, 0.925f)           \
   X(4, 4, 2, 1, 5, 2, 4, 4, true, 0.83f)            \
   X(5, 4, 2, 1, 4, 4, 3, 3, false, 0.90f)           \
   X(6, 2, 4, 1, 4, 4, 3, 3, false, 0.93f)           \
@@ -369,13 +369,18 @@ constexpr int kTileMaxSplits = 8;
 
 struct TilePlan { int shape, tiles_m, tiles_n, splits, chunks_per_split; };
 // Cheapest (shape, number of K ranges) under: 5.5 us for launch, first chunks and output; rounds of 256 workgroups, one
-// per compute unit, of chunk_us per chunk; never less than the weights take from HBM at 5.5 TB/s; fp32 partials written
-// and read back at 4.5 TB/s.  Within 7 % of the best measured shape on the matrices above.
+// per compute unit, of chunk_us per chunk; never less than the weights take from HBM at 6 TB/s; fp32 partials written
+// and read back at 4.5 TB/s.  Alone, over the four projections of three layer widths and 65 to 2048 rows (216 sizes), the choice
+// takes 1.02 times the best shape's time in the mean, 1.14 at worst at the widths of a 7B layer and 1.33 elsewhere (2048 x 2048 at
+// 512 rows, whose K ranges save less than their sum costs).  Constants fitted to those times (1.009, 1.12) lost up to 7 % in
+// whole layers, where the sums of the q|k|v and o projections are the next kernel's.  (5.5 TB/s here kept 3584 x 18944 at 95 to
+// 128 rows on a shape 14 % slower: 45.2 against 39.5 us at 128; 0.95 us for shape 3 kept 37888 x 3584 with the activation at 321
+// to 384 on one 7 % slower: 119 against 112 us at 384.)
 static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool silu) {
   TilePlan best{};
   float best_us = 1e30f;
   const int chunks = (int)(K / 64);
-  const float hbm_us = 8.f + (float)N * (float)K * 2.f / 5.5e6f;
+  const float hbm_us = 8.f + (float)N * (float)K * 2.f / 6.0e6f;
   for (int i = 0; i < kNumShapes; ++i) {
     const int64_t tm = (M + kShapes[i].bm - 1) / kShapes[i].bm, cols = silu ? N / 2 : N, bn = silu ? kShapes[i].bn / 2 : kShapes[i].bn;
     const int64_t tn = (cols + bn - 1) / bn;

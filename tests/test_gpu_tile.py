@@ -64,9 +64,9 @@ def _plan(M, N, K, gate_up):
     (129, 41536, 512, 0, 1, 1), (333, 22816, 512, 0, 2, 1), (129, 20736, 5632, 0, 1, 3), (333, 7296, 18944, 0, 2, 4),
     (257, 22816, 512, 1, 1, 1), (257, 7296, 5632, 1, 1, 5), (200, 33216, 512, 2, 1, 1), (200, 16576, 3584, 2, 1, 2),
     (129, 33216, 1024, 3, 1, 1), (129, 4736, 5632, 3, 1, 7), (65, 33216, 3584, 4, 1, 1), (257, 12416, 512, 4, 3, 1),
-    (65, 16576, 5632, 4, 1, 2), (300, 5856, 2048, 4, 3, 2), (129, 20736, 512, 5, 1, 1), (257, 14496, 512, 5, 2, 1),
-    (129, 4256, 3584, 5, 1, 6), (257, 3616, 3584, 5, 2, 4), (257, 16576, 512, 6, 3, 1), (257, 5536, 2048, 6, 3, 3),
-    (65, 16576, 640, 7, 1, 1), (257, 5536, 512, 7, 3, 1), (65, 5536, 5632, 7, 1, 4), (257, 2816, 2048, 7, 3, 3),
+    (65, 8256, 5632, 4, 1, 4), (300, 5856, 2048, 4, 3, 2), (129, 20736, 512, 5, 1, 1), (257, 14496, 512, 5, 2, 1),
+    (129, 4576, 3584, 5, 1, 6), (257, 3616, 3584, 5, 2, 4), (257, 16576, 512, 3, 2, 1), (257, 5536, 2048, 3, 2, 3), (257, 20736, 512, 6, 3, 1), (257, 6816, 2048, 6, 3, 3),
+    (65, 16576, 640, 7, 1, 1), (257, 5536, 512, 7, 3, 1), (65, 5536, 5632, 7, 1, 5), (257, 2816, 2048, 7, 3, 3),
     (65, 96, 512, 8, 1, 1), (129, 96, 512, 8, 2, 1), (65, 96, 1024, 8, 1, 2), (129, 96, 1024, 8, 2, 2),
     (300, 4608, 3584, 8, 3, 1), (300, 3584, 18944, 6, 3, 6)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -79,7 +79,7 @@ def test_every_shape_of_a_linear_layer(M, N, K, shape, row_tiles, ranges, dtype)
 @pytest.mark.parametrize("M,N,K,shape,row_tiles", [
     (129, 41536, 512, 0, 1), (333, 22816, 512, 0, 2), (333, 28672, 4096, 0, 2), (257, 22816, 512, 1, 1), (300, 37888, 3584, 1, 1),
     (200, 33216, 512, 2, 1), (129, 33216, 1024, 3, 1), (160, 37888, 3584, 3, 1), (100, 37888, 3584, 4, 1), (257, 12416, 512, 4, 3),
-    (129, 20736, 512, 5, 1), (257, 14496, 512, 5, 2), (200, 28672, 4096, 5, 1), (257, 16576, 512, 6, 3), (333, 37888, 3584, 6, 3),
+    (129, 20736, 512, 5, 1), (257, 14496, 512, 5, 2), (200, 28672, 4096, 5, 1), (257, 16576, 512, 3, 2), (333, 37888, 3584, 3, 2), (257, 20736, 512, 6, 3),
     (65, 16576, 640, 7, 1), (257, 5536, 512, 7, 3), (65, 96, 512, 8, 1), (129, 96, 512, 8, 2), (100, 11264, 2048, 8, 1)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_every_shape_of_gate_up(M, N, K, shape, row_tiles, dtype):

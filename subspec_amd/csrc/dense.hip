@@ -297,9 +297,10 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restri
 // registers r and r + 8 of one lane.
 // Measured on the four projections of a 7B layer, weights from HBM: M = 64 16.8 / 14.6 / 50.8 / 34.6 us (q|k|v, o,
 // gate|up with SwiGLU, down with its reduction; the 16 x 16 x 32 kernel above: 16.2 / 14.8 / 64.2 / 37.6); M = 289
-// 33 / 29 / 97 / 70 us (dense_tile_kernel: 20 / 16 / 88 / 58).  At 289 rows the kernel is bound by the activation copies: a chunk is 40 KB per workgroup, LDS
-// holds two of them beside three weight chunks, and one chunk in flight does not cover the L2 latency (M = 256 with
-// three activation slots: 79 us against 94 us with two).
+// 33 / 29 / 97 / 70 us (dense_tile_kernel alone 21.7 / 20.5 / 90 / 57.6; in a forward, behind cold caches and other kernels,
+// 25.6 / 17.8 + its sum in the norm / 94.6 / 54.4 + 7.5).  At 289 rows the kernel is bound by the activation copies: a chunk is
+// 40 KB per workgroup, LDS holds two of them beside three weight chunks, and one chunk in flight does not cover the L2 latency
+// (M = 256 with three activation slots: 79 us against 94 us with two).
 typedef float wd_v16f __attribute__((ext_vector_type(16)));
 typedef uint32_t wd_u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t wd_u2 __attribute__((ext_vector_type(2)));

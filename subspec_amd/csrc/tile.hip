@@ -20,8 +20,8 @@
 //   slots of each ring every chunk waits for a request to HBM (2500 cycles and more).  Three slots of both (256 x 160 at 256
 //   rows: 83 -> 73 us), or three of weights and two of activations with the weights requested half a chunk later (256 x 256,
 //   2048 rows: 490 -> 441 us), are what LDS holds.  Chunks of 32 k in twice as many slots lose (half-line requests).
-// 2048 rows: 441 us = 1.26 PFLOP/s with the activation included (library GEMM alone: 520 us; an 8192^3 product reaches
-// 1.38 PFLOP/s on this card), 289 rows: 87 us (dense_wide_kernel: 106), 128 rows: 54 us = 5.0 TB/s of weights.
+// 2048 rows: 441 to 458 us = 1.21 to 1.26 PFLOP/s with the activation included (library GEMM alone: 520 us; an 8192^3 product
+// reaches 1.38 PFLOP/s on this card), 289 rows: 90 us (dense_wide_kernel: 106), 128 rows: 57 us = 4.8 TB/s of weights.
 #include "dma.h"
 #include <algorithm>
 #include <type_traits>

@@ -153,7 +153,9 @@ __device__ __forceinline__ float warped(float x, const Divisor& temperature) {
 }
 // bf16(float(x / T)) == bf16(float(x * (1 / T))) for every x: a bf16 is one of 128 mantissas times a power of two, and both
 // roundings scale with that power while nothing leaves the normal range (T within 2^+-20; an overflow is infinite either way),
-// so the 128 mantissas decide.  They agree unless a quotient lies within an fp32 ulp of a bf16 midpoint: some 0.4 % of all T.
+// so the 128 mantissas decide.  They agree unless a quotient lies within an fp32 ulp of a bf16 midpoint: 0.05 % of all T in
+// [0.1, 2], but 14 of the 194 with two decimals from 0.05 to 1.99, 0.3, 0.6 and 1.2 among them (2048 x 152064, the whole call:
+// T = 0.8 328 us, T = 0.6 353; 399 and 397 with a division and an exponential per element).
 // (fp16 has 1024 mantissas and results in its subnormal range, fp32 no second rounding: they keep the division.)
 inline bool warp_by_product(int dtype, const Divisor& d) {
   if (dtype != SUBSPEC_BF16 || !(d.t >= 0x1p-20f && d.t <= 0x1p20f)) return false;

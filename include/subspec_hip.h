@@ -473,6 +473,26 @@ int subspec_dense_decoder_layer(const subspec_decoder_layer_dims* dims, const su
                                 void* x, const int32_t* positions, const int32_t* cache_rows, const uint64_t* anc_bits,
                                 void* k_cache, void* v_cache, void* workspace, size_t workspace_bytes, void* stream);
 
+/* n_layers decoder layers one after the other: what n_layers calls of the layer entry points with the same dims, x, positions,
+ * cache_rows, anc_bits and workspace do, bit for bit, with the launches between two layers joined (the reduction of a down
+ * projection, the residual sum and the next layer's RMSNorm).
+ *
+ * weights     host array [n_layers]; k_caches, v_caches: host arrays [n_layers] of device pointers (v_caches NULL: paged)
+ * final_norm  device [hidden], 16-byte aligned, or NULL; with it h_out [n_rows, hidden] receives the RMSNorm of the last
+ *             layer's output (the model's final norm).  x holds that output itself either way.
+ *
+ * Replaces  the loop over decoder layers and the final norm of the HuggingFace models that the draft and the target forward run
+ *           (specdecodes/models/draft_models/classic_sd.py:85-118, specdecodes/models/generators/classic_sd.py:75-109). */
+int subspec_int4_decoder_stack(const subspec_decoder_layer_dims* dims, const subspec_decoder_layer_weights* weights,
+                               int64_t n_layers, void* x, const int32_t* positions, const int32_t* cache_rows,
+                               const uint64_t* anc_bits, void* const* k_caches, void* const* v_caches, const void* final_norm,
+                               void* h_out, void* workspace, size_t workspace_bytes, void* stream);
+
+int subspec_dense_decoder_stack(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights,
+                                int64_t n_layers, void* x, const int32_t* positions, const int32_t* cache_rows,
+                                const uint64_t* anc_bits, void* const* k_caches, void* const* v_caches, const void* final_norm,
+                                void* h_out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* One decoder layer over a chunk of a prompt: the sequence of subspec_dense_decoder_layer with causal attention -- row i is
  * the token at cache row prefix_len + i (cache_rows[i] must say so) and sees every row up to its own.  1 <= n_rows <= 65536;
  * dims->n_tree_slots is ignored, dims->prefix_len_dev must be NULL.
@@ -483,6 +503,12 @@ size_t subspec_prefill_layer_workspace(const subspec_decoder_layer_dims* dims);
 int subspec_prefill_layer(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights, void* x,
                           const int32_t* positions, const int32_t* cache_rows, void* k_cache, void* v_cache, void* workspace,
                           size_t workspace_bytes, void* stream);
+
+/* n_layers of them, as subspec_dense_decoder_stack */
+int subspec_prefill_stack(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights, int64_t n_layers,
+                          void* x, const int32_t* positions, const int32_t* cache_rows, void* const* k_caches,
+                          void* const* v_caches, const void* final_norm, void* h_out, void* workspace, size_t workspace_bytes,
+                          void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * RMSNorm of [rows, hidden] activations in one launch: y = weight * round(x * rsqrt(mean(x^2) + eps)), the sum

@@ -130,6 +130,16 @@ __device__ __forceinline__ void unpack8(dec_u4 v, float* f) {
   }
 }
 template <int DT>
+__device__ __forceinline__ void unpack2(uint32_t v, float* f) {
+  if constexpr (DT == SUBSPEC_BF16) {
+    f[0] = bf16_bits_to_float(v & 0xffffu);
+    f[1] = bf16_bits_to_float(v >> 16);
+  } else {
+    f[0] = f16_bits_to_float(v & 0xffffu);
+    f[1] = f16_bits_to_float(v >> 16);
+  }
+}
+template <int DT>
 __device__ __forceinline__ uint32_t to_bits(float v) {
   if constexpr (DT == SUBSPEC_BF16) {
     return __float_as_uint(round_bf16(v)) >> 16;

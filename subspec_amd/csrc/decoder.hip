@@ -28,47 +28,84 @@
 namespace subspec {
 
 // x[m] (+= delta[m], rounded, written back) ; y[m] = w * round(x * rsqrt(mean(x^2) + eps))
-// One workgroup per row; H % 8 == 0.  kMaxPieces 16-byte pieces per thread cover H <= 256 * 8 * kMaxPieces.
+// One workgroup per row; H % 8 == 0, P 16-byte pieces per thread cover H <= 512 * 8 * P.
 // splits > 0: delta is not a 16-bit tensor yet but `splits` fp32 partial sums [splits][rows][H] of a projection whose K
 // was split over workgroups; they are summed in split order and rounded here (what the projection's own reduction
 // launch would have stored), which saves that launch.
-constexpr int kNormThreads = 256;
-constexpr int kNormMaxPieces = 8;
-template <int DT, bool kAdd>
+// A launch of this size is a chain of memory round trips and nothing else, so there is ONE before the sum of squares: the row, the
+// gain and four partials at a time are requested together.  In the
+// target's forward over 64 rows, with the partials of the o projection: 5.4 us with the gain behind the sum and the partials one
+// after the other, 4.9 now (289 rows 6.0, with six partials of the down projection as well 7.5); an empty launch takes 3.0.
+constexpr int kNormThreads = 512;
+constexpr int kNormMaxPieces = 4;
+template <int DT, bool kAdd, int P>
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(uint16_t* __restrict__ x, const uint16_t* __restrict__ delta,
                                                                    const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
-                                                                   int H, float eps, const float* __restrict__ partial = nullptr,
-                                                                   int splits = 0) {
+                                                                   int H, float eps, const float* __restrict__ partial,
+                                                                   int splits) {
   __shared__ float scratch[kNormThreads / kWave];
   const int m = blockIdx.x, tid = threadIdx.x, pieces = H / 8;
   dec_u4* xr = (dec_u4*)(x + (int64_t)m * H);
-  const dec_u4* dr = (const dec_u4*)(delta + (int64_t)m * H);
-  float v[kNormMaxPieces][8];
-  float ss = 0.f;
+  dec_u4 xv[P], gain[P];
+  float v[P][8];
 #pragma unroll
-  for (int p = 0; p < kNormMaxPieces; ++p) {
-    const int i = p * kNormThreads + tid;
-    if (i < pieces) {
-      unpack8<DT>(xr[i], v[p]);
-      if constexpr (kAdd) {
-        float d[8];
-        if (splits > 0) {
+  for (int p = 0; p < P; ++p) {
+    const int i = min(p * kNormThreads + tid, pieces - 1);
+    xv[p] = xr[i];
+    gain[p] = ((const dec_u4*)w)[i];
+  }
+  if constexpr (kAdd) {
+    if (splits > 0) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) d[j] = 0.f;
-          for (int sp = 0; sp < splits; ++sp) {
-            const float4* pp = (const float4*)(partial + ((int64_t)sp * gridDim.x + m) * H) + 2 * i;
-            const float4 a = pp[0], b = pp[1];
-            d[0] += a.x; d[1] += a.y; d[2] += a.z; d[3] += a.w; d[4] += b.x; d[5] += b.y; d[6] += b.z; d[7] += b.w;
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[p][j] = 0.f;
+      for (int s0 = 0; s0 < splits; s0 += 4) {
+        float4 q[P][4][2];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const int i = min(p * kNormThreads + tid, pieces - 1);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const float4* pp = (const float4*)(partial + ((int64_t)min(s0 + s, splits - 1) * gridDim.x + m) * H) + 2 * i;
+            q[p][s][0] = pp[0];
+            q[p][s][1] = pp[1];
           }
-#pragma unroll
-          for (int j = 0; j < 8; ++j) d[j] = Elem<DT>::round(d[j]);
-        } else {
-          unpack8<DT>(dr[i], d);
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[p][j] = Elem<DT>::round(v[p][j] + d[j]);
-        xr[i] = pack8<DT>(v[p]);
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            if (s0 + s < splits) {
+              const float4 a = q[p][s][0], b = q[p][s][1];
+              v[p][0] += a.x; v[p][1] += a.y; v[p][2] += a.z; v[p][3] += a.w;
+              v[p][4] += b.x; v[p][5] += b.y; v[p][6] += b.z; v[p][7] += b.w;
+            }
       }
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[p][j] = Elem<DT>::round(v[p][j]);
+    } else {
+#pragma unroll
+      for (int p = 0; p < P; ++p) unpack8<DT>(((const dec_u4*)(delta + (int64_t)m * H))[min(p * kNormThreads + tid, pieces - 1)], v[p]);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int i = p * kNormThreads + tid;
+    float xf[8];
+    unpack8<DT>(xv[p], xf);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[p][j] = kAdd ? Elem<DT>::round(xf[j] + v[p][j]) : xf[j];
+      // an fp16 value is taken as a float from here on: both forms of the kernel then compile to the same products (left to itself
+      // the compiler folds the widening into mixed-precision ones in one of them, which round once instead of twice)
+      if constexpr (DT == SUBSPEC_F16) asm volatile("" : "+v"(v[p][j]));
+    }
+    if (i < pieces) {
+      if constexpr (kAdd) xr[i] = pack8<DT>(v[p]);
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss = fmaf(v[p][j], v[p][j], ss);
     }
@@ -76,16 +113,33 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(uint16_t* __r
   const float tot = block_sum<kNormThreads>(ss, scratch);
   const float r = rsqrtf(tot / (float)H + eps);
 #pragma unroll
-  for (int p = 0; p < kNormMaxPieces; ++p) {
+  for (int p = 0; p < P; ++p) {
     const int i = p * kNormThreads + tid;
     if (i < pieces) {
       float wv[8], o[8];
-      unpack8<DT>(((const dec_u4*)w)[i], wv);
+      unpack8<DT>(gain[p], wv);
 #pragma unroll
       for (int j = 0; j < 8; ++j) o[j] = wv[j] * Elem<DT>::round(v[p][j] * r);
       ((dec_u4*)(y + (int64_t)m * H))[i] = pack8<DT>(o);
     }
   }
+}
+// delta null and splits 0: a plain RMSNorm (x is only read)
+template <int DT>
+static void launch_norm(uint16_t* x, const uint16_t* delta, const void* w, uint16_t* y, int64_t rows, int H, float eps,
+                        const float* partial, int splits, hipStream_t st) {
+#define SUBSPEC_NORM(ADD, P)                                                                                                       \
+  hipLaunchKernelGGL((add_rmsnorm_kernel<DT, ADD, P>), dim3((unsigned)rows), dim3(kNormThreads), 0, st, x, delta, (const uint16_t*)w, \
+                     y, H, eps, partial, splits)
+  const bool one = H <= 8 * kNormThreads;
+  if (delta || splits > 0) {
+    if (one) SUBSPEC_NORM(true, 1);
+    else SUBSPEC_NORM(true, kNormMaxPieces);
+  } else {
+    if (one) SUBSPEC_NORM(false, 1);
+    else SUBSPEC_NORM(false, kNormMaxPieces);
+  }
+#undef SUBSPEC_NORM
 }
 
 // act[m, f] = round(silu(gate)) * up with gate = gu[m, f], up = gu[m, F + f]
@@ -107,61 +161,109 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 
 // Rotary embedding (rotate-half form, angle = position * theta^(-2i/D)) of the q and k heads of
 // qkv [M, (Hq + 2 Hkv) * D]; q goes to q_out [Hq, M, D], k and v to rows cache_rows[m] of the
-// layer's [Hkv, S, D] caches.  One wavefront per (row, head); lane i handles dims i and i + D/2.
+// layer's [Hkv, S, D] caches (D = 128).
 // splits > 0: qkv is still `splits` fp32 partial sums [splits][M][(Hq + 2 Hkv) * D] of the projection (K split over
 // workgroups) and `bias` its bias; sum, bias and the rounding to the activation dtype happen here instead of in a
 // reduction launch of their own.
+// A thread takes dims i, i + 1 and their partners D/2 further, 32 lanes a head, eight heads a workgroup; blockIdx.y strides over
+// the groups of eight, so that many rows evaluate their angles once per thread and not once per head.  Bound by launch and round
+// trips up to a few hundred rows (64: 4.8 -> 4.7 us, 256: 7.4 -> 6.2 against one wavefront per (row, head)), then by its 38 MB:
+// 2048 rows of 36 heads 19.7 -> 11.8 us.
+constexpr int kRopeHeads = 8;
 template <int DT>
-__global__ __launch_bounds__(64) void rope_write_kernel(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,
-                                                        const int32_t* __restrict__ cache_rows, uint16_t* __restrict__ q_out,
-                                                        KvRowMap kv, int M, int Hq, int Hkv, int D, float log2_theta,
-                                                        const float* __restrict__ inv_freq_table,
-                                                        const float* __restrict__ partial = nullptr, int splits = 0,
-                                                        const uint16_t* __restrict__ bias = nullptr) {
-  const int m = blockIdx.x, hh = blockIdx.y, i = threadIdx.x;
-  const int half = D / 2;
-  if (i >= half) return;
-  float lo, hi;
-  if (splits > 0) {
-    const int64_t width = (int64_t)(Hq + 2 * Hkv) * D, col = (int64_t)hh * D + i;
-    lo = hi = 0.f;
-    for (int sp = 0; sp < splits; ++sp) {
-      const float* pp = partial + ((int64_t)sp * M + m) * width + col;
-      lo += pp[0];
-      hi += pp[half];
-    }
-    lo = Elem<DT>::round(lo + (bias ? Elem<DT>::load(bias, col) : 0.f));
-    hi = Elem<DT>::round(hi + (bias ? Elem<DT>::load(bias, col + half) : 0.f));
-  } else {
-    const uint16_t* src = qkv + ((int64_t)m * (Hq + 2 * Hkv) + hh) * D;
-    lo = Elem<DT>::load(src, i);
-    hi = Elem<DT>::load(src, i + half);
-  }
-  uint16_t* dst;
-  if (hh < Hq) {
-    dst = q_out + ((int64_t)hh * M + m) * D;
-  } else {
-    // a row outside the layer's cache is dropped: a bad rows tensor must not write beyond the cache
-    uint16_t *kp, *vp;
-    if (!kv_row_ptrs(kv, (hh - Hq) % Hkv, cache_rows[m], &kp, &vp)) return;
-    dst = hh < Hq + Hkv ? kp : vp;
-  }
-  if (hh >= Hq + Hkv) {                                 // value heads are copied
-    Elem<DT>::store(dst, i, lo);
-    Elem<DT>::store(dst, i + half, hi);
-    return;
-  }
+__global__ __launch_bounds__(32 * kRopeHeads) void rope_write_kernel(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,
+                                                                     const int32_t* __restrict__ cache_rows, uint16_t* __restrict__ q_out,
+                                                                     KvRowMap kv, int M, int Hq, int Hkv, float log2_theta,
+                                                                     const float* __restrict__ inv_freq_table,
+                                                                     const float* __restrict__ partial, int splits,
+                                                                     const uint16_t* __restrict__ bias) {
+  constexpr int D = 128, half = D / 2;
+  const int m = blockIdx.x, i = 2 * (threadIdx.x & 31), heads = Hq + 2 * Hkv;
+  const int64_t width = (int64_t)heads * D;
+  const int pos = positions[m], cache_row = cache_rows[m];
   // the caller's table (the values its other code paths use, so that both write identical rows), else theta^(-2i/D)
-  const float inv_freq = inv_freq_table ? inv_freq_table[i] : exp2f(-(float)(2 * i) / (float)D * log2_theta);
-  float s, c;
-  sincosf((float)positions[m] * inv_freq, &s, &c);
-  c = Elem<DT>::round(c);
-  s = Elem<DT>::round(s);
-  // t * cos + rotate_half(t) * sin, each product and the sum rounded like the eager tensor ops
-  const float o_lo = Elem<DT>::round(lo * c) + Elem<DT>::round(-hi * s);
-  const float o_hi = Elem<DT>::round(hi * c) + Elem<DT>::round(lo * s);
-  Elem<DT>::store(dst, i, o_lo);
-  Elem<DT>::store(dst, i + half, o_hi);
+  float freq[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) freq[e] = inv_freq_table ? inv_freq_table[i + e] : exp2f(-(float)(2 * (i + e)) / (float)D * log2_theta);
+  float c[2], s[2];
+  bool angles = false;
+  for (int hh = blockIdx.y * kRopeHeads + (threadIdx.x >> 5); hh < heads; hh += gridDim.y * kRopeHeads) {
+    const int64_t col = (int64_t)hh * D + i;
+    // the head's elements (or its first four partials) are requested, the angles evaluated while they travel
+    uint32_t raw[2] = {0, 0};
+    float bl[2] = {0.f, 0.f}, bh[2] = {0.f, 0.f};
+    dec_f2 a[4], b[4];
+    auto request = [&](int s0) {
+#pragma unroll
+      for (int sp = 0; sp < 4; ++sp) {
+        const float* pp = partial + ((int64_t)min(s0 + sp, splits - 1) * M + m) * width + col;
+        a[sp] = *(const dec_f2*)pp;
+        b[sp] = *(const dec_f2*)(pp + half);
+      }
+    };
+    if (splits > 0) {
+      request(0);
+      if (bias) {                                       // (element loads: the bias may lie at any even address)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          bl[e] = Elem<DT>::load(bias, col + e);
+          bh[e] = Elem<DT>::load(bias, col + half + e);
+        }
+      }
+    } else {
+      const uint16_t* src = qkv + (int64_t)m * width + col;
+      raw[0] = *(const uint32_t*)src;
+      raw[1] = *(const uint32_t*)(src + half);
+    }
+    if (!angles) {
+      angles = true;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        sincosf((float)pos * freq[e], &s[e], &c[e]);
+        c[e] = Elem<DT>::round(c[e]);
+        s[e] = Elem<DT>::round(s[e]);
+      }
+    }
+    float lo[2], hi[2];
+    if (splits > 0) {
+      lo[0] = lo[1] = hi[0] = hi[1] = 0.f;
+      for (int s0 = 0;;) {
+#pragma unroll
+        for (int sp = 0; sp < 4; ++sp)
+          if (s0 + sp < splits) { lo[0] += a[sp][0]; lo[1] += a[sp][1]; hi[0] += b[sp][0]; hi[1] += b[sp][1]; }
+        if ((s0 += 4) >= splits) break;
+        request(s0);
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        lo[e] = Elem<DT>::round(lo[e] + bl[e]);
+        hi[e] = Elem<DT>::round(hi[e] + bh[e]);
+      }
+    } else {
+      unpack2<DT>(raw[0], lo);
+      unpack2<DT>(raw[1], hi);
+    }
+    uint16_t* dst;
+    if (hh < Hq) {
+      dst = q_out + ((int64_t)hh * M + m) * D;
+    } else {
+      // a row outside the layer's cache is dropped: a bad rows tensor must not write beyond the cache
+      uint16_t *kp, *vp;
+      if (!kv_row_ptrs(kv, (hh - Hq) % Hkv, cache_row, &kp, &vp)) continue;
+      dst = hh < Hq + Hkv ? kp : vp;
+    }
+    if (hh < Hq + Hkv) {                                  // value heads are copied
+      // t * cos + rotate_half(t) * sin, each product and the sum rounded like the eager tensor ops
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float a = lo[e], b = hi[e];
+        lo[e] = Elem<DT>::round(a * c[e]) + Elem<DT>::round(-b * s[e]);
+        hi[e] = Elem<DT>::round(b * c[e]) + Elem<DT>::round(a * s[e]);
+      }
+    }
+    *(uint32_t*)(dst + i) = pack2<DT>(lo[0], lo[1]);
+    *(uint32_t*)(dst + i + half) = pack2<DT>(hi[0], hi[1]);
+  }
 }
 
 // Rows 0 .. rows - 1 of a paged layer as contiguous [Hkv, rows, 128] K and V: a prefill's attention reads every row many
@@ -256,6 +358,18 @@ struct LayerWeights {
   Projection qkv, o, gate_up, down;
   bool dense;
 };
+static LayerWeights layer_weights(const subspec_decoder_layer_weights& s) {
+  return {s.input_norm, s.post_norm, s.qkv_bias, {s.qkv_wq, s.qkv_sz}, {s.o_wq, s.o_sz}, {s.gate_up_wq, s.gate_up_sz},
+          {s.down_wq, s.down_sz}, false};
+}
+static LayerWeights layer_weights(const subspec_dense_layer_weights& s) {
+  return {s.input_norm, s.post_norm, s.qkv_bias, {s.qkv_w, nullptr}, {s.o_w, nullptr}, {s.gate_up_w, nullptr}, {s.down_w, nullptr}, true};
+}
+// int4 layers of up to 32 rows: norms and rotary are prologues and output stages of the projections
+static bool int4_norm_prologue(const subspec_decoder_layer_dims& s, bool dense) {
+  return !dense && s.n_rows <= 32 &&
+         subspec_int4_linear_workspace(s.n_rows, (s.n_q_heads + 2 * s.n_kv_heads) * s.head_dim, s.hidden) == 256;
+}
 static int project(const LayerWeights& w, const Projection& p, const void* x, const void* bias, const void* residual, void* y,
                    int dtype, int64_t M, int64_t N, int64_t K, void* sub, size_t sub_bytes, hipStream_t st,
                    int* pending_splits = nullptr) {
@@ -264,10 +378,19 @@ static int project(const LayerWeights& w, const Projection& p, const void* x, co
   return int4_linear_ex(x, (const uint32_t*)p.w, (const uint32_t*)p.sz, bias, residual, y, dtype, M, N, K, 64, sub, sub_bytes, st, pending_splits);
 }
 
+// What a layer of a stack takes over from the one before it and leaves to the next: the down projection's residual sum, the
+// reduction of its fp32 partials and the NEXT RMSNorm are one launch (add_rmsnorm_kernel) instead of two, so a layer of a stack
+// ends with its successor's normalized input.  64 dense rows: 4.7 + 4.8 -> 4.9 us a layer, 2048 rows 20.2 + 7.8 -> 11.4.  The
+// same sums in the same order, the same bits.
+struct StackLink {
+  bool h_ready = false;               // the workspace's h holds this layer's normalized input already
+  const uint16_t* next_norm = nullptr;   // gain of the next RMSNorm, or null: x alone is wanted
+  uint16_t* h_next = nullptr;         // where its output goes; null: the workspace's h
+};
 template <int DT>
 static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w, uint16_t* x,
                      const int32_t* positions, const int32_t* cache_rows, const uint64_t* anc_bits, uint16_t* k_cache,
-                     uint16_t* v_cache, char* ws, hipStream_t st, bool causal = false) {
+                     uint16_t* v_cache, char* ws, hipStream_t st, bool causal = false, StackLink link = {}) {
   const LayerPlan p = layer_plan(s, causal);
   const int M = (int)s.n_rows, H = (int)s.hidden, Hq = (int)s.n_q_heads, Hkv = (int)s.n_kv_heads, D = (int)s.head_dim,
             F = (int)s.intermediate;
@@ -282,20 +405,22 @@ static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w,
   // int4 stack, a level of at most 32 rows: five launches per layer (six with a split-K down projection, seven when
   // the keys are split) -- both norms are prologues of the projections that consume them, rotary + cache write is the
   // output stage of q|k|v, the attention block's residual add the output stage of o_proj
-  const bool fused = !w.dense && M <= 32 && subspec_int4_linear_workspace(M, Q + 2 * KV, H) == 256;
+  const bool fused = int4_norm_prologue(s, w.dense);
   if (fused) {
     if ((rc = int4_qkv_rope_ex(x, (const uint32_t*)w.qkv.w, (const uint32_t*)w.qkv.sz, w.qkv_bias, DT, M, H, w.input_norm, s.rms_eps,
                                positions, cache_rows, q, kv, Hq, s.rope_theta, s.rope_inv_freq, st)))
       return rc;
   } else {
-    hipLaunchKernelGGL((add_rmsnorm_kernel<DT, false>), dim3(M), dim3(kNormThreads), 0, st, x, (const uint16_t*)nullptr,
-                       (const uint16_t*)w.input_norm, h, H, s.rms_eps);
+    if (!link.h_ready)
+      launch_norm<DT>(x, nullptr, w.input_norm, h, M, H, s.rms_eps, nullptr, 0, st);
     // projections whose K is split leave the sum of their partials to the kernel that reads them next
     int pending = 0;
     if ((rc = project(w, w.qkv, h, w.qkv_bias, nullptr, qkv, DT, M, Q + 2 * KV, H, sub, p.sub_bytes, st, &pending))) return rc;
-    hipLaunchKernelGGL((rope_write_kernel<DT>), dim3(M, Hq + 2 * Hkv), dim3(64), 0, st, qkv, positions, cache_rows, q, kv,
-                       M, Hq, Hkv, D, log2f(s.rope_theta), s.rope_inv_freq, (const float*)sub, pending > 1 ? pending : 0,
-                       (const uint16_t*)w.qkv_bias);
+    // few rows: a workgroup per eight heads; from 512 rows a workgroup per row fills the chip and walks all heads
+    const int head_groups = (Hq + 2 * Hkv + kRopeHeads - 1) / kRopeHeads;
+    hipLaunchKernelGGL((rope_write_kernel<DT>), dim3(M, M >= 512 ? 1 : head_groups), dim3(32 * kRopeHeads), 0, st, qkv, positions,
+                       cache_rows, q, kv, M, Hq, Hkv, log2f(s.rope_theta), s.rope_inv_freq, (const float*)sub,
+                       pending > 1 ? pending : 0, (const uint16_t*)w.qkv_bias);
   }
   if (causal) {
     const int64_t rows = s.prefix_len + M;
@@ -320,8 +445,7 @@ static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w,
   } else {
   int pending = 0;
   if ((rc = project(w, w.o, a, nullptr, nullptr, o, DT, M, H, Q, sub, p.sub_bytes, st, &pending))) return rc;
-  hipLaunchKernelGGL((add_rmsnorm_kernel<DT, true>), dim3(M), dim3(kNormThreads), 0, st, x, o, (const uint16_t*)w.post_norm, h, H,
-                     s.rms_eps, (const float*)sub, pending > 1 ? pending : 0);
+  launch_norm<DT>(x, o, w.post_norm, h, M, H, s.rms_eps, (const float*)sub, pending > 1 ? pending : 0, st);
   if (!w.dense) {
     // the activation sits in the output stage of the gate|up projection
     if ((rc = int4_gate_up_silu_ex(h, (const uint32_t*)w.gate_up.w, (const uint32_t*)w.gate_up.sz, nullptr, act, DT, M,
@@ -336,8 +460,34 @@ static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w,
   }
   }
   // down projection with the residual add in its output stage: x = round(round(down(act)) + x)
-  if ((rc = project(w, w.down, act, nullptr, x, x, DT, M, H, F, sub, p.sub_bytes, st))) return rc;
+  int down_splits = 0;
+  if ((rc = project(w, w.down, act, nullptr, x, x, DT, M, H, F, sub, p.sub_bytes, st, link.next_norm ? &down_splits : nullptr))) return rc;
+  if (link.next_norm) {
+    uint16_t* hn = link.h_next ? link.h_next : h;
+    launch_norm<DT>(x, nullptr, link.next_norm, hn, M, H, s.rms_eps, (const float*)sub, down_splits > 1 ? down_splits : 0, st);
+  }
   SUBSPEC_CHECK_HIP(hipGetLastError());
+  return SUBSPEC_OK;
+}
+
+// The layers of a stack one after the other; h_out (with final_norm): RMSNorm of the last layer's output
+template <int DT, typename Weights>
+static int run_stack(const subspec_decoder_layer_dims& s, const Weights* layers, int64_t n_layers, uint16_t* x,
+                     const int32_t* positions, const int32_t* cache_rows, const uint64_t* anc_bits, void* const* k_caches,
+                     void* const* v_caches, const void* final_norm, void* h_out, char* ws, hipStream_t st, bool causal) {
+  StackLink link;
+  for (int64_t i = 0; i < n_layers; ++i) {
+    const LayerWeights w = layer_weights(layers[i]);
+    const bool last = i + 1 == n_layers;
+    // (an int4 layer of up to 32 rows has its norm inside the q|k|v projection: it only takes a final norm behind the stack)
+    const bool own_norm = int4_norm_prologue(s, w.dense);
+    link.next_norm = last ? (const uint16_t*)final_norm : own_norm ? nullptr : (const uint16_t*)layer_weights(layers[i + 1]).input_norm;
+    link.h_next = last ? (uint16_t*)h_out : nullptr;
+    const int rc = run_layer<DT>(s, w, x, positions, cache_rows, anc_bits, (uint16_t*)k_caches[i],
+                                 v_caches ? (uint16_t*)v_caches[i] : nullptr, ws, st, causal, link);
+    if (rc != SUBSPEC_OK) return rc;
+    link.h_ready = link.next_norm != nullptr;
+  }
   return SUBSPEC_OK;
 }
 
@@ -357,12 +507,8 @@ extern "C" int subspec_rms_norm(const void* x, const void* weight, void* y, int 
   if ((uintptr_t)x % 16 || (uintptr_t)weight % 16 || (uintptr_t)y % 16) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "rms_norm: pointers must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   // the kernel only writes x when it also adds: here it reads it
-  if (dtype == SUBSPEC_BF16)
-    hipLaunchKernelGGL((add_rmsnorm_kernel<SUBSPEC_BF16, false>), dim3((unsigned)rows), dim3(kNormThreads), 0, st, (uint16_t*)x,
-                       (const uint16_t*)nullptr, (const uint16_t*)weight, (uint16_t*)y, (int)hidden, eps);
-  else
-    hipLaunchKernelGGL((add_rmsnorm_kernel<SUBSPEC_F16, false>), dim3((unsigned)rows), dim3(kNormThreads), 0, st, (uint16_t*)x,
-                       (const uint16_t*)nullptr, (const uint16_t*)weight, (uint16_t*)y, (int)hidden, eps);
+  if (dtype == SUBSPEC_BF16) launch_norm<SUBSPEC_BF16>((uint16_t*)x, nullptr, weight, (uint16_t*)y, rows, (int)hidden, eps, nullptr, 0, st);
+  else launch_norm<SUBSPEC_F16>((uint16_t*)x, nullptr, weight, (uint16_t*)y, rows, (int)hidden, eps, nullptr, 0, st);
   SUBSPEC_CHECK_HIP(hipGetLastError());
   return SUBSPEC_OK;
 }
@@ -372,9 +518,9 @@ extern "C" size_t subspec_int4_decoder_layer_workspace(const subspec_decoder_lay
   return layer_plan(*dims).total;
 }
 
-static int decoder_layer_entry(const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* x, const int32_t* positions,
-                               const int32_t* cache_rows, const uint64_t* anc_bits, void* k_cache, void* v_cache,
-                               void* workspace, size_t workspace_bytes, void* stream) {
+static int check_layer_call(const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* x, const int32_t* positions,
+                            const int32_t* cache_rows, const uint64_t* anc_bits, void* k_cache, void* v_cache,
+                            void* workspace, size_t workspace_bytes) {
   const int rc = check_dims(dims, w.dense ? kDenseLayerMaxRows : kInt4LayerMaxRows);
   if (rc != SUBSPEC_OK) return rc;
   // the wide dense kernels take weight rows in tiles of 32
@@ -392,6 +538,14 @@ static int decoder_layer_entry(const subspec_decoder_layer_dims* dims, const Lay
   if (!workspace || workspace_bytes < need)
     SUBSPEC_FAIL(SUBSPEC_ERR_WORKSPACE, "decoder_layer: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
   if ((uintptr_t)workspace % 256) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: workspace must be 256-byte aligned");
+  return SUBSPEC_OK;
+}
+
+static int decoder_layer_entry(const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* x, const int32_t* positions,
+                               const int32_t* cache_rows, const uint64_t* anc_bits, void* k_cache, void* v_cache,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  const int rc = check_layer_call(dims, w, x, positions, cache_rows, anc_bits, k_cache, v_cache, workspace, workspace_bytes);
+  if (rc != SUBSPEC_OK) return rc;
   if (dims->dtype == SUBSPEC_BF16)
     return run_layer<SUBSPEC_BF16>(*dims, w, (uint16_t*)x, positions, cache_rows, anc_bits, (uint16_t*)k_cache, (uint16_t*)v_cache,
                                    (char*)workspace, (hipStream_t)stream);
@@ -404,10 +558,7 @@ extern "C" int subspec_int4_decoder_layer(const subspec_decoder_layer_dims* dims
                                           const uint64_t* anc_bits, void* k_cache, void* v_cache, void* workspace,
                                           size_t workspace_bytes, void* stream) {
   if (!weights) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: null weights");
-  const subspec_decoder_layer_weights& s = *weights;
-  const LayerWeights w{s.input_norm, s.post_norm, s.qkv_bias, {s.qkv_wq, s.qkv_sz}, {s.o_wq, s.o_sz},
-                       {s.gate_up_wq, s.gate_up_sz}, {s.down_wq, s.down_sz}, false};
-  return decoder_layer_entry(dims, w, x, positions, cache_rows, anc_bits, k_cache, v_cache, workspace, workspace_bytes, stream);
+  return decoder_layer_entry(dims, layer_weights(*weights), x, positions, cache_rows, anc_bits, k_cache, v_cache, workspace, workspace_bytes, stream);
 }
 
 extern "C" int subspec_dense_decoder_layer(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights,
@@ -415,10 +566,51 @@ extern "C" int subspec_dense_decoder_layer(const subspec_decoder_layer_dims* dim
                                            const uint64_t* anc_bits, void* k_cache, void* v_cache, void* workspace,
                                            size_t workspace_bytes, void* stream) {
   if (!weights) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: null weights");
-  const subspec_dense_layer_weights& s = *weights;
-  const LayerWeights w{s.input_norm, s.post_norm, s.qkv_bias, {s.qkv_w, nullptr}, {s.o_w, nullptr},
-                       {s.gate_up_w, nullptr}, {s.down_w, nullptr}, true};
-  return decoder_layer_entry(dims, w, x, positions, cache_rows, anc_bits, k_cache, v_cache, workspace, workspace_bytes, stream);
+  return decoder_layer_entry(dims, layer_weights(*weights), x, positions, cache_rows, anc_bits, k_cache, v_cache, workspace,
+                             workspace_bytes, stream);
+}
+
+static int check_stack_args(const void* weights, int64_t n_layers, void* const* k_caches, const void* final_norm, const void* h_out) {
+  if (!weights || !k_caches || n_layers < 1) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_stack: null pointer argument or no layers");
+  if (!final_norm != !h_out || (uintptr_t)final_norm % 16 || (uintptr_t)h_out % 16)
+    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_stack: final_norm and h_out go together and are 16-byte aligned");
+  return SUBSPEC_OK;
+}
+
+template <typename Weights>
+static int decoder_stack_entry(const subspec_decoder_layer_dims* dims, const Weights* weights, int64_t n_layers, void* x,
+                               const int32_t* positions, const int32_t* cache_rows, const uint64_t* anc_bits,
+                               void* const* k_caches, void* const* v_caches, const void* final_norm, void* h_out,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_stack_args(weights, n_layers, k_caches, final_norm, h_out);
+  if (rc != SUBSPEC_OK) return rc;
+  for (int64_t i = 0; i < n_layers; ++i)      // every layer is checked before the first one runs
+    if ((rc = check_layer_call(dims, layer_weights(weights[i]), x, positions, cache_rows, anc_bits, k_caches[i],
+                               v_caches ? v_caches[i] : nullptr, workspace, workspace_bytes)))
+      return rc;
+  if (dims->dtype == SUBSPEC_BF16)
+    return run_stack<SUBSPEC_BF16>(*dims, weights, n_layers, (uint16_t*)x, positions, cache_rows, anc_bits, k_caches, v_caches,
+                                   final_norm, h_out, (char*)workspace, (hipStream_t)stream, false);
+  return run_stack<SUBSPEC_F16>(*dims, weights, n_layers, (uint16_t*)x, positions, cache_rows, anc_bits, k_caches, v_caches,
+                                final_norm, h_out, (char*)workspace, (hipStream_t)stream, false);
+}
+
+extern "C" int subspec_int4_decoder_stack(const subspec_decoder_layer_dims* dims, const subspec_decoder_layer_weights* weights,
+                                          int64_t n_layers, void* x, const int32_t* positions, const int32_t* cache_rows,
+                                          const uint64_t* anc_bits, void* const* k_caches, void* const* v_caches,
+                                          const void* final_norm, void* h_out, void* workspace, size_t workspace_bytes,
+                                          void* stream) {
+  return decoder_stack_entry(dims, weights, n_layers, x, positions, cache_rows, anc_bits, k_caches, v_caches, final_norm, h_out,
+                             workspace, workspace_bytes, stream);
+}
+
+extern "C" int subspec_dense_decoder_stack(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights,
+                                           int64_t n_layers, void* x, const int32_t* positions, const int32_t* cache_rows,
+                                           const uint64_t* anc_bits, void* const* k_caches, void* const* v_caches,
+                                           const void* final_norm, void* h_out, void* workspace, size_t workspace_bytes,
+                                           void* stream) {
+  return decoder_stack_entry(dims, weights, n_layers, x, positions, cache_rows, anc_bits, k_caches, v_caches, final_norm, h_out,
+                             workspace, workspace_bytes, stream);
 }
 
 // A prefill takes dense layers whose projections the kernels above cover at its number of rows
@@ -450,28 +642,42 @@ extern "C" size_t subspec_prefill_layer_workspace(const subspec_decoder_layer_di
   return check_prefill(dims) == SUBSPEC_OK ? layer_plan(*dims, true).total : 0;
 }
 
-extern "C" int subspec_prefill_layer(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights, void* x,
-                                     const int32_t* positions, const int32_t* cache_rows, void* k_cache, void* v_cache,
-                                     void* workspace, size_t workspace_bytes, void* stream) {
-  const int rc = check_prefill(dims);
-  if (rc != SUBSPEC_OK) return rc;
-  if (!weights) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: null weights");
-  const subspec_dense_layer_weights& s = *weights;
-  if (!x || !positions || !cache_rows || !k_cache || (!v_cache && !dims->page_indices) || !s.input_norm || !s.post_norm ||
-      !s.qkv_w || !s.o_w || !s.gate_up_w || !s.down_w)
+static int check_prefill_call(const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* x, const int32_t* positions,
+                              const int32_t* cache_rows, void* k_cache, void* v_cache, void* workspace, size_t workspace_bytes) {
+  if (!x || !positions || !cache_rows || !k_cache || (!v_cache && !dims->page_indices) || !w.input_norm || !w.post_norm ||
+      !w.qkv.w || !w.o.w || !w.gate_up.w || !w.down.w)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: null pointer argument");
-  if ((uintptr_t)x % 16 || (uintptr_t)s.input_norm % 16 || (uintptr_t)s.post_norm % 16 || (uintptr_t)k_cache % 16 ||
+  if ((uintptr_t)x % 16 || (uintptr_t)w.input_norm % 16 || (uintptr_t)w.post_norm % 16 || (uintptr_t)k_cache % 16 ||
       (uintptr_t)v_cache % 16)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: x, norm weights and caches must be 16-byte aligned");
   const size_t need = layer_plan(*dims, true).total;
   if (!workspace || workspace_bytes < need)
     SUBSPEC_FAIL(SUBSPEC_ERR_WORKSPACE, "prefill_layer: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
   if ((uintptr_t)workspace % 256) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: workspace must be 256-byte aligned");
-  const LayerWeights w{s.input_norm, s.post_norm, s.qkv_bias, {s.qkv_w, nullptr}, {s.o_w, nullptr},
-                       {s.gate_up_w, nullptr}, {s.down_w, nullptr}, true};
+  return SUBSPEC_OK;
+}
+
+extern "C" int subspec_prefill_stack(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights,
+                                     int64_t n_layers, void* x, const int32_t* positions, const int32_t* cache_rows,
+                                     void* const* k_caches, void* const* v_caches, const void* final_norm, void* h_out,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_prefill(dims);
+  if (rc == SUBSPEC_OK) rc = check_stack_args(weights, n_layers, k_caches, final_norm, h_out);
+  if (rc != SUBSPEC_OK) return rc;
+  for (int64_t i = 0; i < n_layers; ++i)
+    if ((rc = check_prefill_call(dims, layer_weights(weights[i]), x, positions, cache_rows, k_caches[i], v_caches ? v_caches[i] : nullptr,
+                                 workspace, workspace_bytes)))
+      return rc;
   if (dims->dtype == SUBSPEC_BF16)
-    return run_layer<SUBSPEC_BF16>(*dims, w, (uint16_t*)x, positions, cache_rows, nullptr, (uint16_t*)k_cache, (uint16_t*)v_cache,
-                                   (char*)workspace, (hipStream_t)stream, true);
-  return run_layer<SUBSPEC_F16>(*dims, w, (uint16_t*)x, positions, cache_rows, nullptr, (uint16_t*)k_cache, (uint16_t*)v_cache,
-                                (char*)workspace, (hipStream_t)stream, true);
+    return run_stack<SUBSPEC_BF16>(*dims, weights, n_layers, (uint16_t*)x, positions, cache_rows, nullptr, k_caches, v_caches,
+                                   final_norm, h_out, (char*)workspace, (hipStream_t)stream, true);
+  return run_stack<SUBSPEC_F16>(*dims, weights, n_layers, (uint16_t*)x, positions, cache_rows, nullptr, k_caches, v_caches,
+                                final_norm, h_out, (char*)workspace, (hipStream_t)stream, true);
+}
+
+extern "C" int subspec_prefill_layer(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights, void* x,
+                                     const int32_t* positions, const int32_t* cache_rows, void* k_cache, void* v_cache,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+  return subspec_prefill_stack(dims, weights, 1, x, positions, cache_rows, &k_cache, v_cache ? &v_cache : nullptr, nullptr, nullptr,
+                               workspace, workspace_bytes, stream);
 }

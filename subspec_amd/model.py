@@ -159,13 +159,14 @@ class Decoder:
                 make = ops.decoder_layer_weights if packed[0] else ops.dense_layer_weights
                 self._native_make = make
                 resident = min(self.first_streamed, len(self.layers))
-                self._native_weights = [make(w) for w in self.layers[:resident]]
+                tables = [make(w) for w in self.layers[:resident]]
+                self._native_weights = (type(tables[0]) * resident)(*tables) if tables else ()
                 self._native_ws = {}
         return self._native
 
     def _run_native_layers(self, x, positions, rows, anc_bits, prefix_len: int, slots: int,
                            prefix_len_dev: Optional[torch.Tensor] = None, fresh: bool = False) -> torch.Tensor:
-        """``fresh``: ``x`` is a tensor of the caller's own making (the layers work in place and may keep it)."""
+        """Logits of the rows.  ``fresh``: ``x`` is a tensor of the caller's own making (the layers work in place and may keep it)."""
         cfg, cache = self.cfg, self.kv.cache
         n = x.shape[0]
         paged = not cache.contiguous
@@ -188,16 +189,25 @@ class Decoder:
         x = x if fresh and x.is_contiguous() else x.contiguous().clone()
         pos32, rows32 = positions.to(torch.int32), rows.to(torch.int32)          # no copies when they are int32 already
         bits = anc_bits.to(torch.int64).contiguous()
-        for i, w in enumerate(self._native_weights):
-            ops.decoder_layer_(x, dims, w, pos32, rows32, bits, *layer_kv(i), ws)
-        if self.streamer is not None and self.streamer.n:
+        streamed = self.streamer is not None and self.streamer.n
+        normed = None
+        if len(self._native_weights):                # the resident layers, and the final norm behind them, in one call
+            norm = self.norm if not streamed and self._norm_fits(x) else None
+            normed = ops.decoder_stack_(x, dims, self._native_weights, pos32, rows32, bits,
+                                        cache.pool.cache_data if paged else cache.data, ws, norm)
+        if streamed:
             base = self.first_streamed
 
             def step(j, w):                       # w: views into the device slab that holds layer base + j right now
                 ops.decoder_layer_(x, dims, self._native_make(w), pos32, rows32, bits, *layer_kv(base + j), ws)
 
             self.streamer.run(step)
-        return x
+        return self.logits(x) if normed is None else self._head(normed)
+
+    def _norm_fits(self, x: torch.Tensor) -> bool:
+        """Whether the final norm can be the last launch of a one-call stack."""
+        return (self.norm.dtype == x.dtype and self.norm.is_contiguous() and self.norm.data_ptr() % 16 == 0
+                and self.norm.numel() == x.shape[-1] and self.norm.device == x.device)
 
     def _prefill_plan(self, x: torch.Tensor, start: int):
         """What the one-call layers need for a chunk of a prompt, or None where they do not apply: 16-bit device tensors, one
@@ -225,25 +235,30 @@ class Decoder:
         if need == 0:
             return None
         rows = torch.arange(start, start + n, device=x.device, dtype=torch.int32)
-        return {"dims": dims, "rows": rows, "need": need, "ws": None, "paging": paging,
+        return {"dims": dims, "rows": rows, "need": need, "ws": None, "paging": paging, "data": data,
                 "shapes": layer_shapes(cfg), "kv": (lambda i: (data[i], data[i])) if paged else (lambda i: (data[i, 0], data[i, 1]))}
 
     def _prefill_layer(self, plan, i: int, w: Dict[str, torch.Tensor], x: torch.Tensor) -> Optional[torch.Tensor]:
-        """One layer of a prompt chunk on the one-call kernels (in place), or None when this layer's weights are not dense
-        contiguous 16-byte aligned matrices of the expected shapes, or when `_linear` would read more than those (int4 codes,
-        biases other than that of q|k|v)."""
-        if not x.is_contiguous() or any(n + ".wq" in w or (n != "qkv_proj" and w.get(n + ".bias") is not None) for n in QUANTIZED):
+        """One layer of a prompt chunk on the one-call kernels (in place), or None where they do not take it."""
+        if not self._prefill_takes(plan, w, x):
             return None
+        if plan["ws"] is None:
+            plan["ws"] = torch.empty(plan["need"], dtype=torch.uint8, device=x.device)
+        return ops.prefill_layer_(x, plan["dims"], ops.dense_layer_weights(w), plan["rows"], plan["rows"], *plan["kv"](i), plan["ws"])
+
+    def _prefill_takes(self, plan, w: Dict[str, torch.Tensor], x: torch.Tensor) -> bool:
+        """False when this layer's weights are not dense contiguous 16-byte aligned matrices of the expected shapes, or when
+        `_linear` would read more than those (int4 codes, biases other than that of q|k|v)."""
+        if not x.is_contiguous() or any(n + ".wq" in w or (n != "qkv_proj" and w.get(n + ".bias") is not None) for n in QUANTIZED):
+            return False
         for name, shape in plan["shapes"].items():
             t = w.get(name)
             if t is None:
                 if name != "qkv_proj.bias":
-                    return None
+                    return False
             elif (t.shape != shape or t.dtype != x.dtype or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16):
-                return None
-        if plan["ws"] is None:
-            plan["ws"] = torch.empty(plan["need"], dtype=torch.uint8, device=x.device)
-        return ops.prefill_layer_(x, plan["dims"], ops.dense_layer_weights(w), plan["rows"], plan["rows"], *plan["kv"](i), plan["ws"])
+                return False
+        return True
 
     # ------------------------------------------------------------------ pieces
     def _rope(self, t: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
@@ -277,7 +292,15 @@ class Decoder:
 
     def _run_layers(self, x, positions, rows, attn, plan=None) -> torch.Tensor:
         state = {"x": x}
-        for i in range(min(self.first_streamed, len(self.layers))):
+        resident = min(self.first_streamed, len(self.layers))
+        if plan is not None and resident and all(self._prefill_takes(plan, w, x) for w in self.layers[:resident]):
+            if plan["ws"] is None:
+                plan["ws"] = torch.empty(plan["need"], dtype=torch.uint8, device=x.device)
+            tables = [ops.dense_layer_weights(w) for w in self.layers[:resident]]
+            ops.prefill_stack_(x, plan["dims"], (type(tables[0]) * resident)(*tables), plan["rows"], plan["rows"],
+                               plan["data"], plan["ws"])
+            resident = 0
+        for i in range(resident):
             state["x"] = self._layer(i, self.layers[i], state["x"], positions, rows, attn, plan)
         if self.streamer is not None and self.streamer.n:
             base = self.first_streamed
@@ -294,7 +317,10 @@ class Decoder:
         1.09 GB head streams through the dense kernels of this package (152064 x 3584 bf16: 170 us at 8 rows, 198 us at 32
         against 232 / 255 us for the vendor GEMM; 204 us at 64 rows, where the two are level); wider inputs keep the
         vendor GEMM (128 rows: 236 against 261 us)."""
-        h = rms_norm(x, self.norm, self.cfg.rms_norm_eps)
+        return self._head(rms_norm(x, self.norm, self.cfg.rms_norm_eps))
+
+    def _head(self, h: torch.Tensor) -> torch.Tensor:
+        """The language-model head on normalized rows."""
         rows = h.numel() // h.shape[-1]
         V, H = self.lm_head.shape
         if (h.is_cuda and rows <= 64 and h.dtype in (torch.bfloat16, torch.float16) and H % 64 == 0
@@ -356,8 +382,8 @@ class Decoder:
             raise ValueError("a device-side prefix length needs the one-call decoder layers (at most 64 rows; 384 for dense layers)")
         if positions32 is not None and rows32 is not None:
             if native:
-                return self.logits(self._run_native_layers(self.embed[token_ids], positions32, rows32, anc_bits, prefix_len,
-                                                           slots, prefix_len_dev=prefix_len_dev, fresh=True))
+                return self._run_native_layers(self.embed[token_ids], positions32, rows32, anc_bits, prefix_len,
+                                               slots, prefix_len_dev=prefix_len_dev, fresh=True)
             positions, rows = positions32.long(), rows32.long()
         elif depths is None:
             raise ValueError("tree_forward needs `depths`, or positions32 and rows32")
@@ -368,8 +394,8 @@ class Decoder:
             positions = depths.to(self.device) + prefix_len
             rows = torch.arange(prefix_len + first_slot, prefix_len + first_slot + n, device=self.device)
         if native:
-            return self.logits(self._run_native_layers(self.embed[token_ids], positions, rows, anc_bits, prefix_len, slots,
-                                                       prefix_len_dev=prefix_len_dev))
+            return self._run_native_layers(self.embed[token_ids], positions, rows, anc_bits, prefix_len, slots,
+                                           prefix_len_dev=prefix_len_dev)
 
         def attn(i, q):
             return self.kv.cache.tree_attention(i, q, anc_bits, prefix_len, slots).reshape(n, cfg.q_size)

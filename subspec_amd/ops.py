@@ -567,6 +567,60 @@ def prefill_layer_(x: torch.Tensor, dims: "L.DecoderLayerDims", weights: "L.Dens
     return x
 
 
+def _stack_args(x, dims, weights, positions, cache_rows, cache, final_norm, what):
+    """Checks of a stack call; the layers' cache pointers (``cache`` [layers, 2, ...], or a page pool [layers, pages, 2, ...]) and
+    the final norm's pointers."""
+    if positions.dtype != torch.int32 or cache_rows.dtype != torch.int32:
+        raise ValueError(f"{what}: positions / cache_rows must be int32")
+    if not x.is_contiguous() or x.shape != (dims.n_rows, dims.hidden) or positions.numel() != dims.n_rows \
+            or cache_rows.numel() != dims.n_rows:
+        raise ValueError(f"{what}: tensor shapes do not match the dimensions given")
+    n, paged = len(weights), bool(dims.page_indices)
+    if cache.shape[0] < n or not cache[0].is_contiguous() or (not paged and cache.shape[1] != 2):
+        raise ValueError(f"{what}: the cache must hold every layer's K and V contiguously")
+    base, step = cache.data_ptr(), cache.stride(0) * cache.element_size()
+    second = 0 if paged else cache.stride(1) * cache.element_size()
+    pointers = ctypes.c_void_p * n
+    k = pointers(*range(base, base + n * step, step))
+    v = pointers(*range(base + second, base + second + n * step, step))
+    if final_norm is None:
+        return k, v, None, None, None
+    if final_norm.numel() != x.shape[-1] or final_norm.dtype != x.dtype or not final_norm.is_contiguous() or final_norm.device != x.device:
+        raise ValueError(f"{what}: final_norm must be a contiguous [hidden] tensor in the activation dtype")
+    h = torch.empty_like(x)
+    return k, v, h, final_norm.data_ptr(), h.data_ptr()
+
+
+def decoder_stack_(x: torch.Tensor, dims: "L.DecoderLayerDims", weights, positions: torch.Tensor, cache_rows: torch.Tensor,
+                   anc_bits: torch.Tensor, cache: torch.Tensor, workspace: torch.Tensor,
+                   final_norm: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``decoder_layer_`` for the first ``len(weights)`` layers of a stack in one call: ``weights`` is a ctypes array of one pointer
+    table per layer, ``cache`` all layers' K and V (or the page pool).  Updates ``x`` in place; with ``final_norm`` [hidden]
+    returns the RMSNorm of the last layer's output as well."""
+    dev = _require_gpu(x, positions, cache_rows, anc_bits, cache, workspace)
+    k, v, h, norm_ptr, h_ptr = _stack_args(x, dims, weights, positions, cache_rows, cache, final_norm, "decoder stack")
+    if anc_bits.dtype != torch.int64 or anc_bits.numel() != dims.n_rows * ((dims.n_tree_slots + 63) // 64):
+        raise ValueError("decoder stack: anc_bits must be int64 [n_rows, ceil(n_tree_slots / 64)]")
+    name = "subspec_dense_decoder_stack" if weights._type_ is L.DenseLayerWeights else "subspec_int4_decoder_stack"
+    code = getattr(L.lib(), name)(ctypes.byref(dims), weights, len(weights), x.data_ptr(), positions.data_ptr(),
+                                  cache_rows.data_ptr(), anc_bits.data_ptr(), k, v, norm_ptr, h_ptr, workspace.data_ptr(),
+                                  workspace.numel() * workspace.element_size(), _stream(dev))
+    L.check(code, name)
+    return h
+
+
+def prefill_stack_(x: torch.Tensor, dims: "L.DecoderLayerDims", weights, positions: torch.Tensor, cache_rows: torch.Tensor,
+                   cache: torch.Tensor, workspace: torch.Tensor, final_norm: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``prefill_layer_`` for a whole stack in one call (arguments as ``decoder_stack_``)."""
+    dev = _require_gpu(x, positions, cache_rows, cache, workspace)
+    k, v, h, norm_ptr, h_ptr = _stack_args(x, dims, weights, positions, cache_rows, cache, final_norm, "prefill stack")
+    code = L.lib().subspec_prefill_stack(ctypes.byref(dims), weights, len(weights), x.data_ptr(), positions.data_ptr(),
+                                         cache_rows.data_ptr(), k, v, norm_ptr, h_ptr, workspace.data_ptr(),
+                                         workspace.numel() * workspace.element_size(), _stream(dev))
+    L.check(code, "subspec_prefill_stack")
+    return h
+
+
 decoder_layer_ = int4_decoder_layer_     # either weight storage: the pointer table's type selects the entry point
 
 

@@ -1,0 +1,52 @@
+"""A stack in one call against the same layers called one by one: the joined launches sum the same values in the same order, so
+the results are equal bit for bit."""
+import pytest
+import torch
+
+from subspec_amd import model as M, ops
+from subspec_amd.cache import create_kv_cache
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# rows: the int4 kernels of 8, 33 to 64 rows; dense up to 32, 64, more; a prompt.  hidden 4104-wide pieces: one and four per thread
+@pytest.mark.parametrize("kind,rows,hidden", [("int4", 8, 512), ("int4", 40, 512), ("int4", 64, 4224), ("dense", 5, 512),
+                                              ("dense", 64, 4224), ("dense", 289, 512), ("prefill", 300, 512), ("prefill", 513, 4224)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_stack_equals_layers(kind, rows, hidden, dtype):
+    print("stack", kind, rows, hidden, dtype, flush=True)
+    cfg = M.DecoderConfig(num_hidden_layers=3, hidden_size=hidden, num_attention_heads=5, num_key_value_heads=1, head_dim=128,
+                          intermediate_size=8192, vocab_size=64)
+    w = M.init_weights(cfg, rows, DEV, dtype)
+    layers = M.quantize_layers(w["layers"]) if kind == "int4" else w["layers"]
+    kv = create_kv_cache("static", max_cache_len=rows + 70, config=cfg, device=DEV, dtype=dtype)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    kv.cache.data.normal_(generator=g)
+    past, prefix = kv.cache.data.clone(), 50
+    x0 = torch.randn(rows, hidden, generator=g, device=DEV).to(dtype)
+    dims = ops.decoder_layer_dims(dtype, rows, hidden, 8192, 5, 1, 128, rows + 70, prefix, 1 if kind == "prefill" else rows, 1e-6, 1e6)
+    pos = torch.arange(prefix, prefix + rows, dtype=torch.int32, device=DEV)
+    bits = None if kind == "prefill" else ops.ancestor_bits_tensor([-1] + list(range(rows - 1)), device=DEV)
+    make = ops.decoder_layer_weights if kind == "int4" else ops.dense_layer_weights
+    tables = [make(l) for l in layers]
+    need = ops.prefill_layer_workspace(dims) if kind == "prefill" else ops.decoder_layer_workspace(dims)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    want = x0.clone()
+    for i, t in enumerate(tables):
+        args = (kv.cache.k(i), kv.cache.v(i), ws)
+        if kind == "prefill":
+            ops.prefill_layer_(want, dims, t, pos, pos, *args)
+        else:
+            ops.decoder_layer_(want, dims, t, pos, pos, bits, *args)
+    rows_after = kv.cache.data.clone()
+    gain = (torch.rand(hidden, generator=g, device=DEV) + 0.5).to(dtype)
+    for final_norm in (None, gain):
+        kv.cache.data.copy_(past)
+        x = x0.clone()
+        array = (type(tables[0]) * len(tables))(*tables)
+        rest = (kv.cache.data, ws, final_norm)
+        h = ops.prefill_stack_(x, dims, array, pos, pos, *rest) if kind == "prefill" else \
+            ops.decoder_stack_(x, dims, array, pos, pos, bits, *rest)
+        assert torch.isfinite(x).all() and torch.equal(x, want) and torch.equal(kv.cache.data, rows_after)
+        assert h is None if final_norm is None else torch.equal(h, ops.rms_norm(want, gain, 1e-6))

@@ -196,3 +196,47 @@ def test_argument_errors():
                            torch.zeros(65, dtype=torch.int64, device=DEV), 0)
     with pytest.raises(ValueError):
         ops.tree_attention(q[..., :64].contiguous(), k[..., :64].contiguous(), k[..., :64].contiguous(), anc, 8)
+
+
+# the last block count of the kernel for short caches, the first of the ping-pong kernel, the largest tree; ragged last windows
+@pytest.mark.parametrize("n,P", [(289, 920), (289, 990), (300, 1300), (512, 900)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_large_tree_of_one_sequence(dtype, n, P):
+    parents, q, k, v = _case(n + P, 1, 28, 4, n, P, P + n + 40, dtype, depth=40)
+    k[:, :, P + n:] = 1e3                                              # stale rows beyond the tree
+    _check(parents, q, k, v, P, "one sequence")
+    # the same rows over pages in another order: equal bit for bit
+    page = 16
+    table = torch.randperm((P + n + page - 1) // page + 3, generator=torch.Generator().manual_seed(1))[:(P + n + page - 1) // page]
+    pool = torch.full((int(table.max()) + 1, 2, page, 4, 128), float("nan"), dtype=dtype)
+    for part, rows in ((0, k), (1, v)):
+        for r in range(P + n):
+            pool[table[r // page], part, r % page] = rows[0, :, r]
+    anc = ops.ancestor_bits_tensor(parents, device=DEV)
+    got = ops.tree_attention_paged(q.to(DEV), pool.to(DEV), table.to(torch.int32).to(DEV), anc, P)
+    assert torch.equal(got, ops.tree_attention(q.to(DEV), k.to(DEV), v.to(DEV), anc, P))
+
+
+def test_large_tree_shorter_than_its_launch():
+    """A launch laid out for 3000 prefix rows of which the device holds 100: most key chunks are empty."""
+    from subspec_amd import model as M
+    n, bound = 289, 3000
+    cfg = M.DecoderConfig(num_hidden_layers=1, hidden_size=256, num_attention_heads=28, num_key_value_heads=4, head_dim=128,
+                          intermediate_size=256, vocab_size=64)
+    w = M.init_weights(cfg, 4, DEV, torch.bfloat16)["layers"][0]
+    g = torch.Generator(device=DEV).manual_seed(4)
+    x0 = torch.randn(n, 256, generator=g, device=DEV).bfloat16()
+    past = torch.randn(2, 1, 4, bound + n, 128, generator=g, device=DEV).bfloat16()
+    parents, _, _ = W.random_tree(torch.Generator().manual_seed(4), n=n, max_depth=48, max_children=6, vocab=64, chain_depth=40)
+    anc = ops.ancestor_bits_tensor(parents, device=DEV)
+    rows = torch.arange(100, 100 + n, dtype=torch.int32, device=DEV)
+    out = []
+    for prefix, dev in ((100, None), (bound, torch.tensor([100], device=DEV))):
+        dims = ops.decoder_layer_dims(torch.bfloat16, n, 256, 256, 28, 4, 128, bound + n, prefix, n, 1e-6, 1e6, prefix_len_dev=dev)
+        x, kv = x0.clone(), past.clone()
+        ws = torch.full((ops.decoder_layer_workspace(dims),), 0xff, dtype=torch.uint8, device=DEV)
+        ops.decoder_layer_(x, dims, ops.dense_layer_weights(w), rows, rows, anc, kv[0], kv[1], ws)
+        out.append(x.float())
+    assert torch.isfinite(out[1]).all()
+    # the two are cut into other key chunks, whose averages are rounded to bf16 (2^-9 each); then one projection
+    assert (out[0] - out[1]).norm() <= 1e-2 * (out[0] - x0.float()).norm()

@@ -315,17 +315,23 @@ class Decoder:
         """Final norm and the language-model head (HuggingFace ``lm_head`` inside the draft and target forwards,
         specdecodes/models/draft_models/classic_sd.py:10-16, generators/classic_sd.py:102-109).  Up to 64 rows the
         1.09 GB head streams through the dense kernels of this package (152064 x 3584 bf16: 170 us at 8 rows, 198 us at 32
-        against 232 / 255 us for the vendor GEMM; 204 us at 64 rows, where the two are level); wider inputs keep the
-        vendor GEMM (128 rows: 236 against 261 us)."""
+        against 232 / 255 us for the vendor GEMM; 204 us at 64 rows, where the two are level).  From 193 to 384 rows the tiled
+        kernel takes heads that do not stay in the 256 MB memory-side cache (289 rows: 343 against 419 us, 193 rows 285 against
+        319, 384 rows 419 against 452; a 32000 x 2048 head 42 against 38).  The vendor GEMM keeps 65 to 192 rows (96 rows: 221
+        against 232 us, level at 128 and 160) and more than 384."""
         return self._head(rms_norm(x, self.norm, self.cfg.rms_norm_eps))
 
     def _head(self, h: torch.Tensor) -> torch.Tensor:
         """The language-model head on normalized rows."""
         rows = h.numel() // h.shape[-1]
         V, H = self.lm_head.shape
-        if (h.is_cuda and rows <= 64 and h.dtype in (torch.bfloat16, torch.float16) and H % 64 == 0
-                and (V % 32 == 0 if rows > 32 else V % 16 == 0 and V * H * 2 < (1 << 31)) and self.lm_head.is_contiguous()):
-            return ops.dense_linear(h, self.lm_head)
+        if h.is_cuda and h.dtype in (torch.bfloat16, torch.float16) and H % 64 == 0 and self.lm_head.is_contiguous():
+            if rows <= 64:
+                own = V % 32 == 0 if rows > 32 else V % 16 == 0 and V * H * 2 < (1 << 31)
+            else:
+                own = 192 < rows <= 384 and V % 32 == 0 and (1 << 28) <= V * H * 2 < (1 << 31) and self.lm_head.data_ptr() % 16 == 0
+            if own:
+                return ops.dense_linear(h, self.lm_head)
         return F.linear(h, self.lm_head)
 
     # ------------------------------------------------------------------ forwards

@@ -200,3 +200,23 @@ def test_dense_gate_up_projection_with_the_activation_in_its_output_stage(dtype)
         assert differing <= max(1, got.numel() // 1000), (F, K, M, differing)
         ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
         assert ((got.float() - want.float()).abs() <= 2 * ulp * want.float().abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("rows", [192, 193, 289, 384, 385])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_head_of_a_large_tree(rows, dtype):
+    """Rows on both sides of the lines between the tiled kernel and the library, on the smallest head that the former takes."""
+    from subspec_amd import model as M
+    cfg = M.DecoderConfig(num_hidden_layers=1, hidden_size=256, num_attention_heads=2, num_key_value_heads=1, head_dim=128,
+                          intermediate_size=128, vocab_size=524288)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    head = (torch.randn(cfg.vocab_size, 256, generator=g, device=DEV) * 0.05).to(dtype)
+    x = torch.randn(rows, 256, generator=g, device=DEV).to(dtype)
+    kv = create_kv_cache("static", max_cache_len=8, config=cfg, device=DEV, dtype=dtype)
+    d = M.Decoder(cfg, head[:64], [], torch.ones(256, dtype=dtype, device=DEV), head, kv)
+    got = d.logits(x)
+    h = ops.rms_norm(x, torch.ones(256, dtype=dtype, device=DEV), cfg.rms_norm_eps).float()
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)               # one rounding of the result; fp32 sums of 256 products
+    for lo in range(0, cfg.vocab_size, 65536):
+        want = h @ head[lo:lo + 65536].float().t()
+        assert ((got[:, lo:lo + 65536].float() - want).abs() <= eps * want.abs() + 1e-4).all()

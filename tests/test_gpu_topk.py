@@ -147,3 +147,36 @@ def test_draft_probabilities_softmax_with_temperature(dtype):
         assert torch.equal(tok.cpu(), e_tok) and torch.equal(val.cpu(), e_val) and torch.equal(par.cpu(), e_par)
     with pytest.raises(ValueError):
         ops.softmax_temperature(torch.zeros(2, 8, device=DEV), 0.0)
+
+
+# lists on both sides of the small and the large merge, slices of one, two and more tile groups, rows of ties and of distinct values
+@pytest.mark.parametrize("B,L,V,k", [(1, 2, 8192, 64), (1, 2, 8200, 8), (1, 16, 32768, 16), (1, 16, 50257, 64), (3, 8, 16392, 32), (2, 64, 9000, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_merge_of_many_slices(dtype, B, L, V, k):
+    print("topk slices", dtype, B, L, V, k, flush=True)
+    g = torch.Generator().manual_seed(V + k)
+    parent = torch.rand(B, L, generator=g).to(dtype)
+    peaked = torch.softmax(torch.randn(B, L, V, generator=g) * 4, -1).to(dtype)
+    ties = (torch.randint(0, 3, (B, L, V), generator=g) * 0.25).to(dtype)
+    one_leaf = peaked * 1e-3
+    one_leaf[:, L - 1] = peaked[:, L - 1]                              # every winner in one leaf, other lists below the cut
+    for probs in (peaked, ties, one_leaf, torch.zeros_like(peaked)):
+        _check(probs, parent, k)
+
+
+@pytest.mark.parametrize("V,offset", [(4096, 0), (4097, 0), (4104, 0), (8200, 1), (12288, 3), (300000, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_softmax_slices(dtype, V, offset):
+    """Row lengths around the slices, and a first element that no 16-byte piece starts at."""
+    g = torch.Generator().manual_seed(V)
+    logits = (torch.randn(5 * V + offset, generator=g) * 6).to(dtype)
+    logits[offset + 7] = float("-inf")
+    got = ops.softmax_temperature(logits.to(DEV)[offset:].view(5, V), 0.6).cpu()
+    x = (logits[offset:].view(5, V) / 0.6).double()
+    want = torch.softmax(x, -1)
+    # one rounding to 16 bits; in float32 the difference to the maximum (below 128) is off by half an ulp, 2^-18, and exponential,
+    # sum and quotient by a few of 2^-24
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[dtype]
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 1e-38              # half-precision probabilities are subnormal below 6e-5
+    assert ((got.double() - want).abs() <= 1.01 * eps * want + tiny + (2.0 ** -18 + 2.0 ** -20) * want).all()
+    assert got[0, 7] == 0

@@ -326,8 +326,12 @@ template <int DT> __device__ __forceinline__ uint32_t wd_pack2(float a, float b)
   }
 }
 
+template <bool NT>
 __device__ __forceinline__ void wd_dma16(uint32_t lds_base, const uint16_t* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(src) : "memory", "m0");
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(src) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(src) : "memory", "m0");
 }
 template <int N> __device__ __forceinline__ void wd_wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
@@ -343,7 +347,7 @@ struct WideParams {
 // 128 bytes) and of the activations (MT x 32 rows x 128 bytes) sits in a ring slot each; a request moves 1 KB = 8 rows x
 // 128 bytes, whole cache lines.  Copies: wavefronts [0, NWW) bring the weight chunks (WPER requests each per chunk),
 // wavefronts [NWW, NWW + NXW) the activation chunks (ceil(4 MT / NXW) each, at most XPER).
-template <int DT, int WM, int MG, int NTMAX, int SW, int SX, int NWW, int WPER, int NXW, int XPER, bool SILU>
+template <int DT, int WM, int MG, int NTMAX, int SW, int SX, int NWW, int WPER, int NXW, int XPER, bool SILU, bool NT = false>
 __global__ __launch_bounds__(512) void dense_wide_kernel(WideParams p) {
   constexpr int MTMAX = WM * MG;
   __shared__ __attribute__((aligned(16))) uint8_t wd_lds[(SW * NTMAX + SX * MTMAX) * 4096];
@@ -396,19 +400,19 @@ __global__ __launch_bounds__(512) void dense_wide_kernel(WideParams p) {
   const uint32_t cstride = w_wave ? kWStride : xstride;
   constexpr int kWWait = (SW - 2) * WPER, kXWait = (SX - 2) * XPER;
   // chunk s (relative to st0) of this wavefront's ring -> slot
-#define SUBSPEC_WD_ISSUE(S, SLOT)                                                                          \
+#define SUBSPEC_WD_ISSUE(S, SLOT, STREAM)                                                                  \
   do {                                                                                             \
     const int s_ = min((S), nst - 1);                                                              \
     _Pragma("unroll") for (int i_ = 0; i_ < kPer; ++i_)                                            \
-      if (i_ < per) wd_dma16(__builtin_amdgcn_readfirstlane(dst[i_] + (SLOT) * cstride), src[i_] + s_ * 64); \
+      if (i_ < per) wd_dma16<STREAM>(__builtin_amdgcn_readfirstlane(dst[i_] + (SLOT) * cstride), src[i_] + s_ * 64); \
   } while (0)
 
   if (w_wave) {
 #pragma unroll
-    for (int s = 0; s < SW - 1; ++s) SUBSPEC_WD_ISSUE(s, s);
+    for (int s = 0; s < SW - 1; ++s) SUBSPEC_WD_ISSUE(s, s, NT);
   } else if (x_wave) {
 #pragma unroll
-    for (int s = 0; s < SX - 1; ++s) SUBSPEC_WD_ISSUE(s, s);
+    for (int s = 0; s < SX - 1; ++s) SUBSPEC_WD_ISSUE(s, s, false);
   }
 
   // ---- this wavefront's tiles
@@ -448,8 +452,8 @@ __global__ __launch_bounds__(512) void dense_wide_kernel(WideParams p) {
     if (w_wave) wd_wait_vmcnt<kWWait>();
     else if (x_wave) wd_wait_vmcnt<kXWait>();
     __syncthreads();
-    if (w_wave) SUBSPEC_WD_ISSUE(SW - 1, wnext);
-    else if (x_wave) SUBSPEC_WD_ISSUE(SX - 1, xnext);
+    if (w_wave) SUBSPEC_WD_ISSUE(SW - 1, wnext, NT);
+    else if (x_wave) SUBSPEC_WD_ISSUE(SX - 1, xnext, false);
     SUBSPEC_WD_READ(a0, b0, 0);
     for (int it = 0; it < nst; ++it) {
       SUBSPEC_WD_READ(a1, b1, 1);
@@ -474,8 +478,8 @@ __global__ __launch_bounds__(512) void dense_wide_kernel(WideParams p) {
         if (w_wave) wd_wait_vmcnt<kWWait>();
         else if (x_wave) wd_wait_vmcnt<kXWait>();
         __syncthreads();
-        if (w_wave) SUBSPEC_WD_ISSUE(it + SW, wnext);
-        else if (x_wave) SUBSPEC_WD_ISSUE(it + SX, xnext);
+        if (w_wave) SUBSPEC_WD_ISSUE(it + SW, wnext, NT);
+        else if (x_wave) SUBSPEC_WD_ISSUE(it + SX, xnext, false);
         SUBSPEC_WD_READ(a0, b0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -561,11 +565,12 @@ constexpr int kWideMaxRows = 384;
 // spread over the chip by splitting K (partials in fp32, summed in split order by dense_reduce_kernel): two tiles per
 // workgroup for K of a few thousand, four for the long K of a down projection, as many K ranges as keep about 256
 // workgroups, each at least six chunks long.
-struct WidePlan { int wgs, splits, chunks_per_split; };
+struct WidePlan { int wgs, splits, chunks_per_split, tiles; };
 static WidePlan wide_plan(int64_t N, int64_t K, bool silu) {
   const int n_tiles = (int)(N / 32), chunks = (int)(K / 64);
   const int nt = (silu || n_tiles >= 5 * 192) ? 5 : chunks > 128 ? 4 : 2;
   WidePlan pl;
+  pl.tiles = nt;
   pl.wgs = (n_tiles + nt - 1) / nt;
   int splits = silu ? 1 : std::max(1, std::min(8, 256 / pl.wgs));
   splits = std::min(splits, std::max(1, chunks / 6));
@@ -578,10 +583,25 @@ static bool wide_applies(int64_t M, int64_t N) { return M > 32 && M <= kWideMaxR
 template <int DT, bool SILU>
 static void launch_wide(const WideParams& p, const WidePlan& pl, hipStream_t st) {
   const dim3 grid((unsigned)pl.wgs, (unsigned)pl.splits);
-  // rows <= 64: five wavefronts copy weights four chunks deep (the kernel streams); <= 256: three activation slots;
-  // <= 384: two (LDS holds no more beside the weights)
-  if (p.M <= 64)
-    hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 5, 4, 4, 5, 4, 2, 4, SILU>), grid, dim3(512), 0, st, p);
+  // rows <= 64: the kernel streams, each weight byte once, and requests it as streaming data.  That pays only if no line is
+  // requested twice, so the ring has as many tiles as the plan gives a workgroup (rings of five for two or four tiles fill up with
+  // repeats, which come from memory again: 4608 x 3584 15.6 -> 18.3 us); 64 rows, weights from HBM, with the reduction: 37888 x 3584
+  // with the activation 52.0 -> 45.6 us (6.0 TB/s), 3584 x 3584 14.5 -> 13.6, 4608 x 3584 15.7 -> 15.0, 3584 x 18944 33.8 -> 32.6,
+  // 32000 x 2048 36.1 -> 32.6; 152064 x 3584 205 -> 206 (33 rows 196 -> 188).  Deeper rings alone: nothing.
+  // <= 256 rows: three activation slots; <= 384: two (LDS holds no more beside the weights)
+  if (p.M <= 64) {
+    if constexpr (!SILU) {
+      if (pl.tiles == 2) {
+        hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 2, 10, 6, 4, 2, 4, 2, false, true>), grid, dim3(512), 0, st, p);
+        return;
+      }
+      if (pl.tiles == 4) {
+        hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 4, 6, 6, 4, 4, 4, 2, false, true>), grid, dim3(512), 0, st, p);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 5, 4, 4, 5, 4, 2, 4, SILU, true>), grid, dim3(512), 0, st, p);
+  }
   else if (p.M <= 256)
     hipLaunchKernelGGL((dense_wide_kernel<DT, 4, 2, 5, 3, 3, 2, 10, 4, 8, SILU>), grid, dim3(512), 0, st, p);
   else

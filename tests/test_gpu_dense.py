@@ -220,3 +220,17 @@ def test_head_of_a_large_tree(rows, dtype):
     for lo in range(0, cfg.vocab_size, 65536):
         want = h @ head[lo:lo + 65536].float().t()
         assert ((got[:, lo:lo + 65536].float() - want).abs() <= eps * want.abs() + 1e-4).all()
+
+
+# rings of two, four and five weight tiles: fewer chunks of 64 than slots, as many, one more; workgroups with a tile less than the ring
+@pytest.mark.parametrize("M", [33, 64])
+@pytest.mark.parametrize("N,K", [(32, 64), (96, 576), (160, 640), (96, 704), (160, 8256), (224, 8320), (30720, 192), (30752, 256), (30784, 320)])
+def test_streamed_weight_rings(M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(N + K + M)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(N, K, generator=g, device=DEV).bfloat16()
+    want = x.double() @ w.double().t()
+    got = ops.dense_linear(x, w).double()
+    # one rounding to bf16 of a sum whose fp32 error is far below 2^-16 of the sum of the products' magnitudes
+    bound = 2.0 ** -8 * want.abs() + 2.0 ** -16 * (x.double().abs() @ w.double().abs().t())
+    assert ((got - want).abs() <= bound).all()

@@ -8,8 +8,12 @@
 // read of 8 KB feeds TA tiles and the four partial sums meet once, at the end.  Requests return in order, so wavefronts 0..3
 // copy activations (from the L2, a chunk or two ahead) and 4..7 weights (from HBM, three to seven chunks ahead): neither waits
 // behind the other.  A wavefront's requests, operand reads and the scaling of the previous 16 rows are issued between products.
-// What remains is issue: a block is about 50 vector instructions (dequantization; scale and zero point in fp32) and eight
-// products, 0.27 us per tile of a wavefront and chunk beside 0.33 us that a chunk costs at any width.
+// What remains is the vector ALU: a block is about 50 vector instructions (dequantization; scale and zero point in fp32) and eight
+// products, and a wavefront of five tiles issues 268 of the one and 48 of the other per chunk.  They overlap only where they
+// stand next to each other in the code: the scaling of 16 rows sits between the two products of a tile of the next 16 (pinned
+// there: left to itself the compiler sinks it behind all products, which then wait for each other in pairs), the next chunk's
+// codes are dequantized behind the last product of their tile.  37888 x 3584 with the activation, 64 rows: 37.7 -> 34.5 us,
+// 3584 x 18944 29.2 -> 28.0; of the 3.2 us, 1.8 is the order and the rest one v_and_or_b32 a code pair instead of two instructions.
 #include "dma.h"
 #include <algorithm>
 
@@ -116,9 +120,10 @@ __global__ __launch_bounds__(512) void int4_tile_kernel(Int4TileParams p) {
   const uint8_t* const xop1 = lds + kg * 8192 + ln * 128 + ((2 * c + 1) ^ sw) * 16;
   const uint8_t* const wop = lds + kWRing + h * TA * 2048 + kg * 512 + lane * 8;
   const uint8_t* const sop = lds + kWRing + kCodes + h * TA * 256 + kg * 64 + ln * 4;
-  // both constants of ((w >> s) & mask) | magic as run-time values: one v_and_or_b32 (see int4.hip)
-  const uint32_t kmask = 0x000f000fu | (uint32_t)(M >> 30);
-  const uint32_t kmagic = (DT == SUBSPEC_BF16 ? 0x43004300u : 0x64006400u) | ((uint32_t)lane >> 31);
+  // both constants of ((w >> s) & mask) | magic as values the compiler cannot see through, in registers: one v_and_or_b32 (an and
+  // and an or with literals otherwise)
+  uint32_t kmask = 0x000f000fu, kmagic = DT == SUBSPEC_BF16 ? 0x43004300u : 0x64006400u;
+  asm volatile("" : "+s"(kmask), "+v"(kmagic));
   constexpr float kOffset = DT == SUBSPEC_BF16 ? 128.f : 1024.f;
   const uint32_t one2 = DT == SUBSPEC_BF16 ? 0x3f803f80u : 0x3c003c00u;
   const it_u4 ones = it_u4{one2, one2, one2, one2};
@@ -147,33 +152,43 @@ __global__ __launch_bounds__(512) void int4_tile_kernel(Int4TileParams p) {
   if (xrole) wait_vmcnt<(SX - 1) * RX>(); else wait_vmcnt<(SW - 1) * RW>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+  it_u4 b[TA][2];
+  float sc[TA], szo[TA];                                                  // of the chunk whose products were scaled last
+  uint32_t szc[TA];                                                       // (scale, zero) words of the chunk being multiplied
+  it_v4f raw[2][TA], xsum[2];
+  auto dequantize = [&](int t) __attribute__((always_inline)) {
+    auto pair = [&](uint32_t v, int sh) { return ((v >> sh) & kmask) | kmagic; };
+    const uint32_t w0 = w[t].x, w1 = w[t].y;
+    b[t][0] = it_u4{pair(w0, 0), pair(w0, 4), pair(w0, 8), pair(w0, 12)};
+    b[t][1] = it_u4{pair(w1, 0), pair(w1, 4), pair(w1, 8), pair(w1, 12)};
+  };
+  auto scale_tile = [&](int mt, int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr)
+      acc[t][mt][rr] = fmaf(sc[t], raw[mt & 1][t][rr], fmaf(szo[t], xsum[mt & 1][rr], acc[t][mt][rr]));
+    asm volatile("" : "+v"(acc[t][mt][0]), "+v"(acc[t][mt][1]), "+v"(acc[t][mt][2]), "+v"(acc[t][mt][3]));   // (pinned here)
+  };
   read_w(0);
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) read_x(mt, 0);
+#pragma unroll
+  for (int t = 0; t < TA; ++t) {
+    dequantize(t);
+    sc[t] = szo[t] = 0.f;
+    raw[1][t] = it_v4f{0.f, 0.f, 0.f, 0.f};
+  }
+  xsum[1] = it_v4f{0.f, 0.f, 0.f, 0.f};
   for (int it = 0; it < nst; ++it) {
     sync();
     const int xn = xs + 1 == SX ? 0 : xs + 1, wn = ws + 1 == SW ? 0 : ws + 1;
     const uint32_t from = xrole ? xs : ws;
-    it_u4 b[TA][2];
-    float sc[TA], szo[TA];
 #pragma unroll
-    for (int t = 0; t < TA; ++t) {
-      auto pair = [&](uint32_t v, int sh) { return ((v >> sh) & kmask) | kmagic; };
-      const uint32_t w0 = w[t].x, w1 = w[t].y;
-      b[t][0] = it_u4{pair(w0, 0), pair(w0, 4), pair(w0, 8), pair(w0, 12)};
-      b[t][1] = it_u4{pair(w1, 0), pair(w1, 4), pair(w1, 8), pair(w1, 12)};
-      sc[t] = f16_bits_to_float(sz[t] & 0xffffu);
-      szo[t] = -sc[t] * (f16_bits_to_float(sz[t] >> 16) + kOffset);
-    }
+    for (int t = 0; t < TA; ++t) szc[t] = sz[t];
     read_w(wn);
-    it_v4f raw[2][TA], xsum[2];
-    auto scale_tile = [&](int mt, int t) __attribute__((always_inline)) {
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr)
-        acc[t][mt][rr] = fmaf(sc[t], raw[mt & 1][t][rr], fmaf(szo[t], xsum[mt & 1][rr], acc[t][mt][rr]));
-    };
-    // 16 rows at a time; behind their products, so that they are issued while the matrix core works: the next chunk's operands
-    // of these rows and, early, the copies into the slots that this chunk has left
+    // 16 rows at a time; behind their products, so that they are issued while the matrix core works: the scaling of the 16 rows
+    // before (of the last 16 of the chunk before, first), the next chunk's operands of these rows, early the copies into the slots
+    // that this chunk has left, and at the end, tile by tile behind its last product, the next chunk's codes.  Nothing but the
+    // barrier stands between two chunks' products: the two wavefronts of a SIMD run in step, so what one does alone both do.
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
 #pragma unroll
@@ -184,17 +199,29 @@ __global__ __launch_bounds__(512) void int4_tile_kernel(Int4TileParams p) {
       for (int t = 0; t < TA; ++t) {
         r[t] = it_mfma<DT>(x[mt][0], b[t][0], it_v4f{0.f, 0.f, 0.f, 0.f});
         if (t == 0) xsum[mt & 1] = it_mfma<DT>(x[mt][1], ones, xsum[mt & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        scale_tile((mt + 3) & 3, t);
+        if (mt == 0) {
+          sc[t] = f16_bits_to_float(szc[t] & 0xffffu);
+          szo[t] = -sc[t] * (f16_bits_to_float(szc[t] >> 16) + kOffset);
+          asm volatile("" : "+v"(sc[t]), "+v"(szo[t]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
         r[t] = it_mfma<DT>(x[mt][1], b[t][1], r[t]);
-        if (mt > 0) scale_tile(mt - 1, t);
+        if (mt == 3) {
+          dequantize(t);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(b[t][0][e]), "+v"(b[t][1][e]));
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
       read_x(mt, xn);
     }
-#pragma unroll
-    for (int t = 0; t < TA; ++t) scale_tile(3, t);
     xs = xn;
     ws = wn;
   }
+#pragma unroll
+  for (int t = 0; t < TA; ++t) scale_tile(3, t);
   // every copy has landed and every wavefront is done reading the rings: the space is reused
   wait_vmcnt<0>();
   __syncthreads();

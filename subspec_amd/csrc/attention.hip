@@ -403,6 +403,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 // (head, row); a workgroup takes blockDim.x / 32 rows (8, or 2 when the launch would otherwise be
 // too small to fill the chip).  Slot of (bh, chunk c, row) = (bh * chunks + c) * 64 + row; maxima
 // are stored already multiplied by scale * log2(e).
+constexpr int kMergeUpFront = 24;
 template <int DT>
 __global__ __launch_bounds__(256) void tree_attention_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, AttnParams ap, uint16_t* __restrict__ out) {
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(256) void tree_attention_merge_kernel(
   float m = -INFINITY;
   v4f num = {0.f, 0.f, 0.f, 0.f};
   float den = 0.f;
-  constexpr int kUpFront = 24;
+  constexpr int kUpFront = kMergeUpFront;
   if (ap.chunks <= kUpFront) {
     // the usual case (a draft level has 12 to 18 chunks at prefixes of 2000 to 2400): every load of the launch is issued before the
     // first wait -- one round trip instead of two (the maxima first, then the rows); the sums run in the same order
@@ -1312,7 +1313,15 @@ static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_ro
   // a ping-pong workgroup has a compute unit to itself: one more than fit would be a second round
   // for all (5, 6, 7 sequences of 64 rows, 4096 / 4096 / 2000 keys: 46.3 -> 34.5, 53.9 -> 39.3, 43.6 -> 29.3 us)
   if (pl.pingpong) chunks = std::max<int64_t>(1, target_wgs / wgs_per_chunk);
-  chunks = std::min<int64_t>(chunks, std::max<int64_t>(1, blocks / 2));
+  int64_t most = std::max<int64_t>(1, blocks / 2);
+  // A draft level is round trips: the shortest chunks whose merge still has all its loads in flight (three blocks are one chunk and
+  // no merge).  8 rows, 28 : 4 heads, both launches: 1033 keys 12.1 -> 9.8 us, 2056 12.8 -> 11.3; in chunks of two blocks beyond 24
+  // of them 13.6 -> 14.9 at 4104, which therefore takes three.
+  if (win_rows <= 16 && blocks > 3 && blocks <= 4 * kMergeUpFront) {
+    const int64_t per = (blocks + kMergeUpFront - 1) / kMergeUpFront;
+    most = (blocks + per - 1) / per;
+  }
+  chunks = std::min<int64_t>(chunks, most);
   // ... and the partial results (fp32 rows x 128 per head and chunk) are priced against the K / V bytes (16-bit,
   // 2 x kv_len x 128 per KV head): at most twice as many
   const int64_t by_bytes = std::max<int64_t>(1, 2 * (kv_len * hkv) / std::max<int64_t>(1, hq * win_rows));

@@ -522,33 +522,37 @@ extern "C" size_t subspec_int4_decoder_layer_workspace(const subspec_decoder_lay
   return layer_plan(*dims).total;
 }
 
-static int check_layer_call(const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* x, const int32_t* positions,
-                            const int32_t* cache_rows, const uint64_t* anc_bits, void* k_cache, void* v_cache,
-                            void* workspace, size_t workspace_bytes) {
-  const int rc = check_dims(dims, w.dense ? kDenseLayerMaxRows : kInt4LayerMaxRows);
+// what holds for a whole call, and (check_layer) for each of its layers
+static int check_layer_call(const subspec_decoder_layer_dims* dims, bool dense, void* x, const int32_t* positions,
+                            const int32_t* cache_rows, const uint64_t* anc_bits, void* workspace, size_t workspace_bytes) {
+  const int rc = check_dims(dims, dense ? kDenseLayerMaxRows : kInt4LayerMaxRows);
   if (rc != SUBSPEC_OK) return rc;
   // the wide dense kernels take weight rows in tiles of 32
   if (dims->n_rows > 64 && ((dims->n_q_heads + 2 * dims->n_kv_heads) * dims->head_dim % 32 != 0 || dims->hidden % 32 != 0))
     SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "decoder_layer: more than 64 rows need projection widths that are multiples of 32");
-  if (!x || !positions || !cache_rows || !anc_bits || !k_cache || (!v_cache && !dims->page_indices))
-    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: null pointer argument");
-  if (!w.input_norm || !w.post_norm || !w.qkv.w || !w.o.w || !w.gate_up.w || !w.down.w ||
-      (!w.dense && (!w.qkv.sz || !w.o.sz || !w.gate_up.sz || !w.down.sz)))
-    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: null weight pointer");
-  if ((uintptr_t)x % 16 || (uintptr_t)w.input_norm % 16 || (uintptr_t)w.post_norm % 16 || (uintptr_t)k_cache % 16 ||
-      (uintptr_t)v_cache % 16)
-    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: x, norm weights and caches must be 16-byte aligned");
+  if (!x || !positions || !cache_rows || !anc_bits) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: null pointer argument");
+  if ((uintptr_t)x % 16) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: x, norm weights and caches must be 16-byte aligned");
   const size_t need = layer_plan(*dims).total;
   if (!workspace || workspace_bytes < need)
     SUBSPEC_FAIL(SUBSPEC_ERR_WORKSPACE, "decoder_layer: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
   if ((uintptr_t)workspace % 256) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: workspace must be 256-byte aligned");
   return SUBSPEC_OK;
 }
+static int check_layer(const char* what, const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* k_cache, void* v_cache) {
+  if (!k_cache || (!v_cache && !dims->page_indices)) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "%s: null pointer argument", what);
+  if (!w.input_norm || !w.post_norm || !w.qkv.w || !w.o.w || !w.gate_up.w || !w.down.w ||
+      (!w.dense && (!w.qkv.sz || !w.o.sz || !w.gate_up.sz || !w.down.sz)))
+    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "%s: null weight pointer", what);
+  if ((uintptr_t)w.input_norm % 16 || (uintptr_t)w.post_norm % 16 || (uintptr_t)k_cache % 16 || (uintptr_t)v_cache % 16)
+    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "%s: x, norm weights and caches must be 16-byte aligned", what);
+  return SUBSPEC_OK;
+}
 
 static int decoder_layer_entry(const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* x, const int32_t* positions,
                                const int32_t* cache_rows, const uint64_t* anc_bits, void* k_cache, void* v_cache,
                                void* workspace, size_t workspace_bytes, void* stream) {
-  const int rc = check_layer_call(dims, w, x, positions, cache_rows, anc_bits, k_cache, v_cache, workspace, workspace_bytes);
+  int rc = check_layer_call(dims, w.dense, x, positions, cache_rows, anc_bits, workspace, workspace_bytes);
+  if (rc == SUBSPEC_OK) rc = check_layer("decoder_layer", dims, w, k_cache, v_cache);
   if (rc != SUBSPEC_OK) return rc;
   if (dims->dtype == SUBSPEC_BF16)
     return run_layer<SUBSPEC_BF16>(*dims, w, (uint16_t*)x, positions, cache_rows, anc_bits, (uint16_t*)k_cache, (uint16_t*)v_cache,
@@ -587,11 +591,11 @@ static int decoder_stack_entry(const subspec_decoder_layer_dims* dims, const Wei
                                void* const* k_caches, void* const* v_caches, const void* final_norm, void* h_out,
                                void* workspace, size_t workspace_bytes, void* stream) {
   int rc = check_stack_args(weights, n_layers, k_caches, final_norm, h_out);
+  if (rc == SUBSPEC_OK)
+    rc = check_layer_call(dims, layer_weights(weights[0]).dense, x, positions, cache_rows, anc_bits, workspace, workspace_bytes);
   if (rc != SUBSPEC_OK) return rc;
   for (int64_t i = 0; i < n_layers; ++i)      // every layer is checked before the first one runs
-    if ((rc = check_layer_call(dims, layer_weights(weights[i]), x, positions, cache_rows, anc_bits, k_caches[i],
-                               v_caches ? v_caches[i] : nullptr, workspace, workspace_bytes)))
-      return rc;
+    if ((rc = check_layer("decoder_layer", dims, layer_weights(weights[i]), k_caches[i], v_caches ? v_caches[i] : nullptr))) return rc;
   if (dims->dtype == SUBSPEC_BF16)
     return run_stack<SUBSPEC_BF16>(*dims, weights, n_layers, (uint16_t*)x, positions, cache_rows, anc_bits, k_caches, v_caches,
                                    final_norm, h_out, (char*)workspace, (hipStream_t)stream, false);
@@ -646,21 +650,6 @@ extern "C" size_t subspec_prefill_layer_workspace(const subspec_decoder_layer_di
   return check_prefill(dims) == SUBSPEC_OK ? layer_plan(*dims, true).total : 0;
 }
 
-static int check_prefill_call(const subspec_decoder_layer_dims* dims, const LayerWeights& w, void* x, const int32_t* positions,
-                              const int32_t* cache_rows, void* k_cache, void* v_cache, void* workspace, size_t workspace_bytes) {
-  if (!x || !positions || !cache_rows || !k_cache || (!v_cache && !dims->page_indices) || !w.input_norm || !w.post_norm ||
-      !w.qkv.w || !w.o.w || !w.gate_up.w || !w.down.w)
-    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: null pointer argument");
-  if ((uintptr_t)x % 16 || (uintptr_t)w.input_norm % 16 || (uintptr_t)w.post_norm % 16 || (uintptr_t)k_cache % 16 ||
-      (uintptr_t)v_cache % 16)
-    SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: x, norm weights and caches must be 16-byte aligned");
-  const size_t need = layer_plan(*dims, true).total;
-  if (!workspace || workspace_bytes < need)
-    SUBSPEC_FAIL(SUBSPEC_ERR_WORKSPACE, "prefill_layer: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
-  if ((uintptr_t)workspace % 256) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: workspace must be 256-byte aligned");
-  return SUBSPEC_OK;
-}
-
 extern "C" int subspec_prefill_stack(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights,
                                      int64_t n_layers, void* x, const int32_t* positions, const int32_t* cache_rows,
                                      void* const* k_caches, void* const* v_caches, const void* final_norm, void* h_out,
@@ -668,10 +657,14 @@ extern "C" int subspec_prefill_stack(const subspec_decoder_layer_dims* dims, con
   int rc = check_prefill(dims);
   if (rc == SUBSPEC_OK) rc = check_stack_args(weights, n_layers, k_caches, final_norm, h_out);
   if (rc != SUBSPEC_OK) return rc;
+  if (!x || !positions || !cache_rows) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: null pointer argument");
+  if ((uintptr_t)x % 16) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: x, norm weights and caches must be 16-byte aligned");
   for (int64_t i = 0; i < n_layers; ++i)
-    if ((rc = check_prefill_call(dims, layer_weights(weights[i]), x, positions, cache_rows, k_caches[i], v_caches ? v_caches[i] : nullptr,
-                                 workspace, workspace_bytes)))
-      return rc;
+    if ((rc = check_layer("prefill_layer", dims, layer_weights(weights[i]), k_caches[i], v_caches ? v_caches[i] : nullptr))) return rc;
+  const size_t need = layer_plan(*dims, true).total;
+  if (!workspace || workspace_bytes < need)
+    SUBSPEC_FAIL(SUBSPEC_ERR_WORKSPACE, "prefill_layer: workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
+  if ((uintptr_t)workspace % 256) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "prefill_layer: workspace must be 256-byte aligned");
   if (dims->dtype == SUBSPEC_BF16)
     return run_stack<SUBSPEC_BF16>(*dims, weights, n_layers, (uint16_t*)x, positions, cache_rows, nullptr, k_caches, v_caches,
                                    final_norm, h_out, (char*)workspace, (hipStream_t)stream, true);

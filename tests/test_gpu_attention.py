@@ -240,3 +240,13 @@ def test_large_tree_shorter_than_its_launch():
     assert torch.isfinite(out[1]).all()
     # the two are cut into other key chunks, whose averages are rounded to bf16 (2^-9 each); then one projection
     assert (out[0] - out[1]).norm() <= 1e-2 * (out[0] - x0.float()).norm()
+
+
+# key blocks on both sides of every change in the number of blocks per chunk of a draft level
+@pytest.mark.parametrize("blocks", [3, 4, 24, 25, 48, 49, 96, 97])
+@pytest.mark.parametrize("rows,hq,hkv", [(1, 4, 4), (8, 14, 2), (16, 9, 1)])
+def test_chunks_of_a_draft_level(blocks, rows, hq, hkv):
+    for n_keys in (64 * blocks - 63, 64 * blocks):
+        P = n_keys - rows
+        parents, q, k, v = _case(blocks + rows, 2, hq, hkv, rows, P, n_keys + 3, torch.bfloat16)
+        _check(parents, q, k, v, P, "draft level")

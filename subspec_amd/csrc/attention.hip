@@ -975,7 +975,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const int64_t key0 = (int64_t)chunk * ap.chunk_keys;
-  if (key0 >= kv_len) {                                     // (the whole workgroup, before its first barrier)
+  if (__builtin_expect(key0 >= kv_len, 0)) {                // (the whole workgroup, before its first barrier)
     if constexpr (!CAUSAL) {
       // a chunk of a launch laid out for a longer prefix than the device holds: no weight, and no bits a product could trip over
       if (live) {

@@ -160,7 +160,7 @@ class Decoder:
                 self._native_make = make
                 resident = min(self.first_streamed, len(self.layers))
                 tables = [make(w) for w in self.layers[:resident]]
-                self._native_weights = (type(tables[0]) * resident)(*tables) if tables else ()
+                self._native_weights = ops.layer_table(tables) if tables else ()
                 self._native_ws = {}
         return self._native
 
@@ -293,14 +293,19 @@ class Decoder:
     def _run_layers(self, x, positions, rows, attn, plan=None) -> torch.Tensor:
         state = {"x": x}
         resident = min(self.first_streamed, len(self.layers))
-        if plan is not None and resident and all(self._prefill_takes(plan, w, x) for w in self.layers[:resident]):
-            if plan["ws"] is None:
-                plan["ws"] = torch.empty(plan["need"], dtype=torch.uint8, device=x.device)
-            tables = [ops.dense_layer_weights(w) for w in self.layers[:resident]]
-            ops.prefill_stack_(x, plan["dims"], (type(tables[0]) * resident)(*tables), plan["rows"], plan["rows"],
-                               plan["data"], plan["ws"])
-            resident = 0
-        for i in range(resident):
+        done = 0
+        if plan is not None:
+            # the layers in one call -- two calls, so that the device is at work on the first layers while the host looks at the
+            # tensors of the others (a quarter of a millisecond for 28 layers)
+            for end in (min(2, resident), resident):
+                if done == end or not all(self._prefill_takes(plan, w, x) for w in self.layers[done:end]):
+                    break
+                if plan["ws"] is None:
+                    plan["ws"] = torch.empty(plan["need"], dtype=torch.uint8, device=x.device)
+                table = ops.layer_table([ops.dense_layer_weights(w) for w in self.layers[done:end]])
+                ops.prefill_stack_(x, plan["dims"], table, plan["rows"], plan["rows"], plan["data"][done:], plan["ws"])
+                done = end
+        for i in range(done, resident):
             state["x"] = self._layer(i, self.layers[i], state["x"], positions, rows, attn, plan)
         if self.streamer is not None and self.streamer.n:
             base = self.first_streamed

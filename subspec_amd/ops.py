@@ -587,6 +587,11 @@ def prefill_layer_(x: torch.Tensor, dims: "L.DecoderLayerDims", weights: "L.Dens
     return x
 
 
+def layer_table(layers):
+    """Pointer tables of consecutive layers as the array that the stack calls take."""
+    return (type(layers[0]) * len(layers))(*layers)
+
+
 def _stack_args(x, dims, weights, positions, cache_rows, cache, final_norm, what):
     """Checks of a stack call; the layers' cache pointers (``cache`` [layers, 2, ...], or a page pool [layers, pages, 2, ...]) and
     the final norm's pointers."""

@@ -163,8 +163,8 @@ class PreparedTreeVerify:
     token_ids, parents, **kwargs)`` takes what ``tree_verify`` takes, allocates the workspace and the outputs once and
     holds references to all of them; every ``call()`` then only launches, on the stream that was current when the
     object was made, and returns the same output dictionary.  The tensors are read where they are: the caller writes
-    new logits / tokens / parents INTO them between calls.  64 x 152064 fp32 rows: 12.6 us per call against 18 to 20
-    through ``tree_verify(out=...)`` and 26 to 28 when the outputs are allocated per call.
+    new logits / tokens / parents INTO them between calls.  64 x 152064 fp32 rows: 12.6 us per call against 16
+    through ``tree_verify(out=...)``; outputs that are allocated per call add 8.
     """
 
     def __init__(self, logits: torch.Tensor, token_ids: torch.Tensor, parents: torch.Tensor, **kwargs):

@@ -975,18 +975,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const int64_t key0 = (int64_t)chunk * ap.chunk_keys;
-  if (__builtin_expect(key0 >= kv_len, 0)) {                // (the whole workgroup, before its first barrier)
-    if constexpr (!CAUSAL) {
-      // a chunk of a launch laid out for a longer prefix than the device holds: no weight, and no bits a product could trip over
-      if (live) {
-        uint16_t* po = (uint16_t*)part_o + (((int64_t)vbh * ap.chunks + chunk) * 2 + tile) * kTileElems + lane * 4;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) *(uint2*)(po + i * 256) = make_uint2(0, 0);
-        if (g == 0) *(v2f_t*)(part_ml + (((int64_t)vbh * ap.chunks + chunk) * kAttnRows + row) * 2) = v2f_t{-INFINITY, 0.f};
-      }
-    }
-    return;
-  }
+  if (CAUSAL && key0 >= kv_len) return;                     // (the whole workgroup, before its first barrier)
   const int64_t key1 = min(key0 + ap.chunk_keys, kv_len);
   const int nkeys = (int)(key1 - key0);
   const int nb = (nkeys + kKeyBlock - 1) / kKeyBlock;
@@ -1277,18 +1266,18 @@ __global__ __launch_bounds__(256) void causal_attention_merge_kernel(const float
 
 // Launch shape of one window of query rows.
 struct AttnPlan { int threads, rowt, wph, heads_per_wg, chunks; bool mfma32, pingpong; };
-static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_rows, int64_t kv_len, bool one_window,
-                          bool one_sequence) {
+static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_rows, int64_t kv_len, bool one_sequence) {
   AttnPlan pl;
   const int group = (int)(hq / hkv);
   const int64_t blocks = (kv_len + kKeyBlock - 1) / kKeyBlock;
   pl.mfma32 = win_rows > 16;
-  // the ping-pong kernel pays for its set-up over many blocks: (window, head) pairs enough to fill the chip with few key
-  // chunks.  (`one_window`: one sequence of up to 64 rows, where the kernel before it is level and reads pages by itself; the
-  // windows of a larger tree over pages run here on a contiguous copy of the request's rows, so that they equal the
-  // contiguous cache's bit for bit.)  289 rows of one sequence, 28 : 4 heads, whole call: 40.1 -> 35.1 us at 2337 keys, 60.5 -> 44.1
-  // at 4385, but 26.2 -> 28.7 at 989 and 27.2 -> 31.6 at 353: below 20 key blocks the set-up is not paid for.
-  pl.pingpong = pl.mfma32 && !one_window && batch * hq >= 128 && (!one_sequence || blocks >= 20);
+  // the ping-pong kernel pays for its set-up over many blocks: (sequence, head) pairs enough to fill the chip with few key
+  // chunks.  One sequence never takes it, however many windows its tree has: a request's attention over pages equals the contiguous
+  // one bit for bit, and the ping-pong kernel's probabilities are relative to a reference up to 2^8 below the row's maximum, so that
+  // the largest is rounded where it is exactly 1 in the other kernel.  289 rows, 28 : 4 heads, 2337 keys, distance from float64: 2.81e-3
+  // against 2.70e-3 in bf16 and 3.52e-4 against 3.39e-4 in fp16 (scores three times as large: 2.56e-3, 2.39e-3; 3.19e-4, 2.97e-4), for
+  // 35 against 40 us a call; over pages it would need a copy of the rows (200 rows of 32 : 8 heads, 2500 keys: 41 against 34 us).
+  pl.pingpong = pl.mfma32 && !one_sequence && batch * hq >= 128;
   if (win_rows <= 16) {
     // a draft level: a wavefront is a whole head (one 16-row tile), eight heads share the staged keys
     pl.threads = 512; pl.rowt = 1; pl.wph = 1;
@@ -1337,12 +1326,8 @@ static AttnLaunch attn_launch(int64_t batch, int64_t hq, int64_t hkv, int64_t n_
   al.windows = (int)((n_rows + kAttnRows - 1) / kAttnRows);
   al.win_rows = (int)std::min<int64_t>(n_rows, kAttnRows);
   al.vbatch = batch * al.windows;
-  al.pl = attn_plan(al.vbatch, hq, hkv, al.win_rows, kv_len, al.vbatch == 1, batch == 1);
+  al.pl = attn_plan(al.vbatch, hq, hkv, al.win_rows, kv_len, batch == 1);
   return al;
-}
-// the contiguous K and V of a paged request whose windows run on the ping-pong kernel
-static size_t attn_gather_bytes(const AttnLaunch& al, int64_t batch, int64_t hkv, int64_t kv_len) {
-  return batch == 1 && al.pl.pingpong ? (size_t)(2 * hkv * kv_len) * kAttnD * 2 : 0;
 }
 
 }  // namespace subspec
@@ -1359,10 +1344,9 @@ extern "C" size_t subspec_tree_attention_workspace(int64_t batch, int64_t n_q_he
                                                    int64_t prefix_len, int64_t n_tree_slots) {
   if (batch <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads != 0 || n_rows <= 0) return 256;
   const AttnLaunch al = attn_launch(batch, n_q_heads, n_kv_heads, n_rows, prefix_len + n_tree_slots);
-  const size_t gather = attn_gather_bytes(al, batch, n_kv_heads, prefix_len + n_tree_slots);
-  if (al.pl.chunks == 1) return std::max<size_t>(256, gather);
+  if (al.pl.chunks == 1) return 256;
   size_t o_bytes;
-  return attn_partial_bytes(al.vbatch, n_q_heads, al.pl.chunks, &o_bytes) + gather;
+  return attn_partial_bytes(al.vbatch, n_q_heads, al.pl.chunks, &o_bytes);
 }
 
 static int tree_attention_impl(const char* what, const void* q, const void* k_cache, const void* v_cache, void* out, int dtype,
@@ -1417,26 +1401,15 @@ static int tree_attention_impl(const char* what, const void* q, const void* k_ca
   const AttnLaunch al = attn_launch(batch, n_q_heads, n_kv_heads, n_rows, kv_len);
   const AttnPlan& pl = al.pl;
   const int64_t vbatch = al.vbatch;
-  const size_t gather = paged ? attn_gather_bytes(al, batch, n_kv_heads, kv_len) : 0;
-  if (pl.chunks > 1 || gather) {
-    size_t o_bytes = 0;
-    const size_t partials = pl.chunks > 1 ? attn_partial_bytes(vbatch, n_q_heads, pl.chunks, &o_bytes) : 0, need = partials + gather;
+  if (pl.chunks > 1) {
+    size_t o_bytes;
+    const size_t need = attn_partial_bytes(vbatch, n_q_heads, pl.chunks, &o_bytes);
     if (!workspace || workspace_bytes < need)
       SUBSPEC_FAIL(SUBSPEC_ERR_WORKSPACE, "%s: workspace of %zu bytes is smaller than the %zu required", what,
                    workspace_bytes, need);
     if ((uintptr_t)workspace % 16) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "%s: workspace must be 16-byte aligned", what);
     part_o = (float*)workspace;
     part_ml = (float*)((char*)workspace + o_bytes);
-    if (gather) {
-      uint16_t* rows = (uint16_t*)((char*)workspace + partials);
-      gather_pages(make_kv_row_map((void*)k_cache, nullptr, kv_seq_stride, n_kv_heads, paged), kv_len, rows,
-                   rows + n_kv_heads * kv_len * kAttnD, (hipStream_t)stream);
-      k_cache = rows;
-      v_cache = rows + n_kv_heads * kv_len * kAttnD;
-      ap.seq_stride = kv_len;
-      ap.page_table = nullptr;
-      paged = nullptr;
-    }
   }
   hipStream_t st = (hipStream_t)stream;
   {
@@ -1464,7 +1437,7 @@ static int tree_attention_impl(const char* what, const void* q, const void* k_ca
     {                                                                                                              \
       DominantKernelTimer timer(st);                                                                               \
       if (!pl.mfma32) SUBSPEC_ATTN_KERNEL(DT, PAGED, 1, 1, 512);                                                   \
-      else if (pl.pingpong) {                                                                            \
+      else if (pl.pingpong && !PAGED) {                                                                            \
         if (pl.wph == 1) SUBSPEC_ATTNPP_KERNEL(DT, 1); else SUBSPEC_ATTNPP_KERNEL(DT, 2);                          \
       }                                                                                                            \
       else if (pl.wph == 1) SUBSPEC_ATTN32_KERNEL(DT, PAGED, 1, 512);                                              \

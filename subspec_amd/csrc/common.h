@@ -271,8 +271,6 @@ inline KvRowMap make_kv_row_map(void* k_cache, void* v_cache, int64_t seq_stride
   }
   return m;
 }
-// rows 0 .. rows - 1 of a request's pages as contiguous [hkv, rows, 128] K and V (rows outside the pages are left out)
-void gather_pages(const KvRowMap& kv, int64_t rows, void* k_out, void* v_out, hipStream_t st);
 // subspec_tree_attention (batch 1, head_dim 128) with two options of the decoder-layer entry points: prefix_dev (the
 // kernel reads the prefix length from device memory, prefix_len is its upper bound) and pages (k_cache = one layer of
 // a page pool, v_cache unused)

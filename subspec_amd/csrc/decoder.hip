@@ -281,11 +281,6 @@ __global__ __launch_bounds__(256) void gather_pages_kernel(KvRowMap kv, int64_t 
   v_out[o] = ((const dec_u4*)v)[piece];
 }
 
-void gather_pages(const KvRowMap& kv, int64_t rows, void* k_out, void* v_out, hipStream_t st) {
-  const int64_t pieces = rows * kv.hkv * 16;
-  hipLaunchKernelGGL(gather_pages_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, kv, rows, (dec_u4*)k_out, (dec_u4*)v_out);
-}
-
 // rows of one call: the int4 stack serves draft levels and post-verify windows, the dense stack also whole large trees
 constexpr int kInt4LayerMaxRows = 64, kDenseLayerMaxRows = 384, kPrefillMaxRows = 65536;
 struct LayerPlan {
@@ -433,7 +428,8 @@ static int run_layer(const subspec_decoder_layer_dims& s, const LayerWeights& w,
     if (pg) {
       kk = (const uint16_t*)(ws + p.kv);
       vv = kk + KV * rows;
-      gather_pages(kv, rows, ws + p.kv, (uint16_t*)(ws + p.kv) + KV * rows, st);
+      const int64_t pieces = rows * KV / 8;
+      hipLaunchKernelGGL(gather_pages_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, kv, rows, (dec_u4*)kk, (dec_u4*)vv);
     }
     if ((rc = causal_attention(q, kk, vv, a, DT, Hq, Hkv, M, pg ? rows : s.kv_seq_stride, s.prefix_len, 1.f / sqrtf((float)D), sub, st)))
       return rc;

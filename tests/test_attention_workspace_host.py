@@ -1,0 +1,19 @@
+"""Sizes of the attention workspace, from the library's host code alone."""
+import pytest
+
+from subspec_amd import _lib as L
+
+
+def _bytes(batch, hq, hkv, rows, prefix, slots):
+    return L.lib().subspec_tree_attention_workspace(batch, hq, hkv, rows, prefix, slots)
+
+
+@pytest.mark.parametrize("hq,hkv", [(28, 4), (32, 8), (32, 32), (64, 8)])
+@pytest.mark.parametrize("rows", [65, 128, 200, 289, 512])
+def test_large_trees_hold_partials_only(hq, hkv, rows):
+    """The fp32-sized partials of all rows in whole windows, at most 64 chunks of them; nothing that grows with the cache."""
+    windows = (rows + 63) // 64
+    for prefix in (100, 1300, 2048, 8192, 131072):
+        chunks, rest = divmod(_bytes(1, hq, hkv, rows, prefix, rows), windows * hq * 64 * (128 * 4 + 8))
+        assert rest in (0, 256) and chunks <= 64
+    assert _bytes(1, hq, hkv, rows, 65536, rows) == _bytes(1, hq, hkv, rows, 262144, rows)

@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void tree_attention_merge_kernel(
   float den = 0.f;
   constexpr int kUpFront = kMergeUpFront;
   if (ap.chunks <= kUpFront) {
-    // the usual case (a draft level has 12 to 18 chunks at prefixes of 2000 to 2400): every load of the launch is issued before the
+    // the usual case (a draft level has 17 to 20 chunks at prefixes of 2000 to 2400): every load of the launch is issued before the
     // first wait -- one round trip instead of two (the maxima first, then the rows); the sums run in the same order
     v2f_t ml[kUpFront];
     v4f oc[kUpFront];
@@ -1302,19 +1302,25 @@ static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_ro
   // a ping-pong workgroup has a compute unit to itself: one more than fit would be a second round
   // for all (5, 6, 7 sequences of 64 rows, 4096 / 4096 / 2000 keys: 46.3 -> 34.5, 53.9 -> 39.3, 43.6 -> 29.3 us)
   if (pl.pingpong) chunks = std::max<int64_t>(1, target_wgs / wgs_per_chunk);
-  int64_t most = std::max<int64_t>(1, blocks / 2);
-  // A draft level is round trips: the shortest chunks whose merge still has all its loads in flight (three blocks are one chunk and
-  // no merge).  8 rows, 28 : 4 heads, both launches: 1033 keys 12.1 -> 9.8 us, 2056 12.8 -> 11.3; in chunks of two blocks beyond 24
-  // of them 13.6 -> 14.9 at 4104, which therefore takes three.
-  if (win_rows <= 16 && blocks > 3 && blocks <= 4 * kMergeUpFront) {
-    const int64_t per = (blocks + kMergeUpFront - 1) / kMergeUpFront;
-    most = (blocks + per - 1) / per;
-  }
-  chunks = std::min<int64_t>(chunks, most);
   // ... and the partial results (fp32 rows x 128 per head and chunk) are priced against the K / V bytes (16-bit,
   // 2 x kv_len x 128 per KV head): at most twice as many
   const int64_t by_bytes = std::max<int64_t>(1, 2 * (kv_len * hkv) / std::max<int64_t>(1, hq * win_rows));
-  chunks = std::min<int64_t>(chunks, by_bytes);
+  const int64_t wanted = std::min(chunks, by_bytes);
+  chunks = std::min<int64_t>(wanted, std::max<int64_t>(1, blocks / 2));
+  // A draft level is round trips: the shortest chunks whose merge still has all its loads in flight (three blocks are one chunk and
+  // no merge), as long as every workgroup starts at once and the merge stays small.  Both launches: 8 rows of 28 : 4 heads, 1033 keys
+  // 12.1 -> 9.8 us, 2056 12.8 -> 11.3; but two sequences of 16 : 8 heads at 2108 (272 workgroups) 13.7 -> 16.4, one row of 32 : 32 heads
+  // at 1001 (512) 12.1 -> 14.1, 16 rows of two sequences of 28 : 4 at 1516 (21504 partial rows) 14.3 -> 15.4.  Where these are fewer chunks
+  // than half the blocks they save the merge's second pass (8 rows of 28 : 4 heads at 6008 20.4 -> 15.6), unless they
+  // fill a second round for longer (two sequences of 16 : 8 heads at 4801, 416 -> 304 workgroups: 21.6 -> 23.1).
+  if (win_rows <= 16 && blocks > 3 && blocks <= 4 * kMergeUpFront) {
+    const int64_t per = (blocks + kMergeUpFront - 1) / kMergeUpFront, brief = std::min(wanted, (blocks + per - 1) / per);
+    auto rounds = [&](int64_t c) { return (wgs_per_chunk * c + 255) / 256 * ((blocks + c - 1) / c); };
+    const bool one_round = wgs_per_chunk * brief <= 256;
+    if (brief <= chunks ? one_round || rounds(brief) <= rounds(chunks)
+                        : one_round && batch * hq * win_rows * brief <= (brief <= 12 ? 13312 : 10240))
+      chunks = brief;
+  }
   pl.chunks = (int)std::min<int64_t>(chunks, 64);
   return pl;
 }

@@ -278,3 +278,11 @@ def test_chunks_of_a_draft_level(blocks, rows, hq, hkv):
         P = n_keys - rows
         parents, q, k, v = _case(blocks + rows, 2, hq, hkv, rows, P, n_keys + 3, torch.bfloat16)
         _check(parents, q, k, v, P, "draft level")
+
+
+# levels whose short chunks would be more workgroups than compute units, or more partial rows than the merge is worth: chunks of two blocks
+@pytest.mark.parametrize("B,rows,hq,hkv,n_keys", [(2, 8, 16, 8, 2100), (2, 1, 16, 8, 4801), (1, 8, 32, 32, 1008), (4, 16, 32, 32, 266),
+                                                  (2, 16, 28, 4, 1516), (4, 16, 28, 4, 416), (2, 16, 64, 8, 416)])
+def test_chunks_of_a_wide_draft_level(B, rows, hq, hkv, n_keys):
+    parents, q, k, v = _case(n_keys, B, hq, hkv, rows, n_keys - rows, n_keys + 3, torch.bfloat16)
+    _check(parents, q, k, v, n_keys - rows, "wide draft level")

@@ -1264,8 +1264,9 @@ __global__ __launch_bounds__(256) void causal_attention_merge_kernel(const float
       make_uint2(pack2<DT>(num.x * inv, num.y * inv), pack2<DT>(num.z * inv, num.w * inv));
 }
 
-// Launch shape of one window of query rows.
-struct AttnPlan { int threads, rowt, wph, heads_per_wg, chunks; bool mfma32, pingpong; };
+// Launch shape of one window of query rows.  most_chunks: what the workspace is sized for, at least the chunks of this key count and of
+// every smaller one (a draft level has 24 chunks at 3072 keys and 17 at 3073; a workspace serves all prefixes up to the one it was made for).
+struct AttnPlan { int threads, rowt, wph, heads_per_wg, chunks, most_chunks; bool mfma32, pingpong; };
 static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_rows, int64_t kv_len, bool one_sequence) {
   AttnPlan pl;
   const int group = (int)(hq / hkv);
@@ -1307,6 +1308,8 @@ static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_ro
   const int64_t by_bytes = std::max<int64_t>(1, 2 * (kv_len * hkv) / std::max<int64_t>(1, hq * win_rows));
   const int64_t wanted = std::min(chunks, by_bytes);
   chunks = std::min<int64_t>(wanted, std::max<int64_t>(1, blocks / 2));
+  const int64_t most = win_rows <= 16 && blocks > 3 ? std::min(wanted, std::max(chunks, std::min<int64_t>(blocks, kMergeUpFront))) : chunks;
+  pl.most_chunks = (int)std::min<int64_t>(most, 64);
   // A draft level is round trips: the shortest chunks whose merge still has all its loads in flight (three blocks are one chunk and
   // no merge), as long as every workgroup starts at once and the merge stays small.  Both launches: 8 rows of 28 : 4 heads, 1033 keys
   // 12.1 -> 9.8 us, 2056 12.8 -> 11.3; but two sequences of 16 : 8 heads at 2108 (272 workgroups) 13.7 -> 16.4, one row of 32 : 32 heads
@@ -1350,9 +1353,9 @@ extern "C" size_t subspec_tree_attention_workspace(int64_t batch, int64_t n_q_he
                                                    int64_t prefix_len, int64_t n_tree_slots) {
   if (batch <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads != 0 || n_rows <= 0) return 256;
   const AttnLaunch al = attn_launch(batch, n_q_heads, n_kv_heads, n_rows, prefix_len + n_tree_slots);
-  if (al.pl.chunks == 1) return 256;
+  if (al.pl.most_chunks == 1) return 256;
   size_t o_bytes;
-  return attn_partial_bytes(al.vbatch, n_q_heads, al.pl.chunks, &o_bytes);
+  return attn_partial_bytes(al.vbatch, n_q_heads, al.pl.most_chunks, &o_bytes);
 }
 
 static int tree_attention_impl(const char* what, const void* q, const void* k_cache, const void* v_cache, void* out, int dtype,

@@ -179,7 +179,7 @@ __device__ int prune_list(uint64_t* list, int count, uint64_t cut, int* counter)
 template <int DT, int VEC, int U>
 __global__ __launch_bounds__(kTopkThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void topk_slice_kernel(
     const void* __restrict__ probs, const void* __restrict__ parent_probs, int64_t vocab, int leaves, int splits,
-    int64_t chunk, int k, uint64_t* __restrict__ cand, uint64_t* __restrict__ cand_cut,
+    int64_t chunk, int k, uint64_t* __restrict__ cand,
     int64_t* __restrict__ token_ids, void* __restrict__ topk_probs, int64_t* __restrict__ parent_indices) {
   __shared__ uint64_t list[kTopkCap];
   __shared__ uint64_t kth_slot;
@@ -438,47 +438,84 @@ __global__ __launch_bounds__(kTopkThreads) __attribute__((amdgpu_waves_per_eu(8,
     }
     return;
   }
-  // k slots (0: empty) and the slice's k-th best, below which nothing of the whole result can lie (0: fewer than k elements)
+  // k slots, 0: empty
   const int64_t slot0 = (row * splits + c) * kTopkMaxK;
   if (tid < k) cand[slot0 + tid] = tid < cnt ? list[tid] : 0;
-  if (tid == 0) cand_cut[row * splits + c] = tau;
 }
 
-// The best k of all slices' lists.  The largest of the slices' k-th bests is reached by k elements, so it cuts the candidates to
-// little more than k before they are ranked against each other; cuts and candidates are requested together (one round trip).
-// 8 leaves x 152064, k = 8 (512 candidates then, 1216 now): 10.4 us ranking all of them against each other, 5.2 now; with 16 leaves
-// and k = 16 the whole call 93 -> 18 us.
+// The best k of all slices' lists.  Candidates are ranked by counting, which takes their number squared, so a longer list is cut
+// before: of the bests of 16 lanes (four candidates each; 64 or 16 such bests in all), the k-th largest is reached by k candidates.  The
+// lanes of a group hold slots of many lists, so that no leaf or slice with most of the best fills a group of its own.
+// 8 leaves x 152064 bf16, k = 8 (1216 candidates), slices and merge: 19.1 us ranking all, 11.5 cut; where every slice holds k - 1 elements
+// above all others' k-th (a cut by the largest of the slices' k-th bests keeps 1065 of them) 22.7 and 40.7, now 12.5.  16 leaves, k = 16:
+// 94 -> 14.2; 2 leaves, k = 64 36 -> 20.6.  Up to this many candidates ranking all of them is the shorter way (one row in two slices, k = 64:
+// 11.9 us, 14.3 with the cut).
+inline __host__ __device__ int merge_rank_all(int k) { return k <= 8 ? 64 : k <= 32 ? 128 : 256; }
+__device__ __forceinline__ uint64_t row_max(uint64_t v) {               // maximum over the lane's row of 16, in all of them
+  auto step = [&](auto ctrl) __attribute__((always_inline)) {
+    constexpr int kCtrl = decltype(ctrl)::value;                         // row_ror
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)v, kCtrl, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(v >> 32), kCtrl, 0xf, 0xf, true);
+    v = max(v, (uint64_t)hi << 32 | lo);
+  };
+  step(std::integral_constant<int, 0x128>{});
+  step(std::integral_constant<int, 0x124>{});
+  step(std::integral_constant<int, 0x122>{});
+  step(std::integral_constant<int, 0x121>{});
+  return v;
+}
 template <int DT, int THREADS>
 __global__ __launch_bounds__(THREADS) void topk_merge_kernel(
-    const uint64_t* __restrict__ cand, const uint64_t* __restrict__ cand_cut, int64_t vocab, int leaves, int splits,
+    const uint64_t* __restrict__ cand, int64_t vocab, int leaves, int splits,
     int k, int64_t* __restrict__ token_ids, void* __restrict__ topk_probs, int64_t* __restrict__ parent_indices) {
-  constexpr int kPer = 4;                              // leaves * splits * k <= 4 THREADS
+  constexpr int kPer = 4, kGroups = THREADS / 16;      // leaves * splits * k <= 4 THREADS, k <= kGroups
   __shared__ uint64_t list[kPer * THREADS];
-  __shared__ uint64_t wave_cut[THREADS / kWave];
+  __shared__ uint64_t group_best[kGroups], bound;
   __shared__ int total;
-  const int b = blockIdx.x, tid = threadIdx.x;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1);
   const int lists = leaves * splits, slots = lists * k;
-  uint64_t own[kPer];
+  uint64_t own[kPer];                                  // (an empty slot is 0)
 #pragma unroll
   for (int p = 0; p < kPer; ++p) {
     own[p] = 0;
     if (p * THREADS < slots) {                         // (uniform)
-      const uint32_t s = (uint32_t)min(p * THREADS + tid, slots - 1), li = s / (uint32_t)k;
-      own[p] = cand[((int64_t)b * lists + li) * kTopkMaxK + (s - li * (uint32_t)k)];
+      const int mine = p * THREADS + (tid & 15) * kGroups + tid / 16;     // (16 lanes hold slots of many lists)
+      const uint32_t s = (uint32_t)min(mine, slots - 1), li = s / (uint32_t)k;
+      const uint64_t v = cand[((int64_t)b * lists + li) * kTopkMaxK + (s - li * (uint32_t)k)];
+      own[p] = mine < slots ? v : 0;
     }
   }
-  uint64_t cut = 1;                                    // (an empty slot is 0)
-  for (int li = tid; li < lists; li += THREADS) cut = max(cut, cand_cut[(int64_t)b * lists + li]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) cut = max(cut, (uint64_t)__shfl_xor((unsigned long long)cut, o, kWave));
-  if ((tid & (kWave - 1)) == 0) wave_cut[tid / kWave] = cut;
   if (tid == 0) total = 0;
-  __syncthreads();
+  uint64_t cut = 1;
+  if (slots > merge_rank_all(k)) {                         // (uniform)
+    const uint64_t best = row_max(max(max(own[0], own[1]), max(own[2], own[3])));
+    if (tid % 16 == 0) group_best[tid / 16] = best;
+    __syncthreads();
+    if (tid < kWave) {                                 // one wavefront: all of them would queue for the LDS reads
+      const uint64_t mine = group_best[lane % kGroups];
+      int rank = 0;
 #pragma unroll
-  for (int w = 0; w < THREADS / kWave; ++w) cut = max(cut, wave_cut[w]);
+      for (int g = 0; g < kGroups; ++g) rank += group_best[g] > mine || (group_best[g] == mine && g < lane % kGroups);
+      if (rank == k - 1 && lane < kGroups) bound = mine;
+    }
+    __syncthreads();
+    cut = max(cut, bound);
+  } else {
+    __syncthreads();
+  }
+  int kept = 0, before[kPer];                          // of the wavefront
+#pragma unroll
+  for (int p = 0; p < kPer; ++p) {
+    const uint64_t passed = __ballot(own[p] >= cut);
+    before[p] = kept + __builtin_amdgcn_mbcnt_hi((uint32_t)(passed >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)passed, 0));
+    kept += __popcll(passed);
+  }
+  int first = 0;
+  if (lane == 0 && kept) first = atomicAdd(&total, kept);
+  first = __builtin_amdgcn_readfirstlane(first);
 #pragma unroll
   for (int p = 0; p < kPer; ++p)
-    if (p * THREADS + tid < slots && own[p] >= cut) list[atomicAdd(&total, 1)] = own[p];
+    if (own[p] >= cut) list[first + before[p]] = own[p];
   __syncthreads();
   const int cnt = total;
   for (int i = tid; i < cnt; i += THREADS) {
@@ -516,7 +553,7 @@ static bool topk_plan(const void* probs, int dtype, int64_t rows, int64_t vocab,
 
 template <int DT>
 static int run_topk(const void* probs, const void* parent_probs, int64_t batch, int leaves, int64_t vocab, int k,
-                    const TopkPlan& pl, uint64_t* cand, uint64_t* cand_cut, int64_t* token_ids, void* topk_probs,
+                    const TopkPlan& pl, uint64_t* cand, int64_t* token_ids, void* topk_probs,
                     int64_t* parent_indices, hipStream_t st) {
   const dim3 grid(pl.splits, (unsigned)(batch * leaves));
   {
@@ -524,26 +561,26 @@ static int run_topk(const void* probs, const void* parent_probs, int64_t batch, 
     constexpr int kVecFull = DT == SUBSPEC_F32 ? 4 : 8;
     if (pl.vec == 1)
       hipLaunchKernelGGL((topk_slice_kernel<DT, 1, 4>), grid, dim3(kTopkThreads), 0, st, probs, parent_probs, vocab, leaves,
-                         pl.splits, pl.chunk, k, cand, cand_cut, token_ids, topk_probs, parent_indices);
+                         pl.splits, pl.chunk, k, cand, token_ids, topk_probs, parent_indices);
     else if (pl.chunk / kVecFull >= 2 * (int64_t)kTopkThreads * 8)
       hipLaunchKernelGGL((topk_slice_kernel<DT, kVecFull, 8>), grid, dim3(kTopkThreads), 0, st, probs,
-                         parent_probs, vocab, leaves, pl.splits, pl.chunk, k, cand, cand_cut, token_ids, topk_probs,
+                         parent_probs, vocab, leaves, pl.splits, pl.chunk, k, cand, token_ids, topk_probs,
                          parent_indices);
     else if (pl.chunk / kVecFull > 2 * (int64_t)kTopkThreads)
       hipLaunchKernelGGL((topk_slice_kernel<DT, kVecFull, 4>), grid, dim3(kTopkThreads), 0, st, probs,
-                         parent_probs, vocab, leaves, pl.splits, pl.chunk, k, cand, cand_cut, token_ids, topk_probs,
+                         parent_probs, vocab, leaves, pl.splits, pl.chunk, k, cand, token_ids, topk_probs,
                          parent_indices);
     else
       hipLaunchKernelGGL((topk_slice_kernel<DT, kVecFull, 2>), grid, dim3(kTopkThreads), 0, st, probs,
-                         parent_probs, vocab, leaves, pl.splits, pl.chunk, k, cand, cand_cut, token_ids, topk_probs,
+                         parent_probs, vocab, leaves, pl.splits, pl.chunk, k, cand, token_ids, topk_probs,
                          parent_indices);
   }
   const int slots = leaves * pl.splits * k;
-  if (leaves * pl.splits > 1 && slots <= kMergeCap / 4)
+  if (leaves * pl.splits > 1 && (slots <= merge_rank_all(k) || (slots <= kMergeCap / 4 && k <= 8)))
     hipLaunchKernelGGL((topk_merge_kernel<DT, kMergeThreads / 4>), dim3((unsigned)batch), dim3(kMergeThreads / 4), 0, st, cand,
-                       cand_cut, vocab, leaves, pl.splits, k, token_ids, topk_probs, parent_indices);
+                       vocab, leaves, pl.splits, k, token_ids, topk_probs, parent_indices);
   else if (leaves * pl.splits > 1)
-    hipLaunchKernelGGL((topk_merge_kernel<DT, kMergeThreads>), dim3((unsigned)batch), dim3(kMergeThreads), 0, st, cand, cand_cut,
+    hipLaunchKernelGGL((topk_merge_kernel<DT, kMergeThreads>), dim3((unsigned)batch), dim3(kMergeThreads), 0, st, cand,
                      vocab, leaves, pl.splits, k, token_ids, topk_probs, parent_indices);
   SUBSPEC_CHECK_HIP(hipGetLastError());
   return SUBSPEC_OK;
@@ -557,7 +594,7 @@ extern "C" size_t subspec_topk_expand_workspace(int64_t batch, int64_t leaves, i
   (void)vocab; (void)k;
   if (batch <= 0 || leaves <= 0) return 256;
   const size_t lists = (size_t)batch * leaves * kTopkMaxSlices;
-  return align_up(lists * kTopkMaxK * sizeof(uint64_t), 256) + align_up(lists * sizeof(uint64_t), 256);
+  return align_up(lists * kTopkMaxK * sizeof(uint64_t), 256);
 }
 
 extern "C" int subspec_topk_expand(const void* probs, const void* parent_probs, int dtype, int64_t batch,
@@ -584,19 +621,17 @@ extern "C" int subspec_topk_expand(const void* probs, const void* parent_probs, 
   if (!topk_plan(probs, dtype, batch * leaves, vocab, k, (int)leaves, &pl))
     SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "topk_expand: leaves=%lld x k=%d candidates exceed the merge capacity",
                  (long long)leaves, k);
-  const size_t lists = (size_t)batch * leaves * kTopkMaxSlices;
   uint64_t* cand = (uint64_t*)workspace;
-  uint64_t* cand_cut = (uint64_t*)((char*)workspace + align_up(lists * kTopkMaxK * sizeof(uint64_t), 256));
   hipStream_t st = (hipStream_t)stream;
   switch (dtype) {
     case SUBSPEC_F32:
-      return run_topk<SUBSPEC_F32>(probs, parent_probs, batch, (int)leaves, vocab, k, pl, cand, cand_cut, token_ids,
+      return run_topk<SUBSPEC_F32>(probs, parent_probs, batch, (int)leaves, vocab, k, pl, cand, token_ids,
                                    topk_probs, parent_indices, st);
     case SUBSPEC_F16:
-      return run_topk<SUBSPEC_F16>(probs, parent_probs, batch, (int)leaves, vocab, k, pl, cand, cand_cut, token_ids,
+      return run_topk<SUBSPEC_F16>(probs, parent_probs, batch, (int)leaves, vocab, k, pl, cand, token_ids,
                                    topk_probs, parent_indices, st);
     default:
-      return run_topk<SUBSPEC_BF16>(probs, parent_probs, batch, (int)leaves, vocab, k, pl, cand, cand_cut,
+      return run_topk<SUBSPEC_BF16>(probs, parent_probs, batch, (int)leaves, vocab, k, pl, cand,
                                     token_ids, topk_probs, parent_indices, st);
   }
 }

@@ -180,3 +180,22 @@ def test_softmax_slices(dtype, V, offset):
     tiny = 2.0 ** -24 if dtype == torch.float16 else 1e-38              # half-precision probabilities are subnormal below 6e-5
     assert ((got.double() - want).abs() <= 1.01 * eps * want + tiny + (2.0 ** -18 + 2.0 ** -20) * want).all()
     assert got[0, 7] == 0
+
+
+# Rows that leave a cut by the slices' k-th bests nearly all candidates: every stretch of `width` elements holds k - 1 large values,
+# and the k-th of it is small.  One leaf of many, few and many slots, both forms of the merge.
+@pytest.mark.parametrize("B,L,V,k,width", [(1, 8, 152064, 8, 8192), (1, 16, 32768, 16, 8192), (1, 8, 65536, 64, 8192), (2, 2, 40000, 64, 4096),
+                                           (1, 4, 50257, 8, 16384), (1, 64, 9000, 64, 4096), (3, 1, 152064, 32, 16384), (1, 32, 20000, 1, 4096)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_merge_of_crowded_slices(dtype, B, L, V, k, width):
+    print("topk crowded", dtype, B, L, V, k, flush=True)
+    g = torch.Generator().manual_seed(V + k)
+    probs = torch.rand(B, L, V, generator=g) * 1e-3
+    for lo in range(0, V, width):
+        n = min(k - 1, V - lo)
+        probs[:, :, lo:lo + n] = 0.5 + 0.4 * torch.rand(B, L, n, generator=g)
+    parent = torch.rand(B, L, generator=g) * 0.1 + 0.9
+    one_leaf = parent * 1e-2
+    one_leaf[:, L // 2] = 1.0                                          # all of the best in one leaf's lists
+    for p in (parent, one_leaf):
+        _check(probs.to(dtype), p.to(dtype), k)

@@ -27,8 +27,6 @@ constexpr int kTopkCap = 1024;          // candidate slots per workgroup
 constexpr int kTopkPruneAt = 512;       // careful mode prunes above this; one step adds at most 512
 constexpr int kTopkMaxK = 64;
 constexpr int kTopkMaxSlices = 64;
-// Slices of several leaves: two groups of 16-bit tiles.  A slice is a chain of steps behind one load, which a shorter one leaves as
-// it is; only its scan gets shorter: 8 leaves x 152064 8.8 us in slices of 20480, 7.3 in these.
 constexpr int64_t kTopkShortSlice = 8192;
 constexpr int kMergeThreads = 1024;
 constexpr int kMergeCap = 4096;
@@ -538,13 +536,20 @@ static bool topk_plan(const void* probs, int dtype, int64_t rows, int64_t vocab,
   const bool aligned = (vocab % vec_full == 0) && ((uintptr_t)probs % 16 == 0);
   pl->vec = aligned ? vec_full : 1;
   const int64_t quantum = (int64_t)kTopkThreads * pl->vec;
+  // Several leaves: slices of at most 8192 elements (two groups of 16-bit tiles) of equal length, as long as they are few -- a slice is a
+  // chain of steps behind one load, and only its scan gets shorter.  k = 8, 16384-element slices against these: 8 leaves x 152064 (152
+  // slices) 11.9 -> 11.5 us, 8 x 32000 12.0 -> 9.9; 32 x 32000 of 8 rows (1024) 14.1 -> 16.3, 4 x 152064 of 8 rows, k = 1 (608) 10.1 -> 12.2.
+  // One leaf per result, or rows below 16384: slices long enough that short rows need no merge launch (4 x 9000, k = 16: 10.4 -> 11.9).  A
+  // slice much shorter than the others has too few tiles for a bound and ranks all its elements (8192 + 808: 9.0 -> 30.5 us).
+  const int64_t brief = (vocab + kTopkShortSlice - 1) / kTopkShortSlice;
+  const bool cut_short = leaves > 1 && vocab >= 16384 && rows * brief <= (k > 1 ? 512 : 256);
   int64_t splits = (1024 + rows - 1) / rows;
-  // (one leaf per result: slices long enough that short rows need no merge launch)
-  splits = std::min<int64_t>(splits, leaves > 1 ? (vocab + kTopkShortSlice - 1) / kTopkShortSlice : std::max<int64_t>(1, vocab / 16384));
+  splits = std::min<int64_t>(splits, cut_short ? brief : std::max<int64_t>(1, vocab / 16384));
   splits = std::min<int64_t>(splits, std::max<int64_t>(1, kMergeCap / ((int64_t)leaves * k)));
   splits = std::max<int64_t>(1, std::min<int64_t>(splits, kTopkMaxSlices));
+  const int64_t unit = cut_short ? (int64_t)kWave * pl->vec : quantum;
   int64_t chunk = (vocab + splits - 1) / splits;
-  chunk = (chunk + quantum - 1) / quantum * quantum;
+  chunk = (chunk + unit - 1) / unit * unit;
   splits = (vocab + chunk - 1) / chunk;
   pl->splits = (int)splits;
   pl->chunk = chunk;

@@ -199,3 +199,14 @@ def test_merge_of_crowded_slices(dtype, B, L, V, k, width):
     one_leaf[:, L // 2] = 1.0                                          # all of the best in one leaf's lists
     for p in (parent, one_leaf):
         _check(probs.to(dtype), p.to(dtype), k)
+
+
+# on both sides of each line between short and long slices (rows of 16384, 512 short slices, 256 at k = 1), last slices of every length
+@pytest.mark.parametrize("B,L,V,k", [(1, 2, 16383, 8), (1, 2, 16384, 8), (1, 3, 16392, 16), (2, 4, 20008, 64), (8, 16, 32768, 8), (8, 16, 32776, 8),
+                                     (8, 8, 32768, 1), (8, 8, 32776, 1), (1, 4, 24584, 64), (1, 2, 67040, 16)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_lengths_of_slices(dtype, B, L, V, k):
+    print("topk slice lengths", dtype, B, L, V, k, flush=True)
+    g = torch.Generator().manual_seed(V + k)
+    probs = torch.softmax(torch.randn(B, L, V, generator=g) * 3, -1).to(dtype)
+    _check(probs, torch.rand(B, L, generator=g).to(dtype), k)

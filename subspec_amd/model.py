@@ -111,6 +111,21 @@ def _linear(w: Dict[str, torch.Tensor], name: str, x: torch.Tensor) -> torch.Ten
     return F.linear(x, w[name + ".weight"], bias)
 
 
+def tiled_head(rows: int, vocab: int, hidden: int) -> bool:
+    """Whether a 16-bit language-model head over more than 64 rows runs on the tiled kernel of this package.  That kernel and the
+    vendor GEMM cut the head into tiles of 160 and 256 rows, and which of them fills its last round over the 256 compute units
+    decides; both were timed at some 70 heads and 8 row counts between 193 and 384.  Heads of 147456 to 158719 rows (3.6 to 3.9 rounds here)
+    take 0.60 to 1.01 of the GEMM's time up to 320 rows (152064 x 3584, 289 rows: 332 against 414 us) and 0.87 to 0.98 up to 384 where
+    a row has 2560 elements (1024: 1.08); heads of 128000 to 130047 rows of 3072 elements and more 0.73 to 0.95 (2048: 1.06).  At others
+    the GEMM is level or ahead at some row count: 65536 x 2048 1.13 to 1.18, 50304 x 4096 1.06 to 1.11, 32000 x 5120 1.11 to 1.27, 131072 x
+    4096 1.10 to 1.19, 262144 x 1152 1.03 to 1.21, and at all heads with 65 to 192 rows (152064 x 3584, 96 rows: 221 against 232 us)."""
+    if not (192 < rows <= 384 and vocab % 32 == 0 and hidden % 64 == 0 and (1 << 28) <= 2 * vocab * hidden < (1 << 31)):
+        return False
+    if 147456 <= vocab < 158720:
+        return rows <= 320 or hidden >= 2560
+    return 128000 <= vocab < 130048 and hidden >= 3072
+
+
 class Decoder:
     """One decoder stack over a shared KV cache.  ``layers[i]`` holds either bf16 weights or int4
     packed weights; layers from ``first_streamed`` on are fetched through ``streamer``."""
@@ -320,10 +335,8 @@ class Decoder:
         """Final norm and the language-model head (HuggingFace ``lm_head`` inside the draft and target forwards,
         specdecodes/models/draft_models/classic_sd.py:10-16, generators/classic_sd.py:102-109).  Up to 64 rows the
         1.09 GB head streams through the dense kernels of this package (152064 x 3584 bf16: 170 us at 8 rows, 198 us at 32
-        against 232 / 255 us for the vendor GEMM; 204 us at 64 rows, where the two are level).  From 193 to 384 rows the tiled
-        kernel takes heads that do not stay in the 256 MB memory-side cache (289 rows: 343 against 419 us, 193 rows 285 against
-        319, 384 rows 419 against 452; a 32000 x 2048 head 42 against 38).  The vendor GEMM keeps 65 to 192 rows (96 rows: 221
-        against 232 us, level at 128 and 160) and more than 384."""
+        against 232 / 255 us for the vendor GEMM; 204 us at 64 rows, where the two are level).  Wider inputs take the tiled kernel
+        where ``tiled_head`` says so and the vendor GEMM elsewhere."""
         return self._head(rms_norm(x, self.norm, self.cfg.rms_norm_eps))
 
     def _head(self, h: torch.Tensor) -> torch.Tensor:
@@ -334,7 +347,7 @@ class Decoder:
             if rows <= 64:
                 own = V % 32 == 0 if rows > 32 else V % 16 == 0 and V * H * 2 < (1 << 31)
             else:
-                own = 192 < rows <= 384 and V % 32 == 0 and (1 << 28) <= V * H * 2 < (1 << 31) and self.lm_head.data_ptr() % 16 == 0
+                own = tiled_head(rows, V, H) and self.lm_head.data_ptr() % 16 == 0
             if own:
                 return ops.dense_linear(h, self.lm_head)
         return F.linear(h, self.lm_head)

@@ -202,24 +202,31 @@ def test_dense_gate_up_projection_with_the_activation_in_its_output_stage(dtype)
         assert ((got.float() - want.float()).abs() <= 2 * ulp * want.float().abs() + 1e-6).all()
 
 
-@pytest.mark.parametrize("rows", [192, 193, 289, 384, 385])
+# rows on both sides of the lines between the tiled kernel and the library, on heads that the former takes up to 384 rows, up to 320 and never
+@pytest.mark.parametrize("V,H,upto", [(147456, 2560, 384), (158688, 960, 320), (128000, 3072, 384), (131072, 1088, 0), (147424, 960, 0), (158720, 960, 0)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_head_of_a_large_tree(rows, dtype):
-    """Rows on both sides of the lines between the tiled kernel and the library, on the smallest head that the former takes."""
+def test_head_of_a_large_tree(V, H, upto, dtype, monkeypatch):
     from subspec_amd import model as M
-    cfg = M.DecoderConfig(num_hidden_layers=1, hidden_size=256, num_attention_heads=2, num_key_value_heads=1, head_dim=128,
-                          intermediate_size=128, vocab_size=524288)
-    g = torch.Generator(device=DEV).manual_seed(rows)
-    head = (torch.randn(cfg.vocab_size, 256, generator=g, device=DEV) * 0.05).to(dtype)
-    x = torch.randn(rows, 256, generator=g, device=DEV).to(dtype)
+    cfg = M.DecoderConfig(num_hidden_layers=1, hidden_size=H, num_attention_heads=2, num_key_value_heads=1, head_dim=128,
+                          intermediate_size=128, vocab_size=V)
+    g = torch.Generator(device=DEV).manual_seed(V)
+    head = (torch.randn(V, H, generator=g, device=DEV) * 0.05).to(dtype)
     kv = create_kv_cache("static", max_cache_len=8, config=cfg, device=DEV, dtype=dtype)
-    d = M.Decoder(cfg, head[:64], [], torch.ones(256, dtype=dtype, device=DEV), head, kv)
-    got = d.logits(x)
-    h = ops.rms_norm(x, torch.ones(256, dtype=dtype, device=DEV), cfg.rms_norm_eps).float()
-    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)               # one rounding of the result; fp32 sums of 256 products
-    for lo in range(0, cfg.vocab_size, 65536):
-        want = h @ head[lo:lo + 65536].float().t()
-        assert ((got[:, lo:lo + 65536].float() - want).abs() <= eps * want.abs() + 1e-4).all()
+    d = M.Decoder(cfg, head[:64], [], torch.ones(H, dtype=dtype, device=DEV), head, kv)
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)               # one rounding of the result; fp32 sums of up to 3072 products
+    own, calls = ops.dense_linear, []
+    monkeypatch.setattr(ops, "dense_linear", lambda *a: calls.append(a[0].shape[0]) or own(*a))
+    for rows in (192, 193, 289, 320, 321, 384, 385):
+        x = torch.randn(rows, H, generator=g, device=DEV).to(dtype)
+        got = d.logits(x)
+        assert calls == ([rows] if 192 < rows <= upto else []), (V, H, rows)
+        calls.clear()
+        if rows not in (193, 320, 384):
+            continue
+        h = ops.rms_norm(x, torch.ones(H, dtype=dtype, device=DEV), cfg.rms_norm_eps).float()
+        for lo in range(0, V, 65536):
+            want = h @ head[lo:lo + 65536].float().t()
+            assert ((got[:, lo:lo + 65536].float() - want).abs() <= eps * want.abs() + 1e-4).all()
 
 
 # rings of two, four and five weight tiles: fewer chunks of 64 than slots, as many, one more; workgroups with a tile less than the ring

@@ -584,20 +584,25 @@ static bool wide_applies(int64_t M, int64_t N) { return M > 32 && M <= kWideMaxR
 template <int DT, bool SILU>
 static void launch_wide(const WideParams& p, const WidePlan& pl, hipStream_t st) {
   const dim3 grid((unsigned)pl.wgs, (unsigned)pl.splits);
-  // rows <= 64: the kernel streams, each weight byte once, and requests it as streaming data.  That pays only if no line is
-  // requested twice, so the ring has as many tiles as the plan gives a workgroup (rings of five for two or four tiles fill up with
-  // repeats, which come from memory again: 4608 x 3584 15.6 -> 18.3 us); 64 rows, weights from HBM, with the reduction: 37888 x 3584
-  // with the activation 52.0 -> 45.6 us (6.0 TB/s), 3584 x 3584 14.5 -> 13.6, 4608 x 3584 15.7 -> 15.0, 3584 x 18944 33.8 -> 32.6,
-  // 32000 x 2048 36.1 -> 32.6; 152064 x 3584 205 -> 206 (33 rows 196 -> 188).  Deeper rings alone: nothing.
+  // rows <= 64: the kernel streams, each weight byte once.  The ring has as many tiles as the plan gives a workgroup (a ring of five for two
+  // or four tiles fills up with repeats) and four slots: the requests go on behind a range's last chunk, so that every wait names one
+  // count, which is SW - 1 repeats of it for ranges of 7 to 37 chunks, and two workgroups of two tiles share a compute unit's LDS.
+  // 64 rows, weights from HBM, with the reduction, ring of five tiles -> as deep as LDS allows (ten slots of two, six of four) -> four:
+  // 3584 x 3584 13.2 -> 13.3 -> 12.7 us, 4608 x 3584 14.4 -> 14.7 -> 14.0, 4096 x 4096 13.7 -> 14.6 -> 13.7, 4096 x 2048 11.7 -> 12.0
+  // -> 11.0, 8192 x 8192 41.0 -> 37.6 -> 36.6, 3584 x 18944 32.6 -> 32.6 -> 31.5, 4096 x 14336 29.2 -> 31.0 -> 28.9, 3584 x 8960 20.9
+  // -> 22.4 -> 20.2.  Two tiles and five request their weights as streaming data (37888 x 3584 with the activation 52.6 -> 48.3, 32000 x
+  // 2048 31.3 -> 29.6, 152064 x 3584 203 -> 206, 33 rows 200 -> 191; 8192 x 8192 without 38.8), four tiles where ranges are long (52 chunks,
+  // 6144 x 16384: 47.3 -> 44.8; 112, 8192 x 28672: 90.7 -> 82.5; but 18, 3584 x 8960: 20.2 -> 21.7, 37, 3584 x 18944: 31.5 -> 31.9).
   // <= 256 rows: three activation slots; <= 384: two (LDS holds no more beside the weights)
   if (p.M <= 64) {
     if constexpr (!SILU) {
       if (pl.tiles == 2) {
-        hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 2, 10, 6, 4, 2, 4, 2, false, true>), grid, dim3(512), 0, st, p);
+        hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 2, 4, 4, 4, 2, 4, 2, false, true>), grid, dim3(512), 0, st, p);
         return;
       }
       if (pl.tiles == 4) {
-        hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 4, 6, 6, 4, 4, 4, 2, false, true>), grid, dim3(512), 0, st, p);
+        if (pl.chunks_per_split > 44) hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 4, 4, 4, 4, 4, 4, 2, false, true>), grid, dim3(512), 0, st, p);
+        else hipLaunchKernelGGL((dense_wide_kernel<DT, 2, 1, 4, 4, 4, 4, 4, 4, 2, false>), grid, dim3(512), 0, st, p);
         return;
       }
     }

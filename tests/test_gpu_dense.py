@@ -231,7 +231,7 @@ def test_head_of_a_large_tree(V, H, upto, dtype, monkeypatch):
 
 # rings of two, four and five weight tiles: fewer chunks of 64 than slots, as many, one more; workgroups with a tile less than the ring
 @pytest.mark.parametrize("M", [33, 64])
-@pytest.mark.parametrize("N,K", [(32, 64), (96, 576), (160, 640), (96, 704), (160, 8256), (224, 8320), (30720, 192), (30752, 256), (30784, 320)])
+@pytest.mark.parametrize("N,K", [(32, 64), (32, 128), (96, 192), (64, 256), (96, 320), (96, 576), (160, 640), (96, 704), (160, 8256), (224, 8320), (30720, 192), (30752, 256), (30784, 320), (10240, 10240)])
 def test_streamed_weight_rings(M, N, K):
     g = torch.Generator(device=DEV).manual_seed(N + K + M)
     x = torch.randn(M, K, generator=g, device=DEV).bfloat16()

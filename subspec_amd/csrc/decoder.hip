@@ -28,29 +28,32 @@
 namespace subspec {
 
 // x[m] (+= delta[m], rounded, written back) ; y[m] = w * round(x * rsqrt(mean(x^2) + eps))
-// One workgroup per row; H % 8 == 0, P 16-byte pieces per thread cover H <= 512 * 8 * P.
+// One workgroup per row; H % 8 == 0, P 16-byte pieces per thread cover H <= THREADS * 8 * P.
 // splits > 0: delta is not a 16-bit tensor yet but `splits` fp32 partial sums [splits][rows][H] of a projection whose K
 // was split over workgroups; they are summed in split order and rounded here (what the projection's own reduction
 // launch would have stored), which saves that launch.
-// A launch of this size is a chain of memory round trips and nothing else, so there is ONE before the sum of squares: the row, the
-// gain and four partials at a time are requested together.  In the
+// A launch of this size is a chain of memory round trips and nothing else, so there are as few as can be before the sum of squares:
+// one for the row, the gain and the first four partials together, one more for every further four.  In the
 // target's forward over 64 rows, with the partials of the o projection: 5.4 us with the gain behind the sum and the partials one
 // after the other, 4.9 now (289 rows 6.0, with six partials of the down projection as well 7.5); an empty launch takes 3.0.
-constexpr int kNormThreads = 512;
-constexpr int kNormMaxPieces = 4;
-template <int DT, bool kAdd, int P>
-__global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(uint16_t* __restrict__ x, const uint16_t* __restrict__ delta,
+// Few rows take as many threads as there are pieces (64 rows, 3584 wide: 2.6 us with 512 threads, 2.8 with 256 and two pieces each).  From
+// 512 rows on the loads of all workgroups count: small ones, and no more pieces than the row has.  2048 rows, bf16, 512 threads with one
+// or four pieces -> this: 896 wide 4.6 -> 3.6 us, 4096 6.9 -> 6.8, 4104 8.9 -> 6.9, 5120 9.2 -> 7.6, 6144 10.0 -> 8.4 (256 threads and up to
+// eight pieces, bound by a test around each, before the loads moved up: 4.3, 7.0, 7.7, 8.8, 10.3).
+constexpr int kNormMaxHidden = 16384;
+template <int DT, bool kAdd, int THREADS, int P>
+__global__ __launch_bounds__(THREADS) void add_rmsnorm_kernel(uint16_t* __restrict__ x, const uint16_t* __restrict__ delta,
                                                                    const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                                    int H, float eps, const float* __restrict__ partial,
                                                                    int splits) {
-  __shared__ float scratch[kNormThreads / kWave];
+  __shared__ float scratch[THREADS / kWave];
   const int m = blockIdx.x, tid = threadIdx.x, pieces = H / 8;
   dec_u4* xr = (dec_u4*)(x + (int64_t)m * H);
   dec_u4 xv[P], gain[P];
   float v[P][8];
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int i = min(p * kNormThreads + tid, pieces - 1);
+    const int i = min(p * THREADS + tid, pieces - 1);
     xv[p] = xr[i];
     gain[p] = ((const dec_u4*)w)[i];
   }
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(uint16_t* __r
         float4 q[P][4][2];
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-          const int i = min(p * kNormThreads + tid, pieces - 1);
+          const int i = min(p * THREADS + tid, pieces - 1);
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
             const float4* pp = (const float4*)(partial + ((int64_t)min(s0 + s, splits - 1) * gridDim.x + m) * H) + 2 * i;
@@ -88,13 +91,13 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(uint16_t* __r
         for (int j = 0; j < 8; ++j) v[p][j] = Elem<DT>::round(v[p][j]);
     } else {
 #pragma unroll
-      for (int p = 0; p < P; ++p) unpack8<DT>(((const dec_u4*)(delta + (int64_t)m * H))[min(p * kNormThreads + tid, pieces - 1)], v[p]);
+      for (int p = 0; p < P; ++p) unpack8<DT>(((const dec_u4*)(delta + (int64_t)m * H))[min(p * THREADS + tid, pieces - 1)], v[p]);
     }
   }
   float ss = 0.f;
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int i = p * kNormThreads + tid;
+    const int i = p * THREADS + tid;
     float xf[8];
     unpack8<DT>(xv[p], xf);
 #pragma unroll
@@ -110,11 +113,11 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(uint16_t* __r
       for (int j = 0; j < 8; ++j) ss = fmaf(v[p][j], v[p][j], ss);
     }
   }
-  const float tot = block_sum<kNormThreads>(ss, scratch);
+  const float tot = block_sum<THREADS>(ss, scratch);
   const float r = rsqrtf(tot / (float)H + eps);
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int i = p * kNormThreads + tid;
+    const int i = p * THREADS + tid;
     if (i < pieces) {
       float wv[8], o[8];
       unpack8<DT>(gain[p], wv);
@@ -128,17 +131,26 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(uint16_t* __r
 template <int DT>
 static void launch_norm(uint16_t* x, const uint16_t* delta, const void* w, uint16_t* y, int64_t rows, int H, float eps,
                         const float* partial, int splits, hipStream_t st) {
-#define SUBSPEC_NORM(ADD, P)                                                                                                       \
-  hipLaunchKernelGGL((add_rmsnorm_kernel<DT, ADD, P>), dim3((unsigned)rows), dim3(kNormThreads), 0, st, x, delta, (const uint16_t*)w, \
-                     y, H, eps, partial, splits)
-  const bool one = H <= 8 * kNormThreads;
-  if (delta || splits > 0) {
-    if (one) SUBSPEC_NORM(true, 1);
-    else SUBSPEC_NORM(true, kNormMaxPieces);
-  } else {
-    if (one) SUBSPEC_NORM(false, 1);
-    else SUBSPEC_NORM(false, kNormMaxPieces);
+  auto launch = [&](auto threads, auto p) {
+    constexpr int kThreads = decltype(threads)::value, kP = decltype(p)::value;
+    if (delta || splits > 0)
+      hipLaunchKernelGGL((add_rmsnorm_kernel<DT, true, kThreads, kP>), dim3((unsigned)rows), dim3(kThreads), 0, st, x, delta,
+                         (const uint16_t*)w, y, H, eps, partial, splits);
+    else
+      hipLaunchKernelGGL((add_rmsnorm_kernel<DT, false, kThreads, kP>), dim3((unsigned)rows), dim3(kThreads), 0, st, x, delta,
+                         (const uint16_t*)w, y, H, eps, partial, splits);
+  };
+#define SUBSPEC_NORM(THREADS, P) launch(std::integral_constant<int, THREADS>{}, std::integral_constant<int, P>{})
+  if (H <= 2048) SUBSPEC_NORM(256, 1);
+  else if (H <= 8192 && rows >= 512) {
+    if (H <= 4096) SUBSPEC_NORM(256, 2);
+    else if (H <= 6144) SUBSPEC_NORM(256, 3);
+    else SUBSPEC_NORM(256, 4);
   }
+  else if (H <= 4096) SUBSPEC_NORM(512, 1);
+  else if (H <= 8192) SUBSPEC_NORM(512, 2);
+  else if (H <= 12288) SUBSPEC_NORM(512, 3);
+  else SUBSPEC_NORM(512, 4);
 #undef SUBSPEC_NORM
 }
 
@@ -327,9 +339,9 @@ static int check_dims(const subspec_decoder_layer_dims* s, int max_rows) {
   if (s->n_rows < 1 || s->n_rows > max_rows)
     SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "decoder_layer: n_rows=%lld outside 1..%d", (long long)s->n_rows, max_rows);
   if (s->head_dim != 128) SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "decoder_layer: head_dim=%lld (built for 128)", (long long)s->head_dim);
-  if (s->hidden <= 0 || s->hidden % 64 != 0 || s->hidden > 8 * kNormThreads * kNormMaxPieces)
+  if (s->hidden <= 0 || s->hidden % 64 != 0 || s->hidden > kNormMaxHidden)
     SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "decoder_layer: hidden=%lld must be a multiple of 64 and at most %d", (long long)s->hidden,
-                 8 * kNormThreads * kNormMaxPieces);
+                 kNormMaxHidden);
   if (s->intermediate <= 0 || s->intermediate % 64 != 0)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "decoder_layer: intermediate=%lld must be a multiple of 64", (long long)s->intermediate);
   if (s->n_q_heads <= 0 || s->n_kv_heads <= 0 || s->n_q_heads % s->n_kv_heads != 0)
@@ -500,9 +512,9 @@ extern "C" int subspec_rms_norm(const void* x, const void* weight, void* y, int 
   if (dtype != SUBSPEC_BF16 && dtype != SUBSPEC_F16) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "rms_norm: dtype %d not supported (bf16 / fp16)", dtype);
   if (!x || !weight || !y) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "rms_norm: null pointer argument");
   if (rows <= 0 || rows > 0x7fffffff) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "rms_norm: rows=%lld", (long long)rows);
-  if (hidden <= 0 || hidden % 8 != 0 || hidden > 8 * kNormThreads * kNormMaxPieces)
+  if (hidden <= 0 || hidden % 8 != 0 || hidden > kNormMaxHidden)
     SUBSPEC_FAIL(SUBSPEC_ERR_LIMIT, "rms_norm: hidden=%lld must be a multiple of 8 and at most %d", (long long)hidden,
-                 8 * kNormThreads * kNormMaxPieces);
+                 kNormMaxHidden);
   if (!(eps > 0.f)) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "rms_norm: eps out of range");
   if ((uintptr_t)x % 16 || (uintptr_t)weight % 16 || (uintptr_t)y % 16) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "rms_norm: pointers must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;

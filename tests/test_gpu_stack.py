@@ -50,3 +50,21 @@ def test_stack_equals_layers(kind, rows, hidden, dtype):
             ops.decoder_stack_(x, dims, array, pos, pos, bits, *rest)
         assert torch.isfinite(x).all() and torch.equal(x, want) and torch.equal(kv.cache.data, rows_after)
         assert h is None if final_norm is None else torch.equal(h, ops.rms_norm(want, gain, 1e-6))
+
+
+# widths at the ends of every number of threads and pieces per thread, row counts on both sides of the line between them
+@pytest.mark.parametrize("hidden", [8, 2048, 2056, 4096, 4104, 6144, 6152, 8192, 8200, 12288, 12296, 16384])
+@pytest.mark.parametrize("rows", [1, 511, 512])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_norm_at_every_width(dtype, rows, hidden):
+    g = torch.Generator(device=DEV).manual_seed(hidden + rows)
+    x = torch.randn(rows, hidden, generator=g, device=DEV).to(dtype)
+    x[:, -8:] *= 30                                                     # a last piece that counts
+    w = (torch.rand(hidden, generator=g, device=DEV) + 0.5).to(dtype)
+    got = ops.rms_norm(x, w, 1e-6).double()
+    xd = x.double()
+    want = w.double() * (xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-6))
+    # two roundings to 16 bits; the fp32 sum of squares and its root are off by less than 2^-16.  Half-precision values below 2^-14 are
+    # spaced 2^-24: the normalized one is off by 2^-25, times a gain of up to 1.5, the product by another 2^-25
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert ((got - want).abs() <= (2.1 * eps + 2.0 ** -16) * want.abs() + 2.5 * 2.0 ** -25).all()

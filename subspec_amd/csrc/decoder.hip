@@ -553,6 +553,10 @@ static int check_layer(const char* what, const subspec_decoder_layer_dims* dims,
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "%s: null weight pointer", what);
   if ((uintptr_t)w.input_norm % 16 || (uintptr_t)w.post_norm % 16 || (uintptr_t)k_cache % 16 || (uintptr_t)v_cache % 16)
     SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "%s: x, norm weights and caches must be 16-byte aligned", what);
+  // what the projections would refuse in the middle of a stack
+  for (const Projection& p : {w.qkv, w.o, w.gate_up, w.down})
+    if ((uintptr_t)p.w % 16 || (!w.dense && (uintptr_t)p.sz % 16))
+      SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "%s: projection weights must be 16-byte aligned", what);
   return SUBSPEC_OK;
 }
 

@@ -50,6 +50,12 @@ _VERIFY_OUT = (("tokens", "n", torch.int64), ("contexts", "n", torch.int64), ("c
                ("target", "rows", torch.int64), ("entropy", "rows", torch.float32), ("child_prob", "rows", torch.float32))
 
 
+def _named(table, value, default: str):
+    """Entry of ``value`` (any case, blanks around it; empty or None: ``default``), or None.  A name as it stands in the table takes one look."""
+    found = table.get(value) if type(value) is str else None
+    return table.get(str(value or default).strip().lower()) if found is None else found
+
+
 def tree_verify(
     logits: torch.Tensor,            # [B, rows, V] or [rows, V]
     token_ids: torch.Tensor,         # int32 [B, n] or [n], device
@@ -96,14 +102,10 @@ def tree_verify(
     n = token_ids.shape[1]
     if token_ids.shape[0] != B:
         raise ValueError(f"batch mismatch: logits {B} vs tree arrays {token_ids.shape[0]}")
-    method = _METHODS.get(verify_method)
-    if method is None:
-        method = _METHODS.get(str(verify_method or "exact").strip().lower())
+    method = _named(_METHODS, verify_method, "exact")
     if method is None:
         raise ValueError(f"Unsupported verify_method: {verify_method!r} (supported: 'exact', 'lossy')")
-    gate = _GATES.get(threshold_method)
-    if gate is None:
-        gate = _GATES.get(str(threshold_method or "entropy").strip().lower())
+    gate = _named(_GATES, threshold_method, "entropy")
     if gate is None:
         raise ValueError(f"Unsupported threshold_method: {threshold_method!r} (supported: 'entropy', 'prob')")
     logits = logits.contiguous()

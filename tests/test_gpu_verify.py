@@ -423,3 +423,20 @@ def test_large_trees_up_to_the_node_limit(n):
                                     target_tokens=drawn)
             got_t, got_c, got_m = _unpack(smp)
             assert (got_t, got_c, got_m) == (want[0], want[1], want[2]), (n, rows, method, "sampled")
+
+
+def test_method_and_gate_names():
+    """Names in any case, empty values of any type for the default, values that no dictionary can look up."""
+    logits = torch.zeros(1, 2, 64, device=DEV)
+    logits[0, :, 5] = 1
+    tree = (torch.tensor([[3, 5]], dtype=torch.int32, device=DEV), torch.tensor([[-1, 0]], dtype=torch.int32, device=DEV))
+    want = ops.tree_verify(logits, *tree)
+    for value in ("exact", " Exact ", "", None, [], ()):
+        got = ops.tree_verify(logits, *tree, verify_method=value)
+        assert all(torch.equal(got[k], want[k]) for k in ("counts", "target")), value   # (tokens behind the path are never written)
+    for value in ("greedy", ["exact"], {"exact"}, 3):
+        with pytest.raises(ValueError, match="verify_method"):
+            ops.tree_verify(logits, *tree, verify_method=value)
+    for value in ("margin", ["prob"], {1: 2}):
+        with pytest.raises(ValueError, match="threshold_method"):
+            ops.tree_verify(logits, *tree, verify_method="lossy", threshold_method=value)

@@ -68,3 +68,47 @@ def test_norm_at_every_width(dtype, rows, hidden):
     # spaced 2^-24: the normalized one is off by 2^-25, times a gain of up to 1.5, the product by another 2^-25
     eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     assert ((got - want).abs() <= (2.1 * eps + 2.0 ** -16) * want.abs() + 2.5 * 2.0 ** -25).all()
+
+
+# a stack over a page pool in another order, with the prefix length on the host, on the device, and on the device below the launch's bound
+@pytest.mark.parametrize("kind,rows", [("int4", 8), ("int4", 40), ("dense", 64), ("dense", 289)])
+@pytest.mark.parametrize("loose", [None, 0, 900])
+def test_stack_over_pages(kind, rows, loose):
+    print("stack over pages", kind, rows, loose, flush=True)
+    prefix, layers, page, hkv = 1350, 2, 16, 4
+    bound = prefix + (loose or 0)
+    n_pages = (bound + rows + page - 1) // page
+    cfg = M.DecoderConfig(num_hidden_layers=layers, hidden_size=512, num_attention_heads=28, num_key_value_heads=hkv, head_dim=128,
+                          intermediate_size=512, vocab_size=64)
+    w = M.init_weights(cfg, rows, DEV, torch.bfloat16)["layers"]
+    w = M.quantize_layers(w) if kind == "int4" else w
+    make = ops.decoder_layer_weights if kind == "int4" else ops.dense_layer_weights
+    table = ops.layer_table([make(l) for l in w])
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    cache = torch.randn(layers, 2, 1, hkv, n_pages * page, 128, generator=g, device=DEV).bfloat16()
+    order = torch.randperm(n_pages + 3, generator=torch.Generator().manual_seed(1))[:n_pages].to(DEV)
+    pool = torch.full((layers, n_pages + 3, 2, page, hkv, 128), float("nan"), device=DEV, dtype=torch.bfloat16)
+    for i in range(layers):
+        for part in range(2):
+            pool[i, order, part] = cache[i, part, 0].transpose(0, 1).reshape(n_pages, page, hkv, 128)
+    x0 = torch.randn(rows, 512, generator=g, device=DEV).bfloat16()
+    at = torch.arange(prefix, prefix + rows, dtype=torch.int32, device=DEV)
+    bits = ops.ancestor_bits_tensor([-1] + [max(0, i - 3) for i in range(rows - 1)], device=DEV)
+    gain = torch.ones(512, device=DEV, dtype=torch.bfloat16)
+    out = {}
+    for name, data, paging, length, dev in (
+            ("tight", cache.clone(), {}, prefix, None),
+            ("contiguous", cache.clone(), {}, bound, None if loose is None else torch.tensor([prefix], device=DEV)),
+            ("paged", pool, dict(page_indices=order.to(torch.int32), max_pages=n_pages + 3, page_len=page), bound,
+             None if loose is None else torch.tensor([prefix], device=DEV))):
+        dims = ops.decoder_layer_dims(torch.bfloat16, rows, 512, 512, 28, hkv, 128, n_pages * page, length, rows, 1e-6, 1e6,
+                                      prefix_len_dev=dev, **paging)
+        x, ws = x0.clone(), torch.full((ops.decoder_layer_workspace(dims),), 0xff, dtype=torch.uint8, device=DEV)
+        out[name] = (x, ops.decoder_stack_(x, dims, table, at, at, bits, data, ws, gain), data)
+    for a, b in zip(out["paged"][:2], out["contiguous"][:2]):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+    written = out["paged"][2][:, order].permute(0, 2, 4, 1, 3, 5).reshape(layers, 2, 1, hkv, -1, 128)
+    assert torch.equal(written, out["contiguous"][2])
+    # another bound cuts the keys into other chunks: averages that differ by 2^-9 of a layer's update (a tenth of x), and with them the
+    # rounding of some elements of x, by one unit of at most 2^-7 of the element; together well below 2^-8 of x
+    assert (out["paged"][0] - out["tight"][0]).float().norm() <= 2.0 ** -8 * out["tight"][0].float().norm()

@@ -36,10 +36,11 @@ namespace subspec {
 // one for the row, the gain and the first four partials together, one more for every further four.  In the
 // target's forward over 64 rows, with the partials of the o projection: 5.4 us with the gain behind the sum and the partials one
 // after the other, 4.9 now (289 rows 6.0, with six partials of the down projection as well 7.5); an empty launch takes 3.0.
-// Few rows take as many threads as there are pieces (64 rows, 3584 wide: 2.6 us with 512 threads, 2.8 with 256 and two pieces each).  From
-// 512 rows on the loads of all workgroups count: small ones, and no more pieces than the row has.  2048 rows, bf16, 512 threads with one
-// or four pieces -> this: 896 wide 4.6 -> 3.6 us, 4096 6.9 -> 6.8, 4104 8.9 -> 6.9, 5120 9.2 -> 7.6, 6144 10.0 -> 8.4 (256 threads and up to
-// eight pieces, bound by a test around each, before the loads moved up: 4.3, 7.0, 7.7, 8.8, 10.3).
+// Few rows take as many threads as there are pieces (64 rows, 3584 wide: 2.6 us with 512 threads, 2.8 with 256 and two pieces each).  Where
+// that leaves threads without a piece, from 512 rows on the loads of all workgroups count: small ones, and no more pieces than the
+// row has.  2048 rows, bf16, 512 threads with one or four pieces -> this: 896 wide 4.6 -> 3.6 us, 4104 8.9 -> 6.9, 5120 9.2 -> 7.6, 6144
+// 10.0 -> 8.4 (256 threads and up to eight pieces, a test around each, before the loads moved up: 4.3, 7.7, 8.8, 10.3); 4096 wide,
+// 256 threads and two pieces, 6.9 -> 6.8 alone and level in a forward, stays at 512.
 constexpr int kNormMaxHidden = 16384;
 template <int DT, bool kAdd, int THREADS, int P>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_kernel(uint16_t* __restrict__ x, const uint16_t* __restrict__ delta,
@@ -142,12 +143,11 @@ static void launch_norm(uint16_t* x, const uint16_t* delta, const void* w, uint1
   };
 #define SUBSPEC_NORM(THREADS, P) launch(std::integral_constant<int, THREADS>{}, std::integral_constant<int, P>{})
   if (H <= 2048) SUBSPEC_NORM(256, 1);
+  else if (H <= 4096) SUBSPEC_NORM(512, 1);
   else if (H <= 8192 && rows >= 512) {
-    if (H <= 4096) SUBSPEC_NORM(256, 2);
-    else if (H <= 6144) SUBSPEC_NORM(256, 3);
+    if (H <= 6144) SUBSPEC_NORM(256, 3);
     else SUBSPEC_NORM(256, 4);
   }
-  else if (H <= 4096) SUBSPEC_NORM(512, 1);
   else if (H <= 8192) SUBSPEC_NORM(512, 2);
   else if (H <= 12288) SUBSPEC_NORM(512, 3);
   else SUBSPEC_NORM(512, 4);

@@ -347,7 +347,8 @@ class Decoder:
             if rows <= 64:
                 own = V % 32 == 0 if rows > 32 else V % 16 == 0 and V * H * 2 < (1 << 31)
             else:
-                own = tiled_head(rows, V, H) and self.lm_head.data_ptr() % 16 == 0
+                own = (tiled_head(rows, V, H) and self.lm_head.data_ptr() % 16 == 0      # (no gradients there)
+                       and not (torch.is_grad_enabled() and (h.requires_grad or self.lm_head.requires_grad)))
             if own:
                 return ops.dense_linear(h, self.lm_head)
         return F.linear(h, self.lm_head)

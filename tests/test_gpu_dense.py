@@ -229,6 +229,23 @@ def test_head_of_a_large_tree(V, H, upto, dtype, monkeypatch):
             assert ((got[:, lo:lo + 65536].float() - want).abs() <= eps * want.abs() + 1e-4).all()
 
 
+def test_head_of_a_large_tree_keeps_its_gradient():
+    """A head that is being trained: outside no_grad the library's differentiable product, at every number of rows above 64."""
+    from subspec_amd import model as M
+    V, H = 147456, 960
+    cfg = M.DecoderConfig(num_hidden_layers=1, hidden_size=H, num_attention_heads=2, num_key_value_heads=1, head_dim=128,
+                          intermediate_size=128, vocab_size=V)
+    head = torch.full((V, H), 0.01, device=DEV, dtype=torch.bfloat16).requires_grad_()
+    kv = create_kv_cache("static", max_cache_len=8, config=cfg, device=DEV, dtype=torch.bfloat16)
+    d = M.Decoder(cfg, head.detach()[:64], [], torch.ones(H, dtype=torch.bfloat16, device=DEV), head, kv)
+    x = torch.randn(200, H, device=DEV).bfloat16()
+    out = d.logits(x)
+    out[:, 7].float().sum().backward()
+    assert head.grad is not None and head.grad[7].abs().sum() > 0 and head.grad[8].abs().sum() == 0
+    with torch.no_grad():
+        assert not d.logits(x).requires_grad
+
+
 # rings of two, four and five weight tiles: fewer chunks of 64 than slots, as many, one more; workgroups with a tile less than the ring
 @pytest.mark.parametrize("M", [33, 64])
 @pytest.mark.parametrize("N,K", [(32, 64), (32, 128), (96, 192), (64, 256), (96, 320), (96, 576), (160, 640), (96, 704), (160, 8256), (224, 8320), (30720, 192), (30752, 256), (30784, 320), (10240, 10240)])

@@ -295,9 +295,9 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restri
 // instruction: lane -> activation row 32 t + lane % 32, register r -> weight row 8 (r / 4) + 4 (lane / 32) + r % 4.
 // SwiGLU pairs: a "tile" is 16 gate rows + 16 up rows of the same 16 output columns, so gate and up of an element are
 // registers r and r + 8 of one lane.
-// Measured on the four projections of a 7B layer, weights from HBM: M = 64 15.0 / 13.6 / 45.6 / 32.6 us (q|k|v, o,
-// gate|up with SwiGLU, down, reductions included; 16.8 / 14.6 / 50.8 / 34.6 before the weights were streaming data, the
-// 16 x 16 x 32 kernel above: 16.2 / 14.8 / 64.2 / 37.6); M = 289
+// Measured on the four projections of a 7B layer, weights from HBM: M = 64 14.0 / 12.6 / 48.4 / 31.6 us (q|k|v, o,
+// gate|up with SwiGLU, down, reductions included; beside them 14.3 / 13.3 / 52.8 / 32.8 with rings of five tiles whatever
+// a workgroup has and no streaming hint; the 16 x 16 x 32 kernel above: 16.2 / 14.8 / 64.2 / 37.6); M = 289
 // 33 / 29 / 97 / 70 us (dense_tile_kernel alone 21.7 / 20.5 / 90 / 57.6; in a forward, behind cold caches and other kernels,
 // 25.6 / 17.8 + its sum in the norm / 94.6 / 54.4 + 7.5).  At 289 rows the kernel is bound by the activation copies: a chunk is
 // 40 KB per workgroup, LDS holds two of them beside three weight chunks, and one chunk in flight does not cover the L2 latency

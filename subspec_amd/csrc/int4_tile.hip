@@ -312,9 +312,10 @@ struct Int4TilePlan { int shape, units, splits, chunks_per_split; float us; };
 // Cheapest (shape, number of K ranges): 4 us for the launch, rounds of one workgroup per compute unit with 2 us for first chunks
 // and output; the sum over the ranges 2 us (a launch, or part of the consumer's), 0.2 per range and its fp32 partials at
 // 4.5 TB/s.  Fitted to the times of every shape at 78 matrices (512 to 37888 rows of 512 to 18944, weights from HBM) and 33, 48
-// and 64 activation rows: the choice, int4_gemm_kernel included (below), takes 1.006 times the best one's time in the mean, 1.11 at
-// worst (4608 x 3584 shape 2 12.7 us, 3584 x 18944 shape 0 in eleven ranges 27.7, 37888 x 3584 with the activation shape 0 36.0).
-// (Fitted before the scaling stood between the products: shape 0 is 4 to 8 % faster since, the others level.)
+// and 64 activation rows, on the kernel as it was before the scaling stood between the products: the choice, int4_gemm_kernel included
+// (below), took 1.006 times the best one's time in the mean then, 1.11 at worst (4608 x 3584 shape 2 12.7 us, 3584 x 18944 shape 0 in
+// eleven ranges 27.7, 37888 x 3584 with the activation shape 0 36.0).  Shape 0 is 4 to 8 % faster since, the others are level; the
+// constants have not been fitted again, so matrices near a line may be a few percent from their best choice.
 // gate|up never takes shape 2: one pair per workgroup is int4_gemm_kernel's case, several rounds of it lose to shape 1 or 0.
 static Int4TilePlan int4_tile_plan(int64_t M, int64_t N, int64_t K, bool silu) {
   Int4TilePlan best{};

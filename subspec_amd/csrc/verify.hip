@@ -452,13 +452,16 @@ template <> struct RoundBound<SUBSPEC_BF16> { static constexpr float rel = 0x1p-
 //
 // The race key of an element is p / -log(u), evaluated exactly as defined (rounded probability, accurate logarithm, IEEE
 // quotient) only for the few elements that can still win.  -log(u) >= 1 - u, so key <= p / (1 - u), and an element with
-// log2(bound of p) - log2(best key any lane of the wavefront has seen) < log2(1 - u) is skipped.  The test needs no
+// log2(bound of p) - log2(best key any lane of the WORKGROUP has published) < log2(1 - u) is skipped.  The test needs no
 // exponential: its left side is linear in the logit, and the bit pattern of a float, read as an integer, is 2^23 (127 + log2)
-// from below (exact at powers of two, at most 0.087 low), so an element costs six instructions -- unpack, one fused
-// multiply-add, a shift, two conversions, a compare -- and only lets a few more candidates through.
-// What is left is the Philox block: 18 multiplies and 18 exclusive ors per four elements.  Two blocks per lane and trip, the
-// logits of the next trip in flight.  2048 x 152064 bf16 at T = 0.8, rows in the L3: the call 388 -> 317 us, of which the draw takes
-// two thirds, bound by the vector ALU (the multiplies alone are 60 % of it).
+// from below (exact at powers of two, at most 0.087 low).  Both sides are monotone, so the four elements of a block are tested at
+// once with their largest logit and their smallest word -- nine instructions beside the unpacking -- and one by one only in the
+// trips where some block of the wavefront passes.  The bound lives in LDS: a wavefront's records prune the other seven's elements, and
+// before there is one every lane evaluates the most promising element of its trip instead of all eight.
+// What is left is the Philox block, 18 multiplies (about 1.5 times a plain instruction each) and 18 exclusive ors per four elements:
+// 72 of the 112 vector instructions of a trip of two blocks a lane, the logits of the next trip in flight.  Bound by the vector ALU.
+// 2048 x 152064 bf16 at T = 0.8, the call with its statistics pass: 313 -> 274 us against every element tested on its own
+// (175 instructions a trip, a bound for each wavefront; elements evaluated in full: 388).
 // QUAD: the slice starts and ends on multiples of four elements and the rows are aligned for it, so the four logits
 // of a Philox block are one load (8 bytes of a 16-bit row, 16 of an fp32 row) and need no bounds.
 template <int DT, bool QUAD>
@@ -466,12 +469,17 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
     const void* __restrict__ logits, VerifyParams vp, const Part1* __restrict__ part1, Part3* __restrict__ part3) {
   __shared__ float red_f[kRowThreads / kWave];
   __shared__ int red_i[kRowThreads / kWave];
+  __shared__ uint32_t bound;            // log2 of the best key any wavefront has published, kSeenBias added; 0: none yet
+  constexpr float kSeenBias = 256.0f * 0x1p23f;
+  if (threadIdx.x == 0) bound = 0;
+  __syncthreads();
   const int64_t row = blockIdx.y;
   const int c = blockIdx.x;
   const RowStat rs = combine_row<DT>(part1 + row * vp.splits, vp);
   const int64_t c0 = (int64_t)c * vp.chunk;
   const int n = (int)min(vp.chunk, vp.vocab - c0);
   const int blocks = (n + 3) / 4;                      // Philox blocks of the slice
+  auto element = [&](int g, int i) { return (uint32_t)(g + (i >> 2) * kRowThreads) * 4 + (i & 3); };   // i-th of the lane's trip
   const bool warp = vp.temperature.t != 1.0f;
   const float inv_t = warp ? vp.temperature.inv_t : 1.0f;
   const float round_rel = warp ? RoundBound<DT>::rel : 0.f;         // x / T rounded to the dtype, relative
@@ -484,17 +492,21 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
   const float level = !in_range ? INFINITY : (127.0f + (2.02f * round_rel * fmaxf(rs.m, 0.f) + round_abs - rs.m) * kLog2e +
                        log2f((1.0f / rs.S) * (1.0f + 4.0f * RoundBound<DT>::rel + 1e-4f)) + 1e-3f + 1e-6f * fabsf(rs.m)) * 0x1p23f;
   constexpr bool kAbs = RoundBound<DT>::abs > 0.f;      // fp16: a probability may round up to the smallest subnormal
+  constexpr float kFloor = (127.0f + (kAbs ? -24.0f : 0.f)) * 0x1p23f;   // the level of p = abs
   float best = -1.f;
   int idx = 0x7fffffff;
-  float from = INFINITY, floor_from = INFINITY;         // level less log2 of the wavefront's best key; the same for p = abs
-  auto load = [&](int g, float (&xs)[4]) __attribute__((always_inline)) {
-    if constexpr (QUAD) {                              // one load, clamped to the last block of the slice
-      const int64_t at = row * vp.vocab + c0 + (int64_t)min(g, blocks - 1) * 4;
+  // Philox block `lane0 + b kRowThreads` of the trip that begins at block g0, clamped to the last block of the slice; g0 is
+  // uniform, so the address is a scalar base and a 32-bit offset
+  auto load = [&](int g0, int b, float (&xs)[4]) __attribute__((always_inline)) {
+    const int first = min(g0, blocks - 1);
+    const uint32_t at = (uint32_t)min((int)threadIdx.x + b * kRowThreads, blocks - 1 - first);
+    if constexpr (QUAD) {                              // one load
+      const uint8_t* const trip = (const uint8_t*)logits + (row * vp.vocab + c0 + (int64_t)first * 4) * Elem<DT>::kBytes;
       if constexpr (DT == SUBSPEC_F32) {
-        const float4 v = *(const float4*)((const float*)logits + at);
+        const float4 v = *(const float4*)(trip + at * 16u);
         xs[0] = v.x; xs[1] = v.y; xs[2] = v.z; xs[3] = v.w;
       } else {
-        const uint2 v = *(const uint2*)((const uint16_t*)logits + at);
+        const uint2 v = *(const uint2*)(trip + at * 8u);
         if constexpr (DT == SUBSPEC_BF16) {
           xs[0] = __uint_as_float(v.x << 16); xs[1] = __uint_as_float(v.x & 0xffff0000u);
           xs[2] = __uint_as_float(v.y << 16); xs[3] = __uint_as_float(v.y & 0xffff0000u);
@@ -505,55 +517,107 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
       }
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) xs[e] = Elem<DT>::load(logits, row * vp.vocab + c0 + min((int64_t)g * 4 + e, (int64_t)n - 1));
+      for (int e = 0; e < 4; ++e)
+        xs[e] = Elem<DT>::load(logits, row * vp.vocab + c0 + min((int64_t)(first + (int)at) * 4 + e, (int64_t)n - 1));
     }
   };
   constexpr int U = 2;                                 // blocks per lane and trip
   float xs[U][4];
+  uint32_t w[U][4];                                    // complements of the random words
+  // left and right side of the test for one element, or for the largest logit and the smallest word of a block: both sides are
+  // monotone, so a block that fails has no candidate
+  auto score = [&](float x, float from, float floor_from) __attribute__((always_inline)) {
+    float z = fmaf(x, slope, from);                    // (a masked logit's -inf never passes, a NaN row has no candidate)
+    if constexpr (kAbs) z = fmaxf(z, floor_from) + 0x1p23f;
+    return z;
+  };
+  auto below = [&](uint32_t word) __attribute__((always_inline)) {
+    return (float)(int)__float_as_uint((float)(word >> 9));                 // (1 - u) 2^23 - 1/2
+  };
+  auto key_of = [&](float x, uint32_t word) __attribute__((always_inline)) {
+    const float xw = warp ? Elem<DT>::round(div_rn(x, vp.temperature)) : x;
+    const float p = rounded_prob<DT>(xw, rs.m, rs.S);
+    const float u = ((float)(~word >> 9) + 0.5f) * 0x1p-23f;
+    return p / -logf(u);
+  };
+  // nothing that a rarely taken branch does with the words is computed in front of it
+  auto rare = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int b = 0; b < U; ++b) load(threadIdx.x + b * kRowThreads, xs[b]);
+    for (int i = 0; i < U * 4; ++i) asm volatile("" : "+v"(w[i / 4][i % 4]));
+  };
+  // element e of this lane's trip
+  auto pick = [&](int e, float& x, uint32_t& word) __attribute__((always_inline)) {
+    x = xs[0][0];
+    word = w[0][0];
+#pragma unroll
+    for (int i = 1; i < U * 4; ++i) {
+      x = e == i ? xs[i / 4][i % 4] : x;
+      word = e == i ? w[i / 4][i % 4] : word;
+    }
+  };
+  // the best of a wavefront's keys becomes the workgroup's bound, if it is more than the present one
+  auto publish = [&](float key) __attribute__((always_inline)) {
+    key = wave_max(key);
+    if (!(key > 0.f) || (threadIdx.x & (kWave - 1))) return;
+    atomicMax(&bound, __float_as_uint(log2f(key * (0.9999f * 0x1p-23f)) * 0x1p23f + kSeenBias));
+  };
+#pragma unroll
+  for (int b = 0; b < U; ++b) load(0, b, xs[b]);
   for (int g0 = 0; g0 < blocks; g0 += U * kRowThreads) {   // same trip count for every lane: the votes below see whole wavefronts
     const int g = g0 + threadIdx.x;
     float xn[U][4];
 #pragma unroll
-    for (int b = 0; b < U; ++b) load(g + (U + b) * kRowThreads, xn[b]);
-    uint32_t w[U][4];                                  // complements of the random words
-    bool cand[U][4];
-    bool any_cand = false;
+    for (int b = 0; b < U; ++b) load(g0 + U * kRowThreads, b, xn[b]);
+    uint32_t seen_bits = __hip_atomic_load(&bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // used behind the blocks
 #pragma unroll
     for (int b = 0; b < U; ++b)
       philox4x32_10_not((uint32_t)(c0 / 4 + g + b * kRowThreads), (uint32_t)row, vp.offset[0], vp.offset[1], vp.key[0], vp.key[1], w[b]);
+    seen_bits = __builtin_amdgcn_readfirstlane(seen_bits);
+    if (seen_bits == 0) {
+      // nobody has a bound yet: each lane evaluates its most promising element, which only sets the bound
+      rare();
+      float promise = -INFINITY;
+      int at = 0;
+#pragma unroll
+      for (int i = 0; i < U * 4; ++i) {
+        const float s = fmaf(xs[i / 4][i % 4], slope, -below(w[i / 4][i % 4]));
+        if (s > promise && element(g, i) < (uint32_t)n) { promise = s; at = i; }
+      }
+      float x;
+      uint32_t word;
+      pick(at, x, word);
+      const float key = key_of(x, word);
+      publish(element(g, at) < (uint32_t)n && key > 0.f ? key : 0.f);
+      seen_bits = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+    }
+    const float seen = __uint_as_float(seen_bits) - kSeenBias;
+    const float from = seen_bits ? level - seen : INFINITY, floor_from = seen_bits ? kFloor - seen : INFINITY;
+    uint64_t vote = 0;
 #pragma unroll
     for (int b = 0; b < U; ++b) {
-      const bool in = g + b * kRowThreads < blocks;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float z = fmaf(xs[b][e], slope, from);         // (a masked logit's -inf never passes, a NaN row has no candidate)
-        if constexpr (kAbs) z = fmaxf(z, floor_from) + 0x1p23f;
-        const float below = (float)(int)__float_as_uint((float)(w[b][e] >> 9));   // (1 - u) 2^23 - 1/2
-        cand[b][e] = in && z >= below && (QUAD || (g + b * kRowThreads) * 4 + e < n);
-        any_cand |= cand[b][e];
-      }
+      float x;                                         // (fmaxf would quieten its operands first, two more instructions)
+      asm("v_max_f32 %0, %1, %2\n\tv_max3_f32 %0, %0, %3, %4" : "=&v"(x) : "v"(xs[b][0]), "v"(xs[b][1]), "v"(xs[b][2]), "v"(xs[b][3]));
+      const uint32_t word = min(min(w[b][0], w[b][1]), min(w[b][2], w[b][3]));
+      vote |= __ballot(score(x, from, floor_from) >= below(word));
     }
-    // one vote per trip: the threshold only prunes, so refreshing it less often changes no result
-    if (__any(any_cand)) {                             // wavefront-uniform
+    if (vote) {                                        // wavefront-uniform
+      rare();
+      uint32_t cand = 0;
 #pragma unroll
-      for (int b = 0; b < U; ++b) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (cand[b][e]) {
-            const float x = xs[b][e];
-            const float xw = warp ? Elem<DT>::round(div_rn(x, vp.temperature)) : x;
-            const float p = rounded_prob<DT>(xw, rs.m, rs.S);
-            const float u = ((float)(~w[b][e] >> 9) + 0.5f) * 0x1p-23f;
-            const float key = p / -logf(u);
-            if (key > best) { best = key; idx = (int)(c0 + (g + b * kRowThreads) * 4 + e); }   // indices ascend: the first maximum stays
-          }
-        }
+      for (int i = 0; i < U * 4; ++i)
+        if (score(xs[i / 4][i % 4], from, floor_from) >= below(w[i / 4][i % 4]) && element(g, i) < (uint32_t)n) cand |= 1u << i;
+      if (__ballot(cand != 0)) {
+        do {                                           // each lane its next candidate
+          const int i = __ffs(cand) - 1;
+          float x;
+          uint32_t word;
+          pick(i, x, word);
+          const float key = key_of(x, word);
+          if (cand && key > best) { best = key; idx = (int)(c0 + element(g, i)); }   // indices ascend: the first maximum stays
+          cand &= cand - 1;
+        } while (__ballot(cand != 0));
+        publish(best);
       }
-      const float seen = log2f(fmaxf(wave_max(best), 0.f) * (0.9999f * 0x1p-23f)) * 0x1p23f;
-      from = level - seen;
-      if constexpr (kAbs) floor_from = (127.0f + log2f(RoundBound<DT>::abs)) * 0x1p23f - seen;
     }
 #pragma unroll
     for (int b = 0; b < U; ++b)

@@ -90,6 +90,31 @@ def test_draws_at_the_ends_of_the_range(dtype, scale, temperature):
     assert near <= 1
 
 
+@pytest.mark.parametrize("vocab", [1, 3, 4, 7, 8, 511, 2049, 4096, 4104, 16384 + 8, 16384 + 9])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_draws_of_blocks_tested_as_one(dtype, vocab):
+    """Blocks of four whose largest logit and smallest word belong to different elements; trips and slices in which only masked
+    or vanishing elements are left, ahead of and behind the ones that count; last blocks of one to four elements."""
+    g = torch.Generator().manual_seed(vocab)
+    rows = 9
+    logits = torch.randn(rows, vocab, generator=g)
+    logits[1] = 0.0                                       # every element may win
+    logits[2, :-1] = float("-inf")                        # only the last element is left
+    logits[3, 1:] = float("-inf")                         # only the first
+    logits[4, : vocab // 2] = -300.0                      # nothing to win in the first half
+    logits[5, vocab // 2 + 1:] = -300.0
+    logits[6, ::4] += 12.0                                # one strong element a block
+    logits[7] *= 6.0
+    logits[8, torch.arange(vocab) % 4 != 3] = float("-inf")
+    logits[8, -1] = 1.0
+    logits = logits.to(dtype)
+    near = 0
+    for temperature, seed, offset in ((1.0, 21, 3), (0.8, 22, 4), (2.5, 23, 5)):
+        got = ops.sample_tokens(logits.to(DEV), temperature, seed, offset).cpu()
+        near += _check_draws(logits, temperature, got, seed, offset)
+    assert near <= 3
+
+
 def test_draw_frequencies_on_device():
     # 256 rows x 300 offsets of one 16-way distribution: chi-square against the rounded probabilities
     p = torch.tensor([0.25, 0.18, 0.14, 0.10, 0.08, 0.06, 0.05, 0.04, 0.03, 0.02, 0.02, 0.01, 0.01, 0.005, 0.003, 0.002])

@@ -102,6 +102,14 @@ __device__ __forceinline__ float div_rn(float x, const Divisor& d) {
   return fabsf(q) == INFINITY ? q : q1;
 }
 
+// gate / (1 + exp(-gate)) in fp32: the quotient as a product with the reciprocal (v_rcp_f32, 1 ulp), six instructions where the
+// correctly rounded division takes sixteen.  Its callers round the result to 16 bits: of all 97,559 bf16 and fp16 gates below 1e30
+// with a result of at least 1e-36, one does not get the nearest value, as with the division (5.9375 in bf16; there -0.7139 in fp16).
+// Both sides of the quotient are scaled by 1/4, so that the reciprocal of the largest finite denominator is still a normal number.
+__device__ __forceinline__ float silu(float gate) {
+  return 0.25f * gate * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-gate), 0.25f));
+}
+
 // Output element of a linear layer: v = accumulator (+ bias), optionally followed by a residual add with
 // the rounding points of the separate tensor ops it replaces: out = round(round(v) + residual[i]).
 // `residual` may be the output itself (in-place update of the residual stream): the element is read and

@@ -167,7 +167,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
   unpack8<DT>(((const dec_u4*)(gu + m * 2 * F))[p], g);
   unpack8<DT>(((const dec_u4*)(gu + m * 2 * F + F))[p], u);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) g[j] = Elem<DT>::round(g[j] / (1.f + __expf(-g[j]))) * u[j];
+  for (int j = 0; j < 8; ++j) g[j] = Elem<DT>::round(silu(g[j])) * u[j];
   ((dec_u4*)(act + m * F))[p] = pack8<DT>(g);
 }
 

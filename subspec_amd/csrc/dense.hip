@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kDnThreads) void dense_gemm_kernel(
             const int m = mt * 16 + c * 4 + rr;
             if (m >= M) continue;
             const float g = gate_held[mt][rr], u = Elem<DT>::round(v[rr] + bv);
-            Elem<DT>::store(y, (int64_t)m * (N / 2) + f, Elem<DT>::round(g / (1.f + __expf(-g))) * u);
+            Elem<DT>::store(y, (int64_t)m * (N / 2) + f, Elem<DT>::round(silu(g)) * u);
           }
         }
       } else {
@@ -533,7 +533,7 @@ __global__ __launch_bounds__(512) void dense_wide_kernel(WideParams p) {
           for (int e = 0; e < 4; ++e) {
             const float bg = p.bias ? Elem<DT>::load(p.bias, f + e) : 0.f, bu = p.bias ? Elem<DT>::load(p.bias, F + f + e) : 0.f;
             const float gate = Elem<DT>::round(acc[i][k][4 * q + e] + bg), up = Elem<DT>::round(acc[i][k][8 + 4 * q + e] + bu);
-            o[e] = Elem<DT>::round(gate / (1.f + __expf(-gate))) * up;
+            o[e] = Elem<DT>::round(silu(gate)) * up;
           }
           *(wd_u2*)(p.y + (int64_t)m * F + f) = wd_u2{wd_pack2<DT>(o[0], o[1]), wd_pack2<DT>(o[2], o[3])};
         }

@@ -464,7 +464,7 @@ __global__ __launch_bounds__(kI4Threads) void int4_gemm_kernel(
             const int m = mt * 16 + c * 4 + rr;
             if (m >= M) continue;
             const float g = held[mt][rr], u = Elem<DT>::round(v[rr] + bv);
-            Elem<DT>::store(y, (int64_t)m * (N / 2) + f, Elem<DT>::round(g / (1.f + __expf(-g))) * u);
+            Elem<DT>::store(y, (int64_t)m * (N / 2) + f, Elem<DT>::round(silu(g)) * u);
           }
         } else {
           const int u = unit0 + (t >> 1);
@@ -837,7 +837,7 @@ __global__ __launch_bounds__(kR8Threads) void int4_rows8_kernel(
       if constexpr (SILU) {
         // act[m, f] = round(silu(round(gate))) * round(up): the arithmetic of the separate activation kernel
         const float up = Elem<DT>::round(second_raw);
-        Elem<DT>::store(y, (int64_t)m * (N / 2) + (int64_t)u * 16 + ln, Elem<DT>::round(first / (1.f + __expf(-first))) * up);
+        Elem<DT>::store(y, (int64_t)m * (N / 2) + (int64_t)u * 16 + ln, Elem<DT>::round(silu(first)) * up);
       } else if (u < qk_units) {
         // rotary pair (d, d + 64) of head u / 4, d = 16 (u % 4) + ln; t * cos + rotate_half(t) * sin with each
         // product and the sum rounded like the eager tensor ops

@@ -277,7 +277,7 @@ __global__ __launch_bounds__(512) void int4_tile_kernel(Int4TileParams p) {
       const int64_t f = (int64_t)(unit * TA + t) * 16 + ln;
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr)
-        if (m0 + rr < M) Elem<DT>::store(p.y, (m0 + rr) * F + f, Elem<DT>::round(gate[rr] / (1.f + __expf(-gate[rr]))) * up[rr]);
+        if (m0 + rr < M) Elem<DT>::store(p.y, (m0 + rr) * F + f, Elem<DT>::round(silu(gate[rr])) * up[rr]);
     }
   } else {
 #pragma unroll

@@ -20,8 +20,13 @@
 //   slots of each ring every chunk waits for a request to HBM (2500 cycles and more).  Three slots of both (256 x 160 at 256
 //   rows: 83 -> 73 us), or three of weights and two of activations with the weights requested half a chunk later (256 x 256,
 //   2048 rows: 490 -> 441 us), are what LDS holds.  Chunks of 32 k in twice as many slots lose (half-line requests).
-// 2048 rows: 441 to 458 us = 1.21 to 1.26 PFLOP/s with the activation included (library GEMM alone: 520 us; an 8192^3 product
-// reaches 1.38 PFLOP/s on this card), 289 rows: 90 us (dense_wide_kernel: 106), 128 rows: 57 us = 4.8 TB/s of weights.
+// * Output.  A workgroup has its compute unit to itself, so nothing runs beside its output stage: with a division per element and the
+//   bias looked up for every 16 rows it took 24 of 449 us at 2048 rows and 4 of 88 at 289 (activation included).
+// * Weights from HBM (289 rows; the same with every weight request answered by the L2: 69 instead of 88 us, without any copy 61, without
+//   waits for them 81 to 88): requests return in order, and those that wait for HBM hold back the activations behind them.  Neither
+//   the order of the chunks, nor 256-byte requests, nor weights laid out tile by tile change that.
+// 2048 rows: 425 to 435 us = 1.28 to 1.31 PFLOP/s with the activation included (library GEMM alone: 520 us; an 8192^3 product
+// reaches 1.38 PFLOP/s on this card), 289 rows: 84 us (dense_wide_kernel: 106), 128 rows: 57 us = 4.8 TB/s of weights.
 #include "dma.h"
 #include <algorithm>
 #include <type_traits>
@@ -288,54 +293,72 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
     }
     return;
   }
-  // 16 rows at a time through a wavefront-private LDS block, so that rows leave as 16-byte pieces of whole segments
+  // 16 rows at a time through a wavefront-private LDS block, so that rows leave as 16-byte pieces of whole segments.  Each of a
+  // lane's 16 to 100 outputs costs the compute unit eight cycles per instruction while its matrix cores are idle: biases, bounds
+  // and addresses that do not depend on the 16 rows are worked out in front of them, and pairs share their conversions.
   constexpr int kCols = SILU ? TA * 8 : TA * 16;                           // output columns of this wavefront
-  constexpr int kPieces = kCols / 8;
+  constexpr int kPieces = kCols / 8, kRounds = (16 * kPieces + 63) / 64;
   // (two k groups: the block lies in the part of the exchange that only this wavefront reads)
   static_assert(GK == 1 || TA * TB * 1024 >= 16 * kOutRow, "output block inside the exchange");
   uint8_t* const mine = lds + (GK == 2 ? wmn * TA * TB * 1024 : wmn * 16 * kOutRow);
   const int64_t ncol0 = n0 + (int64_t)wn * kCols, ncols = SILU ? F : p.N;
+  float bias[TA][4];                                                       // of acc[i][.][r]
+#pragma unroll
+  for (int i = 0; i < TA; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bias[i][r] = 0.f;
+  if (p.bias) {
+#pragma unroll
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t n = SILU ? n0 + (wn * TA + i) * 8 + 2 * c + (r & 1) : n0 + (wn * TA + i) * 16 + 4 * c + r;
+        if (n < ncols) bias[i][r] = Elem<DT>::load(p.bias, SILU && r >= 2 ? F + n : n);
+      }
+  }
+  const uint8_t* from[kRounds];                                            // this lane's pieces of the block ...
+  int64_t to[kRounds];                                                     // ... and of the first 16 rows
+  int row[kRounds];                                                        // their rows; none: M
+#pragma unroll
+  for (int q = 0; q < kRounds; ++q) {
+    const int pi = q * 64 + lane, r = pi / kPieces, piece = pi % kPieces;
+    from[q] = mine + r * kOutRow + piece * 16;
+    row[q] = r < 16 && ncol0 + piece * 8 < ncols ? m0 + wm * TB * 16 + r : M;
+    to[q] = (int64_t)(m0 + wm * TB * 16 + r) * ncols + ncol0 + piece * 8;
+  }
 #pragma unroll
   for (int k = 0; k < TB; ++k) {
 #pragma unroll
     for (int i = 0; i < TA; ++i) {
+      const float v0 = acc[i][k][0] + bias[i][0], v1 = acc[i][k][1] + bias[i][1];
+      const float v2 = acc[i][k][2] + bias[i][2], v3 = acc[i][k][3] + bias[i][3];
+      const uint32_t lo = pack2<DT>(v0, v1), hi = pack2<DT>(v2, v3);
       if constexpr (SILU) {
-        const int64_t f = n0 + (wn * TA + i) * 8 + 2 * c;
-        float o[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const bool in = p.bias && f + e < F;
-          const float bg = in ? Elem<DT>::load(p.bias, f + e) : 0.f, bu = in ? Elem<DT>::load(p.bias, F + f + e) : 0.f;
-          const float gate = Elem<DT>::round(acc[i][k][e] + bg), up = Elem<DT>::round(acc[i][k][2 + e] + bu);
-          o[e] = Elem<DT>::round(gate / (1.f + __expf(-gate))) * up;
-        }
-        *(uint32_t*)(mine + ln * kOutRow + i * 16 + c * 4) = pack2<DT>(o[0], o[1]);
+        float gate[2], up[2];
+        unpack2<DT>(lo, gate);
+        unpack2<DT>(hi, up);
+        unpack2<DT>(pack2<DT>(silu(gate[0]), silu(gate[1])), gate);
+        *(uint32_t*)(mine + ln * kOutRow + i * 16 + c * 4) = pack2<DT>(gate[0] * up[0], gate[1] * up[1]);
       } else {
-        const int64_t n = n0 + (wn * TA + i) * 16 + 4 * c;
-        float o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = acc[i][k][r] + (p.bias && n + r < p.N ? Elem<DT>::load(p.bias, n + r) : 0.f);
-        *(tl_u2*)(mine + ln * kOutRow + i * 32 + c * 8) = tl_u2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
+        *(tl_u2*)(mine + ln * kOutRow + i * 32 + c * 8) = tl_u2{lo, hi};
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int q = 0; q < (16 * kPieces + 63) / 64; ++q) {
-      const int pi = q * 64 + lane, row = pi / kPieces, piece = pi % kPieces;
-      const int m = m0 + (wm * TB + k) * 16 + row;
-      const int64_t n = ncol0 + piece * 8;
-      if (row < 16 && m < M && n < ncols) {
-        dec_u4 v = *(const dec_u4*)(mine + row * kOutRow + piece * 16);
+    for (int q = 0; q < kRounds; ++q) {
+      if (row[q] + k * 16 < M) {
+        const int64_t at = to[q] + (int64_t)(k * 16) * ncols;
+        dec_u4 v = *(const dec_u4*)from[q];
         if (p.residual) {
           float a[8], b[8];
           unpack8<DT>(v, a);
-          unpack8<DT>(*(const dec_u4*)(p.residual + (int64_t)m * ncols + n), b);
+          unpack8<DT>(*(const dec_u4*)(p.residual + at), b);
 #pragma unroll
           for (int j = 0; j < 8; ++j) a[j] += b[j];
           v = pack8<DT>(a);
         }
-        *(dec_u4*)(p.y + (int64_t)m * ncols + n) = v;
+        *(dec_u4*)(p.y + at) = v;
       }
     }
     __builtin_amdgcn_wave_barrier();

@@ -52,6 +52,35 @@ def test_gate_up_silu(M, N, K, dtype):
     assert ((act - want).abs() <= 4 * ulp * want.abs() + 2 * ulp * up.abs() * 1e-1 + 1e-4).all()
 
 
+@pytest.mark.parametrize("M", [3, 40, 70, 289])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_activation_over_its_range(M, dtype):
+    """gate = x, up = 1 (one weight per row), so the result is round(silu(gate)): gates from both ends of the exponential, tiny
+    and infinite ones, through every dense kernel with the activation in its output stage."""
+    K = 128
+    g = torch.Generator().manual_seed(M)
+    special = torch.tensor([0.0, -0.0, 1e-30, -1e-30, 1.0, -1.0, -16.5, -60.0, -86.5, -87.4, -88.6, -88.8, -92.0, -104.0, -300.0, 88.0, 300.0,
+                            60000.0, -60000.0])
+    gates = torch.cat([special, torch.linspace(-90.0, 20.0, 1024), torch.randn(M * 64, generator=g) * 3])[: M * 64]
+    gates = torch.cat([gates, torch.zeros(M * 64 - gates.numel())]).reshape(M, 64).to(dtype)
+    x = torch.cat([gates, torch.ones(M, 1), torch.zeros(M, K - 65)], dim=1).to(dtype)
+    w = torch.zeros(128, K)
+    w[:64, :64] = torch.eye(64)
+    w[64:, 64] = 1.0
+    act = ops.dense_gate_up_silu(x.to(DEV), w.to(dtype).to(DEV)).cpu().double()
+    exact = gates.double() * torch.sigmoid(gates.double())
+    want = exact.to(dtype).double()
+    # where the exponential leaves fp32's range the result is zero
+    big = gates.double() < -88.0
+    assert (act[big].abs() <= 2 * exact[big].abs()).all()
+    ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    tiny = 2.0 ** (-133 if dtype == torch.bfloat16 else -24)              # the spacing of subnormal results
+    assert ((act - want).abs()[~big] <= ulp * want.abs()[~big] + tiny).all()
+    # an fp32 error of |gate| 2^-23 in the exponential (0.69 |gate| ulps) moves one rounding in 2^15 / |gate| (bf16), 2^12 / |gate|
+    # (fp16); the values repeat, and |gate| is below 90
+    assert (act != want)[~big].double().mean() <= 90 / 2 ** (15 if dtype == torch.bfloat16 else 12)
+
+
 def _plan(M, N, K, gate_up):
     """(tile shape, row tiles, column tiles, K ranges)"""
     plan = (ctypes.c_int32 * 4)()

@@ -455,11 +455,11 @@ template <> struct RoundBound<SUBSPEC_BF16> { static constexpr float rel = 0x1p-
 // log2(bound of p) - log2(best key any lane of the WORKGROUP has published) < log2(1 - u) is skipped.  The test needs no
 // exponential: its left side is linear in the logit, and the bit pattern of a float, read as an integer, is 2^23 (127 + log2)
 // from below (exact at powers of two, at most 0.087 low).  Both sides are monotone, so the four elements of a block are tested at
-// once with their largest logit and their smallest word -- nine instructions beside the unpacking -- and one by one only in the
+// once with their largest logit and their smallest word -- ten instructions beside the unpacking -- and one by one only in the
 // trips where some block of the wavefront passes.  The bound lives in LDS: a wavefront's records prune the other seven's elements, and
 // before there is one every lane evaluates the most promising element of its trip instead of all eight.
 // What is left is the Philox block, 18 multiplies (about 1.5 times a plain instruction each) and 18 exclusive ors per four elements:
-// 72 of the 112 vector instructions of a trip of two blocks a lane, the logits of the next trip in flight.  Bound by the vector ALU.
+// 72 of the 114 vector instructions of a trip of two blocks a lane, the logits of the next trip in flight.  Bound by the vector ALU.
 // 2048 x 152064 bf16 at T = 0.8, the call with its statistics pass: 313 -> 274 us against every element tested on its own
 // (175 instructions a trip, a bound for each wavefront; elements evaluated in full: 388).
 // QUAD: the slice starts and ends on multiples of four elements and the rows are aligned for it, so the four logits
@@ -521,6 +521,8 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
         xs[e] = Elem<DT>::load(logits, row * vp.vocab + c0 + min((int64_t)(first + (int)at) * 4 + e, (int64_t)n - 1));
     }
   };
+  float infinity = INFINITY;                           // (as a value the compiler cannot see through)
+  asm volatile("" : "+s"(infinity));
   constexpr int U = 2;                                 // blocks per lane and trip
   float xs[U][4];
   uint32_t w[U][4];                                    // complements of the random words
@@ -595,8 +597,9 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
     uint64_t vote = 0;
 #pragma unroll
     for (int b = 0; b < U; ++b) {
-      float x;                                         // (fmaxf would quieten its operands first, two more instructions)
-      asm("v_max_f32 %0, %1, %2\n\tv_max3_f32 %0, %0, %3, %4" : "=&v"(x) : "v"(xs[b][0]), "v"(xs[b][1]), "v"(xs[b][2]), "v"(xs[b][3]));
+      // the largest of four as medians with infinity: fmaxf would quieten each operand first
+      const float x = __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(xs[b][0], xs[b][1], infinity),
+                                              __builtin_amdgcn_fmed3f(xs[b][2], xs[b][3], infinity), infinity);
       const uint32_t word = min(min(w[b][0], w[b][1]), min(w[b][2], w[b][3]));
       vote |= __ballot(score(x, from, floor_from) >= below(word));
     }

@@ -451,8 +451,14 @@ int subspec_dense_linear(const void* x, const void* w, const void* bias, void* y
 
 /* How a dense projection over more than 64 rows (gate_up != 0: the gate|up projection with its activation) is cut, for tests
  * and tuning; host only.  plan = {index of the tile shape, row tiles, column tiles, K ranges}; returns 0, or
- * SUBSPEC_ERR_LIMIT where the tiled kernel does not take these sizes (an aligned output assumed). */
+ * SUBSPEC_ERR_LIMIT where the tiled kernel does not take these sizes (an aligned output assumed).  gate_up: the shape that
+ * serves best on its own; subspec_dense_tile_tail says whether two are ahead of it. */
 int subspec_dense_tile_plan(int64_t M, int64_t N, int64_t K, int gate_up, int32_t* plan);
+
+/* gate|up projections of several rounds of the largest tile (index 0) may give their last output columns to smaller tiles of the
+ * same launch.  tail = {index of that shape or -1 (subspec_dense_tile_plan is all there is), its row tiles, its column tiles, first
+ * output column that it takes}; host only, limits as above. */
+int subspec_dense_tile_tail(int64_t M, int64_t N, int64_t K, int32_t* tail);
 
 /* One decoder layer with dense 16-bit projections: same sequence of kernels, arguments, workspace
  * (subspec_int4_decoder_layer_workspace) and limits as subspec_int4_decoder_layer, for the target

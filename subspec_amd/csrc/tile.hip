@@ -50,22 +50,28 @@ struct TileParams {
   const uint16_t* x; const uint16_t* w; const uint16_t* bias; const uint16_t* residual; uint16_t* y; float* partial;
   int M, K; int64_t N;               // N: rows of w (SILU: 2 F)
   int tiles_m, tiles_n, splits, chunks_per_split;
+  int64_t col0;                      // output column at which the first of the tiles_n tiles begins
 };
 
+// LDS of a tile shape: the rings, reused by the output stage
+template <int GM, int GN, int GK, int TA, int TB, int SW, int SX, bool SILU>
+constexpr int tile_lds() {
+  const int rings = SW * GN * TA * 16 * 128 + SX * GM * TB * 16 * 128;
+  const int out = GM * GN * GK * 16 * (TA * (SILU ? 16 : 32) + 16), red = GK > 1 ? GM * GN * TA * TB * 1024 : 0;
+  return std::max(rings, std::max(out, red));
+}
+
+// workgroup `id` of the tiles that p describes
 template <int DT, int GM, int GN, int GK, int TA, int TB, int SW, int SX, bool NT, bool SILU>
-__global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParams p) {
+__device__ __forceinline__ void dense_tile(const TileParams& p, uint8_t* const lds, const int id) {
   constexpr int kWaves = GM * GN * GK;
   constexpr int BM = GM * TB * 16, BN = GN * TA * 16;
   constexpr int kWSlots = BN / 8, kXSlots = BM / 8;                        // 1 KB requests per chunk ...
   constexpr int RW = (kWSlots + kWaves - 1) / kWaves, RX = (kXSlots + kWaves - 1) / kWaves;   // ... of one wavefront
   constexpr uint32_t kWStride = BN * 128, kXStride = BM * 128, kXRing = SW * kWStride;
-  constexpr int kRingBytes = SW * BN * 128 + SX * BM * 128;
   constexpr int kOutRow = TA * (SILU ? 16 : 32) + 16;                     // bytes of a parked output row
-  constexpr int kEpi = kWaves * 16 * kOutRow, kRed = GK > 1 ? GM * GN * TA * TB * 1024 : 0;
-  constexpr int kLds = kRingBytes > kEpi ? (kRingBytes > kRed ? kRingBytes : kRed) : (kEpi > kRed ? kEpi : kRed);
-  static_assert(kLds <= 160 * 1024, "LDS");
+  static_assert(tile_lds<GM, GN, GK, TA, TB, SW, SX, SILU>() <= 160 * 1024, "LDS");
   static_assert(GK <= 2 && SX >= 2 && (SW == SX || (SW == SX + 1 && GK == 1)) , "k groups, ring depths");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 15, c = lane >> 4;
@@ -73,7 +79,7 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
 
   // XCD-aware order: consecutive ids go to different XCDs; each XCD takes a contiguous run of the tile list, rows fastest
   const int total = p.tiles_m * p.tiles_n * p.splits;
-  const int id = blockIdx.x, xcd = id & 7, per = total >> 3, rem = total & 7;
+  const int xcd = id & 7, per = total >> 3, rem = total & 7;
   // The quotients are pinned to scalar registers: the compiler divides in the vector ALU and would keep the tile's origin, and
   // with it the base address of every copy, in vector registers.  A copy's scalar base then comes out of a vector instruction
   // one to four instructions ahead of it, where the architecture asks for five wait states -- which the compiler inserts in front
@@ -85,7 +91,7 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
   asm volatile("" : "+s"(ks));
   const int tm = lin - cell * p.tiles_m, tn = cell - ks * p.tiles_n;
   const int m0 = tm * BM;
-  const int64_t n0 = (int64_t)tn * (SILU ? BN / 2 : BN);                  // SILU: first output column
+  const int64_t n0 = p.col0 + (int64_t)tn * (SILU ? BN / 2 : BN);         // SILU: first output column
   const int64_t F = p.N >> 1;
   const int n_chunks = K >> 6;
   const int st0 = ks * p.chunks_per_split, nst = min(n_chunks, st0 + p.chunks_per_split) - st0;
@@ -365,6 +371,12 @@ __global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParam
   }
 }
 
+template <int DT, int GM, int GN, int GK, int TA, int TB, int SW, int SX, bool NT, bool SILU>
+__global__ __launch_bounds__(GM * GN * GK * 64) void dense_tile_kernel(TileParams p) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[tile_lds<GM, GN, GK, TA, TB, SW, SX, SILU>()];
+  dense_tile<DT, GM, GN, GK, TA, TB, SW, SX, NT, SILU>(p, lds, blockIdx.x);
+}
+
 // ------------------------------------------------------------------ launch shapes
 // Tile shapes and what a chunk of one takes when the chip is full of them (us, measured on the projections of a 7B layer:
 // 4608 / 3584 / 37888 x 3584 and 3584 x 18944 at 65 to 2048 rows).  The shapes of 160 columns cut 37888 rows into 237
@@ -390,7 +402,11 @@ static constexpr TileShape kShapes[] = {
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 constexpr int kTileMaxSplits = 8;
 
-struct TilePlan { int shape, tiles_m, tiles_n, splits, chunks_per_split; };
+struct TilePlan {
+  int shape, tiles_m, tiles_n, splits, chunks_per_split;
+  int tail, tail_tiles_m, tail_tiles_n;                                    // shape of the last columns; none: -1
+  float us;
+};
 // Cheapest (shape, number of K ranges) under: 5.5 us for launch, first chunks and output; rounds of 256 workgroups, one
 // per compute unit, of chunk_us per chunk; never less than the weights take from HBM at 6 TB/s; fp32 partials written
 // and read back at 4.5 TB/s.  Alone, over the four projections of three layer widths and 65 to 2048 rows (216 sizes), the choice
@@ -399,9 +415,33 @@ struct TilePlan { int shape, tiles_m, tiles_n, splits, chunks_per_split; };
 // whole layers, where the sums of the q|k|v and o projections are the next kernel's.  (5.5 TB/s here kept 3584 x 18944 at 95 to
 // 128 rows on a shape 14 % slower: 45.2 against 39.5 us at 128; 0.95 us for shape 3 kept 37888 x 3584 with the activation at 321
 // to 384 on one 7 % slower: 119 against 112 us at 384.)
+// gate|up over several rounds of 256 x 256 tiles: the rounds that fill the chip, and what is left of the columns in the same launch in
+// smaller tiles that fill it once more (a last round of the large ones keeps most of the matrix cores idle).  3 us for the second
+// set of first chunks.  Over 19 row counts from 300 to 2048 at 37888 x 3584, 28672 x 4096 and 11264 x 2048 this takes a tail at 18
+// sizes and is ahead of the best single shape at all of them, by 3 to 11 %: 37888 x 3584 with 1000 rows 238 -> 224 us, 1792 415 ->
+// 381, 2048 434 -> 422; 28672 x 4096 with 600 rows 164 -> 148, 2048 382 -> 364; 11264 x 2048 with 1900 rows 91 -> 83.  At three
+// sizes that it leaves alone a tail would have been 2 to 5 % faster (28672 x 4096 with 1700 and 1792 rows), elsewhere slower.
+#define SUBSPEC_TILE_TAILS(X) X(2) X(4) X(5)
+static void with_tail(TilePlan& best, int64_t M, int64_t N, int64_t K) {
+  const int chunks = (int)(K / 64);
+  const int64_t F = N / 2, tm = (M + kShapes[0].bm - 1) / kShapes[0].bm, tn = (F + kShapes[0].bn / 2 - 1) / (kShapes[0].bn / 2);
+  const int64_t rounds = tm * tn / 256, main_n = rounds * 256 / tm, left = F - main_n * (kShapes[0].bn / 2);
+  const float hbm_us = 8.f + (float)N * (float)K * 2.f / 6.0e6f;           // as in tile_plan
+  if (rounds == 0 || left <= 0) return;
+  auto consider = [&](int i) {
+    const int64_t tail_m = (M + kShapes[i].bm - 1) / kShapes[i].bm, tail_n = (left + kShapes[i].bn / 2 - 1) / (kShapes[i].bn / 2);
+    const float us = std::max(hbm_us, 5.5f + 3.f + (float)chunks * ((float)rounds * kShapes[0].chunk_us +
+                                                                    (float)((tail_m * tail_n + 255) / 256) * kShapes[i].chunk_us));
+    if (us < best.us) best = TilePlan{0, (int)tm, (int)main_n, 1, chunks, i, (int)tail_m, (int)tail_n, us};
+  };
+#define X(ID) consider(ID);
+  SUBSPEC_TILE_TAILS(X)
+#undef X
+}
+
 static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool silu) {
   TilePlan best{};
-  float best_us = 1e30f;
+  best.us = 1e30f;
   const int chunks = (int)(K / 64);
   const float hbm_us = 8.f + (float)N * (float)K * 2.f / 6.0e6f;
   for (int i = 0; i < kNumShapes; ++i) {
@@ -413,13 +453,31 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool silu) {
       const int64_t rounds = (tm * tn * s + 255) / 256;
       float us = std::max(5.5f + (float)rounds * (float)cps * kShapes[i].chunk_us, hbm_us);
       if (s > 1) us += 1.f + 2.f * (float)s * (float)M * (float)N * 4.f / 4.5e6f;
-      if (us < best_us) {
-        best_us = us;
-        best = TilePlan{i, (int)tm, (int)tn, s, cps};
-      }
+      if (us < best.us) best = TilePlan{i, (int)tm, (int)tn, s, cps, -1, 0, 0, us};
     }
   }
   return best;
+}
+
+// Two shapes in one launch (SwiGLU): workgroups below `first` take the tiles of p, the others those of `tail`.
+template <int DT, int TAIL>
+__global__ __launch_bounds__(512) void dense_tile_pair_kernel(TileParams p, TileParams tail, int first) {
+#define X(ID, GM, GN, GK, TA, TB, SW, SX, NT, US) ID == TAIL ? tile_lds<GM, GN, GK, TA, TB, SW, SX, true>() :
+  constexpr int kTailLds = SUBSPEC_TILE_SHAPES(X) 0;
+#undef X
+#define X(ID, GM, GN, GK, TA, TB, SW, SX, NT, US) ID == 0 ? tile_lds<GM, GN, GK, TA, TB, SW, SX, true>() :
+  constexpr int kMainLds = SUBSPEC_TILE_SHAPES(X) 0;
+#undef X
+  __shared__ __attribute__((aligned(16))) uint8_t lds[std::max(kMainLds, kTailLds)];
+  const int id = blockIdx.x;
+#define X(ID, GM, GN, GK, TA, TB, SW, SX, NT, US)                                                                      \
+  if constexpr (ID == 0) {                                                                                             \
+    if (id < first) return dense_tile<DT, GM, GN, GK, TA, TB, SW, SX, false, true>(p, lds, id);                        \
+  } else if constexpr (ID == TAIL) {                                                                                   \
+    return dense_tile<DT, GM, GN, GK, TA, TB, SW, SX, false, true>(tail, lds, id - first);                             \
+  }
+  SUBSPEC_TILE_SHAPES(X)
+#undef X
 }
 
 template <int DT, bool SILU>
@@ -429,6 +487,21 @@ static void launch_tile(TileParams p, const TilePlan& pl, hipStream_t st) {
   p.splits = pl.splits;
   p.chunks_per_split = pl.chunks_per_split;
   const dim3 grid((unsigned)((int64_t)pl.tiles_m * pl.tiles_n * pl.splits));
+  if constexpr (SILU) {
+    if (pl.tail >= 0) {
+      TileParams t = p;
+      t.tiles_m = pl.tail_tiles_m;
+      t.tiles_n = pl.tail_tiles_n;
+      t.col0 = (int64_t)pl.tiles_n * (kShapes[0].bn / 2);
+      const dim3 both(grid.x + (unsigned)(pl.tail_tiles_m * pl.tail_tiles_n));
+      switch (pl.tail) {
+#define X(ID) case ID: hipLaunchKernelGGL((dense_tile_pair_kernel<DT, ID>), both, dim3(512), 0, st, p, t, (int)grid.x); break;
+        SUBSPEC_TILE_TAILS(X)
+#undef X
+      }
+      return;
+    }
+  }
   switch (pl.shape) {
 #define X(ID, GM, GN, GK, TA, TB, SW, SX, NT, US)                                                                       \
   case ID:                                                                                                              \
@@ -459,7 +532,7 @@ int tile_linear(const void* x, const void* w, const void* bias, const void* resi
                 int64_t K, void* workspace, hipStream_t st, int* splits) {
   const TilePlan pl = tile_plan(M, N, K, false);
   const TileParams p{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y,
-                     (float*)workspace, (int)M, (int)K, N, 0, 0, 0, 0};
+                     (float*)workspace, (int)M, (int)K, N, 0, 0, 0, 0, 0};
   *splits = pl.splits;
   DominantKernelTimer timer(st);
   if (dtype == SUBSPEC_BF16) launch_tile<SUBSPEC_BF16, false>(p, pl, st);
@@ -469,9 +542,10 @@ int tile_linear(const void* x, const void* w, const void* bias, const void* resi
 
 int tile_gate_up_silu(const void* x, const void* w, const void* bias, void* act, int dtype, int64_t M, int64_t N, int64_t K,
                       hipStream_t st) {
-  const TilePlan pl = tile_plan(M, N, K, true);
+  TilePlan pl = tile_plan(M, N, K, true);
+  with_tail(pl, M, N, K);
   const TileParams p{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, nullptr, (uint16_t*)act, nullptr,
-                     (int)M, (int)K, N, 0, 0, 0, 0};
+                     (int)M, (int)K, N, 0, 0, 0, 0, 0};
   DominantKernelTimer timer(st);
   if (dtype == SUBSPEC_BF16) launch_tile<SUBSPEC_BF16, true>(p, pl, st);
   else launch_tile<SUBSPEC_F16, true>(p, pl, st);
@@ -489,5 +563,17 @@ extern "C" int subspec_dense_tile_plan(int64_t M, int64_t N, int64_t K, int gate
                  (long long)K);
   const TilePlan pl = tile_plan(M, N, K, gate_up != 0);
   plan[0] = pl.shape; plan[1] = pl.tiles_m; plan[2] = pl.tiles_n; plan[3] = pl.splits;
+  return SUBSPEC_OK;
+}
+
+extern "C" int subspec_dense_tile_tail(int64_t M, int64_t N, int64_t K, int32_t* tail) {
+  using namespace subspec;
+  int32_t plan[4];
+  if (!tail) SUBSPEC_FAIL(SUBSPEC_ERR_ARG, "dense_tile_tail: null pointer");
+  const int code = subspec_dense_tile_plan(M, N, K, 1, plan);
+  if (code != SUBSPEC_OK) return code;
+  TilePlan pl = tile_plan(M, N, K, true);
+  with_tail(pl, M, N, K);
+  tail[0] = pl.tail; tail[1] = pl.tail_tiles_m; tail[2] = pl.tail_tiles_n; tail[3] = pl.tail < 0 ? 0 : pl.tiles_n * (kShapes[0].bn / 2);
   return SUBSPEC_OK;
 }

@@ -88,6 +88,17 @@ def _plan(M, N, K, gate_up):
     return tuple(plan)
 
 
+# M, N, K; shape of the last columns, its row and column tiles (the last of them partial), its first column
+@pytest.mark.parametrize("M,N,K,tail", [
+    (129, 164800, 512, (2, 1, 211, 65536)), (257, 45312, 640, (4, 3, 79, 16384)), (257, 46496, 1024, (5, 2, 108, 16384))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_two_shapes_in_one_launch(M, N, K, tail, dtype):
+    got = (ctypes.c_int32 * 4)()
+    L.check(L.lib().subspec_dense_tile_tail(M, N, K, got), "subspec_dense_tile_tail")
+    assert tuple(got) == tail
+    test_gate_up_silu(M, N, K, dtype)
+
+
 # M, N, K; tile shape, row tiles, K ranges
 @pytest.mark.parametrize("M,N,K,shape,row_tiles,ranges", [
     (129, 41536, 512, 0, 1, 1), (333, 22816, 512, 0, 2, 1), (129, 20736, 5632, 0, 1, 3), (333, 7296, 18944, 0, 2, 4),

@@ -264,7 +264,7 @@ def test_the_parser_of_vector_writes_sees_paths_and_wait_states():
 
 
 @pytest.mark.parametrize("source, kernel, min_kernels", [
-    ("tile.hip", "dense_tile_kernel", 36), ("int4_tile.hip", "int4_tile_kernel", 10),
+    ("tile.hip", "dense_tile_kernel", 36), ("tile.hip", "dense_tile_pair_kernel", 6), ("int4_tile.hip", "int4_tile_kernel", 10),
     ("dense.hip", "dense_wide_kernel", 12), ("attention.hip", "tree_attention_pp_kernel", 8),
 ])
 def test_copies_into_lds_do_not_read_a_scalar_address_too_early(source, kernel, min_kernels, tmp_path):

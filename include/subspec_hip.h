@@ -506,6 +506,12 @@ int subspec_dense_decoder_stack(const subspec_decoder_layer_dims* dims, const su
  * Replaces  the target's forward over a chunk of the prompt (specdecodes/models/generators/base.py:204-263). */
 size_t subspec_prefill_layer_workspace(const subspec_decoder_layer_dims* dims);
 
+/* Order in which the attention of a prefill of n_rows rows behind `prefix` rows starts its (window of 64 rows, key chunk) units, the
+ * same for every KV head; for tests, host only.  entries = capacity x {window or -1 (an empty slot), chunk, keys of a chunk}.  Returns the
+ * number of entries, or -1 for sizes that no prefill has. */
+int64_t subspec_prefill_attention_order(int64_t n_q_heads, int64_t n_kv_heads, int64_t n_rows, int64_t prefix, int32_t* entries,
+                                        int64_t capacity);
+
 int subspec_prefill_layer(const subspec_decoder_layer_dims* dims, const subspec_dense_layer_weights* weights, void* x,
                           const int32_t* positions, const int32_t* cache_rows, void* k_cache, void* v_cache, void* workspace,
                           size_t workspace_bytes, void* stream);

@@ -85,6 +85,7 @@ _SIGNATURES = {
     "subspec_dense_linear": (C.c_int, [_p, _p, _p, _p, C.c_int, _i64, _i64, _i64, _p, _sz, _p]),
     "subspec_dense_tile_plan": (C.c_int, [_i64, _i64, _i64, C.c_int, C.POINTER(C.c_int32)]),
     "subspec_dense_tile_tail": (C.c_int, [_i64, _i64, _i64, C.POINTER(C.c_int32)]),
+    "subspec_prefill_attention_order": (_i64, [_i64, _i64, _i64, _i64, C.POINTER(C.c_int32), _i64]),
     "subspec_dense_decoder_layer": (C.c_int, [C.POINTER(DecoderLayerDims), C.POINTER(DenseLayerWeights), _p, _p, _p, _p,
                                               _p, _p, _p, _sz, _p]),
     "subspec_prefill_layer_workspace": (_sz, [C.POINTER(DecoderLayerDims)]),

@@ -80,7 +80,8 @@ struct AttnParams {
   int chunks;
   int64_t chunk_keys;          // multiple of kKeyBlock
   int pairs_per_kv;            // workgroups (groups of 4 or 8 query heads) per KV head
-  int64_t units;               // batch * hkv * chunks
+  int64_t units;               // batch * hkv * chunks; causal, falling order: hkv * entries of causal_entry
+  int full;                    // causal: entries that are whole chunks; -1: entries window by window
   float scale_log2;            // softmax scale * log2(e)
   // paged cache (one request): row p of K lives at page_table[p >> page_shift], token p & (page_len - 1) of
   // a pool layer [max_pages][2 (K, V)][page_len][hkv][128]; V is v_delta elements behind K
@@ -923,13 +924,58 @@ __device__ __forceinline__ void pp_softmax_phase(int64_t kb, const PPRow& rw, v1
   rf.l += (lsum[0][0] + lsum[0][1]) + (lsum[1][0] + lsum[1][1]);
 }
 
+// The order in which the chunks of a causal call start.  A compute unit holds one workgroup, workgroups start in order, and they are
+// dealt to the 8 XCDs and, there, to the 4 shader engines by their number: where more start than fit and their lengths differ, any
+// pattern but falling lengths meets one of the two.  Window by window, a prompt of 2048 rows (28 : 4 heads: two chunks a window, the
+// second half of them short or empty, 8 (head, chunk) pairs) sent every last chunk to four of the XCDs; with chunks taking turns they
+// went to two of the four engines: 72 to 76 us either way, 57 to 61 in falling order.
+// Falling: whole chunks, then the windows' last ones from long to short.  Window i, counted from the longest, has (at most) `blocks` - i
+// key blocks in chunks of `per`.  Entry e < full: chunk, then window; the others: residue, then every per-th window.  Past the windows,
+// or nothing left over: false.
+// Where everything starts at once, or the windows are of similar length, window by window is ahead: an XCD then reads a chunk of K and V
+// for all windows (700 rows after 1000, falling order: 1 to 4 us more).  The line: more than 256 workgroups, and at most half as many
+// rows before the prompt as in it.  A layer of the three widths of a 3 to 8 billion parameter model, falling against window by window: 600
+// rows 4.7 to 5.4 us less, 700 6.6 to 8.4, 1000 after 250 4.7 to 7.8, 1000 after 500 0.7 to 2.8, 1500 after 500 13 to 16, 2048 7.9 to 15
+// (of 77 to 85); 1300 after 700 2 us more to 0.2 less.
+struct CausalEntry { int window, chunk; bool some; };
+__host__ __device__ inline CausalEntry causal_entry(int e, int full, int windows, int blocks, int per) {
+  if (e < full) {
+    for (int c = 0;; ++c) {
+      const int whole = min(blocks - (c + 1) * per + 1, windows);          // windows with a whole chunk c
+      if (e < whole) return CausalEntry{e, c, true};
+      e -= whole;
+    }
+  }
+  e -= full;
+  const int rounds = (windows + per - 1) / per, rank = e / rounds, copy = e % rounds;
+  const int first = (blocks % per + 1) % per;                              // residue per - 1
+  const int i = windows >= per ? (first + rank) % per + copy * per : (rank + (first < windows ? first : 0)) % windows;
+  return CausalEntry{i, (blocks - i) / per, i < windows && (blocks - i) % per != 0};
+}
+struct CausalOrder { int blocks, per, full, entries; };                   // full -1: window by window
+inline CausalOrder causal_order(int64_t prefix, int64_t n_rows, int windows, int chunks, int64_t chunk_keys, int64_t per_entry) {
+  CausalOrder o;
+  o.per = (int)(chunk_keys / kKeyBlock);
+  if (windows * chunks * per_entry <= 256 || 2 * prefix > n_rows) {
+    o.blocks = 0;
+    o.full = -1;
+    o.entries = windows * chunks;
+    return o;
+  }
+  o.blocks = (int)((prefix + kKeyBlock - 1) / kKeyBlock) + windows;
+  o.full = 0;
+  for (int c = 0; o.blocks - (c + 1) * o.per + 1 > 0; ++c) o.full += std::min(o.blocks - (c + 1) * o.per + 1, windows);
+  o.entries = o.full + (windows + o.per - 1) / o.per * std::min(o.per, windows);
+  return o;
+}
+
 // CAUSAL (a prefill: query row i of the call sits at cache row prefix + i): window w sees prefix + 64 w rows in full and the
 // rows of its own window up to the query's, so its row masks are (2 << row) - 1 and come from no memory.  Windows have
-// different lengths: the longest start first, chunks behind a window's last key end at once, and the partial results of a
-// window cut into several chunks stay fp32 (unnormalised O and sum).
-// 28 : 4 heads, bf16: 2048 rows of a prompt 72 us + 11 us merge, the last 256 of 2048 20 + 9 us (a library's attention with the
+// different lengths (causal_order: which starts when); the partial results of a window cut into several chunks stay fp32
+// (unnormalised O and sum).
+// 28 : 4 heads, bf16: 2048 rows of a prompt 57 to 61 us + 10 us merge, the last 256 of 2048 20 + 7 us (a library's attention with the
 // mask it needs and K / V repeated for the heads: 275 and 190 us).  Bound by the softmax and matrix phases of the blocks, like
-// the tree form; what is left is the uneven length of the windows.
+// the tree form.
 template <int DT, int WPH, bool CAUSAL = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void tree_attention_pp_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
@@ -946,10 +992,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int pair = (int)(slot % (uint32_t)ap.pairs_per_kv);
   const uint32_t unit = (slot / (uint32_t)ap.pairs_per_kv) * (uint32_t)kXcds + (uint32_t)xcd;
   if ((int64_t)unit >= ap.units) return;
-  const int chunk = (int)(unit % (uint32_t)ap.chunks);
-  const uint32_t bkv = unit / (uint32_t)ap.chunks;
-  const int kvh = (int)(bkv % (uint32_t)ap.hkv);
-  const int vb = CAUSAL ? ap.windows - 1 - (int)(bkv / (uint32_t)ap.hkv) : (int)(bkv / (uint32_t)ap.hkv);
+  int chunk, kvh, vb;
+  if (CAUSAL && ap.full >= 0) {
+    kvh = (int)(unit % (uint32_t)ap.hkv);
+    const CausalEntry e = causal_entry((int)(unit / (uint32_t)ap.hkv), ap.full, ap.windows,
+                                       (int)((ap.prefix + kKeyBlock - 1) / kKeyBlock) + ap.windows, (int)(ap.chunk_keys / kKeyBlock));
+    if (!e.some) return;
+    vb = ap.windows - 1 - e.window;
+    chunk = e.chunk;
+  } else {
+    chunk = (int)(unit % (uint32_t)ap.chunks);
+    const uint32_t bkv = unit / (uint32_t)ap.chunks;
+    kvh = (int)(bkv % (uint32_t)ap.hkv);
+    vb = CAUSAL ? ap.windows - 1 - (int)(bkv / (uint32_t)ap.hkv) : (int)(bkv / (uint32_t)ap.hkv);
+  }
   const AttnWindow aw = attn_window(ap, vb);          // (sequence, window of 64 query rows) of this unit
   const int b = aw.b;
   const int group = (int)((uint32_t)ap.hq / (uint32_t)ap.hkv);
@@ -1579,7 +1635,9 @@ int causal_attention(const void* q, const void* k, const void* v, void* out, int
   ap.chunks = pl.chunks;
   ap.chunk_keys = pl.chunk_keys;
   ap.pairs_per_kv = pl.pairs;
-  ap.units = (int64_t)pl.windows * hkv * pl.chunks;
+  const CausalOrder order = causal_order(prefix, n_rows, pl.windows, pl.chunks, pl.chunk_keys, hkv * pl.pairs);
+  ap.units = hkv * order.entries;
+  ap.full = order.full;
   ap.scale_log2 = scale * kLog2e;
   size_t o_bytes = 0;
   attn_partial_bytes(pl.windows, hq, pl.chunks, &o_bytes);
@@ -1592,3 +1650,18 @@ int causal_attention(const void* q, const void* k, const void* v, void* out, int
   return SUBSPEC_OK;
 }
 }  // namespace subspec
+
+extern "C" int64_t subspec_prefill_attention_order(int64_t n_q_heads, int64_t n_kv_heads, int64_t n_rows, int64_t prefix,
+                                                   int32_t* entries, int64_t capacity) {
+  if (n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads != 0 || n_rows <= 0 || prefix < 0 || (capacity > 0 && !entries)) return -1;
+  const CausalPlan pl = causal_plan(n_q_heads, n_kv_heads, n_rows, prefix);
+  const CausalOrder o = causal_order(prefix, n_rows, pl.windows, pl.chunks, pl.chunk_keys, n_kv_heads * pl.pairs);
+  for (int64_t e = 0; e < std::min<int64_t>(o.entries, capacity); ++e) {
+    const CausalEntry c = o.full < 0 ? CausalEntry{(int)(e / pl.chunks), (int)(e % pl.chunks), true}
+                                     : causal_entry((int)e, o.full, pl.windows, o.blocks, o.per);
+    entries[3 * e] = c.some ? pl.windows - 1 - c.window : -1;
+    entries[3 * e + 1] = c.chunk;
+    entries[3 * e + 2] = (int32_t)pl.chunk_keys;
+  }
+  return o.entries;
+}

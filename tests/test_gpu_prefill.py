@@ -1,9 +1,12 @@
 """Prompt chunks on the one-call layers: against a float32 stack of the same weights, with the module-by-module path of the same
 dtype as the yardstick.  Both round at the same points and differ in the order of their sums, so neither may be further from
 float32 than the other by more than that difference; the bounds below are twice the yardstick's own distance."""
+import ctypes
+
 import pytest
 import torch
 
+from subspec_amd import _lib as L
 from subspec_amd import model as M, ops
 from subspec_amd.cache import create_kv_cache
 
@@ -54,6 +57,17 @@ def test_prefill_matches_float32(n, start, dtype, hq, hkv):
         assert native <= 2 * module, (part, native, module)
     rows = out["native"][1]
     assert torch.equal(rows[..., :start, :], past[..., :start, :]) and torch.equal(rows[..., start + n:, :], past[..., start + n:, :])
+
+
+# more workgroups than compute units and windows of very different length: they start in falling order
+@pytest.mark.parametrize("n,start", [(700, 0), (705, 63), (701, 350)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_windows_in_falling_order(n, start, dtype):
+    order = L.lib().subspec_prefill_attention_order
+    entries = (ctypes.c_int32 * 300)()
+    assert 3 * order(16, 16, n, start, entries, 100) <= 300
+    assert entries[0] == entries[3] + 1 and entries[1] == entries[4] == 0       # the longest two windows' first chunks
+    test_prefill_matches_float32(n, start, dtype, 16, 16)
 
 
 @pytest.mark.parametrize("n,start", [(20, 0), (70, 0), (300, 0), (130, 200)])

@@ -34,6 +34,7 @@
 // (405 FLOP/B) is above the chip's ridge, so the bound that applies is the matrix pipe, not HBM.
 #include "common.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace subspec {
 
@@ -82,6 +83,7 @@ struct AttnParams {
   int pairs_per_kv;            // workgroups (groups of 4 or 8 query heads) per KV head
   int64_t units;               // batch * hkv * chunks; causal, falling order: hkv * entries of causal_entry
   int full;                    // causal: entries that are whole chunks; -1: entries window by window
+  bool wide_partials;          // tree_attention32_kernel: a chunk's averages are left in fp32
   float scale_log2;            // softmax scale * log2(e)
   // paged cache (one request): row p of K lives at page_table[p >> page_shift], token p & (page_len - 1) of
   // a pool layer [max_pages][2 (K, V)][page_len][hkv][128]; V is v_delta elements behind K
@@ -714,15 +716,26 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
                                                       pack2<DT>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv));
   } else {
     // the chunk's own softmax-weighted average of V, in the 16-bit dtype (a convex combination of such averages is what the
-    // merge forms, so their rounding error does not grow); every store instruction writes 512 consecutive bytes
+    // merge forms, so their rounding error does not grow), or in fp32 (attn_plan: fewer chunks have fewer probabilities that are
+    // exactly 1); every store instruction writes 512 or 1024 consecutive bytes
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t* po = (uint16_t*)part_o + (((int64_t)vbh * ap.chunks + chunk) * 2 + tile) * kTileElems + lane * 4;
+    const int64_t at = (((int64_t)vbh * ap.chunks + chunk) * 2 + tile) * kTileElems + lane * 4;
+    if (ap.wide_partials) {
 #pragma unroll
-    for (int dt = 0; dt < kAttnD / 32; ++dt)
+      for (int dt = 0; dt < kAttnD / 32; ++dt)
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
-        *(uint2*)(po + (dt * 4 + q4) * 256) = make_uint2(pack2<DT>(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
-                                                         pack2<DT>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv));
+        for (int q4 = 0; q4 < 4; ++q4)
+          *(float4*)(part_o + at + (dt * 4 + q4) * 256) = make_float4(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv,
+                                                                      oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv);
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < kAttnD / 32; ++dt)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+          *(uint2*)((uint16_t*)part_o + at + (dt * 4 + q4) * 256) =
+              make_uint2(pack2<DT>(oacc[dt][4 * q4] * inv, oacc[dt][4 * q4 + 1] * inv),
+                         pack2<DT>(oacc[dt][4 * q4 + 2] * inv, oacc[dt][4 * q4 + 3] * inv));
+    }
     if (g == 0) {
       const int64_t pslot = ((int64_t)vbh * ap.chunks + chunk) * kAttnRows + row;
       *(v2f_t*)(part_ml + pslot * 2) = v2f_t{m_run * ap.scale_log2, l};
@@ -1201,7 +1214,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // and its four elements, of every chunk -- is issued before the first is used, so the launch pays ONE round trip to
 // memory instead of one for the maximum and one for the sums (config 3, B = 8: 6.1 -> 5.3 us); CMAX = 0 is the two-pass
 // form for more chunks, where that many loads up front cost more than they save.
-template <int DT, int CMAX>
+// WIDE: fp32 averages (AttnPlan::wide_partials).
+template <int DT, int CMAX, bool WIDE>
 __global__ __launch_bounds__(256) void tree_attention32_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, AttnParams ap, uint16_t* __restrict__ out) {
   const int tile = blockIdx.x & 1, vbh = blockIdx.x >> 1;
@@ -1212,9 +1226,12 @@ __global__ __launch_bounds__(256) void tree_attention32_merge_kernel(
   const int b = aw.b;
   if (row >= aw.win_rows) return;
   const int64_t slot0 = (int64_t)vbh * ap.chunks * kAttnRows + row;
-  const uint16_t* po = (const uint16_t*)part_o + ((int64_t)vbh * ap.chunks * 2 + tile) * kTileElems + (idx16 * 64 + lane) * 4;
-  auto unpack4 = [](uint2 o, float* f) {
-    if constexpr (DT == SUBSPEC_BF16) {
+  using Four = std::conditional_t<WIDE, float4, uint2>;                    // four elements as they are stored
+  const auto* const po = (const std::conditional_t<WIDE, float, uint16_t>*)part_o + ((int64_t)vbh * ap.chunks * 2 + tile) * kTileElems + (idx16 * 64 + lane) * 4;
+  auto unpack4 = [](Four o, float* f) {
+    if constexpr (WIDE) {
+      f[0] = o.x; f[1] = o.y; f[2] = o.z; f[3] = o.w;
+    } else if constexpr (DT == SUBSPEC_BF16) {
       f[0] = bf16_bits_to_float(o.x & 0xffffu); f[1] = bf16_bits_to_float(o.x >> 16);
       f[2] = bf16_bits_to_float(o.y & 0xffffu); f[3] = bf16_bits_to_float(o.y >> 16);
     } else {
@@ -1226,12 +1243,12 @@ __global__ __launch_bounds__(256) void tree_attention32_merge_kernel(
   float num[4] = {0.f, 0.f, 0.f, 0.f};
   if constexpr (CMAX > 0) {
     v2f_t ml[CMAX];
-    uint2 oc[CMAX];
+    Four oc[CMAX];
 #pragma unroll
     for (int c = 0; c < CMAX; ++c) {
       const int cc = min(c, ap.chunks - 1);              // chunks past the count repeat the last one and get no weight
       ml[c] = *(const v2f_t*)(&part_ml[(slot0 + (int64_t)cc * kAttnRows) * 2]);
-      oc[c] = *(const uint2*)(po + (int64_t)cc * 2 * kTileElems);
+      oc[c] = *(const Four*)(po + (int64_t)cc * 2 * kTileElems);
     }
 #pragma unroll
     for (int c = 0; c < CMAX; ++c) m = fmaxf(m, ml[c][0]);
@@ -1252,7 +1269,7 @@ __global__ __launch_bounds__(256) void tree_attention32_merge_kernel(
 #pragma unroll 8
     for (int c = 0; c < ap.chunks; ++c) {
       const v2f_t ml = *(const v2f_t*)(&part_ml[(slot0 + (int64_t)c * kAttnRows) * 2]);
-      const uint2 o = *(const uint2*)(po + (int64_t)c * 2 * kTileElems);
+      const Four o = *(const Four*)(po + (int64_t)c * 2 * kTileElems);
       const float w = ml[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0] - m) * ml[1];
       float f[4];
       unpack4(o, f);
@@ -1322,7 +1339,7 @@ __global__ __launch_bounds__(256) void causal_attention_merge_kernel(const float
 
 // Launch shape of one window of query rows.  most_chunks: what the workspace is sized for, at least the chunks of this key count and of
 // every smaller one (a draft level has 24 chunks at 3072 keys and 17 at 3073; a workspace serves all prefixes up to the one it was made for).
-struct AttnPlan { int threads, rowt, wph, heads_per_wg, chunks, most_chunks; bool mfma32, pingpong; };
+struct AttnPlan { int threads, rowt, wph, heads_per_wg, chunks, most_chunks; bool mfma32, pingpong, wide_partials; };
 static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_rows, int64_t kv_len, bool one_sequence) {
   AttnPlan pl;
   const int group = (int)(hq / hkv);
@@ -1379,6 +1396,27 @@ static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_ro
     if (brief <= chunks ? one_round || rounds(brief) <= rounds(chunks)
                         : one_round && batch * hq * win_rows * brief <= (brief <= 12 ? 13312 : 10240))
       chunks = brief;
+  }
+  // 33 rows and more: a last round of few workgroups takes as long as a full one, so where chunks of a block or two more save a round,
+  // they are taken (a workgroup costs about three blocks besides its own; an XCD runs 32 large or 64 small ones).  Both launches, bf16: 289
+  // rows of 28 : 4 heads at 2337 keys, 280 -> 240 workgroups, 41.1 -> 36.1 us, at 4385 61.4 -> 45.0; 400 rows 59.0 -> 47.3; 289 rows of
+  // 32 : 8 42.3 -> 36.7, of 16 : 8 31.3 -> 30.7; three sequences of 64 rows of 28 : 4 at 4160 keys 38.5 -> 35.3.  Their averages are left
+  // in fp32 (2 us of what is gained): in 16 bits the results were 0.05 to 0.5 % further from float64 than with the shorter chunks
+  // (2.708e-3 -> 2.712e-3 at 289 rows), in fp32 they are 20 % nearer (2.167e-3).
+  pl.wide_partials = false;
+  if (win_rows > 32 && !pl.pingpong) {
+    const int64_t per_unit = (group + pl.heads_per_wg - 1) / pl.heads_per_wg, fit = target_wgs / kXcds;   // workgroups of an XCD
+    auto per_chunk = [&](int64_t c) { return (blocks + c - 1) / c; };
+    auto rounds = [&](int64_t c) {
+      const int64_t used = (blocks + per_chunk(c) - 1) / per_chunk(c);
+      return ((batch * hkv * used + kXcds - 1) / kXcds * per_unit + fit - 1) / fit;
+    };
+    int64_t fewer = chunks;
+    while (fewer > 1 && rounds(fewer) == rounds(chunks)) --fewer;
+    if (rounds(fewer) < rounds(chunks) && rounds(fewer) * (per_chunk(fewer) + 3) < rounds(chunks) * (per_chunk(chunks) + 3)) {
+      chunks = fewer;
+      pl.wide_partials = true;
+    }
   }
   pl.chunks = (int)std::min<int64_t>(chunks, 64);
   return pl;
@@ -1484,6 +1522,7 @@ static int tree_attention_impl(const char* what, const void* q, const void* k_ca
     ap.chunk_keys = (blocks + pl.chunks - 1) / pl.chunks * kKeyBlock;
     ap.chunks = (int)((kv_len + ap.chunk_keys - 1) / ap.chunk_keys);
     ap.units = vbatch * n_kv_heads * ap.chunks;
+    ap.wide_partials = pl.wide_partials;
     ap.pairs_per_kv = (group + pl.heads_per_wg - 1) / pl.heads_per_wg;
     const dim3 grid((unsigned)((ap.units + kXcds - 1) / kXcds * kXcds * ap.pairs_per_kv));
     const int64_t merge_rows = batch * n_q_heads * ap.win_rows / 8 >= 1024 ? 8 : 2;   // rows per merge workgroup (one window only)
@@ -1497,6 +1536,12 @@ static int tree_attention_impl(const char* what, const void* q, const void* k_ca
 #define SUBSPEC_ATTNPP_KERNEL(DT, WPH)                                                                             \
   hipLaunchKernelGGL((tree_attention_pp_kernel<DT, WPH>), grid, dim3(512), 0, st, (const uint16_t*)q,              \
                      (const uint16_t*)k_cache, (const uint16_t*)v_cache, anc_bits, ap, (uint16_t*)out, part_o, part_ml)
+#define SUBSPEC_ATTN32_MERGE(DT, WIDE)                                                                             \
+  do {                                                                                                             \
+    if (ap.chunks <= 4) hipLaunchKernelGGL((tree_attention32_merge_kernel<DT, 4, WIDE>), mg, dim3(256), 0, st, part_o, part_ml, ap, (uint16_t*)out); \
+    else if (ap.chunks <= 8) hipLaunchKernelGGL((tree_attention32_merge_kernel<DT, 8, WIDE>), mg, dim3(256), 0, st, part_o, part_ml, ap, (uint16_t*)out); \
+    else hipLaunchKernelGGL((tree_attention32_merge_kernel<DT, 0, WIDE>), mg, dim3(256), 0, st, part_o, part_ml, ap, (uint16_t*)out); \
+  } while (0)
 #define SUBSPEC_ATTN_LAUNCH(DT, PAGED)                                                                             \
   do {                                                                                                             \
     {                                                                                                              \
@@ -1512,9 +1557,7 @@ static int tree_attention_impl(const char* what, const void* q, const void* k_ca
     if (ap.chunks > 1) {                                                                                           \
       if (pl.mfma32) {                                                                                             \
         const dim3 mg((unsigned)(vbatch * n_q_heads * 2), 4);                                                      \
-        if (ap.chunks <= 4) hipLaunchKernelGGL((tree_attention32_merge_kernel<DT, 4>), mg, dim3(256), 0, st, part_o, part_ml, ap, (uint16_t*)out); \
-        else if (ap.chunks <= 8) hipLaunchKernelGGL((tree_attention32_merge_kernel<DT, 8>), mg, dim3(256), 0, st, part_o, part_ml, ap, (uint16_t*)out); \
-        else hipLaunchKernelGGL((tree_attention32_merge_kernel<DT, 0>), mg, dim3(256), 0, st, part_o, part_ml, ap, (uint16_t*)out); \
+        if (ap.wide_partials) SUBSPEC_ATTN32_MERGE(DT, true); else SUBSPEC_ATTN32_MERGE(DT, false);                  \
       } else                                                                                                         \
         hipLaunchKernelGGL((tree_attention_merge_kernel<DT>), merge_grid, dim3(merge_rows * 32), 0, st, part_o, part_ml, ap, \
                            (uint16_t*)out);                                                                        \
@@ -1523,6 +1566,7 @@ static int tree_attention_impl(const char* what, const void* q, const void* k_ca
     if (dtype == SUBSPEC_BF16) { if (paged) SUBSPEC_ATTN_LAUNCH(SUBSPEC_BF16, true); else SUBSPEC_ATTN_LAUNCH(SUBSPEC_BF16, false); }
     else { if (paged) SUBSPEC_ATTN_LAUNCH(SUBSPEC_F16, true); else SUBSPEC_ATTN_LAUNCH(SUBSPEC_F16, false); }
 #undef SUBSPEC_ATTN_LAUNCH
+#undef SUBSPEC_ATTN32_MERGE
 #undef SUBSPEC_ATTN32_KERNEL
 #undef SUBSPEC_ATTN_KERNEL
   }

@@ -286,3 +286,13 @@ def test_chunks_of_a_draft_level(blocks, rows, hq, hkv):
 def test_chunks_of_a_wide_draft_level(B, rows, hq, hkv, n_keys):
     parents, q, k, v = _case(n_keys, B, hq, hkv, rows, n_keys - rows, n_keys + 3, torch.bfloat16)
     _check(parents, q, k, v, n_keys - rows, "wide draft level")
+
+
+# chunks whose averages stay in fp32 (fewer chunks than would fill the chip, to save a round of workgroups): up to 4, up to 8, and more
+@pytest.mark.parametrize("B,hq,hkv,n,P", [(1, 28, 4, 390, 2000), (1, 28, 4, 261, 2090), (1, 16, 8, 289, 2048), (3, 28, 4, 50, 4040)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_chunks_that_save_a_round(dtype, B, hq, hkv, n, P):
+    parents, q, k, v = _case(n, B, hq, hkv, n, P, P + n + 3, dtype, depth=20 if n > 64 else 8)
+    k[:, :, P + n:] = 1e3                                              # stale rows beyond the tree must not be read
+    v[:, :, P + n:] = -1e3
+    _check(parents, q, k, v, P, "saves a round")

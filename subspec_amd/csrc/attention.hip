@@ -64,6 +64,25 @@ typedef _Float16 v2h_t __attribute__((ext_vector_type(2)));
 typedef float v2f_t __attribute__((ext_vector_type(2)));
 
 
+// The keys of a 64-key block that one row attends, as bits, for a block that reaches into the tree (kb + 64 > prefix, kb < kv_len):
+// cached rows all, tree rows by the row's bitset (`word`, `next`: its words from the block's first tree row on), none past the last.
+// One mask per row and block and two instructions per score; deciding per score, with 64-bit positions, took ten to fifteen of them and
+// made a masked block two to three times as long as a plain one.  One sequence, bf16, both launches: 289 rows of 28 : 4 heads at 2337
+// keys 36.0 -> 32.8 us, at 589 29.5 -> 21.9, 500 rows at 2548 48.9 -> 37.4; a draft level, all of it 1811.8 -> 1804.7.
+__device__ __forceinline__ uint64_t block_bits(int64_t kb, int64_t prefix, int64_t kv_len, uint64_t word, uint64_t next) {
+  const int off = (int)(kb - prefix);
+  uint64_t m;
+  if (off >= 0) m = (word >> (off & 63)) | (next << 1 << (63 - (off & 63)));
+  else m = (word << -off) | ~(~0ull << -off);
+  const int64_t left = kv_len - kb;
+  return left < 64 ? m & ~(~0ull << left) : m;
+}
+// the score where bit k is set, -inf elsewhere
+__device__ __forceinline__ float where_bit(uint32_t bits, int k, float score) {
+  const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)bits, k, 1);
+  return __uint_as_float((__float_as_uint(score) & keep) | (0xff800000u & ~keep));
+}
+
 // Transposing LDS read of 16-bit elements (ds_read_b64_tr_b16): within each group of 16 lanes,
 // lane i receives element i%4 of the four 8-byte rows addressed by lanes i/4, i/4 + 4, i/4 + 8,
 // i/4 + 12 of the group.
@@ -287,35 +306,28 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int nt = 0; nt < ROWT; ++nt) acc[kt][nt] = mfma32<DT>(a, qreg[nt][ks], acc[kt][nt]);
       }
     }
+    if (plain) {
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      if (plain) {
+      for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
           for (int nt = 0; nt < ROWT; ++nt) {
             s[nt][kt][r] = acc[kt][nt][r];
             mloc[nt] = fmaxf(mloc[nt], acc[kt][nt][r]);
           }
-        }
-      } else {
+    } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t pos = kb + kt * 16 + lg * 4 + r;
-          const bool in_range = pos < kv_len;
-          const bool tree = pos >= prefix;
-          const int rel = tree ? (int)(pos - prefix) : 0;   // tree slot, < 64 * mask_words when in range
-          const int sh = rel & 63;
-          const bool first_word = (rel >> 6) == word0;
+      for (int nt = 0; nt < ROWT; ++nt) {
+        const uint64_t keys = block_bits(kb, prefix, kv_len, bits[nt][0], bits[nt][1]);
+        const uint32_t half[2] = {(uint32_t)keys >> (4 * lg), (uint32_t)(keys >> 32) >> (4 * lg)};
 #pragma unroll
-          for (int nt = 0; nt < ROWT; ++nt) {
-            const uint64_t word = first_word ? bits[nt][0] : bits[nt][1];
-            const bool ok = in_range && (!tree || ((word >> sh) & 1ull));
-            const float t = ok ? acc[kt][nt][r] : -INFINITY;
-            s[nt][kt][r] = t;
-            mloc[nt] = fmaxf(mloc[nt], t);
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            s[nt][kt][r] = where_bit(half[kt >> 1], (kt & 1) * 16 + r, acc[kt][nt][r]);
+            mloc[nt] = fmaxf(mloc[nt], s[nt][kt][r]);
           }
-        }
       }
     }
     // running maximum in units of raw scores (the scale is positive, so the order is the same)
@@ -642,19 +654,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
       // a 64-key block touches at most two consecutive words of the row's bitset (a zero word follows the last)
       const int word0 = min((int)(max(kb - prefix, (int64_t)0) >> 6), SUBSPEC_MAX_TREE_NODES / 64 - 1);
       const uint64_t bits0 = row_ok ? mask_s[row][word0] : 0ull, bits1 = row_ok ? mask_s[row][word0 + 1] : 0ull;
+      const uint64_t keys = block_bits(kb, prefix, kv_len, bits0, bits1);
+      const uint32_t half[2] = {(uint32_t)keys >> (4 * g), (uint32_t)(keys >> 32) >> (4 * g)};
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int64_t pos = kb + t * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
-          const bool in_range = pos < kv_len;
-          const bool tree = pos >= prefix;
-          const int rel = tree ? (int)(pos - prefix) : 0;
-          const uint64_t word = (rel >> 6) == word0 ? bits0 : bits1;
-          const bool ok = in_range && (!tree || ((word >> (rel & 63)) & 1ull));
-          const float tv = ok ? sacc[t][r] : -INFINITY;
-          sacc[t][r] = tv;
-          mloc = fmaxf(mloc, tv);
+          sacc[t][r] = where_bit(half[t], (r >> 2) * 8 + (r & 3), sacc[t][r]);
+          mloc = fmaxf(mloc, sacc[t][r]);
         }
       }
     }
@@ -885,19 +892,12 @@ __device__ __forceinline__ void pp_softmax_phase(int64_t kb, const PPRow& rw, v1
     // a 64-key block touches at most two consecutive words of the row's bitset (a zero word follows the last)
     const int word0 = min((int)(max(kb - rw.prefix, (int64_t)0) >> 6), SUBSPEC_MAX_TREE_NODES / 64 - 1);
     const uint64_t bits0 = rw.row_ok ? rw.mask_row[word0] : 0ull, bits1 = rw.row_ok ? rw.mask_row[word0 + 1] : 0ull;
+    const uint64_t keys = block_bits(kb, rw.prefix, rw.kv_len, bits0, bits1);
+    const uint32_t half[2] = {(uint32_t)keys >> (4 * rw.g), (uint32_t)(keys >> 32) >> (4 * rw.g)};
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t pos = kb + t * 32 + (r >> 2) * 8 + rw.g * 4 + (r & 3);
-        const bool in_range = pos < rw.kv_len;
-        const bool tree = pos >= rw.prefix;
-        const int rel = tree ? (int)(pos - rw.prefix) : 0;
-        const uint64_t word = (rel >> 6) == word0 ? bits0 : bits1;
-        const bool ok = in_range && (!tree || ((word >> (rel & 63)) & 1ull));
-        sacc[t][r] = ok ? sacc[t][r] : -INFINITY;
-      }
-    }
+      for (int r = 0; r < 16; ++r) sacc[t][r] = where_bit(half[t], (r >> 2) * 8 + (r & 3), sacc[t][r]);
   }
   float mt[2] = {-INFINITY, -INFINITY};
 #pragma unroll
@@ -1399,7 +1399,7 @@ static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_ro
   }
   // 33 rows and more: a last round of few workgroups takes as long as a full one, so where chunks of a block or two more save a round,
   // they are taken (a workgroup costs about three blocks besides its own; an XCD runs 32 large or 64 small ones).  Both launches, bf16: 289
-  // rows of 28 : 4 heads at 2337 keys, 280 -> 240 workgroups, 41.1 -> 36.1 us, at 4385 61.4 -> 45.0; 400 rows 59.0 -> 47.3; 289 rows of
+  // rows of 28 : 4 heads at 2337 keys, 280 -> 240 workgroups, 41.1 -> 36.1 us (before block_bits), at 4385 61.4 -> 45.0; 400 rows 59.0 -> 47.3; 289 rows of
   // 32 : 8 42.3 -> 36.7, of 16 : 8 31.3 -> 30.7; three sequences of 64 rows of 28 : 4 at 4160 keys 38.5 -> 35.3.  Their averages are left
   // in fp32 (2 us of what is gained): in 16 bits the results were 0.05 to 0.5 % further from float64 than with the shorter chunks
   // (2.708e-3 -> 2.712e-3 at 289 rows), in fp32 they are 20 % nearer (2.167e-3).

@@ -118,12 +118,18 @@ def tiled_head(rows: int, vocab: int, hidden: int) -> bool:
     take 0.60 to 1.01 of the GEMM's time up to 320 rows (152064 x 3584, 289 rows: 332 against 414 us) and 0.87 to 0.98 up to 384 where
     a row has 2560 elements (1024: 1.08); heads of 128000 to 130047 rows of 3072 elements and more 0.73 to 0.95 (2048: 1.06).  At others
     the GEMM is level or ahead at some row count: 65536 x 2048 1.13 to 1.18, 50304 x 4096 1.06 to 1.11, 32000 x 5120 1.11 to 1.27, 131072 x
-    4096 1.10 to 1.19, 262144 x 1152 1.03 to 1.21, and at all heads with 65 to 192 rows (152064 x 3584, 96 rows: 221 against 232 us)."""
-    if not (192 < rows <= 384 and vocab % 32 == 0 and hidden % 64 == 0 and (1 << 28) <= 2 * vocab * hidden < (1 << 31)):
+    4096 1.10 to 1.19, 262144 x 1152 1.03 to 1.21.  With 65 to 128 rows (nine row counts, bf16 and fp16) heads of 128000 to 130047 rows of
+    4096, 5120 and 8192 elements take 0.75 to 0.90 of its time (128000 x 4096, 96 rows: 189 against 244 us) and those of 147456 to 158719
+    rows of 4096 elements 0.81 to 0.98 (152064, 65 rows: 243 against 300 us); others are level or behind at some row count (147456 x 5120
+    1.11), and with 129 to 192 rows the two are level."""
+    if not (64 < rows <= 384 and vocab % 32 == 0 and hidden % 64 == 0 and (1 << 28) <= 2 * vocab * hidden < (1 << 31)):
         return False
-    if 147456 <= vocab < 158720:
-        return rows <= 320 or hidden >= 2560
-    return 128000 <= vocab < 130048 and hidden >= 3072
+    large, medium = 147456 <= vocab < 158720, 128000 <= vocab < 130048
+    if rows <= 128:
+        return large and 4096 <= hidden < 5120 or medium and hidden >= 4096
+    if rows <= 192:
+        return False
+    return large and (rows <= 320 or hidden >= 2560) or medium and hidden >= 3072
 
 
 class Decoder:

@@ -197,3 +197,19 @@ def test_unaligned_output_takes_the_other_kernel():
     assert room[:4].abs().max() == 0 and room[4 + M * N:].abs().max() == 0
     want = ops.dense_linear(x, w)
     assert ((room[4:4 + M * N].view(M, N).float() - want.float()).abs() <= 2.0 ** -7 * want.float().abs() + 1e-3).all()
+
+
+@pytest.mark.parametrize("rows,own", [(65, True), (97, True), (128, True), (129, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_head_over_65_to_128_rows(rows, own, dtype):
+    """A head of rows of 4096 elements on the kernel that ``tiled_head`` names, against float64."""
+    V, K = 128032, 4096
+    assert model.tiled_head(rows, V, K) == own
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x = torch.randn(rows, K, generator=g, device=DEV).to(dtype)
+    holder = type("Holder", (), {"lm_head": (torch.randn(V, K, generator=g, device=DEV) * K ** -0.5).to(dtype)})()
+    with torch.no_grad():
+        got = model.Decoder._head(holder, x).double()
+    ref = x.double() @ holder.lm_head.double().T
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert ((got - ref).abs() <= ulp * ref.abs() + 1e-4).all()

@@ -179,8 +179,9 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 // reduction launch of their own.
 // A thread takes dims i, i + 1 and their partners D/2 further, 32 lanes a head, eight heads a workgroup; blockIdx.y strides over
 // the groups of eight, so that many rows evaluate their angles once per thread and not once per head.  Bound by launch and round
-// trips up to a few hundred rows (64: 4.8 -> 4.7 us, 256: 7.4 -> 6.2 against one wavefront per (row, head)), then by its 38 MB:
-// 2048 rows of 36 heads 19.7 -> 11.8 us.
+// trips up to a few hundred rows (64: 4.8 -> 4.7 us, 256: 7.4 -> 6.2 against one wavefront per (row, head)), then by its 38 MB and
+// the angles: a workgroup that takes a whole row evaluates each once and requests five groups of heads at a time.
+// 2048 rows of 36 heads 19.7 -> 11.8 us against a wavefront per (row, head), 13.3 -> 10.0 (another box) with both of these.
 constexpr int kRopeHeads = 8;
 template <int DT>
 __global__ __launch_bounds__(32 * kRopeHeads) void rope_write_kernel(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,
@@ -194,10 +195,73 @@ __global__ __launch_bounds__(32 * kRopeHeads) void rope_write_kernel(const uint1
   const int64_t width = (int64_t)heads * D;
   const int pos = positions[m], cache_row = cache_rows[m];
   // the caller's table (the values its other code paths use, so that both write identical rows), else theta^(-2i/D)
+  auto frequency = [&](int d) { return inv_freq_table ? inv_freq_table[d] : exp2f(-(float)(2 * d) / (float)D * log2_theta); };
+  auto angle = [&](float freq, float* sine, float* cosine) {
+    sincosf((float)pos * freq, sine, cosine);
+    *cosine = Elem<DT>::round(*cosine);
+    *sine = Elem<DT>::round(*sine);
+  };
+  float c[2], s[2];
+  auto rotate_and_store = [&](int hh, float (&lo)[2], float (&hi)[2]) {
+    uint16_t* dst;
+    if (hh < Hq) {
+      dst = q_out + ((int64_t)hh * M + m) * D;
+    } else {
+      // a row outside the layer's cache is dropped: a bad rows tensor must not write beyond the cache
+      uint16_t *kp, *vp;
+      if (!kv_row_ptrs(kv, (hh - Hq) % Hkv, cache_row, &kp, &vp)) return;
+      dst = hh < Hq + Hkv ? kp : vp;
+    }
+    if (hh < Hq + Hkv) {                                  // value heads are copied
+      // t * cos + rotate_half(t) * sin, each product and the sum rounded like the eager tensor ops
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float a = lo[e], b = hi[e];
+        lo[e] = Elem<DT>::round(a * c[e]) + Elem<DT>::round(-b * s[e]);
+        hi[e] = Elem<DT>::round(b * c[e]) + Elem<DT>::round(a * s[e]);
+      }
+    }
+    *(uint32_t*)(dst + i) = pack2<DT>(lo[0], lo[1]);
+    *(uint32_t*)(dst + i + half) = pack2<DT>(hi[0], hi[1]);
+  };
+  if (splits == 0 && gridDim.y == 1) {
+    // all heads of a row: five groups' elements are requested before the first is used, and an angle is evaluated once
+    __shared__ float sine[half], cosine[half];
+    constexpr int kBatch = 5;
+    const uint16_t* const src = qkv + (int64_t)m * width + i;
+    const int group = threadIdx.x >> 5, dim = threadIdx.x & (half - 1);
+    const float freq = frequency(dim);
+    bool first = true;
+    for (int h0 = 0; h0 < heads; h0 += kBatch * kRopeHeads) {              // (uniform: a barrier in the first round)
+      uint32_t raw[kBatch][2];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        const uint16_t* const head = src + (int64_t)min(h0 + k * kRopeHeads + group, heads - 1) * D;
+        raw[k][0] = *(const uint32_t*)head;
+        raw[k][1] = *(const uint32_t*)(head + half);
+      }
+      if (first) {
+        first = false;
+        if (threadIdx.x < half) angle(freq, &sine[dim], &cosine[dim]);
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 2; ++e) { s[e] = sine[i + e]; c[e] = cosine[i + e]; }
+      }
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        const int hh = h0 + k * kRopeHeads + group;
+        if (hh >= heads) break;
+        float lo[2], hi[2];
+        unpack2<DT>(raw[k][0], lo);
+        unpack2<DT>(raw[k][1], hi);
+        rotate_and_store(hh, lo, hi);
+      }
+    }
+    return;
+  }
   float freq[2];
 #pragma unroll
-  for (int e = 0; e < 2; ++e) freq[e] = inv_freq_table ? inv_freq_table[i + e] : exp2f(-(float)(2 * (i + e)) / (float)D * log2_theta);
-  float c[2], s[2];
+  for (int e = 0; e < 2; ++e) freq[e] = frequency(i + e);
   bool angles = false;
   for (int hh = blockIdx.y * kRopeHeads + (threadIdx.x >> 5); hh < heads; hh += gridDim.y * kRopeHeads) {
     const int64_t col = (int64_t)hh * D + i;
@@ -230,11 +294,7 @@ __global__ __launch_bounds__(32 * kRopeHeads) void rope_write_kernel(const uint1
     if (!angles) {
       angles = true;
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        sincosf((float)pos * freq[e], &s[e], &c[e]);
-        c[e] = Elem<DT>::round(c[e]);
-        s[e] = Elem<DT>::round(s[e]);
-      }
+      for (int e = 0; e < 2; ++e) angle(freq[e], &s[e], &c[e]);
     }
     float lo[2], hi[2];
     if (splits > 0) {
@@ -255,26 +315,7 @@ __global__ __launch_bounds__(32 * kRopeHeads) void rope_write_kernel(const uint1
       unpack2<DT>(raw[0], lo);
       unpack2<DT>(raw[1], hi);
     }
-    uint16_t* dst;
-    if (hh < Hq) {
-      dst = q_out + ((int64_t)hh * M + m) * D;
-    } else {
-      // a row outside the layer's cache is dropped: a bad rows tensor must not write beyond the cache
-      uint16_t *kp, *vp;
-      if (!kv_row_ptrs(kv, (hh - Hq) % Hkv, cache_row, &kp, &vp)) continue;
-      dst = hh < Hq + Hkv ? kp : vp;
-    }
-    if (hh < Hq + Hkv) {                                  // value heads are copied
-      // t * cos + rotate_half(t) * sin, each product and the sum rounded like the eager tensor ops
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const float a = lo[e], b = hi[e];
-        lo[e] = Elem<DT>::round(a * c[e]) + Elem<DT>::round(-b * s[e]);
-        hi[e] = Elem<DT>::round(b * c[e]) + Elem<DT>::round(a * s[e]);
-      }
-    }
-    *(uint32_t*)(dst + i) = pack2<DT>(lo[0], lo[1]);
-    *(uint32_t*)(dst + i + half) = pack2<DT>(hi[0], hi[1]);
+    rotate_and_store(hh, lo, hi);
   }
 }
 

@@ -986,7 +986,7 @@ inline CausalOrder causal_order(int64_t prefix, int64_t n_rows, int windows, int
 // rows of its own window up to the query's, so its row masks are (2 << row) - 1 and come from no memory.  Windows have
 // different lengths (causal_order: which starts when); the partial results of a window cut into several chunks stay fp32
 // (unnormalised O and sum).
-// 28 : 4 heads, bf16: 2048 rows of a prompt 57 to 61 us + 10 us merge, the last 256 of 2048 20 + 7 us (a library's attention with the
+// 28 : 4 heads, bf16: 2048 rows of a prompt 54 to 61 us + 10 us merge, the last 256 of 2048 18 to 20 + 7 us (a library's attention with the
 // mask it needs and K / V repeated for the heads: 275 and 190 us).  Bound by the softmax and matrix phases of the blocks, like
 // the tree form.
 template <int DT, int WPH, bool CAUSAL = false>
@@ -1350,7 +1350,7 @@ static AttnPlan attn_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t win_ro
   // one bit for bit, and the ping-pong kernel's probabilities are relative to a reference up to 2^8 below the row's maximum, so that
   // the largest is rounded where it is exactly 1 in the other kernel.  289 rows, 28 : 4 heads, 2337 keys, distance from float64: 2.81e-3
   // against 2.70e-3 in bf16 and 3.52e-4 against 3.39e-4 in fp16 (scores three times as large: 2.56e-3, 2.39e-3; 3.19e-4, 2.97e-4), for
-  // 35 against 40 us a call; over pages it would need a copy of the rows (200 rows of 32 : 8 heads, 2500 keys: 41 against 34 us).
+  // 35 us a call (33 here); over pages it would need a copy of the rows (200 rows of 32 : 8 heads, 2500 keys: 41 against 34 us).
   pl.pingpong = pl.mfma32 && !one_sequence && batch * hq >= 128;
   if (win_rows <= 16) {
     // a draft level: a wavefront is a whole head (one 16-row tile), eight heads share the staged keys

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 // the groups of eight, so that many rows evaluate their angles once per thread and not once per head.  Bound by launch and round
 // trips up to a few hundred rows (64: 4.8 -> 4.7 us, 256: 7.4 -> 6.2 against one wavefront per (row, head)), then by its 38 MB and
 // the angles: a workgroup that takes a whole row evaluates each once and requests five groups of heads at a time.
-// 2048 rows of 36 heads 19.7 -> 11.8 us against a wavefront per (row, head), 13.3 -> 10.0 (another box) with both of these.
+// 2048 rows of 36 heads 19.7 -> 11.8 us against a wavefront per (row, head), 13.3 -> 10.0 with both of these.
 constexpr int kRopeHeads = 8;
 template <int DT>
 __global__ __launch_bounds__(32 * kRopeHeads) void rope_write_kernel(const uint16_t* __restrict__ qkv, const int32_t* __restrict__ positions,

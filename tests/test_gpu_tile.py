@@ -81,6 +81,31 @@ def test_activation_over_its_range(M, dtype):
     assert (act != want)[~big].double().mean() <= 90 / 2 ** (15 if dtype == torch.bfloat16 else 12)
 
 
+@pytest.mark.parametrize("M", [3, 40, 70, 289])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_activation_of_every_gate_is_the_nearest_value(M, dtype):
+    """All finite gates of the type with a normal result (gate = x, up = 1, as above) against silu in float64, rounded once: the
+    correctly rounded fp32 quotient of the hardware's exponential misses no bf16 value and one fp16 value (-0.7139)."""
+    K, F = 64 + 64, 64
+    gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
+    exact = gates.double() * torch.sigmoid(gates.double())
+    normal = 2.0 ** (-126 if dtype == torch.bfloat16 else -14)
+    gates = gates[gates.isfinite() & (exact.abs() >= normal) & (gates > -80)]
+    count = gates.numel()
+    rows = -(-count // F)
+    rows = -(-rows // M) * M
+    gates = torch.cat([gates, torch.ones(rows * F - count, dtype=dtype)]).view(rows, F)
+    x = torch.cat([gates, torch.ones(rows, 1, dtype=dtype), torch.zeros(rows, K - F - 1, dtype=dtype)], dim=1).to(DEV)
+    w = torch.zeros(2 * F, K)
+    w[:F, :F] = torch.eye(F)
+    w[F:, F] = 1.0
+    w = w.to(dtype).to(DEV)
+    got = torch.cat([ops.dense_gate_up_silu(x[i:i + M], w) for i in range(0, rows, M)]).cpu().flatten()[:count]
+    gates = gates.flatten()[:count].double()
+    want = (gates * torch.sigmoid(gates)).to(dtype)
+    assert int((got != want).sum()) <= (0 if dtype == torch.bfloat16 else 1), gates[got != want]
+
+
 def _plan(M, N, K, gate_up):
     """(tile shape, row tiles, column tiles, K ranges)"""
     plan = (ctypes.c_int32 * 4)()

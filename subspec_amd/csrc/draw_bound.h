@@ -1,0 +1,20 @@
+// The bound that the wavefronts of a sampled draw share (row_sample_kernel): log2 of a key, as a float whose bits are compared as
+// an unsigned integer.  2^23 (log2(key) - 23 + 256): positive for every fp32 key above zero, so that larger keys have larger bits.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace subspec {
+
+constexpr float kSeenBias = 256.0f * 0x1p23f;
+
+// bits of a positive key, from below (1.5e-4 covers the roundings).  The logarithm comes in front of the scaling: a key below 2^-127
+// would not survive the product, and the bits of -inf are more than any real bound has -- such a slice would evaluate every element
+// to its end.
+__host__ __device__ inline uint32_t seen_bits_of(float key) {
+  const float bits = (log2f(key) - (23.0f + 1.5e-4f)) * 0x1p23f + kSeenBias;
+  return __builtin_bit_cast(uint32_t, bits);
+}
+// 2^23 (log2(key) - 23) again
+__host__ __device__ inline float seen_level(uint32_t bits) { return __builtin_bit_cast(float, bits) - kSeenBias; }
+
+}  // namespace subspec

@@ -28,6 +28,7 @@
 // row maximum; the normalized entropy of a 16-bit row is sum(entr(p)) with p, log p and p*log p
 // each rounded to that dtype, the sum rounded once, divided by float(ln V) and rounded again.
 #include "common.h"
+#include "draw_bound.h"
 #include <string.h>
 #include <mutex>
 #include <algorithm>
@@ -469,8 +470,7 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
     const void* __restrict__ logits, VerifyParams vp, const Part1* __restrict__ part1, Part3* __restrict__ part3) {
   __shared__ float red_f[kRowThreads / kWave];
   __shared__ int red_i[kRowThreads / kWave];
-  __shared__ uint32_t bound;            // log2 of the best key any wavefront has published, kSeenBias added; 0: none yet
-  constexpr float kSeenBias = 256.0f * 0x1p23f;
+  __shared__ uint32_t bound;            // seen_bits_of the best key any wavefront has published; 0: none yet
   if (threadIdx.x == 0) bound = 0;
   __syncthreads();
   const int64_t row = blockIdx.y;
@@ -561,7 +561,7 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
   auto publish = [&](float key) __attribute__((always_inline)) {
     key = wave_max(key);
     if (!(key > 0.f) || (threadIdx.x & (kWave - 1))) return;
-    atomicMax(&bound, __float_as_uint(log2f(key * (0.9999f * 0x1p-23f)) * 0x1p23f + kSeenBias));
+    atomicMax(&bound, seen_bits_of(key));
   };
 #pragma unroll
   for (int b = 0; b < U; ++b) load(0, b, xs[b]);
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
       publish(element(g, at) < (uint32_t)n && key > 0.f ? key : 0.f);
       seen_bits = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
     }
-    const float seen = __uint_as_float(seen_bits) - kSeenBias;
+    const float seen = seen_level(seen_bits);
     const float from = seen_bits ? level - seen : INFINITY, floor_from = seen_bits ? kFloor - seen : INFINITY;
     uint64_t vote = 0;
 #pragma unroll

@@ -115,6 +115,25 @@ def test_draws_of_blocks_tested_as_one(dtype, vocab):
     assert near <= 3
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("low,high", [(85.0, 105.0), (60.0, 90.0), (10.0, 30.0)])
+def test_draws_of_rows_with_one_token_far_above(dtype, low, high):
+    """Probabilities that are subnormal, that round to nothing, or that are just large enough to count, after division by T = 0.2:
+    in front of the token, behind it, and in slices without one; two equal tokens, and one among masked elements."""
+    g = torch.Generator().manual_seed(int(low))
+    rows, vocab, T = 8, 60012, 0.2
+    logits = 20.0 - (low + (high - low) * torch.rand(rows, vocab, generator=g)) * T
+    for r, at in enumerate((0, 17, 30000, vocab - 1, 45001, 59000)):
+        logits[r, at] = 20.0
+    logits[4, 100] = 20.0
+    logits[5, :58000] = float("-inf")
+    logits[6, 40000:] += low * T                          # many that count, behind many that do not
+    logits[7, ::2] = 0.0
+    logits = logits.to(dtype)
+    near = _check_draws(logits, T, ops.sample_tokens(logits.to(DEV), T, 31, 2).cpu(), 31, 2)
+    assert near <= 1
+
+
 def test_draw_frequencies_on_device():
     # 256 rows x 300 offsets of one 16-way distribution: chi-square against the rounded probabilities
     p = torch.tensor([0.25, 0.18, 0.14, 0.10, 0.08, 0.06, 0.05, 0.04, 0.03, 0.02, 0.02, 0.01, 0.01, 0.005, 0.003, 0.002])

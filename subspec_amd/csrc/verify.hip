@@ -457,12 +457,16 @@ template <> struct RoundBound<SUBSPEC_BF16> { static constexpr float rel = 0x1p-
 // exponential: its left side is linear in the logit, and the bit pattern of a float, read as an integer, is 2^23 (127 + log2)
 // from below (exact at powers of two, at most 0.087 low).  Both sides are monotone, so the four elements of a block are tested at
 // once with their largest logit and their smallest word -- ten instructions beside the unpacking -- and one by one only in the
-// trips where some block of the wavefront passes.  The bound lives in LDS: a wavefront's records prune the other seven's elements, and
-// before there is one every lane evaluates the most promising element of its trip instead of all eight.
+// trips where some block of the wavefront passes.  The bound lives in LDS: a wavefront's records prune the other seven's elements.
+// It begins at what the row's largest element reaches with the worst word (least_seen_bits), so that elements more than 28 bits
+// below the maximum's probability are never evaluated, whether or not their slice has a candidate; the first wavefronts of a slice
+// to find one evaluate the most promising element of each lane's trip before the others.
 // What is left is the Philox block, 18 multiplies (about 1.5 times a plain instruction each) and 18 exclusive ors per four elements:
-// 72 of the 114 vector instructions of a trip of two blocks a lane, the logits of the next trip in flight.  Bound by the vector ALU.
+// 72 of the 116 vector instructions of a trip of two blocks a lane, the logits of the next trip in flight.  Bound by the vector ALU.
 // 2048 x 152064 bf16 at T = 0.8, the call with its statistics pass: 313 -> 274 us against every element tested on its own
-// (175 instructions a trip, a bound for each wavefront; elements evaluated in full: 388).
+// (175 instructions a trip, a bound for each wavefront; elements evaluated in full: 388).  512 rows with one token 14 above the
+// others: T = 0.2 147, T = 0.05 143 (rows of ordinary entropy 132); without the bound to begin with 165 and 377, with one for each
+// wavefront 210 and 268; in fp16 161 and 160 (400 and 400; 281 and 280).
 // QUAD: the slice starts and ends on multiples of four elements and the rows are aligned for it, so the four logits
 // of a Philox block are one load (8 bytes of a 16-bit row, 16 of an fp32 row) and need no bounds.
 template <int DT, bool QUAD>
@@ -470,9 +474,7 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
     const void* __restrict__ logits, VerifyParams vp, const Part1* __restrict__ part1, Part3* __restrict__ part3) {
   __shared__ float red_f[kRowThreads / kWave];
   __shared__ int red_i[kRowThreads / kWave];
-  __shared__ uint32_t bound;            // seen_bits_of the best key any wavefront has published; 0: none yet
-  if (threadIdx.x == 0) bound = 0;
-  __syncthreads();
+  __shared__ uint32_t bound;            // seen_bits_of the best key any wavefront has published; at first `least`
   const int64_t row = blockIdx.y;
   const int c = blockIdx.x;
   const RowStat rs = combine_row<DT>(part1 + row * vp.splits, vp);
@@ -491,6 +493,9 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
   const float slope = in_range ? inv_t * (1.0f - round_rel) * kLog2e * 0x1p23f : 0.f;
   const float level = !in_range ? INFINITY : (127.0f + (2.02f * round_rel * fmaxf(rs.m, 0.f) + round_abs - rs.m) * kLog2e +
                        log2f((1.0f / rs.S) * (1.0f + 4.0f * RoundBound<DT>::rel + 1e-4f)) + 1e-3f + 1e-6f * fabsf(rs.m)) * 0x1p23f;
+  const uint32_t least = in_range ? least_seen_bits(rs.pmax) : 0u;
+  if (threadIdx.x == 0) bound = least;
+  __syncthreads();
   constexpr bool kAbs = RoundBound<DT>::abs > 0.f;      // fp16: a probability may round up to the smallest subnormal
   constexpr float kFloor = (127.0f + (kAbs ? -24.0f : 0.f)) * 0x1p23f;   // the level of p = abs
   float best = -1.f;
@@ -575,25 +580,7 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
     for (int b = 0; b < U; ++b)
       philox4x32_10_not((uint32_t)(c0 / 4 + g + b * kRowThreads), (uint32_t)row, vp.offset[0], vp.offset[1], vp.key[0], vp.key[1], w[b]);
     seen_bits = __builtin_amdgcn_readfirstlane(seen_bits);
-    if (seen_bits == 0) {
-      // nobody has a bound yet: each lane evaluates its most promising element, which only sets the bound
-      rare();
-      float promise = -INFINITY;
-      int at = 0;
-#pragma unroll
-      for (int i = 0; i < U * 4; ++i) {
-        const float s = fmaf(xs[i / 4][i % 4], slope, -below(w[i / 4][i % 4]));
-        if (s > promise && element(g, i) < (uint32_t)n) { promise = s; at = i; }
-      }
-      float x;
-      uint32_t word;
-      pick(at, x, word);
-      const float key = key_of(x, word);
-      publish(element(g, at) < (uint32_t)n && key > 0.f ? key : 0.f);
-      seen_bits = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-    }
-    const float seen = seen_level(seen_bits);
-    const float from = seen_bits ? level - seen : INFINITY, floor_from = seen_bits ? kFloor - seen : INFINITY;
+    float seen = seen_level(seen_bits), from = level - seen, floor_from = kFloor - seen;
     uint64_t vote = 0;
 #pragma unroll
     for (int b = 0; b < U; ++b) {
@@ -605,6 +592,24 @@ __global__ __launch_bounds__(kRowThreads) void row_sample_kernel(
     }
     if (vote) {                                        // wavefront-uniform
       rare();
+      if (seen_bits == least) {
+        // nobody has published a key: each lane evaluates its most promising element, which only raises the bound
+        float promise = -INFINITY;
+        int at = 0;
+#pragma unroll
+        for (int i = 0; i < U * 4; ++i) {
+          const float s = fmaf(xs[i / 4][i % 4], slope, -below(w[i / 4][i % 4]));
+          if (s > promise && element(g, i) < (uint32_t)n) { promise = s; at = i; }
+        }
+        float x;
+        uint32_t word;
+        pick(at, x, word);
+        const float key = key_of(x, word);
+        publish(element(g, at) < (uint32_t)n && key > 0.f ? key : 0.f);
+        seen = seen_level(__builtin_amdgcn_readfirstlane(__hip_atomic_load(&bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)));
+        from = level - seen;
+        floor_from = kFloor - seen;
+      }
       uint32_t cand = 0;
 #pragma unroll
       for (int i = 0; i < U * 4; ++i)

@@ -118,18 +118,20 @@ def tiled_head(rows: int, vocab: int, hidden: int) -> bool:
     take 0.60 to 1.01 of the GEMM's time up to 320 rows (152064 x 3584, 289 rows: 332 against 414 us) and 0.87 to 0.98 up to 384 where
     a row has 2560 elements (1024: 1.08); heads of 128000 to 130047 rows of 3072 elements and more 0.73 to 0.95 (2048: 1.06).  At others
     the GEMM is level or ahead at some row count: 65536 x 2048 1.13 to 1.18, 50304 x 4096 1.06 to 1.11, 32000 x 5120 1.11 to 1.27, 131072 x
-    4096 1.10 to 1.19, 262144 x 1152 1.03 to 1.21.  With 65 to 128 rows (nine row counts, bf16 and fp16) heads of 128000 to 130047 rows of
-    4096, 5120 and 8192 elements take 0.75 to 0.90 of its time (128000 x 4096, 96 rows: 189 against 244 us) and those of 147456 to 158719
-    rows of 4096 elements 0.81 to 0.98 (152064, 65 rows: 243 against 300 us); others are level or behind at some row count (147456 x 5120
-    1.11), and with 129 to 192 rows the two are level."""
+    4096 1.10 to 1.19, 262144 x 1152 1.03 to 1.21.  With 65 to 128 rows the length of a row decides: 4096 elements are 8 KB, at which the GEMM
+    reads no head faster than 4.9 TB/s (5.6 with 4608 elements) and the tiled kernel up to 5.9.  29 heads of 96000 such rows and more, nine
+    row counts, bf16 and fp16: 0.66 to 1.00 of its time (128000, 96 rows: 187 against 238 us; 152064, 65 rows: 0.92); at 81920 and 90112
+    of them 0.96 to 1.05.  Heads of longer rows (4608, 5120, 8192) take 0.65 to 1.22 with neighbouring vocabularies on both sides of 1, shorter
+    ones 0.58 to 1.15, and all of them 0.78 to 1.25 with 129 to 192 rows."""
     if not (64 < rows <= 384 and vocab % 32 == 0 and hidden % 64 == 0 and (1 << 28) <= 2 * vocab * hidden < (1 << 31)):
         return False
-    large, medium = 147456 <= vocab < 158720, 128000 <= vocab < 130048
     if rows <= 128:
-        return large and 4096 <= hidden < 5120 or medium and hidden >= 4096
+        return hidden == 4096 and vocab >= 96000
     if rows <= 192:
         return False
-    return large and (rows <= 320 or hidden >= 2560) or medium and hidden >= 3072
+    if 147456 <= vocab < 158720:
+        return rows <= 320 or hidden >= 2560
+    return 128000 <= vocab < 130048 and hidden >= 3072
 
 
 class Decoder:

@@ -31,9 +31,9 @@ def test_every_chunk_once_and_long_ones_first(hq, hkv):
                 assert given == [(w, c) for w in reversed(range(windows)) for c in range(-(-ends[-1] // keys))]
                 continue
             falling += 1
-            blocks = [min(keys, ends[w] - c * keys + 63) // 64 for w, c in given if (w, c) in needed]
-            # the last window may have fewer than 64 rows and with them a block less than its place says
-            assert all(a >= b - 1 for a, b in zip(blocks, blocks[1:])), (rows, prefix, blocks)
+            # the last window as if it had 64 rows: with fewer it may have a block less, but keeps its place
+            blocks = [-(-min(keys, prefix + 64 * (w + 1) - c * keys) // 64) for w, c in given if (w, c) in needed]
+            assert all(a >= b for a, b in zip(blocks, blocks[1:])), (rows, prefix, blocks)
             assert len(order) <= len(needed) + min(windows, keys // 64) + windows // (keys // 64) + 1
     assert falling >= 20
 

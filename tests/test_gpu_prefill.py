@@ -59,15 +59,17 @@ def test_prefill_matches_float32(n, start, dtype, hq, hkv):
     assert torch.equal(rows[..., :start, :], past[..., :start, :]) and torch.equal(rows[..., start + n:, :], past[..., start + n:, :])
 
 
-# more workgroups than compute units and windows of very different length: they start in falling order
-@pytest.mark.parametrize("n,start", [(700, 0), (705, 63), (701, 350)])
+# more workgroups than compute units and windows of very different length: they start in falling order.  Two chunks at the longest
+# windows, and three and more, of which the shorter windows have fewer: every form of the merge over a stride that no window fills
+@pytest.mark.parametrize("n,start,hq,hkv,chunks", [(700, 0, 16, 16, 2), (705, 63, 16, 16, 2), (701, 350, 16, 16, 2), (600, 0, 28, 4, 5),
+                                                   (1000, 63, 28, 4, 3), (1000, 250, 28, 4, 3), (1100, 1, 32, 8, 3), (1000, 333, 7, 1, 11)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_windows_in_falling_order(n, start, dtype):
+def test_windows_in_falling_order(n, start, hq, hkv, chunks, dtype):
     order = L.lib().subspec_prefill_attention_order
-    entries = (ctypes.c_int32 * 300)()
-    assert 3 * order(16, 16, n, start, entries, 100) <= 300
+    entries = (ctypes.c_int32 * 900)()
+    assert order(hq, hkv, n, start, entries, 300) <= 300 and -(-(start + n) // entries[2]) == chunks
     assert entries[0] == entries[3] + 1 and entries[1] == entries[4] == 0       # the longest two windows' first chunks
-    test_prefill_matches_float32(n, start, dtype, 16, 16)
+    test_prefill_matches_float32(n, start, dtype, hq, hkv)
 
 
 @pytest.mark.parametrize("n,start", [(20, 0), (70, 0), (300, 0), (130, 200)])

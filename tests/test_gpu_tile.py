@@ -113,14 +113,19 @@ def _plan(M, N, K, gate_up):
     return tuple(plan)
 
 
+def _tail(M, N, K):
+    """(tile shape of a gate|up projection's last columns, row tiles, column tiles, first column); no such columns: (-1, 0, 0, 0)"""
+    tail = (ctypes.c_int32 * 4)()
+    L.check(L.lib().subspec_dense_tile_tail(M, N, K, tail), "subspec_dense_tile_tail")
+    return tuple(tail)
+
+
 # M, N, K; shape of the last columns, its row and column tiles (the last of them partial), its first column
 @pytest.mark.parametrize("M,N,K,tail", [
     (129, 164800, 512, (2, 1, 211, 65536)), (257, 45312, 640, (4, 3, 79, 16384)), (257, 46496, 1024, (5, 2, 108, 16384))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_two_shapes_in_one_launch(M, N, K, tail, dtype):
-    got = (ctypes.c_int32 * 4)()
-    L.check(L.lib().subspec_dense_tile_tail(M, N, K, got), "subspec_dense_tile_tail")
-    assert tuple(got) == tail
+    assert _tail(M, N, K) == tail
     test_gate_up_silu(M, N, K, dtype)
 
 
@@ -149,20 +154,22 @@ def test_every_shape_of_a_linear_layer(M, N, K, shape, row_tiles, ranges, dtype)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_every_shape_of_gate_up(M, N, K, shape, row_tiles, dtype):
     plan = _plan(M, N, K, 1)
-    assert (plan[0], plan[1], plan[3]) == (shape, row_tiles, 1)
+    assert (plan[0], plan[1], plan[3]) == (shape, row_tiles, 1) and _tail(M, N, K)[0] == -1
     test_gate_up_silu(M, N, K, dtype)
 
 
-# shapes of q|k|v, o, gate|up, down and the K ranges of down, at the widths of a 7B layer and of a wider one
-@pytest.mark.parametrize("rows,widths,shapes,ranges", [(2000, (3584, 28, 4, 18944), (2, 5, 0, 0), 2), (1000, (3584, 28, 4, 18944), (4, 7, 2, 0), 4),
-                                                       (1930, (4096, 32, 8, 14336), (0, 5, 0, 5), 1), (1590, (4096, 32, 8, 14336), (1, 5, 2, 0), 2)])
-def test_shapes_of_long_prompts(rows, widths, shapes, ranges):
+# shapes of q|k|v, o, gate|up (its best alone, which is launched where no last columns follow), down; the K ranges of down; gate|up's last
+# columns (behind the largest shape): at the widths of a 7B layer and of a wider one
+@pytest.mark.parametrize("rows,widths,shapes,ranges,tail", [
+    (2000, (3584, 28, 4, 18944), (2, 5, 0, 0), 2, (2, 8, 32, 16384)), (1000, (3584, 28, 4, 18944), (4, 7, 2, 0), 4, (4, 8, 32, 16384)),
+    (1930, (4096, 32, 8, 14336), (0, 5, 0, 5), 1, (5, 8, 32, 12288)), (1590, (4096, 32, 8, 14336), (1, 5, 2, 0), 2, (-1, 0, 0, 0))])
+def test_shapes_of_long_prompts(rows, widths, shapes, ranges, tail):
     """One whole layer against float32, the module-by-module path of the same dtype as the yardstick: both round at the same
     points, so neither may be twice as far off as the other, in the 2-norm and in any one element."""
     hidden, hq, hkv, mlp = widths
     sizes = [((hq + 2 * hkv) * 128, hidden, 0), (hidden, hq * 128, 0), (2 * mlp, hidden, 1), (hidden, mlp, 0)]
     plans = [_plan(rows, *s) for s in sizes]
-    assert tuple(p[0] for p in plans) == shapes and plans[3][3] == ranges
+    assert tuple(p[0] for p in plans) == shapes and plans[3][3] == ranges and _tail(rows, 2 * mlp, hidden) == tail
     cfg = model.DecoderConfig(num_hidden_layers=1, hidden_size=hidden, num_attention_heads=hq, num_key_value_heads=hkv, head_dim=128,
                           intermediate_size=mlp, vocab_size=512)
     w = model.init_weights(cfg, 1, DEV, torch.bfloat16)

@@ -68,7 +68,7 @@ typedef float v2f_t __attribute__((ext_vector_type(2)));
 // cached rows all, tree rows by the row's bitset (`word`, `next`: its words from the block's first tree row on), none past the last.
 // One mask per row and block and two instructions per score; deciding per score, with 64-bit positions, took ten to fifteen of them and
 // made a masked block two to three times as long as a plain one.  One sequence, bf16, both launches: 289 rows of 28 : 4 heads at 2337
-// keys 36.0 -> 32.8 us, at 589 29.5 -> 21.9, 500 rows at 2548 48.9 -> 37.4; a draft level, all of it 1811.8 -> 1804.7.
+// keys 36.0 -> 32.8 us, at 589 29.5 -> 21.9, 500 rows at 2548 48.9 -> 37.4; a whole draft level, one masked block a launch: level.
 __device__ __forceinline__ uint64_t block_bits(int64_t kb, int64_t prefix, int64_t kv_len, uint64_t word, uint64_t next) {
   const int off = (int)(kb - prefix);
   uint64_t m;
@@ -1640,9 +1640,9 @@ static CausalPlan causal_plan(int64_t hq, int64_t hkv, int64_t n_rows, int64_t p
   pl.chunk_keys = (last + pl.chunks - 1) / pl.chunks * kKeyBlock;
   pl.chunks = pl.most_chunks = (int)((last * kKeyBlock + pl.chunk_keys - 1) / pl.chunk_keys);
   // In falling order (causal_order) a window's last chunk may be short: where there are three and more, chunks of the share and a tenth
-  // instead of equal ones.  A layer of the three widths that causal_order names: 900 rows after 100 5.8 to 8.9 us less, 1000 4.3 to 7.1,
-  // 1000 after 250 0.5 to 3.0, 1200 after 400 6.2 to 10.8, 1500 3.3 to 5.3; two chunks (1800 after 200 and 2048 rows, 8 KV heads) would
-  // take up to 5.9 us more.
+  // instead of equal ones.  Attention with its merge, bf16, 28 : 4, 16 : 8 and 32 : 8 heads: 900 rows after 100 39.0 -> 32.3, 29.8 -> 24.4,
+  // 40.8 -> 34.0 us; 1000 4.5 to 6.7 us less, 1200 after 400 5.0 to 7.9, 1500 3.0 to 4.7; least at 1000 after 250, 0.9 to 1.4 of 28 to 39
+  // (a whole stack of the narrow width is level there).  Two chunks (1800 after 200 and 2048 rows, 8 KV heads) would take up to 5.9 us more.
   const int64_t per = (11 * share + 5) / 10, chunks = (last + per - 1) / per;
   if (pl.chunks > 2 && 2 * prefix <= n_rows && pl.windows * chunks * hkv * pl.pairs > 256) {
     pl.chunk_keys = per * kKeyBlock;

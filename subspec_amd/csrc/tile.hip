@@ -26,7 +26,7 @@
 //   waits for them 81 to 88): requests return in order, and those that wait for HBM hold back the activations behind them.  Neither
 //   the order of the chunks, nor 256-byte requests, nor weights laid out tile by tile change that.
 // 2048 rows: 405 to 435 us = 1.28 to 1.37 PFLOP/s with the activation included (library GEMM alone: 520 us; an 8192^3 product
-// reaches 1.38 PFLOP/s on this card), 289 rows: 84 us (dense_wide_kernel: 106), 128 rows: 57 us = 4.8 TB/s of weights.
+// reaches 1.38 PFLOP/s on this card), 289 rows: 84 to 86 us (dense_wide_kernel: 106), 128 rows: 57 us = 4.8 TB/s of weights.
 #include "dma.h"
 #include <algorithm>
 #include <type_traits>

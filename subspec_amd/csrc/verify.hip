@@ -463,7 +463,7 @@ template <> struct RoundBound<SUBSPEC_BF16> { static constexpr float rel = 0x1p-
 // to find one evaluate the most promising element of each lane's trip before the others.
 // What is left is the Philox block, 18 multiplies (about 1.5 times a plain instruction each) and 18 exclusive ors per four elements:
 // 72 of the 116 vector instructions of a trip of two blocks a lane, the logits of the next trip in flight.  Bound by the vector ALU.
-// 2048 x 152064 bf16 at T = 0.8, the call with its statistics pass: 313 -> 274 us against every element tested on its own
+// 2048 x 152064 bf16 at T = 0.8, the call with its statistics pass: 304 -> 263 us against every element tested on its own
 // (175 instructions a trip, a bound for each wavefront; elements evaluated in full: 388).  512 rows with one token 14 above the
 // others: T = 0.2 147, T = 0.05 143 (rows of ordinary entropy 132); without the bound to begin with 165 and 377, with one for each
 // wavefront 210 and 268; in fp16 161 and 160 (400 and 400; 281 and 280).
